@@ -125,7 +125,7 @@ void free_graph_state(dmm_ctx* ctx) {
   void* bufs[] = {ctx->d_out_off, ctx->d_out_nbr, ctx->d_parent, ctx->d_depth, ctx->d_queue,
                   ctx->d_qoff,    ctx->d_bm[0],   ctx->d_bm[1],  ctx->d_bm[2],
                   ctx->d_score,   ctx->d_contrib[0], ctx->d_contrib[1], ctx->d_score64,
-                  ctx->d_contrib64[0], ctx->d_contrib64[1], ctx->d_err_part, ctx->d_heavy,
+                  ctx->d_contrib64[0], ctx->d_contrib64[1], ctx->d_err_part, ctx->d_heavy, ctx->d_sitems, ctx->d_sstart,
                   ctx->d_gcontrib, ctx->d_seen, ctx->d_levels, ctx->d_bact, ctx->d_baoff,
                   ctx->d_bdepth, ctx->d_items, ctx->d_supers, ctx->d_partial, ctx->d_perm, ctx->d_inv,
                   ctx->d_parent_out, ctx->d_depth_out, ctx->d_score_out, ctx->d_score64_out,
@@ -155,6 +155,8 @@ void free_graph_state(dmm_ctx* ctx) {
   ctx->d_score = ctx->d_contrib[0] = ctx->d_contrib[1] = ctx->d_gcontrib = nullptr;
   ctx->d_score64 = ctx->d_contrib64[0] = ctx->d_contrib64[1] = ctx->d_err_part = nullptr;
   ctx->d_heavy = nullptr;
+  ctx->d_sitems = nullptr;
+  ctx->d_sstart = nullptr;
   ctx->d_items = ctx->d_supers = ctx->d_partial = nullptr;
   ctx->n_items = ctx->n_super = ctx->n_slots = 0;
   ctx->d_seen = ctx->d_levels = nullptr;
@@ -293,7 +295,7 @@ int ensure_pr_state(dmm_ctx* ctx, int mode) {
   }
   if (!ctx->d_err_part) {
     const int64_t parts =
-        std::max<int64_t>(std::max<int64_t>(dmm::pr_light_blocks(ctx) + dmm::pr_heavy_blocks(ctx),
+        std::max<int64_t>(std::max<int64_t>(dmm::pr_serial_blocks(ctx),
                                             dmm::pr_fused_blocks(ctx)),
                           dmm::pr_row_blocks(ctx)) +
         dmm::pr_super_blocks(ctx);
@@ -706,9 +708,30 @@ int dmm_graph_upload(dmm_ctx* ctx, int64_t num_nodes, int64_t vbegin, int64_t ve
       ctx->pr_zero_begin = rows;
     }
   }
+  // The serial mode takes them by length class (powers of two, longest
+  // first, row order inside a class).
+  std::vector<int32_t> by_class(heavy.size());
+  {
+    auto cls = [&](int32_t r) { return __builtin_clzll(static_cast<unsigned long long>(ioff[r + 1] - ioff[r])); };
+    int64_t at[65] = {};
+    for (int32_t r : heavy) at[cls(r) + 1]++;
+    for (int c = 0; c < 64; c++) at[c + 1] += at[c];
+    for (int32_t r : heavy) by_class[at[cls(r)]++] = r;
+  }
   if ((rc = A((void**)&ctx->d_heavy, sizeof(int32_t) * std::max<size_t>(1, heavy.size()), "heavy list"))) return rc;
   if (!heavy.empty())
-    DMM_HIP_CHECK(ctx, hipMemcpy(ctx->d_heavy, heavy.data(), sizeof(int32_t) * heavy.size(), hipMemcpyHostToDevice));
+    DMM_HIP_CHECK(ctx, hipMemcpy(ctx->d_heavy, by_class.data(), sizeof(int32_t) * heavy.size(), hipMemcpyHostToDevice));
+  std::vector<dmm::SerialItem> sitems;
+  std::vector<int32_t> sstart;
+  dmm::serial_plan(ctx->pr_light_begin, ctx->pr_zero_begin, ioff, by_class, ctx->heavy_threshold,
+                   dmm::pr_serial_blocks(ctx), &sitems, &sstart);
+  if ((rc = A(&ctx->d_sitems, sizeof(dmm::SerialItem) * std::max<size_t>(1, sitems.size()), "serial items")) ||
+      (rc = A((void**)&ctx->d_sstart, sizeof(int32_t) * sstart.size(), "serial items")))
+    return rc;
+  if (!sitems.empty())
+    DMM_HIP_CHECK(ctx, hipMemcpy(ctx->d_sitems, sitems.data(), sizeof(dmm::SerialItem) * sitems.size(),
+                                 hipMemcpyHostToDevice));
+  DMM_HIP_CHECK(ctx, hipMemcpy(ctx->d_sstart, sstart.data(), sizeof(int32_t) * sstart.size(), hipMemcpyHostToDevice));
   // Work items of the compensated / FP64 modes: heavy rows whole, rows with
   // more than kPrSplit in-edges cut into kPrSegment-edge segments.
   std::vector<dmm::PrItem> items;

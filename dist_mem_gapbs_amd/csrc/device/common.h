@@ -236,8 +236,10 @@ struct dmm_ctx {
   int64_t err_part_cap = 0;
   dmm::PrCtrl* d_prctrl = nullptr;
   dmm::PrCtrl* h_prctrl = nullptr;
-  int32_t* d_heavy = nullptr;    // vertices with in-degree >= heavy threshold
+  int32_t* d_heavy = nullptr;    // vertices with in-degree >= heavy threshold, longest class first
   int64_t n_heavy = 0;
+  void* d_sitems = nullptr;      // serial mode: work items by workgroup
+  int32_t* d_sstart = nullptr;   // ... first item of each workgroup (+ end)
   void* d_items = nullptr;       // PrItem list (compensated / FP64 modes)
   int64_t n_items = 0;
   void* d_supers = nullptr;      // PrSuper list

@@ -26,6 +26,29 @@ struct PrSuper {
 constexpr int64_t kPrSplit = 2048;    // rows with more in-edges are split
 constexpr int64_t kPrSegment = 2048;  // edges per segment
 
+// Serial mode: work items (dealt to workgroups at upload).  A bundle of 16
+// rows of 1023 edges is the longest item of a small graph when rows go to
+// wavefronts from 1024 on: a whole Kronecker-14 rank takes 305 us with 512
+// and 372 us with 1024 (Kronecker-21 2.42 and 2.35 ms; 256: no change).  A
+// wavefront gathers some 0.1 G/s beside others, so the longest rows need a
+// workgroup: Kronecker-21 2.42 ms from 32768 (or 16384) on, 2.72 from 131072.
+constexpr int64_t kSerialWaveRow = 512;     // rows from here on: a wavefront each
+constexpr int64_t kSerialBlockRow = 32768;  // rows from here on: a workgroup each
+constexpr int kHeavyBundle = 16;            // shorter heavy rows: this many per wavefront
+constexpr int kLightBundle = 64;            // rows below the heavy threshold
+enum : int32_t {
+  kSerialBlock = 0,  // row `first`, by the workgroup
+  kSerialWave = 1,   // row `first`, by a wavefront
+  kSerialHeavy = 2,  // heavy-list entries [first, first + kHeavyBundle)
+  kSerialLight = 3,  // the light ones of rows [first, first + kLightBundle)
+};
+struct SerialItem {
+  int32_t first;
+  int32_t kind;
+};
+void serial_plan(int64_t light_begin, int64_t zero_begin, const int64_t* off, const std::vector<int32_t>& by_class,
+                 int64_t heavy_threshold, int blocks, std::vector<SerialItem>* items, std::vector<int32_t>* start);
+
 // Window-tiled compensated PageRank (degree-ordered whole graphs).
 // Sources are cut into windows of `pr_window` vertices (a tuning value:
 // 16384 or 32768 contributions, 64 or 128 KB of LDS).  Every in-edge sits
@@ -122,7 +145,7 @@ int build_blocks_host(int64_t n, int64_t n_gather, const int64_t* off, const int
 int pr_blocks_build(dmm_ctx* ctx);
 
 int pr_light_blocks(dmm_ctx* ctx);
-int pr_heavy_blocks(dmm_ctx* ctx);
+int pr_serial_blocks(dmm_ctx* ctx);  // workgroups of a serial-mode iteration
 int pr_super_blocks(dmm_ctx* ctx);
 int pr_fused_blocks(dmm_ctx* ctx);  // persistent KAHAN / FP64 kernel
 int pr_row_blocks(dmm_ctx* ctx);    // row kernel of the tiled compensated mode

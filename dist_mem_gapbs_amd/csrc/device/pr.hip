@@ -12,8 +12,8 @@
 //
 // Three arithmetic modes:
 //   FP32_SERIAL  the reference's arithmetic exactly: FP32 sums in ascending
-//                in-neighbour order (thread per vertex; one wave per heavy
-//                vertex folding 64 gathered values in lane order).
+//                in-neighbour order (thread per light row, lane per bundled
+//                row, exact composition of the additions in long rows).
 //   FP32_KAHAN   FP32 storage and gathers, each sum compensated (Knuth's
 //                TwoSum error-free transformation, TAOCP Vol. 2 4.2.2;
 //                partial (sum, error) pairs merged with TwoSum as in
@@ -53,17 +53,20 @@ struct PrArgs {
   const int64_t* in_off;          // local rows
   const int32_t* in_nbr;          // global IDs
   const int64_t* out_off;         // local rows (out-degree for contrib)
-  const int32_t* heavy;           // local rows with in-degree >= kHeavy
+  const int32_t* heavy;           // local rows with in-degree >= heavy_threshold, longest class first
   const PrItem* items;            // heavy rows / segments of split rows
   const PrSuper* supers;          // split rows and their segment slots
   double2* partial;               // per-segment partial sums
   int64_t nloc, n_heavy, n_items, n_super;
+  const SerialItem* sitems;       // serial mode: each workgroup's items
+  const int32_t* sstart;          // ... first item of each workgroup (+ end)
   int64_t n_gather;               // entries of the gathered contribution vector
   int64_t light_begin, light_end; // light-row range (heavy rows inside are skipped)
   int64_t zero_begin;             // rows [zero_begin, nloc) have no in-edges
   int heavy_threshold;
   double* err_part;               // [light | heavy-or-items | super] blocks
-  int light_blocks, heavy_blocks, super_blocks;
+  int serial_hub;                     // contributions [0, serial_hub) go to LDS (serial mode)
+  int super_blocks;
   int main_blocks;                // error partials written before the combine
   PrCtrl* ctrl;
   double* err_trace;              // per-iteration error
@@ -129,63 +132,438 @@ __device__ __forceinline__ double finish_f64(const PrArgs& a, int64_t lu, double
   return fabs(nw - old_score);
 }
 
-// ---- FP32_SERIAL ----------------------------------------------------------
-
-__global__ __launch_bounds__(kThreads) void k_serial_light(PrArgs a, const float* __restrict__ cin,
-                                                           float* __restrict__ cout,
-                                                           float* __restrict__ score) {
-  __shared__ double red[kThreads / 64];
-  if (a.ctrl->pad) return;  // converged
-  double err = 0;
-  const int64_t gtid = int64_t(blockIdx.x) * kThreads + threadIdx.x;
-  const int64_t gsize = int64_t(gridDim.x) * kThreads;
-  for (int64_t u = gtid; u < a.nloc; u += gsize) {
-    const int64_t s = a.in_off[u], e = a.in_off[u + 1];
-    if (e - s >= a.heavy_threshold) continue;
-    float incoming_total = 0;
-    // In-neighbour order, as src/pr.cc:57-59; the loads run kLightUnroll
-    // ahead of the adds, which keep their order.
-    int64_t k = s;
-    for (; k + kLightUnroll <= e; k += kLightUnroll) {
-      int32_t v[kLightUnroll];
-      float x[kLightUnroll];
-#pragma unroll
-      for (int j = 0; j < kLightUnroll; j++) v[j] = a.in_nbr[k + j];
-#pragma unroll
-      for (int j = 0; j < kLightUnroll; j++) x[j] = cin[v[j]];
-#pragma unroll
-      for (int j = 0; j < kLightUnroll; j++) incoming_total += x[j];
-    }
-    for (; k < e; k++) incoming_total += cin[a.in_nbr[k]];
-    err += finish_f32(a, u, incoming_total, score, cout);
-  }
-  double t = block_err_sum(err, red);
-  if (threadIdx.x == 0) a.err_part[blockIdx.x] = t;
+// Inclusive prefix sum over the 64 lanes from DPP lane moves (row_shr
+// 1/2/4/8 inside 16-lane rows, row_bcast 15 and 31 across): no LDS traffic.
+__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
+  v += __builtin_amdgcn_update_dpp(0u, v, 0x111, 0xf, 0xf, true);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0u, v, 0x112, 0xf, 0xf, true);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0u, v, 0x114, 0xf, 0xf, true);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0u, v, 0x118, 0xf, 0xf, true);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0u, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0u, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+  return v;
 }
 
-__global__ __launch_bounds__(kThreads) void k_serial_heavy(PrArgs a, const float* __restrict__ cin,
-                                                           float* __restrict__ cout,
-                                                           float* __restrict__ score) {
-  __shared__ double red[kThreads / 64];
-  if (a.ctrl->pad) return;
-  const int lane = lane_id();
-  const int64_t wave = (int64_t(blockIdx.x) * kThreads + threadIdx.x) >> 6;
-  const int64_t nwaves = (int64_t(gridDim.x) * kThreads) >> 6;
-  double err = 0;
-  for (int64_t h = wave; h < a.n_heavy; h += nwaves) {
-    const int64_t u = a.heavy[h];
-    const int64_t s = a.in_off[u], e = a.in_off[u + 1];
-    float incoming_total = 0;  // wave-uniform running sum, ascending order
-    for (int64_t k = s; k < e; k += 64) {
-      const int64_t kk = k + lane;
-      const float x = kk < e ? cin[a.in_nbr[kk]] : 0.0f;
-      const int cnt = static_cast<int>(min<int64_t>(64, e - k));
-      for (int i = 0; i < cnt; i++) incoming_total += __shfl(x, i, 64);
-    }
-    if (lane == 0) err += finish_f32(a, u, incoming_total, score, cout);
+// Block-wide copy of cnt entries from src into LDS (room for kBytes, a
+// multiple of 16) with all 16-byte loads of a thread issued before its
+// stores (one round trip instead of one per element): whole when cnt fills
+// the room, else the loads past the last whole one repeat it and a tail
+// follows.  A src that is not 16-byte aligned is copied entry by entry.
+template <typename T, int kBytes, int kBlock = kFusedThreads>
+__device__ __forceinline__ void lds_fill(T* dst, const T* __restrict__ src, int cnt) {
+  constexpr int kPer = kBytes / 16 / kBlock;
+  constexpr int kVec = 16 / sizeof(T);
+  static_assert(kBytes % (16 * kBlock) == 0, "fill size");
+  const int n4 = (reinterpret_cast<uintptr_t>(src) & 15) == 0 ? cnt / kVec : 0;
+  if (n4 > 0) {
+    float4 v[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; i++)
+      v[i] = reinterpret_cast<const float4*>(src)[min(static_cast<int>(threadIdx.x) + i * kBlock, n4 - 1)];
+#pragma unroll
+    for (int i = 0; i < kPer; i++)
+      if (static_cast<int>(threadIdx.x) + i * kBlock < n4) reinterpret_cast<float4*>(dst)[threadIdx.x + i * kBlock] = v[i];
   }
-  double t = block_err_sum(err, red);
-  if (threadIdx.x == 0) a.err_part[a.light_blocks + blockIdx.x] = t;
+  for (int j = n4 * kVec + threadIdx.x; j < cnt; j += kBlock) dst[j] = src[j];
+}
+
+template <typename T>
+__device__ __forceinline__ T hub_gather(const T* hub, int hub_n, const T* __restrict__ cin, int32_t u) {
+  T x;
+  if (u < hub_n)
+    x = hub[u];
+  else
+    x = cin[u];
+  return x;
+}
+
+// ---- FP32_SERIAL ----------------------------------------------------------
+//
+// The reference's arithmetic: each row's contributions added one by one in
+// FP32, in in-neighbour order (src/pr.cc:57-59).  The order of the additions
+// is fixed, not who does them; rows are taken by length:
+//   bundles      kLightBundle rows (below heavy_threshold) or kHeavyBundle
+//                rows per wavefront, gathered together and coalesced, one
+//                lane adding each row
+//   long rows    from kSerialWaveRow on by a wavefront, from kSerialBlockRow
+//                on by a workgroup, by exact composition (serial_fold)
+// What bounds it: the gathers beyond the LDS hub, some 200 G/s (a cache line
+// into L1 for each), and per CU about 1/256 of that, so items are dealt to
+// the CUs by their edges (serial_plan).  Kronecker-21, per iteration: 260 us;
+// 2150 us with a wavefront per heavy row adding shuffled values one by one
+// (the longest row, some 10^5 edges, took that long), 340 us with these
+// items strided over small workgroups without the hub, 327 us with the hub
+// and strided.
+//
+// Long rows by composition.  While the running sum S stays inside one binade
+// [2^E, 2^(E+1)), S is an integer multiple of u = 2^(E-23), and adding x >= 0
+// adds the integer rn(x / u), except that an exact half goes to the even
+// neighbour, which depends only on the parity of S / u.  So every run of
+// additions inside a binade is a pair (what it adds to an even S, to an odd
+// S), and pairs compose associatively: lanes build their own kSerialPer
+// elements' pairs and a scan over the wavefront composes them, in order, with
+// exact integers.  The element where S leaves the binade is found from the
+// scan; the lane that holds it adds its elements one by one, and the scan
+// goes on behind that lane with the new binade.  S only grows, so a row of d
+// elements crosses at most about log2(d) + 30 binades.  Negative or non-finite
+// contributions, and sums below 2^-103, are added one lane after another.
+
+constexpr int kSerialThreads = 1024;
+constexpr int kSerialWaves = kSerialThreads / 64;
+constexpr int kSerialHub = 28672;         // contributions in LDS (112 KB, whole 16-byte loads per thread)
+constexpr int kSerialPer = 8;             // edges per lane and step
+constexpr int kHeavyCols = 64 * kSerialPer / kHeavyBundle;  // edges of each row per step of a bundle
+constexpr int kLightCols = 64 * kSerialPer / kLightBundle;
+constexpr int kHeavyPitch = kHeavyCols + 4;  // LDS floats from row to row: no two rows of a read on one bank
+constexpr int kLightPitch = kLightCols + 2;
+constexpr int kStageFloats = kHeavyBundle * kHeavyPitch > kLightBundle * kLightPitch ? kHeavyBundle * kHeavyPitch
+                                                                                     : kLightBundle * kLightPitch;
+constexpr unsigned kBinadeEnd = 1u << 24;
+
+__device__ __forceinline__ float lane_value(float x, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
+}
+
+// Whether composition works from S: positive, normal, both its unit and the
+// reciprocal of the unit normal.
+__device__ __forceinline__ bool composable(float S) {
+  const unsigned eb = __float_as_uint(S) >> 23;  // a set sign bit makes it >= 256
+  return eb >= 24u && eb <= 254u;
+}
+__device__ __forceinline__ unsigned units_of(float S) { return (__float_as_uint(S) & 0x7FFFFFu) | 0x800000u; }
+// The float of `units` (below kBinadeEnd) in S's binade.
+__device__ __forceinline__ float from_units(float S, unsigned units) {
+  return __uint_as_float((__float_as_uint(S) & 0xFF800000u) | (units & 0x7FFFFFu));
+}
+
+__device__ __forceinline__ bool all_plain(const float (&x)[kSerialPer]) {
+  bool ok = true;
+#pragma unroll
+  for (int j = 0; j < kSerialPer; j++) ok = ok && x[j] >= 0.0f && x[j] < __builtin_inff();
+  return __ballot(!ok) == 0ull;
+}
+
+// The lane's pair under S's unit: what its elements add to an even and to an
+// odd multiple, each saturated at kBinadeEnd (past any binade's end).
+__device__ __forceinline__ void lane_pair(float S, const float (&x)[kSerialPer], unsigned& a0, unsigned& a1) {
+  const float scale = __uint_as_float((277u - (__float_as_uint(S) >> 23)) << 23);  // 1 / u
+  a0 = a1 = 0;
+#pragma unroll
+  for (int j = 0; j < kSerialPer; j++) {
+    const float t = fminf(x[j] * scale, 16777216.0f);  // exact below the clamp (or far below one half)
+    const float r = rintf(t);                          // half to even
+    const float d = t - r;
+    const unsigned c0 = static_cast<unsigned>(r);
+    const unsigned c1 = fabsf(d) == 0.5f ? static_cast<unsigned>(t + d) : c0;  // the other neighbour of a half
+    a0 += (a0 & 1u) ? c1 : c0;
+    a1 += (a1 & 1u) ? c0 : c1;
+  }
+  a0 = min(a0, kBinadeEnd);
+  a1 = min(a1, kBinadeEnd);
+}
+
+// Inclusive scan over the lanes of what they add to S (its parity is
+// `odd`).  Without halves (both entries equal in every lane) a plain sum.
+__device__ __forceinline__ unsigned pair_scan(unsigned a0, unsigned a1, unsigned odd) {
+  if (__ballot(a0 != a1) == 0ull) return wave_scan_u32(a0);
+  const int lane = lane_id();
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const unsigned p0 = __shfl_up(a0, d, 64), p1 = __shfl_up(a1, d, 64);
+    if (lane >= d) {
+      const unsigned n0 = p0 + ((p0 & 1u) ? a1 : a0);
+      const unsigned n1 = p1 + ((p1 & 1u) ? a0 : a1);
+      a0 = n0;
+      a1 = n1;
+    }
+  }
+  return odd ? a1 : a0;
+}
+
+// S after adding the wavefront's elements in lane order (lane i holds the
+// elements [i * kSerialPer, (i + 1) * kSerialPer)); S is wave-uniform.
+__device__ __forceinline__ float serial_fold(float S, const float (&x)[kSerialPer], int lane) {
+  const bool plain = all_plain(x);
+  for (int from = 0; from < 64;) {
+    int at = from;  // the lane whose elements are added one by one
+    if (plain && composable(S)) {
+      unsigned a0, a1;
+      lane_pair(S, x, a0, a1);
+      if (lane < from) a0 = a1 = 0;
+      const unsigned si = units_of(S);
+      const unsigned incl = pair_scan(a0, a1, si & 1u);
+      const unsigned long long over = __ballot(si + incl >= kBinadeEnd);
+      if (over == 0ull) return from_units(S, si + __builtin_amdgcn_readlane(incl, 63));
+      at = __builtin_ctzll(over);
+      if (at > from) S = from_units(S, si + __builtin_amdgcn_readlane(incl, at - 1));
+    }
+    float r = S;
+#pragma unroll
+    for (int j = 0; j < kSerialPer; j++) r += x[j];
+    S = lane_value(r, at);
+    from = at + 1;
+  }
+  return S;
+}
+
+// The contributions of the first n vertices, in LDS, and a zero behind the
+// room for them.
+struct SerialHub {
+  const float* lds;
+  int n;
+};
+
+// The contributions of kSerialPer edges on their way.  A wavefront's loads
+// are unconditional (lanes without work read a spare place), so that every
+// path issues the same number: a step's IDs are waited for with the previous
+// step's gathers in flight, and its gathers with the next step's.
+struct SerialStep {
+  int32_t v[kSerialPer];  // sources, -1: no edge
+  float g[kSerialPer];    // what lies beyond the hub
+  __device__ __forceinline__ void load(const SerialHub& hub, const float* __restrict__ cin) {
+#pragma unroll
+    for (int j = 0; j < kSerialPer; j++) g[j] = cin[v[j] >= hub.n ? v[j] : 0];
+  }
+  __device__ __forceinline__ void take(const SerialHub& hub, float (&x)[kSerialPer]) const {
+    float l[kSerialPer];
+#pragma unroll
+    for (int j = 0; j < kSerialPer; j++)
+      l[j] = hub.lds[static_cast<unsigned>(v[j]) < static_cast<unsigned>(hub.n) ? v[j] : kSerialHub];
+    // No edge adds +0, which changes no sum here (they start at +0).
+#pragma unroll
+    for (int j = 0; j < kSerialPer; j++) x[j] = v[j] >= hub.n ? g[j] : l[j];
+  }
+};
+
+// Source IDs of in-edges [k, k + kSerialPer) of a row that ends at e and has
+// at least kSerialPer: past the end the last kSerialPer, of which keep_ids
+// drops the ones below k.
+__device__ __forceinline__ void load_ids(const int32_t* __restrict__ nbr, int64_t k, int64_t e,
+                                         int32_t (&v)[kSerialPer]) {
+  __builtin_memcpy(v, nbr + min(k, e - kSerialPer), sizeof(v));  // rows start at any 4-byte address
+}
+__device__ __forceinline__ void keep_ids(int64_t k, int64_t e, const int32_t (&raw)[kSerialPer], SerialStep& st) {
+  const int drop = static_cast<int>(max<int64_t>(0, min<int64_t>(kSerialPer, k - (e - kSerialPer))));
+#pragma unroll
+  for (int j = 0; j < kSerialPer; j++) st.v[j] = j >= drop ? raw[j] : -1;
+}
+
+// The steps of one row, kLanes lanes wide, handed to f(x) in order.
+template <int kLanes, typename F>
+__device__ __forceinline__ void row_steps(const int32_t* __restrict__ nbr, const SerialHub& hub,
+                                          const float* __restrict__ cin, int64_t s, int64_t e, int lane, F&& f) {
+  constexpr int64_t kStep = int64_t(kLanes) * kSerialPer;
+  int64_t k = s + int64_t(lane) * kSerialPer;
+  int32_t raw[kSerialPer];
+  SerialStep cur, next;
+  load_ids(nbr, k, e, raw);
+  keep_ids(k, e, raw, cur);
+  load_ids(nbr, k + kStep, e, raw);
+  cur.load(hub, cin);
+  for (int64_t at = s; at < e; at += kStep) {
+    k += kStep;
+    keep_ids(k, e, raw, next);
+    load_ids(nbr, k + kStep, e, raw);
+    next.load(hub, cin);
+    float x[kSerialPer];
+    cur.take(hub, x);
+    f(x);
+    cur = next;
+  }
+}
+
+struct SerialLds {
+  float hub[kSerialHub + 4];
+  float stage[kSerialWaves][kStageFloats];
+  unsigned p0[2][kSerialWaves], p1[2][kSerialWaves];
+  float sum[2];
+  double red[kSerialWaves];
+};
+static_assert(sizeof(SerialLds) <= 160 * 1024, "one workgroup per CU");
+
+// A very long row by the workgroup.  Each round every wavefront not yet
+// folded in offers the pair of its elements under the sum's binade; they are
+// taken in wave order until one would leave the binade, which that wavefront
+// then folds itself.
+__device__ __forceinline__ float serial_block_row(const PrArgs& a, const SerialHub& hub,
+                                                  const float* __restrict__ cin, int64_t s, int64_t e, SerialLds& L) {
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float S = 0.0f;
+  int buf = 0;  // the exchange words alternate, so one barrier separates their uses
+  row_steps<kSerialThreads>(a.in_nbr, hub, cin, s, e, threadIdx.x, [&](const float (&x)[kSerialPer]) {
+    const bool plain = all_plain(x);
+    for (int from = 0; from < kSerialWaves;) {
+      const bool can = composable(S);  // the same in every wavefront
+      if (can && wave >= from) {
+        unsigned a0 = kBinadeEnd, a1 = kBinadeEnd;
+        if (plain) {
+          unsigned l0, l1;
+          lane_pair(S, x, l0, l1);
+          if (__ballot(l0 != l1) == 0ull) {
+            a0 = a1 = __builtin_amdgcn_readlane(wave_scan_u32(l0), 63);
+          } else {
+            a0 = __builtin_amdgcn_readlane(pair_scan(l0, l1, 0u), 63);
+            a1 = __builtin_amdgcn_readlane(pair_scan(l0, l1, 1u), 63);
+          }
+        }
+        if (lane == 0) {
+          L.p0[buf][wave] = min(a0, kBinadeEnd);
+          L.p1[buf][wave] = min(a1, kBinadeEnd);
+        }
+      }
+      __syncthreads();
+      if (can) {
+        unsigned si = units_of(S);
+        for (; from < kSerialWaves; from++) {
+          const unsigned add = (si & 1u) ? L.p1[buf][from] : L.p0[buf][from];
+          if (si + add >= kBinadeEnd) break;
+          si += add;
+        }
+        S = from_units(S, si);
+      }
+      if (from < kSerialWaves) {
+        if (wave == from) {
+          const float r = serial_fold(S, x, lane);
+          if (lane == 0) L.sum[buf] = r;
+        }
+        __syncthreads();
+        S = L.sum[buf];
+        from++;
+      }
+      buf ^= 1;
+    }
+  });
+  __syncthreads();  // the exchange words are free for the next row
+  return S;
+}
+
+// kRows rows by one wavefront, lane i adding the row [s, s + len) it holds
+// (len 0: none): the wavefront gathers kCols edges of every row at a time
+// and stages them in LDS.  Returns the lane's sum.
+template <int kRows, int kCols, int kPitch>
+__device__ __forceinline__ float serial_bundle(const int32_t* __restrict__ nbr, const SerialHub& hub,
+                                               const float* __restrict__ cin, int64_t s, int len, int lane,
+                                               float* stage) {
+  static_assert(kRows * kCols == 64 * kSerialPer, "a step's edges");
+  constexpr int kPass = 64 / kCols;  // rows per load
+  const int col = lane % kCols;
+  int64_t base[kSerialPer];
+  int left[kSerialPer];
+#pragma unroll
+  for (int j = 0; j < kSerialPer; j++) {
+    const int r = j * kPass + lane / kCols;
+    base[j] = __shfl(s, r, 64) + col;
+    left[j] = __shfl(len, r, 64) - col;
+  }
+  int longest = len;
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) longest = max(longest, __shfl_xor(longest, d, 64));
+  longest = __builtin_amdgcn_readfirstlane(longest);
+  int32_t raw[kSerialPer];
+  SerialStep cur, next;
+  auto load = [&](int c) {
+#pragma unroll
+    for (int j = 0; j < kSerialPer; j++) raw[j] = nbr[c < left[j] ? base[j] + c : 0];
+  };
+  auto keep = [&](int c, SerialStep& st) {
+#pragma unroll
+    for (int j = 0; j < kSerialPer; j++) st.v[j] = c < left[j] ? raw[j] : -1;
+  };
+  if (longest == 0) return 0.0f;
+  load(0);
+  keep(0, cur);
+  load(kCols);
+  cur.load(hub, cin);
+  float sum = 0.0f;
+  using Quad = float __attribute__((ext_vector_type(kPitch % 4 == 0 ? 4 : 2)));
+  constexpr int kQuad = sizeof(Quad) / 4;
+  const Quad* mine = reinterpret_cast<const Quad*>(stage + (lane % kRows) * kPitch);
+  float* put = stage + (lane / kCols) * kPitch + col;
+  for (int c = 0; c < longest; c += kCols) {
+    keep(c + kCols, next);
+    load(c + 2 * kCols);
+    next.load(hub, cin);
+    float x[kSerialPer];
+    cur.take(hub, x);
+    // LDS operations of one wavefront complete in order: only the compiler's
+    // order needs holding between the writes and the other lanes' reads.
+#pragma unroll
+    for (int j = 0; j < kSerialPer; j++) put[j * kPass * kPitch] = x[j];
+    __asm__ volatile("" ::: "memory");
+#pragma unroll
+    for (int q = 0; q < kCols / kQuad; q++) {
+      const Quad z = mine[q];
+#pragma unroll
+      for (int i = 0; i < kQuad; i++) sum += z[i];
+    }
+    __asm__ volatile("" ::: "memory");
+    cur = next;
+  }
+  return sum;
+}
+
+// One iteration, one workgroup per CU: it fills its hub, takes its very long
+// rows, its wavefronts take the rest of its items in turn, and the rows
+// without in-edges go to all threads.
+__global__ __launch_bounds__(kSerialThreads) void k_serial(PrArgs a, const float* __restrict__ cin,
+                                                           float* __restrict__ cout, float* __restrict__ score) {
+  __shared__ SerialLds L;
+  if (a.ctrl->pad) return;  // converged
+  const SerialHub hub{L.hub, a.serial_hub};
+  if (hub.n > 0) lds_fill<float, kSerialHub * 4, kSerialThreads>(L.hub, cin, hub.n);
+  if (threadIdx.x == 0) L.hub[kSerialHub] = 0.0f;
+  __syncthreads();
+  double err = 0;
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int i = a.sstart[blockIdx.x];
+  const int end = a.sstart[blockIdx.x + 1];
+  for (; i < end && a.sitems[i].kind == kSerialBlock; i++) {
+    const int64_t u = a.sitems[i].first;
+    const float sum = serial_block_row(a, hub, cin, a.in_off[u], a.in_off[u + 1], L);
+    if (threadIdx.x == 0) err += finish_f32(a, u, sum, score, cout);
+  }
+  for (i += wave; i < end; i += kSerialWaves) {
+    const SerialItem it = a.sitems[i];
+    if (it.kind == kSerialWave) {
+      const int64_t s = a.in_off[it.first], e = a.in_off[it.first + 1];
+      float sum = 0.0f;
+      row_steps<64>(a.in_nbr, hub, cin, s, e, lane,
+                    [&](const float (&x)[kSerialPer]) { sum = serial_fold(sum, x, lane); });
+      if (lane == 0) err += finish_f32(a, it.first, sum, score, cout);
+      continue;
+    }
+    // Rows of the heavy list, or neighbouring rows of which the heavy ones
+    // are someone else's.
+    const bool heavy = it.kind == kSerialHeavy;
+    const int64_t at = int64_t(it.first) + lane;
+    int64_t row = -1;
+    if (heavy) {
+      if (lane < kHeavyBundle && at < a.n_heavy) row = a.heavy[at];
+    } else if (at < a.zero_begin) {
+      row = at;
+    }
+    int64_t s = 0;
+    int len = 0;
+    if (row >= 0) {
+      s = a.in_off[row];
+      const int64_t d = a.in_off[row + 1] - s;
+      if (!heavy && d >= a.heavy_threshold)
+        row = -1;
+      else
+        len = static_cast<int>(d);
+    }
+    const float sum =
+        heavy ? serial_bundle<kHeavyBundle, kHeavyCols, kHeavyPitch>(a.in_nbr, hub, cin, s, len, lane, L.stage[wave])
+              : serial_bundle<kLightBundle, kLightCols, kLightPitch>(a.in_nbr, hub, cin, s, len, lane, L.stage[wave]);
+    if (row >= 0) err += finish_f32(a, row, sum, score, cout);
+  }
+  for (int64_t u = a.zero_begin + int64_t(blockIdx.x) * kSerialThreads + threadIdx.x; u < a.nloc;
+       u += int64_t(gridDim.x) * kSerialThreads)
+    err += finish_f32(a, u, 0.0f, score, cout);
+  const double t = block_err_sum<kSerialThreads>(err, L.red);
+  if (threadIdx.x == 0) a.err_part[blockIdx.x] = t;
 }
 
 // ---- FP32_KAHAN -------------------------------------------------------------
@@ -249,36 +627,6 @@ __device__ __forceinline__ double finish_t(const PrArgs& a, int64_t lu, float in
 }
 __device__ __forceinline__ double finish_t(const PrArgs& a, int64_t lu, double in, double* score, double* cout) {
   return finish_f64(a, lu, in, score, cout);
-}
-
-// Block-wide copy of `bytes` (a multiple of 16) from src into LDS with all
-// 16-byte loads of a thread issued before its stores (one round trip
-// instead of one per element); entries at or beyond cnt are not read.
-template <typename T, int kBytes>
-__device__ __forceinline__ void lds_fill(T* dst, const T* __restrict__ src, int cnt) {
-  constexpr int kVec = 16 / sizeof(T);
-  constexpr int kPer = kBytes / 16 / kFusedThreads;
-  static_assert(kBytes % (16 * kFusedThreads) == 0, "fill size");
-  if (cnt * static_cast<int>(sizeof(T)) >= kBytes) {
-    float4 v[kPer];
-#pragma unroll
-    for (int i = 0; i < kPer; i++) v[i] = reinterpret_cast<const float4*>(src)[threadIdx.x + i * kFusedThreads];
-#pragma unroll
-    for (int i = 0; i < kPer; i++) reinterpret_cast<float4*>(dst)[threadIdx.x + i * kFusedThreads] = v[i];
-  } else {
-    for (int j = threadIdx.x; j < cnt; j += kFusedThreads) dst[j] = src[j];
-  }
-  (void)kVec;
-}
-
-template <typename T>
-__device__ __forceinline__ T hub_gather(const T* hub, int hub_n, const T* __restrict__ cin, int32_t u) {
-  T x;
-  if (u < hub_n)
-    x = hub[u];
-  else
-    x = cin[u];
-  return x;
 }
 
 template <typename T>
@@ -385,18 +733,6 @@ __device__ __forceinline__ double seg_scan(double v, int lane, int seg) {
   if (((lane >> 4) & 1) && (lane & ~15) - 1 >= seg) v += t;
   t = dpp_move<0x143, 0xc>(v);  // row_bcast:31 -> rows 2 and 3 get lane 31
   if (lane >= 32 && 31 >= seg) v += t;
-  return v;
-}
-
-// Inclusive prefix sum over the 64 lanes from DPP lane moves (the
-// unsegmented form of seg_scan): no LDS traffic.
-__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
-  v += __builtin_amdgcn_update_dpp(0u, v, 0x111, 0xf, 0xf, true);  // row_shr:1
-  v += __builtin_amdgcn_update_dpp(0u, v, 0x112, 0xf, 0xf, true);  // row_shr:2
-  v += __builtin_amdgcn_update_dpp(0u, v, 0x114, 0xf, 0xf, true);  // row_shr:4
-  v += __builtin_amdgcn_update_dpp(0u, v, 0x118, 0xf, 0xf, true);  // row_shr:8
-  v += __builtin_amdgcn_update_dpp(0u, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
-  v += __builtin_amdgcn_update_dpp(0u, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
   return v;
 }
 
@@ -1124,12 +1460,6 @@ __global__ __launch_bounds__(kThreads) void k_init_f64(PrArgs a, double* score, 
   }
 }
 
-// The serial mode has no combine step: clear the combine blocks' partials.
-__global__ void k_zero_err(PrArgs a) {
-  for (int i = threadIdx.x; i < a.super_blocks; i += blockDim.x)
-    a.err_part[a.main_blocks + i] = 0.0;
-}
-
 __global__ void k_reset_ctrl(PrCtrl* c) {
   c->pad = 0;
   c->ticket = 0;
@@ -1151,10 +1481,13 @@ PrArgs make_args(dmm_ctx* ctx) {
   a.n_super = ctx->n_super;
   a.heavy_threshold = ctx->heavy_threshold;
   a.err_part = ctx->d_err_part;
-  a.light_blocks = pr_light_blocks(ctx);
-  a.heavy_blocks = pr_heavy_blocks(ctx);
+  a.sitems = static_cast<const SerialItem*>(ctx->d_sitems);
+  a.sstart = ctx->d_sstart;
+  // In the degree order the first vertices receive most gathers; in another
+  // order they do only if they are most of the vertices.
+  a.serial_hub = ctx->relabeled || ctx->n <= 2 * kSerialHub ? static_cast<int>(std::min<int64_t>(kSerialHub, ctx->n)) : 0;
   a.super_blocks = pr_super_blocks(ctx);
-  a.main_blocks = a.light_blocks + a.heavy_blocks;
+  a.main_blocks = 0;
   a.n_gather = ctx->n;
   a.light_begin = ctx->pr_light_begin;
   a.light_end = ctx->pr_light_end;
@@ -1177,10 +1510,9 @@ void launch_iteration(dmm_ctx* ctx, PrArgs a, int mode, int it, const void* gcon
   if (mode == DMM_PR_FP32_SERIAL) {
     const float* cin = gcontrib ? static_cast<const float*>(gcontrib) : ctx->d_contrib[it & 1];
     float* cout = contrib_out ? contrib_out : ctx->d_contrib[(it + 1) & 1];
-    a.main_blocks = a.light_blocks + a.heavy_blocks;
-    hipLaunchKernelGGL(k_serial_light, dim3(a.light_blocks), dim3(kThreads), 0, s, a, cin, cout, score_f);
-    hipLaunchKernelGGL(k_serial_heavy, dim3(a.heavy_blocks), dim3(kThreads), 0, s, a, cin, cout, score_f);
-    hipLaunchKernelGGL(k_zero_err, dim3(1), dim3(kThreads), 0, s, a);
+    a.main_blocks = pr_serial_blocks(ctx);
+    a.super_blocks = 0;
+    hipLaunchKernelGGL(k_serial, dim3(a.main_blocks), dim3(kSerialThreads), 0, s, a, cin, cout, score_f);
   } else {
     const int fb = pr_fused_blocks(ctx);
     a.main_blocks = fb;
@@ -1259,11 +1591,58 @@ int pr_light_blocks(dmm_ctx* ctx) {
       1, std::min<int64_t>(int64_t(std::max(1, ctx->cu_count)) * 8, ceil_div(ctx->nloc, kThreads))));
 }
 
-int pr_heavy_blocks(dmm_ctx* ctx) {
-  const int64_t work = std::max(ctx->n_heavy, ctx->n_items);
-  return static_cast<int>(std::max<int64_t>(
-      1, std::min<int64_t>(int64_t(std::max(1, ctx->cu_count)) * 8, ceil_div(work * 64, kThreads))));
+// Deals the rows to the serial kernel's workgroups: longest first, each to
+// the workgroup with the fewest edges so far.  Static, so that every run adds
+// the error terms in the same order.  by_class: the heavy rows, longest
+// power-of-two class first.
+void serial_plan(int64_t light_begin, int64_t zero_begin, const int64_t* off, const std::vector<int32_t>& by_class,
+                 int64_t heavy_threshold, int blocks, std::vector<SerialItem>* items, std::vector<int32_t>* start) {
+  struct Load {
+    int64_t edges;
+    int32_t block;
+    bool operator<(const Load& o) const { return edges != o.edges ? edges > o.edges : block > o.block; }
+  };
+  std::vector<Load> heap;
+  for (int32_t b = 0; b < blocks; b++) heap.push_back({0, b});
+  std::make_heap(heap.begin(), heap.end());
+  struct Dealt {
+    SerialItem it;
+    int32_t block;
+  };
+  std::vector<Dealt> dealt;
+  auto deal = [&](int32_t first, int32_t kind, int64_t edges) {
+    std::pop_heap(heap.begin(), heap.end());
+    heap.back().edges += edges;
+    dealt.push_back({{first, kind}, heap.back().block});
+    std::push_heap(heap.begin(), heap.end());
+  };
+  auto len = [&](int64_t r) { return off[r + 1] - off[r]; };
+  constexpr int64_t kItemCost = 128;  // an item's own steps, in edges
+  size_t h = 0;
+  for (; h < by_class.size() && len(by_class[h]) >= kSerialBlockRow; h++)
+    deal(by_class[h], kSerialBlock, len(by_class[h]));
+  for (; h < by_class.size() && len(by_class[h]) >= kSerialWaveRow; h++)
+    deal(by_class[h], kSerialWave, len(by_class[h]) + kItemCost);
+  for (; h < by_class.size(); h += kHeavyBundle) {
+    int64_t edges = 0;
+    for (size_t i = h; i < std::min(by_class.size(), h + kHeavyBundle); i++) edges += len(by_class[i]);
+    deal(static_cast<int32_t>(h), kSerialHeavy, edges + kItemCost);
+  }
+  for (int64_t r = light_begin; r < zero_begin; r += kLightBundle) {
+    int64_t edges = 0;
+    for (int64_t i = r; i < std::min(zero_begin, r + kLightBundle); i++)
+      if (len(i) < heavy_threshold) edges += len(i);
+    deal(static_cast<int32_t>(r), kSerialLight, edges + kItemCost);
+  }
+  start->assign(blocks + 1, 0);
+  for (const Dealt& d : dealt) (*start)[d.block + 1]++;
+  for (int b = 0; b < blocks; b++) (*start)[b + 1] += (*start)[b];
+  items->resize(dealt.size());
+  std::vector<int32_t> at(start->begin(), start->end() - 1);
+  for (const Dealt& d : dealt) (*items)[at[d.block]++] = d.it;
 }
+
+int pr_serial_blocks(dmm_ctx* ctx) { return std::max(1, ctx->cu_count); }
 
 int pr_fused_blocks(dmm_ctx* ctx) {
   const int64_t lanes = std::max(ctx->nloc * kGroup, ctx->n_items * 64);
@@ -1466,7 +1845,7 @@ int pr_block_iteration_noalloc(dmm_ctx* ctx, const float* d_gcontrib, float* d_s
   unsigned char* base = ctx->scratch;
   if (!base) return set_err(ctx, DMM_ERR_STATE, "the context has no scratch address");
   PrArgs a = make_args(ctx);
-  const int parts = mode == DMM_PR_FP32_SERIAL ? a.light_blocks + a.heavy_blocks + a.super_blocks
+  const int parts = mode == DMM_PR_FP32_SERIAL ? pr_serial_blocks(ctx)
                     : ctx->bp_ready ? pr_bsum_blocks(ctx) + pr_bsplit_blocks(ctx)
                                     : pr_fused_blocks(ctx) + a.super_blocks;
   if (parts > kScratchErrParts)
