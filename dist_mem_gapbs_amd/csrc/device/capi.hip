@@ -104,15 +104,15 @@ void drop_tiles(dmm_ctx* ctx) {
   if (ctx->tiles_ready) drop_graphs(ctx);
   ctx->tiles_ready = false;
   // The PE-block propagation layout.
-  void* bbufs[] = {ctx->d_bp_src, ctx->d_bp_wstart, ctx->d_bp_wlen, ctx->d_bp_wseg, ctx->d_bp_seg_e,
+  void* bbufs[] = {ctx->d_bp_src, ctx->d_bp_wstart, ctx->d_bp_wlen, ctx->d_bp_wseg, ctx->d_bp_wgroup, ctx->d_bp_groups,
                    ctx->d_bp_seg_d, ctx->d_bp_brow, ctx->d_bp_units, ctx->d_bp_splits, ctx->d_bp_val,
-                   ctx->d_bp_part};
+                   ctx->d_bp_part, ctx->d_bp_rows};
   for (void* p : bbufs) dmm::dev_free(p);
   ctx->dev_bytes -= ctx->bp_bytes;
   ctx->bp_bytes = 0;
-  ctx->d_bp_src = ctx->d_bp_wstart = ctx->d_bp_wlen = ctx->d_bp_wseg = ctx->d_bp_seg_e = nullptr;
+  ctx->d_bp_src = ctx->d_bp_wstart = ctx->d_bp_wlen = ctx->d_bp_wseg = ctx->d_bp_wgroup = ctx->d_bp_groups = nullptr;
   ctx->d_bp_seg_d = ctx->d_bp_brow = ctx->d_bp_units = ctx->d_bp_splits = ctx->d_bp_val = nullptr;
-  ctx->d_bp_part = nullptr;
+  ctx->d_bp_part = ctx->d_bp_rows = nullptr;
   ctx->n_bp_windows = ctx->n_bp_units = ctx->n_bp_splits = ctx->n_bp_buckets = 0;
   ctx->bp_ready = false;
 }

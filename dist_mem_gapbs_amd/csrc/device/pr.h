@@ -104,18 +104,50 @@ int pr_tiles_build(dmm_ctx* ctx);
 // anywhere in the whole graph): propagation layout.  Pass 1 copies one
 // window of kBWin contributions into LDS at a time and writes each in-edge's
 // contribution to the edge's place in the bucket-major array; pass 2 sums
-// each bucket's rows exactly, as 128-bit fixed-point integers in LDS.
+// each bucket's rows exactly, as 128-bit fixed-point integers.  Two bucket
+// shapes:
+//   fine    a bucket's contributions fit LDS: pass 2 sorts them there by row
+//           (static places) and sums each row's run in registers
+//   coarse  a bucket's row accumulators fit LDS: pass 2 adds every
+//           contribution with LDS atomics.  Only for blocks with more fine
+//           buckets than a window's segment table holds (some 125 M
+//           in-edges): the atomics run at about 350 G/s, and a block that does
+//           not fill the CUs with buckets of 2^19 edges waits for the largest.
+//           Kronecker-23, block 3 of 8, pass 1 + pass 2: coarse 52 + 281 us,
+//           fine 61 + 75 us.
 constexpr int kBWin = 32768;             // sources per window (128 KB of LDS)
-constexpr int kBRows = 8192;             // rows per bucket (its accumulators fill 128 KB of LDS)
-constexpr int64_t kBEdges = 1 << 19;     // in-edges per bucket, and per unit of a one-row bucket
-constexpr int kBSegMax = 4000;           // buckets a window's segment table may hold
+struct BlockShape {
+  int64_t rows;   // rows per bucket
+  int64_t edges;  // in-edges per bucket, and per unit of a one-row bucket
+  bool fine;
+};
+constexpr int kBRows = 8192;             // coarse: the accumulators fill 128 KB of LDS
+constexpr int64_t kBEdges = 1 << 19;
+constexpr int kFineRows = 2048;
+constexpr int kFineEdges = 16384;        // with the row sums 72 KB of LDS: two workgroups per CU
+constexpr int kFineLeast = 1024;         // ... of a small block, so that its buckets reach more CUs
+constexpr int kFineLong = 256;           // rows from here on are summed by the workgroup,
+constexpr int kFineMid = 8;              // from here on by eight lanes, shorter ones by a thread
+constexpr BlockShape kCoarse = {kBRows, kBEdges, false};
+constexpr BlockShape kFine = {kFineRows, kFineEdges, true};
+constexpr int kBSegMax = 8000;           // buckets a window's segment table may hold (beside the window in LDS)
 constexpr int kBPer = 8;                 // edges per thread in pass 1 (window starts padded to it)
 struct BlockUnit {  // pass 2 work: bucket rows [row0, row0 + nrows), edges [e0, e1)
   int32_t row0;
   int32_t nrows;
   int32_t slot;  // >= 0: a part of a one-row bucket, its sum goes to partial slot `slot`
+  int32_t nlong; // fine: rows of kFineLong in-edges and more (the first in its part of `rows`)
+  int32_t nmid;  // ... of kFineMid and more
   int32_t pad;
   int64_t e0, e1;
+};
+struct BlockGroup {   // 64 consecutive edges of a window
+  uint64_t starts;    // bit k: edge k + 1 of the group begins a segment
+  int32_t first;      // the segment, in the window, of the group's edge 0
+  int32_t pad;
+};
+struct FineRow {  // row `row` of a fine bucket: places [start, start + len)
+  uint16_t row, start, len, pad;
 };
 struct BlockSplit {  // a one-row bucket in parts: partial slots [first, first + count)
   int32_t row;
@@ -130,16 +162,20 @@ struct BlockHost {
   std::vector<int64_t> wseg;       // first segment of each window (+ end)
   std::vector<int32_t> seg_e;      // segment start inside its window
   std::vector<int32_t> seg_d;      // segment destination minus seg_e
-  std::vector<uint16_t> brow_off;  // bucket-major row offsets inside the bucket
+  std::vector<int64_t> wgroup;     // first group of 64 edges of each window (+ end)
+  std::vector<BlockGroup> groups;  // per group: where segments start in it
+  std::vector<uint16_t> brow_off;  // bucket-major; coarse: row offset inside the bucket, fine: place, rows by length
+  std::vector<FineRow> rows;       // fine: per bucket (from its first row on), longest class first
   std::vector<BlockUnit> units;
   std::vector<BlockSplit> splits;
   int32_t n_slots = 0, n_windows = 0;
   int64_t n_buckets = 0;
 };
 // Builds the propagation layout of an in-CSR of n rows with sources in
-// [0, n_gather).  Returns DMM_OK or an error code (message in *err).
-int build_blocks_host(int64_t n, int64_t n_gather, const int64_t* off, const int32_t* nbr, BlockHost* out,
-                      std::string* err);
+// [0, n_gather) with buckets of the given shape.  Returns DMM_OK or an error
+// code (message in *err; DMM_ERR_CAPACITY also for too many buckets).
+int build_blocks_host(int64_t n, int64_t n_gather, const int64_t* off, const int32_t* nbr, const BlockShape& shape,
+                      BlockHost* out, std::string* err);
 // Builds it from the device CSR (host work, once per upload, at the first
 // compensated block iteration).
 int pr_blocks_build(dmm_ctx* ctx);

@@ -70,6 +70,7 @@ struct PrArgs {
   int main_blocks;                // error partials written before the combine
   PrCtrl* ctrl;
   double* err_trace;              // per-iteration error
+  double* err_out;                // the iteration's error again, for the caller (may be NULL)
   const PrParams* prm;
 };
 
@@ -1116,15 +1117,18 @@ struct BpArgs {
   const int64_t* wstart;
   const int32_t* wlen;
   const int64_t* wseg;
-  const int32_t* seg_e;
   const int32_t* seg_d;
+  const int64_t* wgroup;
+  const BlockGroup* groups;
   const uint16_t* brow;
+  const FineRow* rows;
   const BlockUnit* units;
   const BlockSplit* splits;
   float* val;
   float* spare;     // val[m]: the stores of lanes past a window's end
   long long* part;  // (lo, hi) per partial slot
   int32_t nwin;
+  int32_t wparts;   // workgroups that share a window
   int64_t n_units, n_splits;
 };
 
@@ -1181,33 +1185,37 @@ __device__ __forceinline__ float fx_value(unsigned long long lo, long long hi) {
   return neg ? -f : f;
 }
 
-// Pass 1: persistent workgroups take windows in turn.  A window's
-// contributions and segment table go to LDS.  A wavefront takes kBPer
-// groups of 64 consecutive edges at a time, lane l the l-th edge of each
-// group, so every store instruction writes 64 consecutive destinations
-// inside a segment (segments average tens of edges).  The group's first
-// segment is found once per wavefront by binary search; each lane steps
-// from it to its own edge's segment.  The next round's source offsets are
-// loaded before this round's stores.
+// Pass 1: persistent workgroups take windows in turn, or parts of one where
+// there are fewer windows than CUs.  A window's contributions and segment
+// table go to LDS.  A wavefront takes kBPer groups of 64 consecutive edges at
+// a time, lane l the l-th edge of each group, so every store instruction
+// writes 64 consecutive destinations inside a segment (segments average tens
+// of edges).  A lane's segment is the group's first plus the segment starts
+// up to its edge, counted in the group's mask.  The next round's source
+// offsets and masks are loaded before this round's stores.
 __global__ __launch_bounds__(kBPropThreads) void k_bprop(BpArgs b, const float* __restrict__ cin, int64_t n_gather,
                                                          const PrCtrl* ctrl) {
   __shared__ float win[kBWin];
-  __shared__ int32_t se[kBSegMax + 1];
   __shared__ int32_t sd[kBSegMax];
   if (ctrl->pad) return;
   const int lane = lane_id();
   const int wv = threadIdx.x >> 6;
   constexpr int kRound = 64 * kBPer;                         // edges per wavefront round
   constexpr int kStride = (kBPropThreads / 64) * kRound;     // edges per workgroup round
-  for (int32_t w = blockIdx.x; w < b.nwin; w += gridDim.x) {
+  for (int32_t item = blockIdx.x; item < b.nwin * b.wparts; item += gridDim.x) {
+    const int32_t w = item % b.nwin, part = item / b.nwin;
     const int64_t base = int64_t(w) * kBWin;
     const int cnt = static_cast<int>(min<int64_t>(kBWin, n_gather - base));
     const int64_t s0 = b.wseg[w];
     const int ns = static_cast<int>(b.wseg[w + 1] - s0);
-    const int len = b.wlen[w];
+    // This part's edges [begin, len) of the window (whole rounds).
+    const int per = (b.wlen[w] + b.wparts * kStride - 1) / (b.wparts * kStride) * kStride;
+    const int begin = part * per;
+    const int len = min(b.wlen[w], begin + per);
+    if (begin >= len) continue;
     const uint16_t* src = b.src + b.wstart[w];
     __syncthreads();  // the previous window's readers are done
-    if (cnt == kBWin) {
+    if (cnt == kBWin && (reinterpret_cast<uintptr_t>(cin) & 15) == 0) {
       const float4* s4 = reinterpret_cast<const float4*>(cin + base);
       float4* d4 = reinterpret_cast<float4*>(win);
       constexpr int kPer = kBWin / 4 / kBPropThreads;
@@ -1219,68 +1227,351 @@ __global__ __launch_bounds__(kBPropThreads) void k_bprop(BpArgs b, const float* 
     } else {
       for (int j = threadIdx.x; j < cnt; j += kBPropThreads) win[j] = cin[base + j];
     }
-    for (int k = threadIdx.x; k < ns; k += kBPropThreads) {
-      se[k] = b.seg_e[s0 + k];
-      sd[k] = b.seg_d[s0 + k];
-    }
-    if (threadIdx.x == 0) se[ns] = len;
+    for (int k = threadIdx.x; k < ns; k += kBPropThreads) sd[k] = b.seg_d[s0 + k];
+    const BlockGroup* groups = b.groups + b.wgroup[w];
+    const int last_group = (b.wlen[w] - 1) >> 6;
     __syncthreads();
-    // A wavefront's next round of source offsets loads at the start of the
+    // A wavefront's next round of offsets and masks loads at the start of the
     // current round, into one of two buffers that alternate (no copy, which
     // would wait).  Vector loads and stores complete in issue order; with
     // unconditional loads (index clamped into the window) and stores, every
     // path issues the same count, so the next round waits for its offsets
     // with a count that leaves this round's stores in flight.
-    auto load_round = [&](int c, uint32_t (&qr)[kBPer]) {
-#pragma unroll
-      for (int k = 0; k < kBPer; k++) qr[k] = src[min(c + lane + 64 * k, len - 1)];
+    struct Round {
+      uint32_t q[kBPer];
+      BlockGroup g;  // lane k: the round's k-th group
     };
-    auto round = [&](int c0, const uint32_t (&q)[kBPer], uint32_t (&qn)[kBPer]) {
-      load_round(c0 + kStride, qn);
-      int lo = 0, hi = ns;  // the last segment with se <= c0 (the same for every lane)
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (se[mid] <= c0) lo = mid; else hi = mid;
-      }
-      // Every lane stores kBPer times (lanes past the window's end into the
+    auto load_round = [&](int c, Round& r) {
+#pragma unroll
+      for (int k = 0; k < kBPer; k++) r.q[k] = src[min(c + lane + 64 * k, len - 1)];
+      r.g = groups[min((c >> 6) + (lane & (kBPer - 1)), last_group)];
+    };
+    auto round = [&](int c0, const Round& r, Round& next) {
+      load_round(c0 + kStride, next);
+      // Every lane stores kBPer times (lanes past the part's end into the
       // spare slot), so every path issues the same number of stores.
 #pragma unroll
       for (int k = 0; k < kBPer; k++) {
         const int i = c0 + lane + 64 * k;
-        int sg = lo;
-        float* dst = b.spare;
-        if (i < len) {
-          while (se[sg + 1] <= i) sg++;
-          dst = b.val + int64_t(sd[sg]) + i;
-        }
-        *dst = win[q[k]];
-        lo = __shfl(sg, 63);  // lane 63 holds the group's last edge: the next group starts in its segment or later
+        const unsigned lo = __builtin_amdgcn_readlane(static_cast<unsigned>(r.g.starts), k);
+        const unsigned hi = __builtin_amdgcn_readlane(static_cast<unsigned>(r.g.starts >> 32), k);
+        const int sg = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, __builtin_amdgcn_readlane(r.g.first, k)));
+        float* dst = b.val + int64_t(sd[min(sg, ns - 1)]) + i;
+        *(i < len ? dst : b.spare) = win[r.q[k]];
       }
     };
-    if (len > 0) {
-      int c0 = wv * kRound;
-      uint32_t qa[kBPer], qb[kBPer];
-      load_round(c0, qa);
+    int c0 = begin + wv * kRound;
+    if (c0 < len) {
+      Round ra, rb;
+      load_round(c0, ra);
 #pragma unroll
-      for (int k = 0; k < kBPer; k++) __asm__ volatile("" ::"v"(qa[k]));
-      while (c0 < len) {
-        round(c0, qa, qb);
+      for (int k = 0; k < kBPer; k++) __asm__ volatile("" ::"v"(ra.q[k]));
+      __asm__ volatile("" ::"v"(ra.g.first));
+      for (;;) {
+        round(c0, ra, rb);
         c0 += kStride;
         if (c0 >= len) break;
-        round(c0, qb, qa);
+        round(c0, rb, ra);
         c0 += kStride;
+        if (c0 >= len) break;
       }
     }
   }
 }
 
-// Pass 2: persistent workgroups take units in turn.  A bucket of several
-// rows accumulates in LDS (128-bit integer per row: the low word by a
+// A unit of one row, by the workgroup: summed in registers.
+constexpr int kBSumUnroll = 8;
+__device__ __forceinline__ void one_row_unit(const PrArgs& a, const BpArgs& b, const BlockUnit& U,
+                                             unsigned long long* rlo, long long* rhi, double& err, float* cout,
+                                             float* score) {
+  constexpr int64_t kStep = int64_t(kBSumThreads) * kBSumUnroll;
+  const int tid = threadIdx.x;
+  const int lane = lane_id();
+  const int wave = tid >> 6;
+  unsigned long long lo = 0;
+  long long hi = 0;
+  for (int64_t e = U.e0 + tid; e < U.e1; e += kStep) {
+    float v[kBSumUnroll];
+#pragma unroll
+    for (int j = 0; j < kBSumUnroll; j++) v[j] = e + j * kBSumThreads < U.e1 ? b.val[e + j * kBSumThreads] : 0.0f;
+#pragma unroll
+    for (int j = 0; j < kBSumUnroll; j++) {
+      unsigned long long xl;
+      long long xh;
+      fx_of(v[j], xl, xh);
+      fx_add(lo, hi, xl, xh);
+    }
+  }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    const unsigned long long ol = __shfl_xor(lo, d);
+    const long long oh = __shfl_xor(hi, d);
+    fx_add(lo, hi, ol, oh);
+  }
+  if (lane == 0) {
+    rlo[wave] = lo;
+    rhi[wave] = hi;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    unsigned long long tl = 0;
+    long long th = 0;
+    for (int w = 0; w < kBSumThreads / 64; w++) fx_add(tl, th, rlo[w], rhi[w]);
+    if (U.slot >= 0) {
+      b.part[2 * int64_t(U.slot)] = static_cast<long long>(tl);
+      b.part[2 * int64_t(U.slot) + 1] = th;
+    } else {
+      err += finish_f32(a, U.row0, fx_value(tl, th), score, cout);
+    }
+  }
+  __syncthreads();
+}
+
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ long long dpp_move64(long long x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(x), kCtrl, kRowMask, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(x >> 32), kCtrl, kRowMask, 0xf, true);
+  return (static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo);
+}
+
+// Sum over groups of kLanes lanes (1, 8 or 64), valid in a group's last lane.
+template <int kCtrl, int kRowMask, typename T>
+__device__ __forceinline__ T dpp_moved(T x) {
+  long long b;
+  __builtin_memcpy(&b, &x, 8);
+  b = dpp_move64<kCtrl, kRowMask>(b);
+  __builtin_memcpy(&x, &b, 8);
+  return x;
+}
+template <int kLanes, typename T>
+__device__ __forceinline__ T group_sum(T x) {
+  if (kLanes > 1) {
+    x += dpp_moved<0x111, 0xf>(x);  // row_shr:1
+    x += dpp_moved<0x112, 0xf>(x);  // row_shr:2
+    x += dpp_moved<0x114, 0xf>(x);  // row_shr:4
+  }
+  if (kLanes == 64) {
+    x += dpp_moved<0x118, 0xf>(x);  // row_shr:8
+    x += dpp_moved<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3
+    x += dpp_moved<0x143, 0xc>(x);  // row_bcast:31 into rows 2 and 3
+  }
+  return x;
+}
+
+// Exact sums of contributions (multiples of 2^-kFxShift), as two doubles
+// where every |c| of the unit is 0 or in [2^-57, 1/4] (FineHalves), else as
+// 128-bit integers (FineFixed).
+//
+// Halves: c = h + l with h the nearest multiple of 2^-40 and l a multiple of
+// 2^-80 of at most 2^-41.  A unit has at most 2^14 values, so sums of h stay
+// at most 2^52 units and sums of l at most 2^53: neither is ever rounded, in
+// any order, and h + l is the exact sum.  Five double additions a value where
+// the integers take some twenty instructions.
+constexpr float kHalvesMin = 0x1p-57f, kHalvesMax = 0.25f;
+static_assert(kFineEdges <= 1 << 14, "exact sums of halves");
+
+struct FineHalves {
+  double h = 0.0, l = 0.0;
+  __device__ __forceinline__ void add(float c) {
+    constexpr double kRound = 0x1.8p12;  // adding it rounds to multiples of 2^-40
+    const double d = static_cast<double>(c);
+    const double t = (d + kRound) - kRound;
+    h += t;
+    l += d - t;
+  }
+  template <int kLanes>
+  __device__ __forceinline__ void reduce() {
+    h = group_sum<kLanes>(h);
+    l = group_sum<kLanes>(l);
+  }
+  // To a row's accumulator in LDS (two words, zeroed), from any wavefront.
+  __device__ __forceinline__ void add_to(unsigned long long* a, unsigned long long* b) const {
+    atomicAdd(reinterpret_cast<double*>(a), h);
+    atomicAdd(reinterpret_cast<double*>(b), l);
+  }
+  static __device__ __forceinline__ FineHalves of(unsigned long long a, unsigned long long b) {
+    FineHalves r;
+    __builtin_memcpy(&r.h, &a, 8);
+    __builtin_memcpy(&r.l, &b, 8);
+    return r;
+  }
+  // h + l rounded once to FP32: rounded to odd in double (which keeps, in its
+  // last bit, that something was cut off), then to nearest.
+  __device__ __forceinline__ float value() const {
+    const double s = h + l;
+    const double bb = s - h;
+    const double e = (h - (s - bb)) + (l - bb);
+    long long bits = __double_as_longlong(s);
+    if (e != 0.0 && (bits & 1) == 0) bits += (e > 0.0) == (s > 0.0) ? 1 : -1;
+    return static_cast<float>(__longlong_as_double(bits));
+  }
+};
+
+struct FineFixed {
+  unsigned long long lo = 0;
+  long long hi = 0;
+  __device__ __forceinline__ void add(float c) {
+    unsigned long long xl;
+    long long xh;
+    fx_of(c, xl, xh);
+    fx_add(lo, hi, xl, xh);
+  }
+  // Three limbs of 48 bits, whose sums over lanes carry nothing.
+  template <int kLanes>
+  __device__ __forceinline__ void reduce() {
+    if (kLanes == 1) return;
+    constexpr unsigned long long kMask = (1ull << 48) - 1;
+    const long long l0 = group_sum<kLanes>(static_cast<long long>(lo & kMask));
+    const long long l1 =
+        group_sum<kLanes>(static_cast<long long>(((lo >> 48) | (static_cast<unsigned long long>(hi) << 16)) & kMask));
+    const long long l2 = group_sum<kLanes>(hi >> 32);
+    lo = static_cast<unsigned long long>(l0);
+    hi = l2 << 32;
+    fx_add(lo, hi, static_cast<unsigned long long>(l1) << 48, l1 >> 16);
+  }
+  __device__ __forceinline__ void add_to(unsigned long long* a, unsigned long long* b) const {
+    const unsigned long long old = atomicAdd(a, lo);
+    atomicAdd(b, static_cast<unsigned long long>(hi) + (old + lo < old ? 1 : 0));
+  }
+  static __device__ __forceinline__ FineFixed of(unsigned long long a, unsigned long long b) {
+    FineFixed r;
+    r.lo = a;
+    r.hi = static_cast<long long>(b);
+    return r;
+  }
+  __device__ __forceinline__ float value() const { return fx_value(lo, hi); }
+};
+
+// The exact sum of places [begin, end), by kLanes lanes of which this is the
+// sub-th, kFineAhead reads ahead; valid in the last one.
+constexpr int kFineAhead = 4;
+template <typename Acc, int kLanes>
+__device__ __forceinline__ Acc fine_sum(const float* place, int begin, int end, int sub) {
+  Acc acc;
+  for (int k = begin + sub; k < end; k += kLanes * kFineAhead) {
+    float x[kFineAhead];
+#pragma unroll
+    for (int j = 0; j < kFineAhead; j++) x[j] = place[min(k + j * kLanes, end - 1)];
+#pragma unroll
+    for (int j = 0; j < kFineAhead; j++) acc.add(k + j * kLanes < end ? x[j] : 0.0f);
+  }
+  acc.template reduce<kLanes>();
+  return acc;
+}
+
+constexpr int kFineLongs = kFineEdges / kFineLong;
+static_assert(kFineLongs <= 64, "a lane per long row");
+
+struct FineLds {
+  float place[kFineEdges];
+  float sums[kFineRows];
+  unsigned long long la[kFineLongs], lb[kFineLongs];  // the long rows' accumulators
+  int fixed;  // the unit last found with a contribution outside the halves' range
+};
+
+// The row sums of a unit whose contributions are in place.
+template <typename Acc>
+__device__ __forceinline__ void fine_rows(const BlockUnit& U, const FineRow* rows, FineLds& L) {
+  constexpr int kWaves = kBSumThreads / 64;
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int short0 = U.nlong + U.nmid;
+  if (U.nlong > 0) {
+    // The long rows hold places [0, end): this wavefront's share, row by row.
+    const FineRow mine = rows[min(lane, U.nlong - 1)];
+    const int end = __builtin_amdgcn_readlane(mine.start + mine.len, U.nlong - 1);
+    const int per = (end + kWaves - 1) / kWaves;
+    const int p1 = min(end, (wave + 1) * per);
+    int p = wave * per;
+    int i = __popcll(__ballot(lane < U.nlong && mine.start <= p)) - 1;
+    while (p < p1) {
+      const int stop = min(p1, __builtin_amdgcn_readlane(mine.start + mine.len, i));
+      const Acc acc = fine_sum<Acc, 64>(L.place, p, stop, lane);
+      if (lane == 63) acc.add_to(&L.la[i], &L.lb[i]);
+      p = stop;
+      i++;
+    }
+  }
+  for (int i0 = U.nlong + wave * 8; i0 < short0; i0 += kWaves * 8) {
+    const int i = i0 + (lane >> 3);
+    const FineRow r = rows[min(i, short0 - 1)];
+    const Acc acc = fine_sum<Acc, 8>(L.place, r.start, r.start + r.len, lane & 7);
+    if (i < short0 && (lane & 7) == 7) L.sums[r.row] = acc.value();
+  }
+  for (int i = short0 + threadIdx.x; i < U.nrows; i += kBSumThreads) {
+    const FineRow r = rows[i];
+    L.sums[r.row] = fine_sum<Acc, 1>(L.place, r.start, r.start + r.len, 0).value();
+  }
+  if (U.nlong > 0) {
+    __syncthreads();
+    const int i = threadIdx.x;
+    if (i < U.nlong) L.sums[rows[i].row] = Acc::of(L.la[i], L.lb[i]).value();
+  }
+}
+
+// Pass 2, fine buckets: a unit's contributions go to their places in LDS,
+// rows by length, and each row's run is summed in registers: short rows by a
+// thread, middling ones by eight lanes, and the long ones' places are shared
+// out evenly, each wavefront adding what it has of a row to the row's
+// accumulator; then the rows finish, in order.  One LDS write and one read
+// per edge where the coarse pass has 64-bit atomics.
+__global__ __launch_bounds__(kBSumThreads, 8) void k_bfine(PrArgs a, BpArgs b, float* __restrict__ cout,
+                                                           float* __restrict__ score) {
+  __shared__ FineLds L;
+  __shared__ unsigned long long rlo[kBSumThreads / 64];
+  __shared__ long long rhi[kBSumThreads / 64];
+  __shared__ double red[kBSumThreads / 64];
+  if (a.ctrl->pad) return;
+  double err = 0;
+  const int tid = threadIdx.x;
+  constexpr int kPer = kFineEdges / kBSumThreads;
+  if (tid == 0) L.fixed = -1;  // no unit
+  __syncthreads();
+  for (int u = blockIdx.x; u < b.n_units; u += gridDim.x) {
+    const BlockUnit U = b.units[u];
+    if (U.nrows == 1) {
+      one_row_unit(a, b, U, rlo, rhi, err, cout, score);
+      continue;
+    }
+    const int n = static_cast<int>(U.e1 - U.e0);
+    if (n > 0) {
+      // All loads first (past the end the last edge again), then the stores.
+      float v[kPer];
+      int at[kPer];
+#pragma unroll
+      for (int j = 0; j < kPer; j++) {
+        const int64_t e = U.e0 + min(tid + j * kBSumThreads, n - 1);
+        v[j] = b.val[e];
+        at[j] = b.brow[e];
+      }
+      bool halves = true;
+#pragma unroll
+      for (int j = 0; j < kPer; j++) {
+        L.place[at[j]] = v[j];
+        const float c = fabsf(v[j]);
+        halves = halves && (c == 0.0f || (c >= kHalvesMin && c <= kHalvesMax));
+      }
+      if (!halves) L.fixed = u;
+    }
+    if (tid < kFineLongs) L.la[tid] = L.lb[tid] = 0;
+    __syncthreads();
+    if (L.fixed != u)
+      fine_rows<FineHalves>(U, b.rows + U.row0, L);
+    else
+      fine_rows<FineFixed>(U, b.rows + U.row0, L);
+    __syncthreads();
+    for (int r = tid; r < U.nrows; r += kBSumThreads) err += finish_f32(a, int64_t(U.row0) + r, L.sums[r], score, cout);
+  }
+  const double t = block_err_sum<kBSumThreads>(err, red);
+  if (threadIdx.x == 0) a.err_part[blockIdx.x] = t;
+}
+
+// Pass 2, coarse buckets: persistent workgroups take units in turn.  A bucket
+// of several rows accumulates in LDS (128-bit integer per row: the low word by a
 // 64-bit atomic add, its carry and the high word by a second); a one-row
 // unit in registers, reduced over the workgroup.  Rows finish here, except
 // the parts of a one-row bucket beyond kBEdges edges, whose sums go to
 // partial slots for k_bsplit.
-constexpr int kBSumUnroll = 8;
 __global__ __launch_bounds__(kBSumThreads) void k_bsum(PrArgs a, BpArgs b, float* __restrict__ cout,
                                                        float* __restrict__ score) {
   __shared__ unsigned long long alo[kBRows];
@@ -1291,49 +1582,11 @@ __global__ __launch_bounds__(kBSumThreads) void k_bsum(PrArgs a, BpArgs b, float
   if (a.ctrl->pad) return;
   double err = 0;
   const int tid = threadIdx.x;
-  const int lane = lane_id();
-  const int wave = tid >> 6;
   constexpr int64_t kStep = int64_t(kBSumThreads) * kBSumUnroll;
   for (int64_t u = blockIdx.x; u < b.n_units; u += gridDim.x) {
     const BlockUnit U = b.units[u];
     if (U.nrows == 1) {
-      unsigned long long lo = 0;
-      long long hi = 0;
-      for (int64_t e = U.e0 + tid; e < U.e1; e += kStep) {
-        float v[kBSumUnroll];
-#pragma unroll
-        for (int j = 0; j < kBSumUnroll; j++) v[j] = e + j * kBSumThreads < U.e1 ? b.val[e + j * kBSumThreads] : 0.0f;
-#pragma unroll
-        for (int j = 0; j < kBSumUnroll; j++) {
-          unsigned long long xl;
-          long long xh;
-          fx_of(v[j], xl, xh);
-          fx_add(lo, hi, xl, xh);
-        }
-      }
-#pragma unroll
-      for (int d = 32; d >= 1; d >>= 1) {
-        const unsigned long long ol = __shfl_xor(lo, d);
-        const long long oh = __shfl_xor(hi, d);
-        fx_add(lo, hi, ol, oh);
-      }
-      if (lane == 0) {
-        rlo[wave] = lo;
-        rhi[wave] = hi;
-      }
-      __syncthreads();
-      if (tid == 0) {
-        unsigned long long tl = 0;
-        long long th = 0;
-        for (int w = 0; w < kBSumThreads / 64; w++) fx_add(tl, th, rlo[w], rhi[w]);
-        if (U.slot >= 0) {
-          b.part[2 * int64_t(U.slot)] = static_cast<long long>(tl);
-          b.part[2 * int64_t(U.slot) + 1] = th;
-        } else {
-          err += finish_f32(a, U.row0, fx_value(tl, th), score, cout);
-        }
-      }
-      __syncthreads();
+      one_row_unit(a, b, U, rlo, rhi, err, cout, score);
       continue;
     }
     for (int r = tid; r < U.nrows; r += kBSumThreads) {
@@ -1425,6 +1678,7 @@ __global__ __launch_bounds__(kThreads) void k_reduce(PrArgs a) {
     const unsigned it = c->ticket;
     c->err = t;
     if (it < DMM_MAX_PR_ITERS) a.err_trace[it] = t;
+    if (a.err_out) *a.err_out = t;
     c->ticket = it + 1;
     if (t < a.prm->eps) c->pad = 1;
   }
@@ -1494,6 +1748,7 @@ PrArgs make_args(dmm_ctx* ctx) {
   a.zero_begin = ctx->pr_zero_begin;
   a.ctrl = ctx->d_prctrl;
   a.err_trace = ctx->d_err_trace;
+  a.err_out = nullptr;
   a.prm = reinterpret_cast<const PrParams*>(ctx->d_prparams);
   return a;
 }
@@ -1529,22 +1784,29 @@ void launch_iteration(dmm_ctx* ctx, PrArgs a, int mode, int it, const void* gcon
       b.wstart = static_cast<const int64_t*>(ctx->d_bp_wstart);
       b.wlen = static_cast<const int32_t*>(ctx->d_bp_wlen);
       b.wseg = static_cast<const int64_t*>(ctx->d_bp_wseg);
-      b.seg_e = static_cast<const int32_t*>(ctx->d_bp_seg_e);
+      b.wgroup = static_cast<const int64_t*>(ctx->d_bp_wgroup);
+      b.groups = static_cast<const BlockGroup*>(ctx->d_bp_groups);
       b.seg_d = static_cast<const int32_t*>(ctx->d_bp_seg_d);
       b.brow = static_cast<const uint16_t*>(ctx->d_bp_brow);
+      b.rows = static_cast<const FineRow*>(ctx->d_bp_rows);
       b.units = static_cast<const BlockUnit*>(ctx->d_bp_units);
       b.splits = static_cast<const BlockSplit*>(ctx->d_bp_splits);
       b.val = static_cast<float*>(ctx->d_bp_val);
       b.spare = b.val + ctx->m_in;
       b.part = static_cast<long long*>(ctx->d_bp_part);
       b.nwin = static_cast<int32_t>(ctx->n_bp_windows);
+      // A block with fewer windows than CUs has several workgroups copy each.
+      b.wparts = std::max<int32_t>(1, std::max(1, ctx->cu_count) / std::max(1, b.nwin));
       b.n_units = ctx->n_bp_units;
       b.n_splits = ctx->n_bp_splits;
       hipLaunchKernelGGL(k_bprop, dim3(std::max(1, ctx->cu_count)), dim3(kBPropThreads), 0, s, b, cin, a.n_gather,
                          a.ctrl);
       a.main_blocks = pr_bsum_blocks(ctx);
       a.super_blocks = pr_bsplit_blocks(ctx);
-      hipLaunchKernelGGL(k_bsum, dim3(a.main_blocks), dim3(kBSumThreads), 0, s, a, b, cout, score_f);
+      if (ctx->bp_fine)
+        hipLaunchKernelGGL(k_bfine, dim3(a.main_blocks), dim3(kBSumThreads), 0, s, a, b, cout, score_f);
+      else
+        hipLaunchKernelGGL(k_bsum, dim3(a.main_blocks), dim3(kBSumThreads), 0, s, a, b, cout, score_f);
       if (a.super_blocks > 0)
         hipLaunchKernelGGL(k_bsplit, dim3(a.super_blocks), dim3(kThreads), 0, s, a, b, cout, score_f);
     } else if (ctx->tiles_ready && !gcontrib) {
@@ -1653,7 +1915,9 @@ int pr_fused_blocks(dmm_ctx* ctx) {
 int pr_row_blocks(dmm_ctx* ctx) { return kRowGroupsPerCU * std::max(1, ctx->cu_count); }
 
 int pr_bsum_blocks(dmm_ctx* ctx) {
-  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(std::max(1, ctx->cu_count), ctx->n_bp_units)));
+  const int64_t per_cu = ctx->bp_fine ? 2 : 1;  // by LDS
+  return static_cast<int>(
+      std::max<int64_t>(1, std::min<int64_t>(per_cu * std::max(1, ctx->cu_count), ctx->n_bp_units)));
 }
 
 int pr_bsplit_blocks(dmm_ctx* ctx) { return static_cast<int>(ceil_div(ctx->n_bp_splits, kThreads)); }
@@ -1819,10 +2083,6 @@ __global__ void k_scratch_prep(unsigned char* base, PrParams p) {
   }
 }
 
-__global__ void k_scratch_err(const unsigned char* base, double* err_out) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *err_out = reinterpret_cast<const PrCtrl*>(base + kScratchCtrl)->err;
-}
-
 }  // namespace
 
 int scratch_init(dmm_ctx* ctx) {
@@ -1857,6 +2117,7 @@ int pr_block_iteration_noalloc(dmm_ctx* ctx, const float* d_gcontrib, float* d_s
   a.prm = reinterpret_cast<const PrParams*>(base + kScratchParams);
   a.ctrl = reinterpret_cast<PrCtrl*>(base + kScratchCtrl);
   a.err_trace = reinterpret_cast<double*>(base + kScratchTrace);
+  a.err_out = d_err;
   a.err_part = reinterpret_cast<double*>(base + kScratchErr);
   a.partial = reinterpret_cast<double2*>(base + kScratchSegs);
   // Constants as the reference computes them in float (src/pr.cc:39, 45-46);
@@ -1874,7 +2135,6 @@ int pr_block_iteration_noalloc(dmm_ctx* ctx, const float* d_gcontrib, float* d_s
   p.pad = 0;
   hipLaunchKernelGGL(k_scratch_prep, dim3(1), dim3(64), 0, ctx->stream, base, p);
   launch_iteration(ctx, a, mode, 0, d_gcontrib, d_scores, d_contrib_out);
-  hipLaunchKernelGGL(k_scratch_err, dim3(1), dim3(64), 0, ctx->stream, base, d_err);
   DMM_HIP_CHECK(ctx, hipGetLastError());
   DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
   return DMM_OK;

@@ -4,21 +4,23 @@
 //
 // Sources are cut into windows of kBWin vertices (one window of
 // contributions fills a workgroup's LDS); rows into buckets of at most
-// kBRows consecutive rows and kBEdges in-edges (a row with more in-edges is
-// a bucket of its own, summed in units of at most kBEdges edges).  Edge
-// (u -> r) belongs to segment (window u / kBWin, bucket of r).
+// shape.rows consecutive rows and shape.edges in-edges (a row with more
+// in-edges is a bucket of its own, summed in units of at most that many).
+// Edge (u -> r) belongs to segment (window u / kBWin, bucket of r).
 //
 //   window-major array (pass 1 reads it): per window its edges' 16-bit
 //     source offsets, segment by segment in bucket order, the window's
 //     start padded to a multiple of kBPer edges;
 //   bucket-major array (pass 1 writes it, pass 2 reads it): per bucket its
 //     edges' contributions, segment by segment in window order, and beside
-//     it (static) each edge's row offset inside its bucket.
+//     it (static) each edge's row offset inside its bucket (coarse) or its
+//     place among the bucket's edges, rows by length (fine).
 // The i-th edge of a segment sits at the i-th place of the segment in both
 // arrays.  Per window, the segment table gives each non-empty segment's
-// start inside the window and its destination in the bucket-major array
-// (stored as destination - start, so an edge's destination is that plus
-// its index in the window).
+// destination in the bucket-major array (stored as destination - start, so an
+// edge's destination is that plus its index in the window), and per group of
+// 64 edges of the window a mask says where segments start, so that a lane
+// counts its segment instead of searching for it.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -30,8 +32,8 @@
 
 namespace dmm {
 
-int build_blocks_host(int64_t n, int64_t n_gather, const int64_t* off, const int32_t* nbr, BlockHost* out,
-                      std::string* err) {
+int build_blocks_host(int64_t n, int64_t n_gather, const int64_t* off, const int32_t* nbr, const BlockShape& shape,
+                      BlockHost* out, std::string* err) {
   const int nt = resolve_threads(0);
   const int64_t m = off[n];
   if (m >= (int64_t(1) << 31) || n_gather >= (int64_t(1) << 31)) {
@@ -45,7 +47,7 @@ int build_blocks_host(int64_t n, int64_t n_gather, const int64_t* off, const int
     int64_t rows = 0, edges = 0;
     for (int64_t r = 0; r < n; r++) {
       const int64_t d = off[r + 1] - off[r];
-      if (rows > 0 && (rows == kBRows || edges + d > kBEdges)) {
+      if (rows > 0 && (rows == shape.rows || edges + d > shape.edges)) {
         brow.push_back(static_cast<int32_t>(r));
         rows = edges = 0;
       }
@@ -110,31 +112,77 @@ int build_blocks_host(int64_t n, int64_t n_gather, const int64_t* off, const int
     }
     wseg[w + 1] = static_cast<int64_t>(seg_e.size());
   }
-  // 5. Fill both arrays, bucket by bucket (disjoint segments).
+  // Where segments start, per group of 64 edges.
+  std::vector<int64_t> wgroup(nwin + 1, 0);
+  for (int32_t w = 0; w < nwin; w++) wgroup[w + 1] = wgroup[w] + (wlen[w] + 63) / 64;
+  std::vector<BlockGroup> groups(wgroup[nwin]);
+  parallel_dynamic(nwin, nt, 1, [&](int64_t w) {
+    int32_t k = 0;
+    const int32_t* se = seg_e.data() + wseg[w];
+    const int32_t ns = static_cast<int32_t>(wseg[w + 1] - wseg[w]);
+    for (int64_t g = wgroup[w]; g < wgroup[w + 1]; g++) {
+      const int32_t e0 = static_cast<int32_t>(g - wgroup[w]) * 64;
+      while (k + 1 < ns && se[k + 1] <= e0) k++;
+      groups[g] = {0, k, 0};
+      for (int32_t j = k + 1; j < ns && se[j] < e0 + 64; j++) groups[g].starts |= uint64_t(1) << (se[j] - e0 - 1);
+    }
+  });
+  // 5. Fine buckets: rows by length, longest first (row order inside a length
+  // class of powers of two, so that the rows of a wavefront are alike), and
+  // their runs of places in that order.
+  std::vector<FineRow> rows(shape.fine ? n : 0);
+  std::vector<int32_t> place(shape.fine ? n : 0, 0);  // each row's next place
+  std::vector<int32_t> nlong(nb, 0), nmid(nb, 0);
+  if (shape.fine)
+    parallel_dynamic(nb, nt, 16, [&](int64_t b) {
+      if (brow[b + 1] - brow[b] == 1) return;  // one-row units need no order
+      auto len = [&](int64_t r) { return off[r + 1] - off[r]; };
+      auto cls = [&](int64_t r) {  // 0: longest, 64: empty
+        return len(r) == 0 ? 64 : __builtin_clzll(static_cast<unsigned long long>(len(r)));
+      };
+      int64_t at[66] = {};
+      for (int64_t r = brow[b]; r < brow[b + 1]; r++) {
+        at[cls(r) + 1]++;
+        nlong[b] += len(r) >= kFineLong;
+        nmid[b] += len(r) >= kFineMid && len(r) < kFineLong;
+      }
+      for (int c = 0; c < 65; c++) at[c + 1] += at[c];
+      for (int64_t r = brow[b]; r < brow[b + 1]; r++)
+        rows[brow[b] + at[cls(r)]++] = {static_cast<uint16_t>(r - brow[b]), 0, static_cast<uint16_t>(len(r)), 0};
+      int32_t next = 0;
+      for (int64_t i = brow[b]; i < brow[b + 1]; i++) {
+        rows[i].start = static_cast<uint16_t>(next);
+        place[brow[b] + rows[i].row] = next;
+        next += rows[i].len;
+      }
+    });
+  // 6. Fill both arrays, bucket by bucket (disjoint segments).
   std::vector<uint16_t> src(std::max<int64_t>(1, wstart[nwin]), 0);
   std::vector<uint16_t> brow_off(std::max<int64_t>(1, m), 0);
   parallel_dynamic(nb, nt, 16, [&](int64_t b) {
+    const bool places = shape.fine && brow[b + 1] - brow[b] > 1;
     for (int64_t r = brow[b]; r < brow[b + 1]; r++)
       for (int64_t e = off[r]; e < off[r + 1]; e++) {
         const int32_t u = nbr[e];
         const size_t k = static_cast<size_t>(u / kBWin) * nb + b;
         src[wpos[k]++] = static_cast<uint16_t>(u % kBWin);
-        brow_off[bpos[k]++] = static_cast<uint16_t>(r - brow[b]);
+        brow_off[bpos[k]++] = static_cast<uint16_t>(places ? place[r]++ : r - brow[b]);
       }
   });
-  // 6. Units: a bucket whole, or a one-row bucket beyond kBEdges in parts
+  // 7. Units: a bucket whole, or a one-row bucket beyond shape.edges in parts
   // whose sums go to partial slots.
   std::vector<BlockUnit> units;
   std::vector<BlockSplit> splits;
   int32_t slots = 0;
   for (int64_t b = 0; b < nb; b++) {
     const int64_t e0 = bstart[b], e1 = bstart[b + 1];
-    if (e1 - e0 <= kBEdges) {
-      units.push_back({brow[b], brow[b + 1] - brow[b], -1, 0, e0, e1});
+    if (e1 - e0 <= shape.edges) {
+      units.push_back({brow[b], brow[b + 1] - brow[b], -1, nlong[b], nmid[b], 0, e0, e1});
       continue;
     }
     const int32_t first = slots;
-    for (int64_t e = e0; e < e1; e += kBEdges) units.push_back({brow[b], 1, slots++, 0, e, std::min(e1, e + kBEdges)});
+    for (int64_t e = e0; e < e1; e += shape.edges)
+      units.push_back({brow[b], 1, slots++, 0, 0, 0, e, std::min(e1, e + shape.edges)});
     splits.push_back({brow[b], first, slots - first, 0});
   }
   out->src.swap(src);
@@ -143,7 +191,10 @@ int build_blocks_host(int64_t n, int64_t n_gather, const int64_t* off, const int
   out->wseg.swap(wseg);
   out->seg_e.swap(seg_e);
   out->seg_d.swap(seg_d);
+  out->wgroup.swap(wgroup);
+  out->groups.swap(groups);
   out->brow_off.swap(brow_off);
+  out->rows.swap(rows);
   out->units.swap(units);
   out->splits.swap(splits);
   out->n_slots = slots;
@@ -164,6 +215,18 @@ int upload_vec(dmm_ctx* ctx, void** dst, const std::vector<T>& v, const char* wh
 
 }  // namespace
 
+// Fine buckets of a block with m in-edges: as large as LDS allows, in a small
+// block so that every workgroup (two per CU) has one.  Larger blocks gain
+// nothing from smaller buckets that would divide evenly: Kronecker-23, block
+// 3 of 8 (33 M edges, 4.5 full buckets per workgroup): pass 2 75 us, 90 us
+// with buckets of 13900 edges.
+BlockShape fine_shape(int64_t m, int cus) {
+  BlockShape shape = kFine;
+  const int64_t groups = 2 * std::max(1, cus);
+  shape.edges = std::min<int64_t>(kFineEdges, std::max<int64_t>(kFineLeast, ceil_div(m, groups)));
+  return shape;
+}
+
 int pr_blocks_build(dmm_ctx* ctx) {
   const int64_t n = ctx->nloc;
   const int64_t m = ctx->m_in;
@@ -174,7 +237,10 @@ int pr_blocks_build(dmm_ctx* ctx) {
   BlockHost bh;
   std::string err;
   const int64_t held = ctx->dev_bytes;
-  int rc = build_blocks_host(n, ctx->n, off.data(), nbr.data(), &bh, &err);
+  // Fine buckets where a window's segment table holds them.
+  int rc = build_blocks_host(n, ctx->n, off.data(), nbr.data(), fine_shape(m, ctx->cu_count), &bh, &err);
+  ctx->bp_fine = rc == DMM_OK;
+  if (rc == DMM_ERR_CAPACITY) rc = build_blocks_host(n, ctx->n, off.data(), nbr.data(), kCoarse, &bh, &err);
   if (rc) return set_err(ctx, rc, "%s", err.c_str());
   std::vector<int64_t>().swap(off);
   std::vector<int32_t>().swap(nbr);
@@ -182,9 +248,11 @@ int pr_blocks_build(dmm_ctx* ctx) {
       (rc = upload_vec(ctx, &ctx->d_bp_wstart, bh.wstart, "PR block window starts")) ||
       (rc = upload_vec(ctx, &ctx->d_bp_wlen, bh.wlen, "PR block window lengths")) ||
       (rc = upload_vec(ctx, &ctx->d_bp_wseg, bh.wseg, "PR block window segments")) ||
-      (rc = upload_vec(ctx, &ctx->d_bp_seg_e, bh.seg_e, "PR block segment starts")) ||
+      (rc = upload_vec(ctx, &ctx->d_bp_wgroup, bh.wgroup, "PR block groups")) ||
+      (rc = upload_vec(ctx, &ctx->d_bp_groups, bh.groups, "PR block groups")) ||
       (rc = upload_vec(ctx, &ctx->d_bp_seg_d, bh.seg_d, "PR block segment destinations")) ||
       (rc = upload_vec(ctx, &ctx->d_bp_brow, bh.brow_off, "PR block row offsets")) ||
+      (rc = upload_vec(ctx, &ctx->d_bp_rows, bh.rows, "PR block rows")) ||
       (rc = upload_vec(ctx, &ctx->d_bp_units, bh.units, "PR block units")) ||
       (rc = upload_vec(ctx, &ctx->d_bp_splits, bh.splits, "PR block split rows")) ||
       // One spare slot past the m contributions takes the propagation
@@ -239,25 +307,12 @@ float host_fx_value(__int128 v) {
   return neg ? -f : f;
 }
 
-}  // namespace
-
-}  // namespace dmm
-
-// Host check of the PE-block propagation layout (no GPU): builds it, checks
-// every index the kernels use against its buffer and that every edge reaches
-// its row once, and replays pass 1 and pass 2 with the kernels' arithmetic.
-extern "C" int dmm_pr_blocks_check(int64_t n, int64_t n_gather, const int64_t* off, const int32_t* nbr,
-                                   const float* contrib, float* incoming, int64_t* stats) {
-  using namespace dmm;
-  if (n < 0 || !off || (off[n] > 0 && !nbr) || !contrib || !incoming || !stats)
-    return set_err(nullptr, DMM_ERR_INVALID, "dmm_pr_blocks_check: bad arguments");
+// Checks every index the kernels use against its buffer and that every edge
+// reaches its row once, and replays pass 1 and pass 2 with the kernels'
+// arithmetic.
+int check_blocks(const BlockHost& bh, const BlockShape& shape, int64_t n, int64_t n_gather, const int64_t* off,
+                 const float* contrib, float* incoming) {
   const int64_t m = off[n];
-  for (int64_t e = 0; e < m; e++)
-    if (nbr[e] < 0 || nbr[e] >= n_gather) return set_err(nullptr, DMM_ERR_GRAPH, "source outside [0, n_gather)");
-  BlockHost bh;
-  std::string err;
-  int rc = build_blocks_host(n, n_gather, off, nbr, &bh, &err);
-  if (rc) return set_err(nullptr, rc, "%s", err.c_str());
   auto bad = [](const char* what) { return set_err(nullptr, DMM_ERR_GRAPH, "block layout: %s", what); };
   const int32_t nwin = bh.n_windows;
   if (static_cast<int32_t>(bh.wstart.size()) != nwin + 1 || static_cast<int32_t>(bh.wseg.size()) != nwin + 1 ||
@@ -276,28 +331,19 @@ extern "C" int dmm_pr_blocks_check(int64_t n, int64_t n_gather, const int64_t* o
     if (ns > 0 && bh.seg_e[s0] != 0) return bad("first segment");
     for (int k = 1; k < ns; k++)
       if (bh.seg_e[s0 + k] <= bh.seg_e[s0 + k - 1] || bh.seg_e[s0 + k] >= len) return bad("segment starts");
-    for (int i0 = 0; i0 < len; i0 += kBPer) {
-      int lo = 0, hi = ns;
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (bh.seg_e[s0 + mid] <= i0) lo = mid; else hi = mid;
-      }
-      int next = lo + 1 < ns ? bh.seg_e[s0 + lo + 1] : len;
-      int64_t dst = int64_t(bh.seg_d[s0 + lo]) + i0;
-      for (int k = 0; k < kBPer && i0 + k < len; k++) {
-        const int i = i0 + k;
-        if (i == next) {
-          lo++;
-          next = lo + 1 < ns ? bh.seg_e[s0 + lo + 1] : len;
-          dst = int64_t(bh.seg_d[s0 + lo]) + i;
-        }
-        const uint16_t s = bh.src[bh.wstart[w] + i];
-        if (s >= cnt) return bad("source offset");
-        if (dst < 0 || dst >= m || hit[dst]) return bad("destination");
-        hit[dst] = 1;
-        val[dst] = contrib[base + s];
-        dst++;
-      }
+    if (bh.wgroup[w + 1] - bh.wgroup[w] != (len + 63) / 64) return bad("groups");
+    for (int i = 0; i < len; i++) {
+      const BlockGroup& g = bh.groups[bh.wgroup[w] + i / 64];
+      const int k = i % 64;
+      const int sg = g.first + __builtin_popcountll(k ? g.starts << (64 - k) : 0);
+      if (sg < 0 || sg >= ns || bh.seg_e[s0 + sg] > i || (sg + 1 < ns && bh.seg_e[s0 + sg + 1] <= i))
+        return bad("group segments");
+      const int64_t dst = int64_t(bh.seg_d[s0 + sg]) + i;
+      const uint16_t s = bh.src[bh.wstart[w] + i];
+      if (s >= cnt) return bad("source offset");
+      if (dst < 0 || dst >= m || hit[dst]) return bad("destination");
+      hit[dst] = 1;
+      val[dst] = contrib[base + s];
     }
   }
   for (int64_t e = 0; e < m; e++)
@@ -309,7 +355,7 @@ extern "C" int dmm_pr_blocks_check(int64_t n, int64_t n_gather, const int64_t* o
   std::vector<char> done(std::max<int64_t>(1, n), 0);
   int64_t next_e = 0;
   for (const BlockUnit& u : bh.units) {
-    if (u.e0 != next_e || u.e1 < u.e0 || u.nrows < 1 || u.nrows > kBRows || u.e1 - u.e0 > kBEdges ||
+    if (u.e0 != next_e || u.e1 < u.e0 || u.nrows < 1 || u.nrows > shape.rows || u.e1 - u.e0 > shape.edges ||
         u.row0 < 0 || int64_t(u.row0) + u.nrows > n)
       return bad("unit");
     next_e = u.e1;
@@ -317,7 +363,7 @@ extern "C" int dmm_pr_blocks_check(int64_t n, int64_t n_gather, const int64_t* o
       if (u.nrows != 1 || u.slot >= bh.n_slots) return bad("split unit");
       __int128 s = 0;
       for (int64_t e = u.e0; e < u.e1; e++) {
-        if (bh.brow_off[e] != 0) return bad("split unit row");
+        if (!shape.fine && bh.brow_off[e] != 0) return bad("split unit row");
         s += host_fx_of(val[e]);
       }
       part[u.slot] = s;
@@ -326,9 +372,36 @@ extern "C" int dmm_pr_blocks_check(int64_t n, int64_t n_gather, const int64_t* o
     }
     if (off[u.row0 + u.nrows] - off[u.row0] != u.e1 - u.e0) return bad("unit edges differ from its rows' in-edges");
     std::vector<__int128> acc(u.nrows, 0);
-    for (int64_t e = u.e0; e < u.e1; e++) {
-      if (bh.brow_off[e] >= u.nrows) return bad("row offset");
-      acc[bh.brow_off[e]] += host_fx_of(val[e]);
+    if (shape.fine && u.nrows > 1) {
+      // As k_bfine: every contribution to its place, then each row's run.
+      if (u.nlong > kFineEdges / kFineLong) return bad("long rows");
+      std::vector<float> place(u.e1 - u.e0);
+      std::vector<char> set(u.e1 - u.e0, 0);
+      for (int64_t e = u.e0; e < u.e1; e++) {
+        const int64_t at = bh.brow_off[e];
+        if (at >= u.e1 - u.e0 || set[at]) return bad("place in row order");
+        set[at] = 1;
+        place[at] = val[e];
+      }
+      std::vector<char> taken(u.nrows, 0);
+      int64_t next_place = 0;
+      for (int32_t i = 0; i < u.nrows; i++) {
+        const FineRow fr = bh.rows[u.row0 + i];
+        const int32_t r = fr.row;
+        if (r >= u.nrows || taken[r]) return bad("row order");
+        taken[r] = 1;
+        const int64_t s = next_place, e = s + (off[u.row0 + r + 1] - off[u.row0 + r]);
+        if (fr.start != s || fr.len != e - s) return bad("row places");
+        next_place = e;
+        if ((e - s >= kFineLong) != (i < u.nlong) || (e - s >= kFineMid) != (i < u.nlong + u.nmid))
+          return bad("row classes");
+        for (int64_t k = s; k < e; k++) acc[r] += host_fx_of(place[k]);
+      }
+    } else {
+      for (int64_t e = u.e0; e < u.e1; e++) {
+        if (bh.brow_off[e] >= u.nrows) return bad("row offset");
+        acc[bh.brow_off[e]] += host_fx_of(val[e]);
+      }
     }
     for (int32_t r = 0; r < u.nrows; r++) {
       incoming[u.row0 + r] = host_fx_value(acc[r]);
@@ -351,7 +424,41 @@ extern "C" int dmm_pr_blocks_check(int64_t n, int64_t n_gather, const int64_t* o
   }
   for (int64_t r = 0; r < n; r++)
     if (done[r] != 1) return bad("row not finished exactly once");
-  stats[0] = nwin;
+  return DMM_OK;
+}
+
+}  // namespace
+
+}  // namespace dmm
+
+// Host check of the PE-block propagation layout (no GPU): the coarse layout,
+// and fine ones where the block has them, whose sums must be the same.
+extern "C" int dmm_pr_blocks_check(int64_t n, int64_t n_gather, const int64_t* off, const int32_t* nbr,
+                                   const float* contrib, float* incoming, int64_t* stats) {
+  using namespace dmm;
+  if (n < 0 || !off || (off[n] > 0 && !nbr) || !contrib || !incoming || !stats)
+    return set_err(nullptr, DMM_ERR_INVALID, "dmm_pr_blocks_check: bad arguments");
+  for (int64_t e = 0; e < off[n]; e++)
+    if (nbr[e] < 0 || nbr[e] >= n_gather) return set_err(nullptr, DMM_ERR_GRAPH, "source outside [0, n_gather)");
+  BlockHost bh;
+  std::string err;
+  int rc = build_blocks_host(n, n_gather, off, nbr, kCoarse, &bh, &err);
+  if (rc) return set_err(nullptr, rc, "%s", err.c_str());
+  if ((rc = check_blocks(bh, kCoarse, n, n_gather, off, contrib, incoming))) return rc;
+  // The largest and the smallest fine buckets the GPU uses.
+  BlockShape least = kFine;
+  least.edges = kFineLeast;
+  for (const BlockShape& shape : {kFine, least}) {
+    BlockHost fine;
+    rc = build_blocks_host(n, n_gather, off, nbr, shape, &fine, &err);
+    if (rc == DMM_ERR_CAPACITY) continue;
+    if (rc) return set_err(nullptr, rc, "%s", err.c_str());
+    std::vector<float> again(std::max<int64_t>(1, n), 0.0f);
+    if ((rc = check_blocks(fine, shape, n, n_gather, off, contrib, again.data()))) return rc;
+    if (n > 0 && std::memcmp(again.data(), incoming, sizeof(float) * n) != 0)
+      return set_err(nullptr, DMM_ERR_GRAPH, "block layout: fine and coarse sums differ");
+  }
+  stats[0] = bh.n_windows;
   stats[1] = bh.n_buckets;
   stats[2] = static_cast<int64_t>(bh.units.size());
   stats[3] = static_cast<int64_t>(bh.splits.size());
