@@ -33,6 +33,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 namespace dmm {
@@ -56,6 +57,7 @@ struct BCtrl {
   int sweeps;
   int error;
   int pad;
+  uint64_t live;                      // lanes with a vertex in F[level]
   int level_kind[DMM_MAX_STEPS];
   long long level_active[DMM_MAX_STEPS];
 };
@@ -80,6 +82,8 @@ struct BArgs {
   int64_t m;          // directed edges of the block (td threshold base)
   int td_div;
   int undirected;     // in-CSR == out-CSR
+  const int32_t* heavy;       // rows by in-degree class, longest first:
+  int64_t n_giant, n_wide;    // the leading ones of kSweepGiant and, after them, kSweepWide in-edges and more
 };
 
 struct TdLds {
@@ -92,6 +96,7 @@ struct TdLds {
 
 struct SmallLds {
   int64_t red[kPartWidth][kThreads / 64];
+  uint64_t found[2][kThreads / 64];
   int64_t scan_c[kThreads / 64 + 1];
   int64_t scan_d[kThreads / 64 + 1];
 };
@@ -100,6 +105,35 @@ union BLds {
   TdLds td;
   SmallLds sm;
 };
+
+// The OR of x over the wavefront, in every lane.
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ uint64_t dpp_or(uint64_t x) {
+  const unsigned lo = __builtin_amdgcn_update_dpp(0u, static_cast<unsigned>(x), kCtrl, kRowMask, 0xf, true);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0u, static_cast<unsigned>(x >> 32), kCtrl, kRowMask, 0xf, true);
+  return x | (static_cast<uint64_t>(hi) << 32) | lo;
+}
+__device__ __forceinline__ uint64_t wave_or(uint64_t x) {
+  x = dpp_or<0x111, 0xf>(x);  // row_shr:1
+  x = dpp_or<0x112, 0xf>(x);  // row_shr:2
+  x = dpp_or<0x114, 0xf>(x);  // row_shr:4
+  x = dpp_or<0x118, 0xf>(x);  // row_shr:8
+  x = dpp_or<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3
+  x = dpp_or<0x143, 0xc>(x);  // row_bcast:31 into rows 2 and 3
+  return (static_cast<uint64_t>(static_cast<unsigned>(__builtin_amdgcn_readlane(static_cast<int>(x >> 32), 63))) << 32) |
+         static_cast<unsigned>(__builtin_amdgcn_readlane(static_cast<int>(x), 63));
+}
+// ... over the workgroup; scratch: one word per wavefront, in LDS.
+template <int kBlock>
+__device__ __forceinline__ uint64_t block_or(uint64_t x, uint64_t* scratch) {
+  x = wave_or(x);
+  if (lane_id() == 0) scratch[threadIdx.x >> 6] = x;
+  __syncthreads();
+  x = 0;
+  for (int w = 0; w < kBlock / 64; w++) x |= scratch[w];
+  __syncthreads();
+  return x;
+}
 
 __device__ void zero_next_next(const BArgs& a, int level) {
   // F[level + 2] is written by atomics if level + 1 runs top-down.  Its
@@ -261,6 +295,49 @@ __device__ __forceinline__ int64_t sweep_row(const int32_t* __restrict__ in_nbr,
   return stop;
 }
 
+// Rows beyond kSweepWide in-edges: by a wavefront (kWaves 1) or a workgroup
+// (its kWaves), kWideUnroll edges per lane and round, stopping as soon as
+// every needed lane is found.  An 8-lane group took 256 edges a round, so a
+// hub's row was the sweep: 318 us for one level of a Kronecker-17 batch.
+constexpr int kWideUnroll = 8;
+template <int kWaves>
+__device__ __forceinline__ int64_t wide_row(const int32_t* __restrict__ in_nbr, int64_t b, int64_t e, uint64_t need,
+                                            const uint64_t* __restrict__ front, uint64_t (*red)[kThreads / 64],
+                                            int& buf, uint64_t* found) {
+  constexpr int64_t kRound = int64_t(kWaves) * 64 * kWideUnroll;
+  const int t = kWaves == 1 ? lane_id() : static_cast<int>(threadIdx.x);
+  uint64_t acc = 0;
+  int64_t k0 = b;
+  for (; k0 < e; k0 += kRound) {
+    int32_t v[kWideUnroll];
+#pragma unroll
+    for (int j = 0; j < kWideUnroll; j++) {
+      const int64_t k = k0 + j * (kWaves * 64) + t;
+      v[j] = in_nbr[min(k, e - 1)];  // past the end the last edge again
+    }
+    uint64_t x = 0;
+#pragma unroll
+    for (int j = 0; j < kWideUnroll; j++) x |= front[v[j]];
+    x = wave_or(x);
+    if (kWaves > 1) {
+      // The words alternate, so one barrier separates their uses.
+      if (lane_id() == 0) red[buf][threadIdx.x >> 6] = x;
+      __syncthreads();
+      x = 0;
+#pragma unroll
+      for (int w = 0; w < kWaves; w++) x |= red[buf][w];
+      buf ^= 1;
+    }
+    acc |= x;
+    if ((acc & need) == need) {
+      k0 += kRound;
+      break;
+    }
+  }
+  *found = acc & need;
+  return min(k0, e);
+}
+
 __device__ void bu_phase(const BArgs& a, BCtrl* c, SmallLds& L, int level) {
   const uint64_t* __restrict__ Fl = a.levels + level * a.nloc;
   uint64_t* __restrict__ Fn = a.levels + (level + 1) * a.nloc;
@@ -269,7 +346,46 @@ __device__ void bu_phase(const BArgs& a, BCtrl* c, SmallLds& L, int level) {
   const int sub = threadIdx.x & (kGroup - 1);
   const int64_t grp = (int64_t(blockIdx.x) * kThreads + threadIdx.x) / kGroup;
   const int64_t ngrp = (int64_t(gridDim.x) * kThreads) / kGroup;
+  // A lane whose frontier is empty finds nothing any more: rows out of its
+  // reach do not look for it (a source in a small component would have every
+  // sweep read every edge).
+  const uint64_t lanes = a.lanes & c->live;
+  uint64_t any = 0;  // lanes found
   int64_t scanned = 0, cnt = 0, degs = 0;
+  // The wide rows first: giant ones by a workgroup, the others by a
+  // wavefront, neighbouring ones by different workgroups.
+  int buf = 0;
+  auto wide = [&](int64_t u, auto waves, bool writer) {
+    const uint64_t fl = Fl[u], s = a.seen[u] | fl;
+    const uint64_t need = lanes & ~s;
+    uint64_t nxt = 0;
+    int64_t ex = 0;
+    if (need) {
+      const int64_t b = in_off[u];
+      ex = wide_row<waves.value>(in_nbr, b, in_off[u + 1], need, Fl, L.found, buf, &nxt) - b;
+    }
+    if (writer) {
+      scanned += ex;
+      Fn[u] = nxt;
+      any |= nxt;
+      if (fl | nxt) a.seen[u] = s | nxt;
+      const int64_t d = nxt ? a.out_off[u + 1] - a.out_off[u] : 0;
+      if (d > 0) {
+        cnt++;
+        degs += d;
+      }
+    }
+  };
+  for (int64_t i = blockIdx.x; i < a.n_giant; i += gridDim.x) {
+    // Every thread reads the row's seen word before a barrier that the writer
+    // passes before it writes; without one (nothing needed) the word written
+    // leaves nothing needed either.
+    wide(a.heavy[i], std::integral_constant<int, kThreads / 64>(), threadIdx.x == 0);
+    __syncthreads();
+  }
+  for (int64_t i = int64_t(threadIdx.x >> 6) * gridDim.x + blockIdx.x; i < a.n_wide;
+       i += int64_t(gridDim.x) * (kThreads / 64))
+    wide(a.heavy[a.n_giant + i], std::integral_constant<int, 1>(), lane_id() == 0);
   // Rows from bend on have no in-edges; their F[L + 1] words stay zero.
   // A group loads its next row's words and bounds at the start of the
   // current row and waits for them before the current row's stores: on
@@ -293,12 +409,13 @@ __device__ void bu_phase(const BArgs& a, BCtrl* c, SmallLds& L, int level) {
   };
   auto row = [&](int64_t u, const RowHead& h, RowHead& hn) {
     hn = load_head(u + ngrp);
+    if (h.e - h.b >= kSweepWide) return;  // a wide row
     const uint64_t s = h.seen | h.fl;
-    const uint64_t need = a.lanes & ~s;
+    const uint64_t need = lanes & ~s;
     uint64_t nxt = 0;
     if (need && h.e > h.b) {
       const int64_t stop = sweep_row<kSweepUnroll>(in_nbr, h.b, h.e, sub, need, Fl, nullptr, nullptr, &nxt);
-      scanned += stop - h.b;
+      if (sub == 0) scanned += stop - h.b;
     }
     // Out-degree of a found row: its in-row length when in-CSR == out-CSR.
     int64_t d = 0;
@@ -306,6 +423,7 @@ __device__ void bu_phase(const BArgs& a, BCtrl* c, SmallLds& L, int level) {
     __asm__ volatile("" ::"v"(hn.seen), "v"(hn.fl), "v"(hn.b), "v"(hn.e) : "memory");
     if (sub == 0) {
       Fn[u] = nxt;
+      any |= nxt;
       if (h.fl | nxt) a.seen[u] = s | nxt;
       if (d > 0) {
         cnt++;
@@ -323,17 +441,17 @@ __device__ void bu_phase(const BArgs& a, BCtrl* c, SmallLds& L, int level) {
     row(u, hb, ha);
     u += ngrp;
   }
-  // Each group counted its scan in every lane; keep one lane's count.
-  if (sub != 0) scanned = 0;
+  __syncthreads();  // the giant rows' words are read
   const int64_t s0 = block_sum<kThreads>(scanned, L.red[0]);
   const int64_t s1 = block_sum<kThreads>(cnt, L.red[1]);
   const int64_t s2 = block_sum<kThreads>(degs, L.red[2]);
+  const uint64_t s3 = block_or<kThreads>(any, L.found[0]);
   if (threadIdx.x == 0) {
     int64_t* p = a.part + blockIdx.x * kPartWidth;
     p[0] = s0;
     p[1] = s1;
     p[2] = s2;
-    p[3] = 0;
+    p[3] = static_cast<int64_t>(s3);
   }
 }
 
@@ -350,8 +468,11 @@ __device__ void count_or_write(const BArgs& a, BCtrl* c, SmallLds& L, int level)
   const int64_t v0 = min(a.bend, int64_t(blockIdx.x) * vpb), v1 = min(a.bend, v0 + vpb);
   if (!kWrite) {
     int64_t cnt = 0, degs = 0;
+    uint64_t any = 0;
     for (int64_t u = v0 + threadIdx.x; u < v1; u += kThreads) {
-      if (Fl[u]) {
+      const uint64_t f = Fl[u];
+      any |= f;
+      if (f) {
         const int64_t d = a.out_off[u + 1] - a.out_off[u];
         if (d > 0) {
           cnt++;
@@ -361,12 +482,13 @@ __device__ void count_or_write(const BArgs& a, BCtrl* c, SmallLds& L, int level)
     }
     const int64_t sc = block_sum<kThreads>(cnt, L.red[0]);
     const int64_t sd = block_sum<kThreads>(degs, L.red[1]);
+    const uint64_t so = block_or<kThreads>(any, L.found[0]);
     if (threadIdx.x == 0) {
       int64_t* p = a.part + blockIdx.x * kPartWidth;
       p[0] = sc;
       p[1] = sd;
       p[2] = 0;
-      p[3] = 0;
+      p[3] = static_cast<int64_t>(so);
     }
     return;
   }
@@ -440,15 +562,18 @@ __global__ __launch_bounds__(kPostThreads) void k_bpost(BArgs a, int nblocks) {
   const int phase = c->phase;
   if (phase != kBTD && phase != kBBU && phase != kBCount && phase != kBWrite) return;
   int64_t s0 = 0, s1 = 0, s2 = 0;
+  uint64_t s3 = 0;
   if (phase == kBBU || phase == kBCount) {
     for (int b = threadIdx.x; b < nblocks; b += kPostThreads) {
       s0 += a.part[b * kPartWidth + 0];
       s1 += a.part[b * kPartWidth + 1];
       s2 += a.part[b * kPartWidth + 2];
+      s3 |= static_cast<uint64_t>(a.part[b * kPartWidth + 3]);
     }
     s0 = block_sum<kPostThreads>(s0, red[0]);
     s1 = block_sum<kPostThreads>(s1, red[1]);
     s2 = block_sum<kPostThreads>(s2, red[2]);
+    s3 = block_or<kPostThreads>(s3, reinterpret_cast<uint64_t*>(red[3]));
   }
   if (phase == kBCount) {
     int64_t carry_c = 0, carry_d = 0;
@@ -484,6 +609,7 @@ __global__ __launch_bounds__(kPostThreads) void k_bpost(BArgs a, int nblocks) {
       }
       return;
     }
+    c->live = s3;
     c->sweeps = c->sweeps + 1;
     c->sweep_scanned_total += s0;
     // A sweep's partials are not in vertex order: a top-down level next
@@ -494,6 +620,7 @@ __global__ __launch_bounds__(kPostThreads) void k_bpost(BArgs a, int nblocks) {
     return;
   }
   if (phase == kBCount) {
+    c->live = s3;
     c->acount = s0;
     c->aedges = s1;
     choose_next(a, c, s0, s1, true);
@@ -559,6 +686,7 @@ __global__ void k_binit2(BArgs a, const int32_t* srcs, int nsrc) {
   c->pend_cnt = cnt;
   c->pend_degs = degs;
   c->level = 0;
+  c->live = a.lanes;
   c->done = 0;
   c->cur = 0;
   c->nlevels = 1;
@@ -676,6 +804,9 @@ BArgs make_args(dmm_ctx* ctx, int nsrc, int td_div) {
   a.m = std::max<int64_t>(1, ctx->m_out);
   a.td_div = std::max(1, td_div);
   a.undirected = ctx->directed ? 0 : 1;
+  a.heavy = ctx->d_heavy;
+  a.n_giant = ctx->n_giant;
+  a.n_wide = ctx->n_wide;
   return a;
 }
 

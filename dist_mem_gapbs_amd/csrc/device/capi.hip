@@ -716,7 +716,15 @@ int dmm_graph_upload(dmm_ctx* ctx, int64_t num_nodes, int64_t vbegin, int64_t ve
     int64_t at[65] = {};
     for (int32_t r : heavy) at[cls(r) + 1]++;
     for (int c = 0; c < 64; c++) at[c + 1] += at[c];
-    for (int32_t r : heavy) by_class[at[cls(r)]++] = r;
+    ctx->n_giant = ctx->n_wide = 0;
+    for (int32_t r : heavy) {
+      by_class[at[cls(r)]++] = r;
+      const int64_t d = ioff[r + 1] - ioff[r];
+      if (d >= dmm::kSweepGiant)
+        ctx->n_giant++;
+      else if (d >= dmm::kSweepWide)
+        ctx->n_wide++;
+    }
   }
   if ((rc = A((void**)&ctx->d_heavy, sizeof(int32_t) * std::max<size_t>(1, heavy.size()), "heavy list"))) return rc;
   if (!heavy.empty())

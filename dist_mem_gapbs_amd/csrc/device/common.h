@@ -23,6 +23,13 @@ constexpr int kMaxGridPerCU = 32;   // upper bound of workgroups per CU
 constexpr int kPartWidth = 4;       // int64 partials per workgroup
 constexpr int kRecentSearches = 32; // searches sizing the device-loop chain
 constexpr int kHeadNbrs = 4;        // in-neighbours per row in the head array
+// Batched sweep: rows from here on by a wavefront, a workgroup (powers of
+// two, so that they lead the list by classes).  64 lanes on Kronecker graphs,
+// whole call: 131 K vertices 1108 us with 8-lane groups for all rows, 769
+// with 512 / 16384, 755 with 512 / 4096; 900 K vertices 4.29, 1.91, 1.87 ms.
+// 256 or 1024 for the first: within 2%.
+constexpr int64_t kSweepWide = 512;
+constexpr int64_t kSweepGiant = 4096;
 
 // What the host needs of a finished device-loop search, written by its
 // last kernel into mapped host memory (no copy back).
@@ -238,6 +245,7 @@ struct dmm_ctx {
   dmm::PrCtrl* h_prctrl = nullptr;
   int32_t* d_heavy = nullptr;    // vertices with in-degree >= heavy threshold, longest class first
   int64_t n_heavy = 0;
+  int64_t n_giant = 0, n_wide = 0;  // its leading rows of kSweepGiant and, after them, kSweepWide in-edges and more
   void* d_sitems = nullptr;      // serial mode: work items by workgroup
   int32_t* d_sstart = nullptr;   // ... first item of each workgroup (+ end)
   void* d_items = nullptr;       // PrItem list (compensated / FP64 modes)

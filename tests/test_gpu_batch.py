@@ -217,3 +217,32 @@ def test_block_level_edge_cases(dmm, orc):
         if b == 0:
             assert kinds == {L.DMM_STEP_TD, L.DMM_STEP_BU}
     ctx.close()
+
+
+@pytest.mark.parametrize("hub", [511, 512, 4095, 4096, 9000])
+@pytest.mark.parametrize("directed", [False, True])
+def test_batch_wide_rows_and_dead_lanes(dmm, orc, hub, directed):
+    """Rows at the edges of the sweep's row classes (an 8-lane group, a
+    wavefront, a workgroup), whose lanes come from few of their many
+    in-neighbours, beside small components whose lanes die early: rows out of
+    their reach stop looking for them, depths stay exact."""
+    rng = np.random.default_rng([hub, directed])
+    ring = np.arange(3000)
+    pairs = [np.stack((np.arange(3000, 3000 + hub), np.zeros(hub, np.int64)), 1),  # leaves -> hub 0
+             np.stack((ring, np.roll(ring, -1)), 1),
+             rng.integers(0, 3000, (9000, 2)),
+             np.stack((rng.integers(0, 3000, hub), np.arange(3000, 3000 + hub)), 1)]
+    base = 3000 + hub
+    for k in range(20):  # components of 1 .. 20 edges in a row
+        pairs.append(np.stack((np.arange(base, base + k + 1), np.arange(base + 1, base + k + 2)), 1))
+        base += k + 2
+    g = csr_from_pairs(dmm, np.concatenate(pairs), base, symmetrize=not directed)
+    og = orc.CSR.of(g)
+    srcs = np.concatenate((rng.integers(0, 3000 + hub, 40), rng.integers(3000 + hub, base, 24))).astype(np.int32)
+    with dmm.Context(0) as c:
+        c.upload(g)
+        for td_div in (1, 1000000):  # pushed and swept levels
+            depth, _ = c.bfs_batch64(srcs, td_div=td_div)
+            for i, s in enumerate(srcs):
+                ref = orc.bfs_depth(og, int(s))
+                assert np.array_equal(depth[i], np.where(ref < 0, 255, ref).astype(np.uint8)), (i, s, td_div)
