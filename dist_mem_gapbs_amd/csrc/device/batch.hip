@@ -728,6 +728,7 @@ __device__ __forceinline__ uint64_t depth_bytes(const uint64_t* m, int g) {
 // sets lane s in plane j when bit j of L is set); an unreached lane gets
 // every plane bit, so its byte comes out as 255.
 __global__ __launch_bounds__(kThreads) void k_bdepth(BArgs a, uint8_t* out, int nsrc, const int32_t* perm) {
+  if (a.ctrl->done != 1) return;  // levels are missing: queued again behind them
   const int nlev = a.ctrl->nlevels;
   const int64_t gtid = int64_t(blockIdx.x) * kThreads + threadIdx.x;
   const int64_t gsize = int64_t(gridDim.x) * kThreads;
@@ -761,6 +762,7 @@ __global__ __launch_bounds__(kThreads) void k_bdepth(BArgs a, uint8_t* out, int 
 // Sum over lanes of the out-degrees of reached vertices (GTEPS numerator).
 __global__ __launch_bounds__(kThreads) void k_breach(BArgs a) {
   __shared__ int64_t red[kThreads / 64];
+  if (a.ctrl->done != 1) return;  // levels are missing, and a WRITE may need the partials
   const int nlev = a.ctrl->nlevels;
   const int64_t gtid = int64_t(blockIdx.x) * kThreads + threadIdx.x;
   const int64_t gsize = int64_t(gridDim.x) * kThreads;
@@ -776,6 +778,7 @@ __global__ __launch_bounds__(kThreads) void k_breach(BArgs a) {
 
 __global__ __launch_bounds__(kThreads) void k_breach_sum(BArgs a, int nblocks, int64_t* out) {
   __shared__ int64_t red[kThreads / 64];
+  if (a.ctrl->done != 1) return;
   int64_t s = 0;
   for (int b = threadIdx.x; b < nblocks; b += kThreads) s += a.part[b * kPartWidth];
   s = block_sum<kThreads>(s, red);
@@ -1262,7 +1265,7 @@ int ensure_levels(dmm_ctx* ctx, int64_t cap) {
 
 }  // namespace
 
-size_t batch_ctrl_bytes() { return sizeof(BCtrl); }
+size_t batch_ctrl_bytes() { return sizeof(BCtrl) + sizeof(int64_t); }  // and, on the host, the reached edges
 
 int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth,
               const dmm_batch_params* params, dmm_batch_stats* stats) {
@@ -1323,18 +1326,36 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
       ctx->batch_graph_key = key;
     }
     BCtrl* h = reinterpret_cast<BCtrl*>(ctx->h_bctrl);
+    int64_t* h_reached = reinterpret_cast<int64_t*>(h + 1);
+    // What follows the levels is queued behind them, before it is known that
+    // they are done (it reads only the state they left): one wait for all,
+    // and again in the rare case that levels were missing.
+    auto finish = [&]() -> int {
+      DMM_HIP_CHECK(ctx, hipEventRecord(ctx->ev_b, ctx->stream));
+      if (want_depth) {
+        hipLaunchKernelGGL(k_bdepth, dim3(blocks), dim3(kThreads), 0, ctx->stream, a, ctx->d_bdepth, nsrc,
+                           ctx->relabeled ? static_cast<const int32_t*>(ctx->d_perm) : nullptr);
+        DMM_HIP_CHECK(ctx, hipEventRecord(ctx->ev_b, ctx->stream));
+      }
+      if (stats) {
+        hipLaunchKernelGGL(k_breach, dim3(blocks), dim3(kThreads), 0, ctx->stream, a);
+        hipLaunchKernelGGL(k_breach_sum, dim3(1), dim3(kThreads), 0, ctx->stream, a, blocks, ctx->d_scratch64);
+        DMM_HIP_CHECK(ctx, hipMemcpyAsync(h_reached, ctx->d_scratch64, sizeof(int64_t), hipMemcpyDeviceToHost,
+                                          ctx->stream));
+      }
+      DMM_HIP_CHECK(ctx, hipGetLastError());
+      DMM_HIP_CHECK(ctx, hipMemcpyAsync(h, ctx->d_bctrl, sizeof(BCtrl), hipMemcpyDeviceToHost, ctx->stream));
+      DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+      return DMM_OK;
+    };
     DMM_HIP_CHECK(ctx, hipEventRecord(ctx->ev_a, ctx->stream));
     DMM_HIP_CHECK(ctx, hipGraphLaunch(ctx->batch_graph, ctx->stream));
-    DMM_HIP_CHECK(ctx, hipEventRecord(ctx->ev_b, ctx->stream));
-    DMM_HIP_CHECK(ctx, hipMemcpyAsync(h, ctx->d_bctrl, sizeof(BCtrl), hipMemcpyDeviceToHost, ctx->stream));
-    DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+    if ((rc = finish())) return rc;
     int guard = 0;
     while (h->done == 0 && !h->error) {
       if (++guard > 100000) return set_err(ctx, DMM_ERR_STATE, "batched BFS did not terminate");
       DMM_HIP_CHECK(ctx, hipGraphLaunch(ctx->batch_cont, ctx->stream));
-      DMM_HIP_CHECK(ctx, hipEventRecord(ctx->ev_b, ctx->stream));
-      DMM_HIP_CHECK(ctx, hipMemcpyAsync(h, ctx->d_bctrl, sizeof(BCtrl), hipMemcpyDeviceToHost, ctx->stream));
-      DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+      if ((rc = finish())) return rc;
     }
     if (h->error) return set_err(ctx, DMM_ERR_STATE, "batched BFS active list invariant violated");
     if (h->done == 3) {
@@ -1346,14 +1367,8 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
       continue;
     }
     if (want_depth) {
-      hipLaunchKernelGGL(k_bdepth, dim3(blocks), dim3(kThreads), 0, ctx->stream, a, ctx->d_bdepth, nsrc,
-                         ctx->relabeled ? static_cast<const int32_t*>(ctx->d_perm) : nullptr);
-      DMM_HIP_CHECK(ctx, hipGetLastError());
-      DMM_HIP_CHECK(ctx, hipEventRecord(ctx->ev_b, ctx->stream));
-      if (depth)
-        DMM_HIP_CHECK(ctx, hipMemcpyAsync(depth, ctx->d_bdepth, int64_t(nsrc) * ctx->nloc, hipMemcpyDeviceToHost,
-                                          ctx->stream));
-      DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+      const ReadPart part = {depth, ctx->d_bdepth, static_cast<size_t>(int64_t(nsrc) * ctx->nloc)};
+      if (depth && (rc = read_out(ctx, &part, 1))) return rc;
       ctx->bdepth_nsrc = nsrc;
     }
     float ms = 0;
@@ -1376,15 +1391,7 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
     }
     ctx->batch_valid = true;
     ctx->batch_last_level = h->level;
-    if (stats) {
-      int64_t* out = ctx->d_scratch64;
-      hipLaunchKernelGGL(k_breach, dim3(blocks), dim3(kThreads), 0, ctx->stream, a);
-      hipLaunchKernelGGL(k_breach_sum, dim3(1), dim3(kThreads), 0, ctx->stream, a, blocks, out);
-      int64_t r = 0;
-      DMM_HIP_CHECK(ctx, hipMemcpyAsync(&r, out, sizeof(r), hipMemcpyDeviceToHost, ctx->stream));
-      DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-      stats->reached_edges = r;
-    }
+    if (stats) stats->reached_edges = *h_reached;
     return DMM_OK;
   }
   return set_err(ctx, DMM_ERR_CAPACITY, "batched BFS level storage could not be grown");
@@ -1393,10 +1400,8 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
 int batch_read_depth(dmm_ctx* ctx, uint8_t* depth) {
   if (!ctx->batch_valid || ctx->bdepth_nsrc <= 0)
     return set_err(ctx, DMM_ERR_STATE, "the last batched BFS wrote no depths");
-  DMM_HIP_CHECK(ctx, hipMemcpyAsync(depth, ctx->d_bdepth, int64_t(ctx->bdepth_nsrc) * ctx->nloc,
-                                    hipMemcpyDeviceToHost, ctx->stream));
-  DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-  return DMM_OK;
+  const ReadPart part = {depth, ctx->d_bdepth, static_cast<size_t>(int64_t(ctx->bdepth_nsrc) * ctx->nloc)};
+  return read_out(ctx, &part, 1);
 }
 
 int batch_read_level(dmm_ctx* ctx, int32_t level, uint64_t* words) {
@@ -1415,10 +1420,8 @@ int batch_read_level(dmm_ctx* ctx, int32_t level, uint64_t* words) {
                      ctx->relabeled ? static_cast<const int32_t*>(ctx->d_perm) : nullptr, ctx->nloc,
                      ctx->d_words_tmp);
   DMM_HIP_CHECK(ctx, hipGetLastError());
-  DMM_HIP_CHECK(ctx, hipMemcpyAsync(words, ctx->d_words_tmp, sizeof(uint64_t) * ctx->nloc, hipMemcpyDeviceToHost,
-                                    ctx->stream));
-  DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-  return DMM_OK;
+  const ReadPart part = {words, ctx->d_words_tmp, sizeof(uint64_t) * ctx->nloc};
+  return read_out(ctx, &part, 1);
 }
 
 int batch_block_level(dmm_ctx* ctx, const uint64_t* front, const uint64_t* seen, uint64_t* next,
@@ -1523,7 +1526,8 @@ int batch_block_level(dmm_ctx* ctx, const uint64_t* front, const uint64_t* seen,
   DMM_HIP_CHECK(ctx, hipGetLastError());
   int64_t scanned = 0;
   BlockCtrl hc;
-  DMM_HIP_CHECK(ctx, hipMemcpyAsync(next, ctx->d_bnext, sizeof(uint64_t) * ctx->nloc, hipMemcpyDeviceToHost, ctx->stream));
+  const ReadPart part = {next, ctx->d_bnext, sizeof(uint64_t) * ctx->nloc};
+  if ((rc = read_out(ctx, &part, 1))) return rc;
   DMM_HIP_CHECK(ctx, hipMemcpyAsync(&scanned, ctx->d_scratch64, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
   DMM_HIP_CHECK(ctx, hipMemcpyAsync(&hc, bc, sizeof(BlockCtrl), hipMemcpyDeviceToHost, ctx->stream));
   DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));

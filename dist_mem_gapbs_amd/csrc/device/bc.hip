@@ -695,14 +695,10 @@ int bc_read(dmm_ctx* ctx, int32_t* depth, uint64_t* path_counts, uint64_t* succ)
   if (!ctx->bc_valid) return set_err(ctx, DMM_ERR_STATE, "no Brandes forward result on the ctx");
   const int64_t n = ctx->nloc;
   const int64_t words = (ctx->m_out + 63) / 64;
-  hipStream_t s = ctx->stream;
-  if (depth) DMM_HIP_CHECK(ctx, hipMemcpyAsync(depth, ctx->d_bc_depth, sizeof(int32_t) * n, hipMemcpyDeviceToHost, s));
-  if (path_counts)
-    DMM_HIP_CHECK(ctx, hipMemcpyAsync(path_counts, ctx->d_bc_pc, sizeof(uint64_t) * n, hipMemcpyDeviceToHost, s));
-  if (succ && words > 0)
-    DMM_HIP_CHECK(ctx, hipMemcpyAsync(succ, ctx->d_bc_succ, sizeof(uint64_t) * words, hipMemcpyDeviceToHost, s));
-  DMM_HIP_CHECK(ctx, hipStreamSynchronize(s));
-  return DMM_OK;
+  const ReadPart parts[] = {{depth, ctx->d_bc_depth, sizeof(int32_t) * n},
+                            {path_counts, ctx->d_bc_pc, sizeof(uint64_t) * n},
+                            {succ, ctx->d_bc_succ, sizeof(uint64_t) * words}};
+  return read_out(ctx, parts, 3);
 }
 
 }  // namespace dmm

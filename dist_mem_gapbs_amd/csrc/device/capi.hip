@@ -128,7 +128,7 @@ void free_graph_state(dmm_ctx* ctx) {
                   ctx->d_contrib64[0], ctx->d_contrib64[1], ctx->d_err_part, ctx->d_heavy, ctx->d_sitems, ctx->d_sstart,
                   ctx->d_gcontrib, ctx->d_seen, ctx->d_levels, ctx->d_bact, ctx->d_baoff,
                   ctx->d_bdepth, ctx->d_items, ctx->d_supers, ctx->d_partial, ctx->d_perm, ctx->d_inv,
-                  ctx->d_parent_out, ctx->d_depth_out, ctx->d_score_out, ctx->d_score64_out,
+                  ctx->d_parent_out, ctx->d_score_out, ctx->d_score64_out,
                   ctx->d_words_tmp, ctx->d_gfront, ctx->d_bseen, ctx->d_bnext, ctx->d_gnz,
                   ctx->d_bsegs, ctx->d_head, ctx->d_poff, ctx->d_ptgt, ctx->d_flist, ctx->d_blkctrl,
                   ctx->d_bc_depth, ctx->d_bc_pc, ctx->d_bc_succ, ctx->d_bc_queue, ctx->d_bc_part,
@@ -440,7 +440,7 @@ int dmm_ctx_create(int32_t device, dmm_ctx** out) {
       hipHostMalloc((void**)&ctx->h_flags, sizeof(dmm::LoopFlags), hipHostMallocMapped) != hipSuccess ||
       hipHostGetDevicePointer(&ctx->hd_params, ctx->h_params, 0) != hipSuccess ||
       hipHostGetDevicePointer((void**)&ctx->hd_flags, ctx->h_flags, 0) != hipSuccess ||
-      hipHostMalloc((void**)&ctx->h_prctrl, sizeof(dmm::PrCtrl), hipHostMallocDefault) != hipSuccess ||
+      hipHostMalloc((void**)&ctx->h_prctrl, sizeof(dmm::PrCtrl) + sizeof(double) * DMM_MAX_PR_ITERS, hipHostMallocDefault) != hipSuccess ||
       hipHostMalloc(&ctx->h_prparams, dmm::kPrParamsBytes, hipHostMallocDefault) != hipSuccess ||
       hipHostMalloc(&ctx->h_bctrl, dmm::batch_ctrl_bytes(), hipHostMallocDefault) != hipSuccess ||
       hipHostMalloc(&ctx->h_bsrc, 64 * sizeof(int32_t), hipHostMallocDefault) != hipSuccess ||
@@ -465,6 +465,7 @@ void dmm_ctx_destroy(dmm_ctx* ctx) {
   (void)hipSetDevice(ctx->device);
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   free_graph_state(ctx);
+  dmm::read_free(ctx);
   void* bufs[] = {ctx->d_ctrl, ctx->d_params, ctx->d_scratch64, ctx->d_prctrl, ctx->d_prparams,
                   ctx->d_err_trace, ctx->d_bctrl, ctx->d_bsrc, ctx->d_part};
   for (void* p : bufs) dmm::dev_free(p);
@@ -632,9 +633,9 @@ int dmm_graph_upload(dmm_ctx* ctx, int64_t num_nodes, int64_t vbegin, int64_t ve
     dmm::degree_order(rows, out_offsets, &ctx->h_perm, &inv);
     if ((rc = A((void**)&ctx->d_perm, sizeof(int32_t) * rows, "layout permutation")) ||
         (rc = A((void**)&ctx->d_inv, sizeof(int32_t) * rows, "layout inverse")) ||
-        (rc = A((void**)&ctx->d_parent_out, sizeof(int32_t) * rows, "parent (original IDs)")) ||
-        (rc = A((void**)&ctx->d_depth_out, sizeof(int32_t) * rows, "depth (original IDs)")))
+        (rc = A((void**)&ctx->d_parent_out, 2 * sizeof(int32_t) * rows, "parent and depth (original IDs)")))
       return rc;
+    ctx->d_depth_out = ctx->d_parent_out + rows;  // read out in one piece
     DMM_HIP_CHECK(ctx, hipMemcpy(ctx->d_perm, ctx->h_perm.data(), sizeof(int32_t) * rows, hipMemcpyHostToDevice));
     DMM_HIP_CHECK(ctx, hipMemcpy(ctx->d_inv, inv.data(), sizeof(int32_t) * rows, hipMemcpyHostToDevice));
     if ((rc = dmm::relabel_upload(ctx, out_offsets, out_neighs, inv, &new_out_off, &ctx->d_out_off, &ctx->d_out_nbr)))
@@ -881,12 +882,8 @@ int dmm_bfs_read(dmm_ctx* ctx, int32_t* parent, int32_t* depth) {
     return set_err(ctx, DMM_ERR_STATE, "the last BFS did not track depths (pass a depth buffer to dmm_bfs)");
   const int32_t* dp = ctx->relabeled ? ctx->d_parent_out : ctx->d_parent;
   const int32_t* dd = ctx->relabeled ? ctx->d_depth_out : ctx->d_depth;
-  if (parent)
-    DMM_HIP_CHECK(ctx, hipMemcpyAsync(parent, dp, sizeof(int32_t) * ctx->nloc, hipMemcpyDeviceToHost, ctx->stream));
-  if (depth)
-    DMM_HIP_CHECK(ctx, hipMemcpyAsync(depth, dd, sizeof(int32_t) * ctx->nloc, hipMemcpyDeviceToHost, ctx->stream));
-  DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-  return DMM_OK;
+  const dmm::ReadPart parts[] = {{parent, dp, sizeof(int32_t) * ctx->nloc}, {depth, dd, sizeof(int32_t) * ctx->nloc}};
+  return dmm::read_out(ctx, parts, 2);
 }
 
 int dmm_step_init(dmm_ctx* ctx, int32_t source) {
@@ -1121,12 +1118,11 @@ int dmm_pr_pull(dmm_ctx* ctx, int32_t max_iters, double epsilon, int32_t mode, v
   std::memset(st, 0, sizeof(*st));
   if ((rc = dmm::pr_run(ctx, max_iters, epsilon, mode, st))) return rc;
   if (scores) {
-    if (mode == DMM_PR_FP64)
-      DMM_HIP_CHECK(ctx, hipMemcpy(scores, ctx->relabeled ? ctx->d_score64_out : ctx->d_score64,
-                                   sizeof(double) * ctx->nloc, hipMemcpyDeviceToHost));
-    else
-      DMM_HIP_CHECK(ctx, hipMemcpy(scores, ctx->relabeled ? ctx->d_score_out : ctx->d_score,
-                                   sizeof(float) * ctx->nloc, hipMemcpyDeviceToHost));
+    const bool d = mode == DMM_PR_FP64;
+    const void* src = ctx->relabeled ? (d ? static_cast<void*>(ctx->d_score64_out) : ctx->d_score_out)
+                                     : (d ? static_cast<void*>(ctx->d_score64) : ctx->d_score);
+    const dmm::ReadPart part = {scores, src, (d ? sizeof(double) : sizeof(float)) * ctx->nloc};
+    if ((rc = dmm::read_out(ctx, &part, 1))) return rc;
   }
   st->host_ms = now_ms() - t0;
   return DMM_OK;

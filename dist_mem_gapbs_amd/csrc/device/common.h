@@ -98,6 +98,8 @@ enum : int {
   kPhaseDone = 5,
 };
 
+constexpr int kReadSlots = 8;  // pieces of a read in flight (readout.hip)
+
 struct PrCtrl {
   double err;          // L1 change of the last iteration
   unsigned int ticket; // iterations run
@@ -243,6 +245,9 @@ struct dmm_ctx {
   int64_t err_part_cap = 0;
   dmm::PrCtrl* d_prctrl = nullptr;
   dmm::PrCtrl* h_prctrl = nullptr;
+  char* h_ring = nullptr;        // pinned staging of reads (readout.hip)
+  size_t ring_bytes = 0;
+  hipEvent_t ring_events[dmm::kReadSlots] = {};
   int32_t* d_heavy = nullptr;    // vertices with in-degree >= heavy threshold, longest class first
   int64_t n_heavy = 0;
   int64_t n_giant = 0, n_wide = 0;  // its leading rows of kSweepGiant and, after them, kSweepWide in-edges and more
@@ -314,6 +319,16 @@ int set_err(dmm_ctx* ctx, int code, const char* fmt, ...);
 // Device allocation that records failures as DMM_ERR_NOMEM.
 int dev_alloc(dmm_ctx* ctx, void** p, size_t bytes, const char* what);
 void dev_free(void* p);
+
+// Copies results to the caller's buffers (a part without one is skipped)
+// behind everything queued on the stream; returns when they have arrived.
+struct ReadPart {
+  void* dst;
+  const void* src;
+  size_t bytes;
+};
+int read_out(dmm_ctx* ctx, const ReadPart* parts, int nparts);
+void read_free(dmm_ctx* ctx);
 
 // A transient device buffer; its bytes count towards the context's device
 // memory only while it is held.

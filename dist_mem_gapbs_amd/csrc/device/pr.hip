@@ -1978,6 +1978,12 @@ int pr_run(dmm_ctx* ctx, int32_t max_iters, double epsilon, int32_t mode, dmm_pr
   DMM_HIP_CHECK(ctx, hipEventRecord(ctx->ev_b, ctx->stream));
   DMM_HIP_CHECK(ctx, hipMemcpyAsync(ctx->h_prctrl, ctx->d_prctrl, sizeof(PrCtrl), hipMemcpyDeviceToHost,
                                     ctx->stream));
+  // The error trace too: one wait for both.
+  double* h_trace = reinterpret_cast<double*>(ctx->h_prctrl + 1);
+  const int trace = std::min(max_iters, DMM_MAX_PR_ITERS);
+  if (stats && trace > 0)
+    DMM_HIP_CHECK(ctx, hipMemcpyAsync(h_trace, ctx->d_err_trace, sizeof(double) * trace, hipMemcpyDeviceToHost,
+                                      ctx->stream));
   DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
   ctx->pr_mode = mode;
   if (stats) {
@@ -1987,9 +1993,7 @@ int pr_run(dmm_ctx* ctx, int32_t max_iters, double epsilon, int32_t mode, dmm_pr
     stats->iters = iters;
     stats->total_ms = ms;
     stats->iter_ms = iters > 0 ? ms / iters : 0;
-    const int nt = std::min(iters, DMM_MAX_PR_ITERS);
-    if (nt > 0)
-      DMM_HIP_CHECK(ctx, hipMemcpy(stats->err, ctx->d_err_trace, sizeof(double) * nt, hipMemcpyDeviceToHost));
+    std::copy(h_trace, h_trace + std::min(iters, trace), stats->err);
     const int64_t m = ctx->m_in, nl = ctx->nloc;
     stats->alg_bytes_per_iter = (mode == DMM_PR_FP64) ? 12 * m + 32 * nl + 8 : 8 * m + 20 * nl + 8;
   }

@@ -1,0 +1,44 @@
+"""Results read out through the pinned ring: sizes around one piece, several
+pieces, helper threads and the ring's reuse arrive whole, from runs of
+different sizes on one context, also into buffers at odd addresses."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import dist_mem_gapbs_amd._lib as L
+
+pytestmark = pytest.mark.gpu
+
+
+def _graph(dmm, n):
+    rng = np.random.default_rng(n)
+    return dmm.from_edgelist(rng.integers(0, n, (8 * n, 2)).astype(np.int32), n)
+
+
+# 64 lanes of n bytes: up to 512 KB in one piece, from 2 MB on with helpers,
+# beyond 16 MB with slots used again.
+@pytest.mark.parametrize("n", [100, 8191, 8192, 8193, 16384, 16385, 32767, 32769, 262144, 262147, 450001])
+def test_batch_depths_arrive_whole(dmm, orc, n):
+    g = _graph(dmm, n)
+    og = orc.CSR.of(g)
+    srcs = dmm.pick_sources(g, 64)
+    with dmm.Context(0) as c:
+        c.upload(g)
+        out = np.empty(64 * n + 3, np.uint8)[3:]  # an odd address
+        rc = c._lib.dmm_bfs_batch64(c._h, L.ptr(srcs, C.c_int32), 64, L.ptr(out, C.c_uint8), None, None)
+        assert rc == 0
+        depth = out.reshape(64, n)
+        for i in range(0, 64, 7 if n > 100000 else 1):
+            ref = orc.bfs_depth(og, int(srcs[i]))
+            assert np.array_equal(depth[i], np.where(ref < 0, 255, ref).astype(np.uint8))
+        assert np.array_equal(c.batch_read_depth(64), depth)
+        # A smaller and a two-part read behind it.
+        parent, d, _ = c.DOBFS(int(srcs[0]))
+        ref = orc.bfs_depth(og, int(srcs[0]))
+        assert np.array_equal(d, ref)
+        assert orc.bfs_verify(og, int(srcs[0]), parent)[0]
+        only, none = c.bfs_read(depth=False)
+        assert none is None and np.array_equal(only, parent)
+        _, only = c.bfs_read(parent=False)
+        assert np.array_equal(only, ref)
