@@ -326,6 +326,7 @@ struct ReadPart {
   void* dst;
   const void* src;
   size_t bytes;
+  bool joined = false;  // src follows the previous part's in the same allocation
 };
 int read_out(dmm_ctx* ctx, const ReadPart* parts, int nparts);
 void read_free(dmm_ctx* ctx);

@@ -38,6 +38,7 @@ struct Piece {
   char* dst;
   const char* src;
   size_t bytes;
+  bool joined;
 };
 
 }  // namespace
@@ -66,7 +67,9 @@ static int read_pieces(dmm_ctx* ctx, const ReadPart* parts, int nparts) {
     if (!parts[i].dst) continue;
     char* d = static_cast<char*>(parts[i].dst);
     const char* s = static_cast<const char*>(parts[i].src);
-    for (size_t o = 0; o < parts[i].bytes; o += slot) pieces.push_back({d + o, s + o, std::min(slot, parts[i].bytes - o)});
+    const bool joined = parts[i].joined && i > 0 && parts[i - 1].dst;
+    for (size_t o = 0; o < parts[i].bytes; o += slot)
+      pieces.push_back({d + o, s + o, std::min(slot, parts[i].bytes - o), joined && o == 0});
   }
   const int n = static_cast<int>(pieces.size());
   // Slot s holds the pieces s, s + slots, ...  The ring grows to what a read
@@ -97,12 +100,13 @@ static int read_pieces(dmm_ctx* ctx, const ReadPart* parts, int nparts) {
     return DMM_OK;
   }
   if (total <= kSmallRead) {
-    // Parts that follow one another in device memory come in one piece.
+    // Joined parts come in one piece.  (That two parts' addresses follow one
+    // another does not say so: a copy must not span allocations.)
     size_t at = 0;
     for (int i = 0; i < n;) {
       size_t run = pieces[i].bytes;
       int j = i + 1;
-      for (; j < n && pieces[j].src == pieces[i].src + run; j++) run += pieces[j].bytes;
+      for (; j < n && pieces[j].joined; j++) run += pieces[j].bytes;
       DMM_HIP_CHECK(ctx, hipMemcpyAsync(ctx->h_ring + at, pieces[i].src, run, hipMemcpyDeviceToHost, ctx->stream));
       at += run;
       i = j;

@@ -42,3 +42,20 @@ def test_batch_depths_arrive_whole(dmm, orc, n):
         assert none is None and np.array_equal(only, parent)
         _, only = c.bfs_read(parent=False)
         assert np.array_equal(only, ref)
+
+
+# Whole pages: allocations of these sizes may follow one another in device
+# memory, and a copy must not run from one into the next.
+@pytest.mark.parametrize("n", [1024, 2048, 4096, 8192])
+def test_parts_of_separate_allocations(dmm, orc, n):
+    g = _graph(dmm, n)
+    og = orc.CSR.of(g)
+    s = int(dmm.pick_sources(g, 1)[0])
+    with dmm.Context(0) as c:
+        c.set_layout(L.DMM_LAYOUT_NATURAL)
+        c.upload(g)
+        depth, counts, _, _ = c.bc_forward(s)
+        assert np.array_equal(depth, orc.bfs_depth(og, s))
+        assert counts[s] == 1 and (counts[depth > 0] > 0).all()
+        parent, depth, _ = c.DOBFS(s)
+        assert np.array_equal(depth, orc.bfs_depth(og, s)) and orc.bfs_verify(og, s, parent)[0]
