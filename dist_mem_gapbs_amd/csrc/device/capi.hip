@@ -300,10 +300,10 @@ int ensure_pr_state(dmm_ctx* ctx, int mode) {
                           dmm::pr_row_blocks(ctx)) +
         dmm::pr_super_blocks(ctx);
     const int64_t bparts = dmm::pr_bsum_blocks(ctx) + dmm::pr_bsplit_blocks(ctx);
-    if ((rc = dmm::dev_alloc(ctx, (void**)&ctx->d_err_part, sizeof(double) * std::max(parts, bparts),
+    ctx->err_part_half = std::max(parts, bparts);  // iterations alternate between two halves
+    if ((rc = dmm::dev_alloc(ctx, (void**)&ctx->d_err_part, 2 * sizeof(double) * ctx->err_part_half,
                              "error partials")))
       return rc;
-    ctx->err_part_cap = std::max(parts, bparts);
   }
   return DMM_OK;
 }

@@ -242,7 +242,7 @@ struct dmm_ctx {
   int32_t n_windows = 0;
   // Rows of the light loop and the in-degree-0 tail (see the upload).
   int64_t pr_light_begin = 0, pr_light_end = 0, pr_zero_begin = 0;
-  int64_t err_part_cap = 0;
+  int64_t err_part_half = 0;  // entries of each of d_err_part's two halves
   dmm::PrCtrl* d_prctrl = nullptr;
   dmm::PrCtrl* h_prctrl = nullptr;
   char* h_ring = nullptr;        // pinned staging of reads (readout.hip)

@@ -74,6 +74,49 @@ struct PrArgs {
   const PrParams* prm;
 };
 
+// What an iteration's first kernel needs of the iteration before.
+struct PrPrev {
+  const double* part;   // its error partials
+  int parts;
+  int it;               // this iteration's number: 0 has none before it
+  PrCtrl* ctrl;
+  double* err_trace;
+  const PrParams* prm;
+};
+
+// Start of an iteration's first kernel: every workgroup sums the previous
+// iteration's error partials in the same order and stops if that iteration
+// converged (src/pr.cc:66-68); workgroup 0 records the error and the stop
+// decision for the kernels that follow.  ctrl->ticket counts the iterations
+// run; ctrl->pad != 0 marks convergence and turns the remaining captured
+// iterations into no-ops.  A kernel of its own for this took 5 us an
+// iteration.  scratch: kBlock / 64 + 1 doubles of LDS, free again on return.
+template <int kBlock>
+__device__ __forceinline__ bool pr_begin(const PrPrev& p, double* scratch) {
+  if (p.it == 0) return true;
+  double x = 0;
+  for (int i = threadIdx.x; i < p.parts; i += kBlock) x += p.part[i];
+  // Workgroup 0 may be writing the mark: one thread reads it for all.
+  const double mark = threadIdx.x == 0 && p.ctrl->pad ? 1.0 : 0.0;
+  x = wave_sum(x);
+  if (lane_id() == 0) scratch[threadIdx.x >> 6] = x;
+  if (threadIdx.x == 0) scratch[kBlock / 64] = mark;
+  __syncthreads();
+  double t = 0;
+  for (int w = 0; w < kBlock / 64; w++) t += scratch[w];
+  const bool over = scratch[kBlock / 64] != 0.0;
+  __syncthreads();
+  if (over) return false;
+  const bool converged = t < p.prm->eps;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    p.ctrl->err = t;
+    p.ctrl->ticket = p.it;
+    if (p.it <= DMM_MAX_PR_ITERS) p.err_trace[p.it - 1] = t;
+    if (converged) p.ctrl->pad = 1;
+  }
+  return !converged;
+}
+
 __device__ __forceinline__ void two_sum(float a, float b, float& s, float& e) {
   s = a + b;
   const float bb = s - a;
@@ -378,7 +421,7 @@ struct SerialLds {
   float stage[kSerialWaves][kStageFloats];
   unsigned p0[2][kSerialWaves], p1[2][kSerialWaves];
   float sum[2];
-  double red[kSerialWaves];
+  double red[kSerialWaves + 1];
 };
 static_assert(sizeof(SerialLds) <= 160 * 1024, "one workgroup per CU");
 
@@ -507,10 +550,10 @@ __device__ __forceinline__ float serial_bundle(const int32_t* __restrict__ nbr, 
 // One iteration, one workgroup per CU: it fills its hub, takes its very long
 // rows, its wavefronts take the rest of its items in turn, and the rows
 // without in-edges go to all threads.
-__global__ __launch_bounds__(kSerialThreads) void k_serial(PrArgs a, const float* __restrict__ cin,
+__global__ __launch_bounds__(kSerialThreads) void k_serial(PrArgs a, PrPrev prev, const float* __restrict__ cin,
                                                            float* __restrict__ cout, float* __restrict__ score) {
   __shared__ SerialLds L;
-  if (a.ctrl->pad) return;  // converged
+  if (!pr_begin<kSerialThreads>(prev, L.red)) return;
   const SerialHub hub{L.hub, a.serial_hub};
   if (hub.n > 0) lds_fill<float, kSerialHub * 4, kSerialThreads>(L.hub, cin, hub.n);
   if (threadIdx.x == 0) L.hub[kSerialHub] = 0.0f;
@@ -631,11 +674,11 @@ __device__ __forceinline__ double finish_t(const PrArgs& a, int64_t lu, double i
 }
 
 template <typename T>
-__global__ __launch_bounds__(kFusedThreads) void k_fused(PrArgs a, const T* __restrict__ cin,
+__global__ __launch_bounds__(kFusedThreads) void k_fused(PrArgs a, PrPrev prev, const T* __restrict__ cin,
                                                          T* __restrict__ cout, T* __restrict__ score) {
   __shared__ T hub[kHubBytes / sizeof(T)];
-  __shared__ double red[kFusedThreads / 64];
-  if (a.ctrl->pad) return;  // converged
+  __shared__ double red[kFusedThreads / 64 + 1];
+  if (!pr_begin<kFusedThreads>(prev, red)) return;
   const int hub_n = static_cast<int>(min<int64_t>(kHubBytes / sizeof(T), a.n_gather));
   lds_fill<T, kHubBytes>(hub, cin, hub_n);
   __syncthreads();
@@ -868,11 +911,11 @@ __device__ __forceinline__ void chunk_ready(const ChunkLoad& l) {
 // contributions into LDS at a time and its wavefronts take the window's
 // chunks in turn, each loading its next chunk before it sums the current.
 template <int kWin>
-__global__ __launch_bounds__(kTileThreads) void k_tile(TileArgs t, const float* __restrict__ cin, int64_t n_gather,
-                                                      const PrCtrl* ctrl) {
+__global__ __launch_bounds__(kTileThreads) void k_tile(TileArgs t, PrPrev prev, const float* __restrict__ cin,
+                                                      int64_t n_gather) {
   __shared__ float win[kWin];
-  __shared__ float stage_all[kTileThreads / 64][kChunkPieces];
-  if (ctrl->pad) return;  // converged
+  __shared__ __align__(8) float stage_all[kTileThreads / 64][kChunkPieces];
+  if (!pr_begin<kTileThreads>(prev, reinterpret_cast<double*>(stage_all))) return;
   const int64_t per = (t.n_chunks + gridDim.x - 1) / gridDim.x;
   const int64_t c0 = min(t.n_chunks, int64_t(blockIdx.x) * per), c1 = min(t.n_chunks, c0 + per);
   const int lane = lane_id();
@@ -1662,10 +1705,8 @@ __global__ __launch_bounds__(kThreads) void k_bsplit(PrArgs a, BpArgs b, float* 
 
 // ---- iteration bookkeeping --------------------------------------------------
 
-// Sums the error partials in a fixed order; records the error and the stop
-// decision (src/pr.cc:66-68).  ctrl->pad != 0 marks convergence and turns
-// the remaining captured iterations into no-ops; ctrl->ticket counts
-// iterations run.
+// The last iteration's error (the others' are reduced by the kernel that
+// follows them, pr_begin).
 __global__ __launch_bounds__(kThreads) void k_reduce(PrArgs a) {
   __shared__ double red[kThreads / 64];
   PrCtrl* c = a.ctrl;
@@ -1753,28 +1794,44 @@ PrArgs make_args(dmm_ctx* ctx) {
   return a;
 }
 
-// One iteration on ctx->stream.  With gcontrib (a PE block's iteration from
+// Error partials an iteration of `mode` writes (block: a PE block's iteration
+// from the global contributions).
+int pr_error_parts(dmm_ctx* ctx, int mode, bool block) {
+  if (mode == DMM_PR_FP32_SERIAL) return pr_serial_blocks(ctx);
+  if (mode == DMM_PR_FP32_KAHAN && block && ctx->bp_ready) return pr_bsum_blocks(ctx) + pr_bsplit_blocks(ctx);
+  if (mode == DMM_PR_FP32_KAHAN && !block && ctx->tiles_ready) return pr_row_blocks(ctx);
+  return pr_fused_blocks(ctx) + pr_super_blocks(ctx);
+}
+
+// One iteration on ctx->stream; the last one also reduces its own error.
+// With gcontrib (a PE block's iteration from
 // the global contribution vector) the FP32 modes may write the scores and
 // the block's new contributions to score_out / contrib_out instead of the
 // context's own buffers.
-void launch_iteration(dmm_ctx* ctx, PrArgs a, int mode, int it, const void* gcontrib, float* score_out = nullptr,
-                      float* contrib_out = nullptr) {
+void launch_iteration(dmm_ctx* ctx, PrArgs a, int mode, int it, bool last, const void* gcontrib,
+                      float* score_out = nullptr, float* contrib_out = nullptr) {
   hipStream_t s = ctx->stream;
   const int sb = a.super_blocks;
+  // The error partials alternate between two halves: a kernel that writes its
+  // own may still be reading the previous iteration's.
+  double* const part0 = a.err_part;
+  PrPrev prev{part0 + (it & 1 ? 0 : ctx->err_part_half), 0, it, a.ctrl, a.err_trace, a.prm};
+  if (it & 1) a.err_part = part0 + ctx->err_part_half;
+  prev.parts = pr_error_parts(ctx, mode, gcontrib != nullptr);
   float* const score_f = score_out ? score_out : ctx->d_score;
   if (mode == DMM_PR_FP32_SERIAL) {
     const float* cin = gcontrib ? static_cast<const float*>(gcontrib) : ctx->d_contrib[it & 1];
     float* cout = contrib_out ? contrib_out : ctx->d_contrib[(it + 1) & 1];
     a.main_blocks = pr_serial_blocks(ctx);
     a.super_blocks = 0;
-    hipLaunchKernelGGL(k_serial, dim3(a.main_blocks), dim3(kSerialThreads), 0, s, a, cin, cout, score_f);
+    hipLaunchKernelGGL(k_serial, dim3(a.main_blocks), dim3(kSerialThreads), 0, s, a, prev, cin, cout, score_f);
   } else {
     const int fb = pr_fused_blocks(ctx);
     a.main_blocks = fb;
     if (mode == DMM_PR_FP64) {
       const double* cin = gcontrib ? static_cast<const double*>(gcontrib) : ctx->d_contrib64[it & 1];
       double* cout = ctx->d_contrib64[(it + 1) & 1];
-      hipLaunchKernelGGL(k_fused<double>, dim3(fb), dim3(kFusedThreads), 0, s, a, cin, cout, ctx->d_score64);
+      hipLaunchKernelGGL(k_fused<double>, dim3(fb), dim3(kFusedThreads), 0, s, a, prev, cin, cout, ctx->d_score64);
       hipLaunchKernelGGL(k_f64_super, dim3(sb), dim3(kThreads), 0, s, a, cout, ctx->d_score64);
     } else if (ctx->bp_ready && gcontrib) {
       const float* cin = static_cast<const float*>(gcontrib);
@@ -1830,20 +1887,20 @@ void launch_iteration(dmm_ctx* ctx, PrArgs a, int mode, int it, const void* gcon
       t.n_blocks = ctx->n_row_blocks;
       const int tb = std::max(1, ctx->cu_count);
       if (ctx->tiles_window == 16384)
-        hipLaunchKernelGGL(k_tile<16384>, dim3(tb), dim3(kTileThreads), 0, s, t, cin, a.n_gather, a.ctrl);
+        hipLaunchKernelGGL(k_tile<16384>, dim3(tb), dim3(kTileThreads), 0, s, t, prev, cin, a.n_gather);
       else
-        hipLaunchKernelGGL(k_tile<32768>, dim3(tb), dim3(kTileThreads), 0, s, t, cin, a.n_gather, a.ctrl);
+        hipLaunchKernelGGL(k_tile<32768>, dim3(tb), dim3(kTileThreads), 0, s, t, prev, cin, a.n_gather);
       a.main_blocks = pr_row_blocks(ctx);
       a.super_blocks = 0;
       hipLaunchKernelGGL(k_rows, dim3(a.main_blocks), dim3(kRowThreads), 0, s, a, t, cout, ctx->d_score);
     } else {
       const float* cin = gcontrib ? static_cast<const float*>(gcontrib) : ctx->d_contrib[it & 1];
       float* cout = contrib_out ? contrib_out : ctx->d_contrib[(it + 1) & 1];
-      hipLaunchKernelGGL(k_fused<float>, dim3(fb), dim3(kFusedThreads), 0, s, a, cin, cout, score_f);
+      hipLaunchKernelGGL(k_fused<float>, dim3(fb), dim3(kFusedThreads), 0, s, a, prev, cin, cout, score_f);
       hipLaunchKernelGGL(k_kahan_super, dim3(sb), dim3(kThreads), 0, s, a, cout, score_f);
     }
   }
-  hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kThreads), 0, s, a);
+  if (last) hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kThreads), 0, s, a);
 }
 
 }  // namespace
@@ -1958,7 +2015,7 @@ int pr_run(dmm_ctx* ctx, int32_t max_iters, double epsilon, int32_t mode, dmm_pr
     else
       hipLaunchKernelGGL(k_init_f32, dim3(ib), dim3(kThreads), 0, ctx->stream, a, ctx->d_score,
                          ctx->d_contrib[0]);
-    for (int it = 0; it < max_iters; it++) launch_iteration(ctx, a, mode, it, nullptr);
+    for (int it = 0; it < max_iters; it++) launch_iteration(ctx, a, mode, it, it + 1 == max_iters, nullptr);
     // Scores back to the caller's IDs.
     if (ctx->relabeled) {
       if (mode == DMM_PR_FP64)
@@ -2028,7 +2085,7 @@ int pr_block_iteration(dmm_ctx* ctx, const float* gcontrib_host, float* scores_i
   // The timed region starts after the host copies have landed.
   DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
   DMM_HIP_CHECK(ctx, hipEventRecord(ctx->ev_a, ctx->stream));
-  launch_iteration(ctx, a, mode, 0, ctx->d_gcontrib);
+  launch_iteration(ctx, a, mode, 0, true, ctx->d_gcontrib);
   DMM_HIP_CHECK(ctx, hipEventRecord(ctx->ev_b, ctx->stream));
   DMM_HIP_CHECK(ctx, hipGetLastError());
   DMM_HIP_CHECK(ctx, hipMemcpyAsync(scores_inout, ctx->d_score, sizeof(float) * ctx->nloc,
@@ -2109,9 +2166,7 @@ int pr_block_iteration_noalloc(dmm_ctx* ctx, const float* d_gcontrib, float* d_s
   unsigned char* base = ctx->scratch;
   if (!base) return set_err(ctx, DMM_ERR_STATE, "the context has no scratch address");
   PrArgs a = make_args(ctx);
-  const int parts = mode == DMM_PR_FP32_SERIAL ? pr_serial_blocks(ctx)
-                    : ctx->bp_ready ? pr_bsum_blocks(ctx) + pr_bsplit_blocks(ctx)
-                                    : pr_fused_blocks(ctx) + a.super_blocks;
+  const int parts = pr_error_parts(ctx, mode, true);
   if (parts > kScratchErrParts)
     return set_err(ctx, DMM_ERR_CAPACITY, "%d error partials exceed the %d the scratch array holds", parts,
                    kScratchErrParts);
@@ -2138,7 +2193,7 @@ int pr_block_iteration_noalloc(dmm_ctx* ctx, const float* d_gcontrib, float* d_s
   p.init_d = static_cast<double>(p.init_f);
   p.pad = 0;
   hipLaunchKernelGGL(k_scratch_prep, dim3(1), dim3(64), 0, ctx->stream, base, p);
-  launch_iteration(ctx, a, mode, 0, d_gcontrib, d_scores, d_contrib_out);
+  launch_iteration(ctx, a, mode, 0, true, d_gcontrib, d_scores, d_contrib_out);
   DMM_HIP_CHECK(ctx, hipGetLastError());
   DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
   return DMM_OK;
