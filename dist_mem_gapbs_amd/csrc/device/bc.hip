@@ -36,17 +36,20 @@
 // After either direction the depth-L bitmap is compacted in ascending
 // order into the next queue, its degree prefix, rank words and compact
 // path counts: a count pass and a write pass over kBcWW words per
-// wavefront, with a one-workgroup scan of the wavefronts' counts between
-// them.  The write pass clears the bitmap behind it.
+// wavefront.  The write pass takes the wavefronts' prefixes itself, each
+// workgroup summing the counts before its own, or from a one-workgroup scan
+// where there are more than kBcFusedScan of them; it clears the bitmap
+// behind it.
 //
-// The level loop runs on the device: the scan also updates a control
-// block (the frontier's sizes, the level, the unvisited out-edges R and
-// the direction of the next level), and every kernel reads it at start,
-// so a level is a fixed sequence of launches -- pull, successor pass,
-// top-down pass (the direction not taken returns at once), count, scan,
-// write -- and kBcLevels levels are captured in one graph.  Levels after
-// the last frontier return at once.  The host launches the graph until
-// the control block, mirrored to mapped memory, says the search is done.
+// The level loop runs on the device: the write pass (or the scan) also sets
+// the next level's control block (the frontier's sizes, the level, the
+// unvisited out-edges R and the direction), and every kernel reads its
+// level's at start, so a level is a fixed sequence of launches -- pull or
+// top-down pass, successor pass beside the count, (scan,) write -- and
+// kBcLevels levels are captured in one graph.  Two control blocks alternate,
+// so a level's never changes while its kernels read it.  Levels after the
+// last frontier return at once.  The host launches the graph until the
+// control block, mirrored to mapped memory, says the search is done.
 //
 // Successor bits are set with one atomicOr per run of lanes whose edge
 // positions are consecutive inside a bitmap word.  Depths, counts and bits
@@ -73,7 +76,10 @@ constexpr int kBcLight = 64;      // longest row an 8-lane group takes
 constexpr int kBcWW = 16;         // bitmap words per wavefront in the compaction
 constexpr int kBcPartWidth = 4;   // per such wavefront: found, queued (out-degree >= 1), their out-degree sum, pad
 constexpr int kBcScanThreads = 1024;
-constexpr int kBcLevels = 8;      // levels per captured graph
+constexpr int kBcLevels = 8;      // levels per captured graph (even: each graph starts on control block 0)
+// Compaction wavefronts up to which every workgroup of the write pass sums
+// the counts itself (24 bytes each, from L2), which saves a launch per level.
+constexpr int kBcFusedScan = 2048;
 
 // The level loop's state (device memory; see the file comment).
 struct BcCtl {
@@ -85,8 +91,6 @@ struct BcCtl {
   int levels;       // frontiers with at least one vertex so far
   int pull;         // this level runs bottom-up
   int done;         // no level is left to run
-  int scans;        // scans run: the write pass after a scan runs once,
-  int writes;       // while writes (set by the next count pass) trails scans
   int marks;        // this pulled level sets its successor bits in the pull
   int pad;
 };
@@ -102,6 +106,28 @@ constexpr long long kBcMarkRatio = 8;
 struct BcWord {
   unsigned long long bits;
   long long pre;
+};
+
+// What the kernels of a level read and write.
+struct BcArgs {
+  const int64_t* in_off;
+  const int32_t* in_nbr;
+  const int64_t* out_off;
+  const int32_t* out_nbr;
+  int64_t n, nw;
+  int32_t* depth;
+  unsigned long long* pc;
+  unsigned long long* succ;
+  unsigned long long* fnew;  // the depth-L bitmap
+  int32_t* queue;
+  int64_t* qoff;
+  unsigned long long* pcq;
+  BcWord* rank;
+  const int32_t* mirror;
+  int64_t* part;             // per compaction wavefront
+  int64_t nparts;
+  int marks_ok;
+  unsigned long long* host;  // mapped flags
 };
 
 int grid_of(int64_t items) {
@@ -149,7 +175,6 @@ __global__ __launch_bounds__(kCThreads) void k_bc_init(int64_t n, int64_t words,
     c.levels = 1;
     c.pull = d * kBcPull > c.R ? 1 : 0;
     c.done = d == 0 ? 1 : 0;
-    c.scans = c.writes = 0;
     c.marks = marks_ok && c.pull && d > kBcMarkRatio * c.R ? 1 : 0;
     c.pad = 0;
     *ctl = c;
@@ -188,25 +213,35 @@ __device__ __forceinline__ void succ_or(unsigned long long* __restrict__ succ, i
 // >= 1, so qoff is strictly increasing and a chunk spans at most kBcChunk
 // entries.
 template <bool kTopDown>
-__global__ __launch_bounds__(kCThreads) void k_bc_expand(const int64_t* __restrict__ off,
-                                                         const int32_t* __restrict__ nbr,
-                                                         const int32_t* __restrict__ queue,
-                                                         const int64_t* __restrict__ qoff,
-                                                         const unsigned long long* __restrict__ pcq,
-                                                         const BcCtl* __restrict__ ctl, int32_t* __restrict__ depth,
-                                                         unsigned long long* __restrict__ pc,
-                                                         unsigned long long* __restrict__ succ,
-                                                         unsigned long long* __restrict__ fnew) {
-  __shared__ int32_t rel[kBcChunk];    // entry's first edge, relative to the chunk (0 if before it)
-  __shared__ int64_t base[kBcChunk];   // out_off[u] - qoff[entry]: edge e sits at base + e
-  __shared__ unsigned long long pcu[kTopDown ? kBcChunk : 1];
-  __shared__ int64_t ie[2];
-  if (ctl->done || ctl->pull == (kTopDown ? 1 : 0) || (!kTopDown && ctl->marks)) return;
+struct ExpandLds {
+  int32_t rel[kBcChunk];    // entry's first edge, relative to the chunk (0 if before it)
+  int64_t base[kBcChunk];   // out_off[u] - qoff[entry]: edge e sits at base + e
+  unsigned long long pcu[kTopDown ? kBcChunk : 1];
+  int64_t ie[2];
+};
+
+// By workgroups [0, nblocks), of which this is the block-th.
+template <bool kTopDown>
+__device__ void bc_expand(const BcArgs& g, const BcCtl* __restrict__ ctl, ExpandLds<kTopDown>& L, int block,
+                          int nblocks) {
+  const int64_t* __restrict__ off = g.out_off;
+  const int32_t* __restrict__ nbr = g.out_nbr;
+  const int32_t* __restrict__ queue = g.queue;
+  const int64_t* __restrict__ qoff = g.qoff;
+  const unsigned long long* __restrict__ pcq = g.pcq;
+  int32_t* __restrict__ depth = g.depth;
+  unsigned long long* __restrict__ pc = g.pc;
+  unsigned long long* __restrict__ succ = g.succ;
+  unsigned long long* __restrict__ fnew = g.fnew;
+  int32_t* const rel = L.rel;
+  int64_t* const base = L.base;
+  unsigned long long* const pcu = L.pcu;
+  int64_t* const ie = L.ie;
   const int64_t F = ctl->Fq, T = ctl->T;
   const int32_t level = ctl->level;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  for (int64_t e0 = int64_t(blockIdx.x) * kBcChunk; e0 < T; e0 += int64_t(gridDim.x) * kBcChunk) {
+  for (int64_t e0 = int64_t(block) * kBcChunk; e0 < T; e0 += int64_t(nblocks) * kBcChunk) {
     const int64_t e1 = min(T, e0 + int64_t(kBcChunk));
     if (tid < 128) {
       const int64_t r = wave_last_le(qoff, 0, F, tid < 64 ? e0 : e1 - 1);
@@ -319,18 +354,18 @@ __device__ __forceinline__ void pull_terms(const int32_t* u, int64_t e, int stri
 
 // Bottom-up level (see the file comment): wavefront per word w of the
 // depth-L bitmap fnew, which it writes whole.
-__global__ __launch_bounds__(kCThreads) void k_bc_pull(const int64_t* __restrict__ in_off,
-                                                       const int32_t* __restrict__ in_nbr, int64_t n, int64_t nw,
-                                                       const BcCtl* __restrict__ ctl, int32_t* __restrict__ depth,
-                                                       unsigned long long* __restrict__ pc,
-                                                       const BcWord* __restrict__ rank,
-                                                       const unsigned long long* __restrict__ pcq,
-                                                       const int32_t* __restrict__ mirror,
-                                                       unsigned long long* __restrict__ succ,
-                                                       unsigned long long* __restrict__ fnew) {
-  if (ctl->done || !ctl->pull) return;
+__device__ void bc_pull(const BcArgs& g, const BcCtl* __restrict__ ctl) {
+  const int64_t* __restrict__ in_off = g.in_off;
+  const int32_t* __restrict__ in_nbr = g.in_nbr;
+  const int64_t n = g.n, nw = g.nw;
+  int32_t* __restrict__ depth = g.depth;
+  unsigned long long* __restrict__ pc = g.pc;
+  const BcWord* __restrict__ rank = g.rank;
+  const unsigned long long* __restrict__ pcq = g.pcq;
+  unsigned long long* __restrict__ succ = g.succ;
+  unsigned long long* __restrict__ fnew = g.fnew;
   const int32_t level = ctl->level;
-  if (!ctl->marks) mirror = nullptr;  // the successor pass sets this level's bits
+  const int32_t* __restrict__ mirror = ctl->marks ? g.mirror : nullptr;  // else the successor pass sets this level's bits
   const int lane = lane_id();
   const int sub = lane & (kBcGroup - 1);
   const int grp = lane / kBcGroup;
@@ -401,6 +436,16 @@ __global__ __launch_bounds__(kCThreads) void k_bc_pull(const int64_t* __restrict
   }
 }
 
+// A level's expansion in its direction.
+__global__ __launch_bounds__(kCThreads) void k_bc_level(BcArgs g, const BcCtl* __restrict__ ctl) {
+  __shared__ ExpandLds<true> L;
+  if (ctl->done) return;
+  if (ctl->pull)
+    bc_pull(g, ctl);
+  else
+    bc_expand<true>(g, ctl, L, blockIdx.x, gridDim.x);
+}
+
 // The mirror: for in-edge position e of row v (in-neighbour u), the
 // position of the out-edge u -> v in u's out-row, by binary search.  Out-rows
 // that are not strictly increasing, or an in-edge without its out-edge,
@@ -436,12 +481,11 @@ __global__ __launch_bounds__(kCThreads) void k_bc_mirror(const int64_t* __restri
 // Compaction of the depth-L bitmap, first pass: wavefront g takes words
 // [g * kBcWW, (g + 1) * kBcWW) and counts the vertices found there, those
 // of out-degree >= 1 (queued) and their out-degree sum.
-__global__ __launch_bounds__(kCThreads) void k_bc_count(const int64_t* __restrict__ off,
-                                                        const unsigned long long* __restrict__ fnew, int64_t nw,
-                                                        BcCtl* __restrict__ ctl, int64_t* __restrict__ part) {
-  // The previous level's write pass has run (stream order).
-  if (blockIdx.x == 0 && threadIdx.x == 0) ctl->writes = ctl->scans;
-  if (ctl->done) return;
+__device__ void bc_count(const BcArgs& a) {
+  const int64_t* __restrict__ off = a.out_off;
+  const unsigned long long* __restrict__ fnew = a.fnew;
+  const int64_t nw = a.nw;
+  int64_t* __restrict__ part = a.part;
   const int lane = lane_id();
   const int64_t g = (int64_t(blockIdx.x) * kCThreads + threadIdx.x) >> 6;
   const int64_t w0 = g * kBcWW;
@@ -471,14 +515,50 @@ __global__ __launch_bounds__(kCThreads) void k_bc_count(const int64_t* __restric
   }
 }
 
-// One workgroup: exclusive prefixes of the wavefronts' queued counts and
-// degree sums (in place), qoff[F] = T, and the control block's next level
-// (mirrored to the host's flags).
-__global__ __launch_bounds__(kBcScanThreads) void k_bc_scan(int64_t* __restrict__ part, int64_t nparts,
-                                                            int64_t* __restrict__ qoff, int marks_ok,
-                                                            BcCtl* __restrict__ ctl, unsigned long long* __restrict__ host) {
-  __shared__ int64_t wt[3][kBcScanThreads / 64];
+// What follows the expansion: the count pass by workgroups [0, cgrid), the
+// successor bits of a pulled level that did not set them by the others.
+__global__ __launch_bounds__(kCThreads) void k_bc_after(BcArgs g, const BcCtl* __restrict__ ctl, int cgrid) {
+  __shared__ ExpandLds<false> L;
   if (ctl->done) return;
+  if (static_cast<int>(blockIdx.x) < cgrid)
+    bc_count(g);
+  else if (ctl->pull && !ctl->marks)
+    bc_expand<false>(g, ctl, L, blockIdx.x - cgrid, gridDim.x - cgrid);
+}
+
+// The next level's control block from this one's and the counted frontier
+// (ta vertices, tp of them queued, td their out-edges), mirrored to the
+// host's flags; qoff[F] = T.
+__device__ __forceinline__ void bc_next(const BcArgs& g, const BcCtl& ctl, BcCtl* __restrict__ next, int64_t ta,
+                                        int64_t tp, int64_t td) {
+  g.qoff[tp] = td;
+  BcCtl c = ctl;
+  c.F = ta;
+  c.T = td;
+  c.Fq = tp;
+  c.R -= td;
+  c.level += 1;
+  c.levels += ta > 0 ? 1 : 0;
+  c.pull = td * kBcPull > c.R ? 1 : 0;
+  c.done = (ta == 0 || td == 0) ? 1 : 0;
+  c.marks = g.marks_ok && c.pull && td > kBcMarkRatio * c.R ? 1 : 0;
+  *next = c;
+  g.host[0] = static_cast<unsigned long long>(c.done);
+  g.host[1] = static_cast<unsigned long long>(c.levels);
+  g.host[2] = static_cast<unsigned long long>(ta);
+}
+
+// One workgroup: exclusive prefixes of the wavefronts' queued counts and
+// degree sums (in place), and the next control block.
+__global__ __launch_bounds__(kBcScanThreads) void k_bc_scan(BcArgs g, const BcCtl* __restrict__ ctl,
+                                                            BcCtl* __restrict__ next) {
+  __shared__ int64_t wt[3][kBcScanThreads / 64];
+  if (ctl->done) {
+    if (threadIdx.x == 0) *next = *ctl;
+    return;
+  }
+  int64_t* __restrict__ part = g.part;
+  const int64_t nparts = g.nparts;
   const int lane = lane_id();
   const int wave = threadIdx.x >> 6;
   const int64_t per = (nparts + kBcScanThreads - 1) / kBcScanThreads;
@@ -515,47 +595,76 @@ __global__ __launch_bounds__(kBcScanThreads) void k_bc_scan(int64_t* __restrict_
     ep += pj;
     ed += dj;
   }
-  if (threadIdx.x == 0) {
-    qoff[tp] = td;
-    BcCtl c = *ctl;
-    c.F = ta;
-    c.T = td;
-    c.Fq = tp;
-    c.R -= td;
-    c.level += 1;
-    c.levels += ta > 0 ? 1 : 0;
-    c.pull = td * kBcPull > c.R ? 1 : 0;
-    c.done = (ta == 0 || td == 0) ? 1 : 0;
-    c.marks = marks_ok && c.pull && td > kBcMarkRatio * c.R ? 1 : 0;
-    c.scans += 1;
-    *ctl = c;
-    host[0] = static_cast<unsigned long long>(c.done);
-    host[1] = static_cast<unsigned long long>(c.levels);
-    host[2] = static_cast<unsigned long long>(ta);
-  }
+  if (threadIdx.x == 0) bc_next(g, *ctl, next, ta, tp, td);
 }
 
 // Second pass, same words per wavefront: the queue (ascending vertices of
 // out-degree >= 1), its degree prefix, the compact path counts and the
 // rank words, from the wavefront's prefixes; then the words are cleared
 // for the next level.
-__global__ __launch_bounds__(kCThreads) void k_bc_write(const int64_t* __restrict__ off,
-                                                        unsigned long long* __restrict__ fnew, int64_t nw,
-                                                        const int64_t* __restrict__ part,
-                                                        const unsigned long long* __restrict__ pc,
-                                                        int32_t* __restrict__ queue, int64_t* __restrict__ qoff,
-                                                        unsigned long long* __restrict__ pcq,
-                                                        BcWord* __restrict__ rank, const BcCtl* __restrict__ ctl) {
-  // Runs once after each scan, also after the one that ended the search.
-  if (ctl->scans == ctl->writes) return;
+template <bool kScanned>
+__global__ __launch_bounds__(kCThreads) void k_bc_write(BcArgs a, const BcCtl* __restrict__ ctl,
+                                                        BcCtl* __restrict__ next) {
+  __shared__ int64_t red[5][kCWaves];
+  if (ctl->done) {
+    if (!kScanned && blockIdx.x == 0 && threadIdx.x == 0) *next = *ctl;
+    return;
+  }
+  const int64_t* __restrict__ off = a.out_off;
+  unsigned long long* __restrict__ fnew = a.fnew;
+  const int64_t* __restrict__ part = a.part;
+  const unsigned long long* __restrict__ pc = a.pc;
+  int32_t* __restrict__ queue = a.queue;
+  int64_t* __restrict__ qoff = a.qoff;
+  unsigned long long* __restrict__ pcq = a.pcq;
+  BcWord* __restrict__ rank = a.rank;
+  const int64_t nw = a.nw;
   const int lane = lane_id();
-  const int64_t g = (int64_t(blockIdx.x) * kCThreads + threadIdx.x) >> 6;
+  const int wave = threadIdx.x >> 6;
+  const int64_t g = int64_t(blockIdx.x) * kCWaves + wave;
+  int64_t pos = 0, deg = 0;  // the wavefront's prefixes
+  if (kScanned) {
+    if (g < a.nparts) {
+      pos = part[g * kBcPartWidth + 1];
+      deg = part[g * kBcPartWidth + 2];
+    }
+  } else {
+    // Totals, and the sums before this workgroup's wavefronts.
+    const int64_t g0 = int64_t(blockIdx.x) * kCWaves;
+    int64_t t[5] = {0, 0, 0, 0, 0};
+    for (int64_t j = threadIdx.x; j < a.nparts; j += kCThreads) {
+      const int64_t pa = part[j * kBcPartWidth], pp = part[j * kBcPartWidth + 1], pd = part[j * kBcPartWidth + 2];
+      t[0] += pa;
+      t[1] += pp;
+      t[2] += pd;
+      t[3] += j < g0 ? pp : 0;
+      t[4] += j < g0 ? pd : 0;
+    }
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+      t[k] = wave_sum(t[k]);
+      if (lane == 0) red[k][wave] = t[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+      t[k] = 0;
+#pragma unroll
+      for (int w = 0; w < kCWaves; w++) t[k] += red[k][w];
+    }
+    pos = t[3];
+    deg = t[4];
+    for (int64_t j = g0; j < min(g, a.nparts); j++) {
+      pos += part[j * kBcPartWidth + 1];
+      deg += part[j * kBcPartWidth + 2];
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) bc_next(a, *ctl, next, t[0], t[1], t[2]);
+  }
   const int64_t w0 = g * kBcWW;
   if (w0 >= nw) return;  // whole wavefronts
   const bool own = lane < kBcWW && w0 + lane < nw;
   const unsigned long long mine = own ? fnew[w0 + lane] : 0ull;
   if (own) fnew[w0 + lane] = 0;
-  int64_t pos = part[g * kBcPartWidth + 1], deg = part[g * kBcPartWidth + 2];
   unsigned long long word[kBcWW];
   int64_t d[kBcWW];
 #pragma unroll
@@ -604,7 +713,7 @@ int bc_forward(dmm_ctx* ctx, int32_t source, int32_t* depth, uint64_t* path_coun
         (rc = dev_alloc(ctx, reinterpret_cast<void**>(&ctx->d_bc_pcq), sizeof(uint64_t) * n,
                         "BC frontier path counts")) ||
         (rc = dev_alloc(ctx, reinterpret_cast<void**>(&ctx->d_bc_rank), sizeof(BcWord) * nw, "BC frontier ranks")) ||
-        (rc = dev_alloc(ctx, &ctx->d_bc_ctl, sizeof(BcCtl), "BC level control")) ||
+        (rc = dev_alloc(ctx, &ctx->d_bc_ctl, 2 * sizeof(BcCtl), "BC level control")) ||
         (rc = dev_alloc(ctx, reinterpret_cast<void**>(&ctx->d_bc_bm), sizeof(uint64_t) * nw, "BC level bitmap")))
       return rc;
   }
@@ -649,21 +758,39 @@ int bc_forward(dmm_ctx* ctx, int32_t source, int32_t* depth, uint64_t* path_coun
     const int pgrid = static_cast<int>(std::min<int64_t>(cap, ceil_div(nw, kCWaves)));
     const int egrid = static_cast<int>(std::min<int64_t>(cap, ceil_div(m, kBcChunk)));
     const int cgrid = static_cast<int>(ceil_div(nparts, kCWaves));
+    BcArgs a;
+    a.in_off = ctx->d_in_off;
+    a.in_nbr = ctx->d_in_nbr;
+    a.out_off = ctx->d_out_off;
+    a.out_nbr = ctx->d_out_nbr;
+    a.n = n;
+    a.nw = nw;
+    a.depth = d_depth;
+    a.pc = d_pc;
+    a.succ = d_succ;
+    a.fnew = fnew;
+    a.queue = ctx->d_bc_queue;
+    a.qoff = ctx->d_bc_qoff;
+    a.pcq = d_pcq;
+    a.rank = d_rank;
+    a.mirror = mirror;
+    a.part = ctx->d_bc_part;
+    a.nparts = nparts;
+    a.marks_ok = mirror ? 1 : 0;
+    a.host = d_host;
     hipGraph_t g = nullptr;
     DMM_HIP_CHECK(ctx, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
     for (int k = 0; k < kBcLevels; k++) {
-      hipLaunchKernelGGL(k_bc_pull, dim3(pgrid), dim3(kCThreads), 0, s, ctx->d_in_off, ctx->d_in_nbr, n, nw, d_ctl,
-                         d_depth, d_pc, d_rank, d_pcq, mirror, d_succ, fnew);
-      hipLaunchKernelGGL(k_bc_expand<false>, dim3(egrid), dim3(kCThreads), 0, s, ctx->d_out_off, ctx->d_out_nbr,
-                         ctx->d_bc_queue, ctx->d_bc_qoff, d_pcq, d_ctl, d_depth, d_pc, d_succ, fnew);
-      hipLaunchKernelGGL(k_bc_expand<true>, dim3(egrid), dim3(kCThreads), 0, s, ctx->d_out_off, ctx->d_out_nbr,
-                         ctx->d_bc_queue, ctx->d_bc_qoff, d_pcq, d_ctl, d_depth, d_pc, d_succ, fnew);
-      hipLaunchKernelGGL(k_bc_count, dim3(cgrid), dim3(kCThreads), 0, s, ctx->d_out_off, fnew, nw, d_ctl,
-                         ctx->d_bc_part);
-      hipLaunchKernelGGL(k_bc_scan, dim3(1), dim3(kBcScanThreads), 0, s, ctx->d_bc_part, nparts, ctx->d_bc_qoff,
-                         mirror ? 1 : 0, d_ctl, d_host);
-      hipLaunchKernelGGL(k_bc_write, dim3(cgrid), dim3(kCThreads), 0, s, ctx->d_out_off, fnew, nw, ctx->d_bc_part,
-                         d_pc, ctx->d_bc_queue, ctx->d_bc_qoff, d_pcq, d_rank, d_ctl);
+      BcCtl* const cur = d_ctl + (k & 1);
+      BcCtl* const next = d_ctl + ((k + 1) & 1);
+      hipLaunchKernelGGL(k_bc_level, dim3(std::max(1, std::max(pgrid, egrid))), dim3(kCThreads), 0, s, a, cur);
+      hipLaunchKernelGGL(k_bc_after, dim3(cgrid + egrid), dim3(kCThreads), 0, s, a, cur, cgrid);
+      if (nparts > kBcFusedScan) {
+        hipLaunchKernelGGL(k_bc_scan, dim3(1), dim3(kBcScanThreads), 0, s, a, cur, next);
+        hipLaunchKernelGGL(k_bc_write<true>, dim3(cgrid), dim3(kCThreads), 0, s, a, cur, next);
+      } else {
+        hipLaunchKernelGGL(k_bc_write<false>, dim3(cgrid), dim3(kCThreads), 0, s, a, cur, next);
+      }
     }
     hipError_t e = hipStreamEndCapture(s, &g);
     if (e != hipSuccess) return set_err(ctx, DMM_ERR_HIP, "BC capture failed: %s", hipGetErrorString(e));
