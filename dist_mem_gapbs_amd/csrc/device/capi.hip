@@ -732,7 +732,7 @@ int dmm_graph_upload(dmm_ctx* ctx, int64_t num_nodes, int64_t vbegin, int64_t ve
     DMM_HIP_CHECK(ctx, hipMemcpy(ctx->d_heavy, by_class.data(), sizeof(int32_t) * heavy.size(), hipMemcpyHostToDevice));
   std::vector<dmm::SerialItem> sitems;
   std::vector<int32_t> sstart;
-  dmm::serial_plan(ctx->pr_light_begin, ctx->pr_zero_begin, ioff, by_class, ctx->heavy_threshold,
+  dmm::serial_plan(rows, ctx->pr_light_begin, ctx->pr_zero_begin, ioff, by_class, ctx->heavy_threshold,
                    dmm::pr_serial_blocks(ctx), &sitems, &sstart);
   if ((rc = A(&ctx->d_sitems, sizeof(dmm::SerialItem) * std::max<size_t>(1, sitems.size()), "serial items")) ||
       (rc = A((void**)&ctx->d_sstart, sizeof(int32_t) * sstart.size(), "serial items")))

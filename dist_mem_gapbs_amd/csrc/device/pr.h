@@ -34,6 +34,10 @@ constexpr int64_t kPrSegment = 2048;  // edges per segment
 // workgroup: Kronecker-21 2.42 ms from 32768 (or 16384) on, 2.72 from 131072.
 constexpr int64_t kSerialWaveRow = 512;     // rows from here on: a wavefront each
 constexpr int64_t kSerialBlockRow = 32768;  // rows from here on: a workgroup each
+// ... in a small graph: halved down to this while the CUs would have less than
+// such a row each (200 K vertices, 20 iterations: 816 us; 936 from 32768 on;
+// least 1024 or 4096: no change).
+constexpr int64_t kSerialBlockLeast = 2048;
 constexpr int kHeavyBundle = 16;            // shorter heavy rows: this many per wavefront
 constexpr int kLightBundle = 64;            // rows below the heavy threshold
 enum : int32_t {
@@ -46,7 +50,7 @@ struct SerialItem {
   int32_t first;
   int32_t kind;
 };
-void serial_plan(int64_t light_begin, int64_t zero_begin, const int64_t* off, const std::vector<int32_t>& by_class,
+void serial_plan(int64_t rows, int64_t light_begin, int64_t zero_begin, const int64_t* off, const std::vector<int32_t>& by_class,
                  int64_t heavy_threshold, int blocks, std::vector<SerialItem>* items, std::vector<int32_t>* start);
 
 // Window-tiled compensated PageRank (degree-ordered whole graphs).

@@ -1914,7 +1914,7 @@ int pr_light_blocks(dmm_ctx* ctx) {
 // the workgroup with the fewest edges so far.  Static, so that every run adds
 // the error terms in the same order.  by_class: the heavy rows, longest
 // power-of-two class first.
-void serial_plan(int64_t light_begin, int64_t zero_begin, const int64_t* off, const std::vector<int32_t>& by_class,
+void serial_plan(int64_t rows, int64_t light_begin, int64_t zero_begin, const int64_t* off, const std::vector<int32_t>& by_class,
                  int64_t heavy_threshold, int blocks, std::vector<SerialItem>* items, std::vector<int32_t>* start) {
   struct Load {
     int64_t edges;
@@ -1936,9 +1936,12 @@ void serial_plan(int64_t light_begin, int64_t zero_begin, const int64_t* off, co
     std::push_heap(heap.begin(), heap.end());
   };
   auto len = [&](int64_t r) { return off[r + 1] - off[r]; };
+  const int64_t off_end = off[rows];
   constexpr int64_t kItemCost = 128;  // an item's own steps, in edges
+  int64_t block_row = kSerialBlockRow;
+  while (block_row > kSerialBlockLeast && block_row * blocks > off_end) block_row /= 2;
   size_t h = 0;
-  for (; h < by_class.size() && len(by_class[h]) >= kSerialBlockRow; h++)
+  for (; h < by_class.size() && len(by_class[h]) >= block_row; h++)
     deal(by_class[h], kSerialBlock, len(by_class[h]));
   for (; h < by_class.size() && len(by_class[h]) >= kSerialWaveRow; h++)
     deal(by_class[h], kSerialWave, len(by_class[h]) + kItemCost);
