@@ -22,11 +22,12 @@
 //   bottom-up (pull) sweep over all u: need = lanes & ~(seen[u] | F[L][u]);
 //             OR F[L][v] over in(u) until every needed lane is found;
 //             F[L+1][u] = found & need (full overwrite);
-// and a one-workgroup post kernel reduces the per-workgroup partials and
-// picks the next direction: top-down while the next frontier's out-edges
-// are fewer than M / td_div (tuned).  The active list for a top-down level
-// is compacted from F[L+1] in ascending vertex order (COUNT, scan, WRITE),
-// so no phase uses a same-address atomic.  A chain of these launches is
+// and the next launch picks the next direction from the per-workgroup
+// partials: top-down while the next frontier's out-edges are fewer than
+// M / td_div (tuned).  The active list for a top-down level is compacted
+// from F[L+1] in ascending vertex order (COUNT, WRITE), so no phase uses a
+// same-address atomic.  Each launch (k_bslot) starts with that choice, made
+// by every workgroup on its own copy of the loop state; a chain of them is
 // captured in a hipGraph.
 #include "batch.h"
 
@@ -41,25 +42,54 @@ namespace dmm {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kPostThreads = 1024;  // the one-workgroup post kernel
 constexpr int kItems = 2;
 constexpr int kEPB = kThreads * kItems;
 constexpr int kGroup = 8;  // lanes per vertex in the bottom-up sweep
+// Workgroups: as many per CU as asked for (or tuned), but no more than one per
+// kBatchRows rows between one and kBatchMostPerCU per CU: the step kernel's
+// registers leave room for five, and every workgroup reads every partial.
+// 64 lanes with 1, 2, 4, 8, 16 per CU: 22 K Kronecker vertices 173, 180, 200,
+// 264, 455 us; 131 K 221, 200, 203, 258, 428; 900 K 788, 565, 497, 589, 849;
+// 3.7 M uniform 5.00, 4.41, 4.36, 4.55, 4.62 ms.
+constexpr int64_t kBatchRows = 256;
+constexpr int kBatchMostPerCU = 4;
 
 enum : int { kBTD = 1, kBBU = 2, kBCount = 3, kBWrite = 4, kBDone = 5 };
 
-struct BCtrl {
+// Loop state.  Slot k reads head k & 1 and writes the other, so a head never
+// changes while a slot's workgroups read it.
+struct BHead {
   long long acount, aedges;           // active list size / its out-edges
   long long pend_cnt, pend_degs;      // counted next frontier
   long long sweep_scanned_total;      // edges scanned by all sweeps
+  uint64_t live;                      // lanes with a vertex in F[level]
   int level, phase, done, cur;        // cur = active list buffer index
   int nlevels;
   int sweeps;
   int error;
+  int ran;                            // the phase the slot ran, its post pending
+  int used;                           // slots that ran one
   int pad;
-  uint64_t live;                      // lanes with a vertex in F[level]
+};
+constexpr int kBHeadWords = sizeof(BHead) / 8;
+static_assert(sizeof(BHead) % 8 == 0 && kBHeadWords <= 64, "a head is copied as 8-byte words by one wave");
+
+struct BCtrl {
+  BHead h[2];
+  int slot_error;                     // raised by a step
+  int pad;
   int level_kind[DMM_MAX_STEPS];
   long long level_active[DMM_MAX_STEPS];
+};
+
+// What a step takes from the loop state, and where it reports.
+struct BIo {
+  int64_t acount, aedges;
+  uint64_t live;
+  int cur;
+  int* error;
+  int64_t* part;                      // this slot's partials [gridDim.x][kPartWidth]
+  int64_t base_c, base_d;             // WRITE: the workgroup's prefixes of the counted partials
 };
 
 struct BArgs {
@@ -77,7 +107,8 @@ struct BArgs {
   int64_t* aoff0;
   int64_t* aoff1;
   BCtrl* ctrl;
-  int64_t* part;      // [gridDim.x][kPartWidth]
+  int64_t* part;      // [2][gridDim.x][kPartWidth], the slots' in turn
+  int64_t part_half;  // offset of the second
   uint64_t lanes;     // mask of used lanes
   int64_t m;          // directed edges of the block (td threshold base)
   int td_div;
@@ -145,12 +176,12 @@ __device__ void zero_next_next(const BArgs& a, int level) {
   for (int64_t i = gtid; i < a.bend; i += gsize) z[i] = 0;
 }
 
-__device__ void td_phase(const BArgs& a, BCtrl* c, TdLds& L, int level) {
-  const int cur = c->cur;
+__device__ void td_phase(const BArgs& a, const BIo& io, TdLds& L, int level) {
+  const int cur = io.cur;
   const int32_t* q = cur ? a.act1 : a.act0;
   const int64_t* qoff = cur ? a.aoff1 : a.aoff0;
-  const int64_t F = c->acount;
-  const int64_t T = c->aedges;
+  const int64_t F = io.acount;
+  const int64_t T = io.aedges;
   const uint64_t* Fl = a.levels + level * a.nloc;
   uint64_t* Fn = a.levels + (level + 1) * a.nloc;
   const int tid = threadIdx.x;
@@ -172,7 +203,7 @@ __device__ void td_phase(const BArgs& a, BCtrl* c, TdLds& L, int level) {
     // Listed vertices have out-degree >= 1: a chunk spans <= kEPB + 1 of them.
     int nv = static_cast<int>(L.ie[1] - i0 + 1);
     if (nv > kEPB + 2) {
-      if (tid == 0) c->error = 1;
+      if (tid == 0) *io.error = 1;
       nv = kEPB + 2;
     }
     for (int i = tid; i < nv; i += kThreads) {
@@ -222,7 +253,7 @@ __device__ void td_phase(const BArgs& a, BCtrl* c, TdLds& L, int level) {
     }
     __syncthreads();
   }
-  if (threadIdx.x < kPartWidth) a.part[blockIdx.x * kPartWidth + threadIdx.x] = 0;
+  if (threadIdx.x < kPartWidth) io.part[blockIdx.x * kPartWidth + threadIdx.x] = 0;
 }
 
 // Bottom-up sweep: kGroup lanes per vertex, strided over its in-neighbours,
@@ -234,15 +265,15 @@ __device__ void td_phase(const BArgs& a, BCtrl* c, TdLds& L, int level) {
 // reads kGroup edges (rows whose needed lanes are all found there stop
 // early), later rounds keep kUnroll frontier-word loads in flight per lane;
 // the group ORs them and the scan stops once every needed lane is found.
-// The whole-graph sweep uses kSweepUnroll; the PE-block kernels, which probe
-// the non-zero bitmaps first and stop earlier, use kBlockUnroll.  nz (may be
-// NULL) is a
-// non-zero bitmap of the frontier words (bit v), with a summary bitmap nz2
-// (bit w set iff nz word w != 0, so 256 KB for 2^27 vertices, resident in
-// L2); both are probed before a word load, so sparse frontiers cost one L2
-// probe per edge.
+// The whole-graph sweep uses kSweepUnroll (16 leaves registers for five
+// workgroups per CU; 32: four, 3% slower on Kronecker graphs); the PE-block
+// kernels, which probe the non-zero bitmaps first and stop earlier, use
+// kBlockUnroll.  nz (may be NULL) is a non-zero bitmap of the frontier words
+// (bit v), with a summary bitmap nz2 (bit w set iff nz word w != 0, so 256 KB
+// for 2^27 vertices, resident in L2); both are probed before a word load, so
+// sparse frontiers cost one L2 probe per edge.
 // Returns the end of the examined range; *found = the needed lanes found.
-constexpr int kSweepUnroll = 32;
+constexpr int kSweepUnroll = 16;
 constexpr int kBlockUnroll = 4;
 template <int kUnroll>
 __device__ __forceinline__ int64_t sweep_row(const int32_t* __restrict__ in_nbr, int64_t b, int64_t e,
@@ -338,7 +369,7 @@ __device__ __forceinline__ int64_t wide_row(const int32_t* __restrict__ in_nbr, 
   return min(k0, e);
 }
 
-__device__ void bu_phase(const BArgs& a, BCtrl* c, SmallLds& L, int level) {
+__device__ void bu_phase(const BArgs& a, const BIo& io, SmallLds& L, int level) {
   const uint64_t* __restrict__ Fl = a.levels + level * a.nloc;
   uint64_t* __restrict__ Fn = a.levels + (level + 1) * a.nloc;
   const int64_t* __restrict__ in_off = a.in_off;
@@ -349,7 +380,7 @@ __device__ void bu_phase(const BArgs& a, BCtrl* c, SmallLds& L, int level) {
   // A lane whose frontier is empty finds nothing any more: rows out of its
   // reach do not look for it (a source in a small component would have every
   // sweep read every edge).
-  const uint64_t lanes = a.lanes & c->live;
+  const uint64_t lanes = a.lanes & io.live;
   uint64_t any = 0;  // lanes found
   int64_t scanned = 0, cnt = 0, degs = 0;
   // The wide rows first: giant ones by a workgroup, the others by a
@@ -447,7 +478,7 @@ __device__ void bu_phase(const BArgs& a, BCtrl* c, SmallLds& L, int level) {
   const int64_t s2 = block_sum<kThreads>(degs, L.red[2]);
   const uint64_t s3 = block_or<kThreads>(any, L.found[0]);
   if (threadIdx.x == 0) {
-    int64_t* p = a.part + blockIdx.x * kPartWidth;
+    int64_t* p = io.part + blockIdx.x * kPartWidth;
     p[0] = s0;
     p[1] = s1;
     p[2] = s2;
@@ -458,10 +489,10 @@ __device__ void bu_phase(const BArgs& a, BCtrl* c, SmallLds& L, int level) {
 // COUNT / WRITE over the frontier words F[level]: contiguous vertex ranges
 // per workgroup in ascending order; listed = nonzero word and out-degree >= 1.
 template <bool kWrite>
-__device__ void count_or_write(const BArgs& a, BCtrl* c, SmallLds& L, int level) {
+__device__ void count_or_write(const BArgs& a, const BIo& io, SmallLds& L, int level) {
   // Workgroup b owns the contiguous range [v0, v1) and walks it in tiles
   // of kThreads consecutive vertices (coalesced); WRITE orders entries by
-  // a block scan per tile on top of the workgroup's prefix from k_bpost.
+  // a block scan per tile on top of the workgroup's prefix.
   // Levels >= 1 have no lanes from bend on.
   const uint64_t* Fl = a.levels + level * a.nloc;
   const int64_t vpb = (a.bend + gridDim.x - 1) / gridDim.x;
@@ -484,7 +515,7 @@ __device__ void count_or_write(const BArgs& a, BCtrl* c, SmallLds& L, int level)
     const int64_t sd = block_sum<kThreads>(degs, L.red[1]);
     const uint64_t so = block_or<kThreads>(any, L.found[0]);
     if (threadIdx.x == 0) {
-      int64_t* p = a.part + blockIdx.x * kPartWidth;
+      int64_t* p = io.part + blockIdx.x * kPartWidth;
       p[0] = sc;
       p[1] = sd;
       p[2] = 0;
@@ -492,11 +523,11 @@ __device__ void count_or_write(const BArgs& a, BCtrl* c, SmallLds& L, int level)
     }
     return;
   }
-  const int cur = c->cur;
+  const int cur = io.cur;
   int32_t* oq = cur ? a.act0 : a.act1;
   int64_t* oqoff = cur ? a.aoff0 : a.aoff1;
-  int64_t pos = a.part[blockIdx.x * kPartWidth + 0];
-  int64_t run = a.part[blockIdx.x * kPartWidth + 1];
+  int64_t pos = io.base_c;
+  int64_t run = io.base_d;
   for (int64_t t = v0; t < v1; t += kThreads) {
     const int64_t u = t + threadIdx.x;
     int64_t d = 0;
@@ -514,123 +545,162 @@ __device__ void count_or_write(const BArgs& a, BCtrl* c, SmallLds& L, int level)
   }
 }
 
-__global__ __launch_bounds__(kThreads) void k_bstep(BArgs a) {
-  __shared__ BLds lds;
-  BCtrl* c = a.ctrl;
-  const int phase = c->phase;
-  const int level = c->level;
-  switch (phase) {
-    case kBTD:
-      zero_next_next(a, level);
-      td_phase(a, c, lds.td, level);
-      break;
-    case kBBU:
-      zero_next_next(a, level);
-      bu_phase(a, c, lds.sm, level);
-      break;
-    case kBCount: count_or_write<false>(a, c, lds.sm, level); break;
-    case kBWrite: count_or_write<true>(a, c, lds.sm, level); break;
-    default: break;
-  }
-}
-
-__device__ void choose_next(const BArgs& a, BCtrl* c, long long cnt, long long degs, bool have_list) {
-  c->pend_cnt = cnt;
-  c->pend_degs = degs;
+__device__ void choose_next(const BArgs& a, BHead& h, long long cnt, long long degs, bool have_list) {
+  h.pend_cnt = cnt;
+  h.pend_degs = degs;
   if (cnt == 0) {
-    c->phase = kBDone;
-    c->done = 1;
-    c->nlevels = c->level + 1;  // F[level] is empty
+    h.phase = kBDone;
+    h.done = 1;
+    h.nlevels = h.level + 1;  // F[level] is empty
     return;
   }
-  if (c->level + 1 >= a.level_cap) {
-    c->phase = kBDone;  // out of level storage: the host grows and reruns
-    c->done = 3;
+  if (h.level + 1 >= a.level_cap) {
+    h.phase = kBDone;  // out of level storage: the host grows and reruns
+    h.done = 3;
     return;
   }
   if (degs * a.td_div < a.m)
-    c->phase = have_list ? kBWrite : kBCount;
+    h.phase = have_list ? kBWrite : kBCount;
   else
-    c->phase = kBBU;
+    h.phase = kBBU;
 }
 
-__global__ __launch_bounds__(kPostThreads) void k_bpost(BArgs a, int nblocks) {
-  __shared__ int64_t red[kPartWidth][kPostThreads / 64];
-  __shared__ int64_t sc[kPostThreads / 64 + 1];
-  __shared__ int64_t sd[kPostThreads / 64 + 1];
-  BCtrl* c = a.ctrl;
-  const int phase = c->phase;
-  if (phase != kBTD && phase != kBBU && phase != kBCount && phase != kBWrite) return;
-  int64_t s0 = 0, s1 = 0, s2 = 0;
-  uint64_t s3 = 0;
-  if (phase == kBBU || phase == kBCount) {
-    for (int b = threadIdx.x; b < nblocks; b += kPostThreads) {
-      s0 += a.part[b * kPartWidth + 0];
-      s1 += a.part[b * kPartWidth + 1];
-      s2 += a.part[b * kPartWidth + 2];
-      s3 |= static_cast<uint64_t>(a.part[b * kPartWidth + 3]);
-    }
-    s0 = block_sum<kPostThreads>(s0, red[0]);
-    s1 = block_sum<kPostThreads>(s1, red[1]);
-    s2 = block_sum<kPostThreads>(s2, red[2]);
-    s3 = block_or<kPostThreads>(s3, reinterpret_cast<uint64_t*>(red[3]));
-  }
-  if (phase == kBCount) {
-    int64_t carry_c = 0, carry_d = 0;
-    for (int base = 0; base < nblocks; base += kPostThreads) {
-      const int b = base + threadIdx.x;
-      const int64_t vc = b < nblocks ? a.part[b * kPartWidth + 0] : 0;
-      const int64_t vd = b < nblocks ? a.part[b * kPartWidth + 1] : 0;
-      int64_t tc, td;
-      const int64_t ec = block_excl_scan<kPostThreads>(vc, sc, &tc);
-      const int64_t ed = block_excl_scan<kPostThreads>(vd, sd, &td);
-      if (b < nblocks) {
-        a.part[b * kPartWidth + 0] = carry_c + ec;
-        a.part[b * kPartWidth + 1] = carry_d + ed;
-      }
-      carry_c += tc;
-      carry_d += td;
-    }
-  }
-  if (threadIdx.x != 0) return;
-  const int level = c->level;
+// The loop state after a step of phase h.ran with totals s0..s2 and the OR
+// s3 of its partials (one thread); c (may be null) takes the level's record.
+__device__ void post_update(const BArgs& a, BHead& h, BCtrl* c, int64_t s0, int64_t s1, int64_t s2, uint64_t s3) {
+  const int phase = h.ran;
+  const int level = h.level;
+  h.used += 1;
   if (phase == kBTD || phase == kBBU) {
-    if (level < DMM_MAX_STEPS) {
+    if (c && level < DMM_MAX_STEPS) {
       c->level_kind[level] = phase == kBTD ? DMM_STEP_TD : DMM_STEP_BU;
-      c->level_active[level] = c->acount;
+      c->level_active[level] = h.acount;
     }
-    c->level = level + 1;
-    c->nlevels = level + 2;  // F[0 .. level + 1] hold frontiers
+    h.level = level + 1;
+    h.nlevels = level + 2;  // F[0 .. level + 1] hold frontiers
     if (phase == kBTD) {
-      c->phase = kBCount;
-      if (c->level + 1 >= a.level_cap) {
-        c->phase = kBDone;
-        c->done = 3;
+      h.phase = kBCount;
+      if (h.level + 1 >= a.level_cap) {
+        h.phase = kBDone;
+        h.done = 3;
       }
       return;
     }
-    c->live = s3;
-    c->sweeps = c->sweeps + 1;
-    c->sweep_scanned_total += s0;
+    h.live = s3;
+    h.sweeps += 1;
+    h.sweep_scanned_total += s0;
     // A sweep's partials are not in vertex order: a top-down level next
     // needs COUNT + WRITE.
-    c->acount = s1;
-    c->aedges = s2;
-    choose_next(a, c, s1, s2, false);
+    h.acount = s1;
+    h.aedges = s2;
+    choose_next(a, h, s1, s2, false);
     return;
   }
   if (phase == kBCount) {
-    c->live = s3;
-    c->acount = s0;
-    c->aedges = s1;
-    choose_next(a, c, s0, s1, true);
+    h.live = s3;
+    h.acount = s0;
+    h.aedges = s1;
+    choose_next(a, h, s0, s1, true);
     return;
   }
   // WRITE: the written list is the active list of this level.
-  c->cur = 1 - c->cur;
-  c->acount = c->pend_cnt;
-  c->aedges = c->pend_degs;
-  c->phase = kBTD;
+  h.cur = 1 - h.cur;
+  h.acount = h.pend_cnt;
+  h.aedges = h.pend_degs;
+  h.phase = kBTD;
+}
+
+// Slot k (parity = k & 1): every workgroup first applies the post of slot k-1
+// to its own copy of the loop state -- the same inputs (head[parity] and slot
+// k-1's partials) give every workgroup the same result, which workgroup 0
+// records -- and then runs the step that it scheduled.  The kernel boundary
+// between slots is the only synchronisation.  A one-workgroup post kernel
+// between the steps took 4.5 to 9 us a step.
+struct SlotLds {
+  union {
+    BHead h;
+    long long w[kBHeadWords];
+  } sh;
+  int64_t red[6][kThreads / 64];
+  int64_t base_c, base_d;
+};
+
+__global__ __launch_bounds__(kThreads, 4) void k_bslot(BArgs a, int parity) {
+  __shared__ BLds lds;
+  __shared__ SlotLds L;
+  BCtrl* c = a.ctrl;
+  const int tid = threadIdx.x;
+  const int me = blockIdx.x, G = gridDim.x;
+  const int64_t* pin = a.part + (parity ^ 1) * a.part_half;
+  // All loads of the prologue before its first wait, but for grids beyond
+  // kRound * kThreads workgroups.
+  const long long hw = reinterpret_cast<const long long*>(&c->h[parity])[min(tid, kBHeadWords - 1)];
+  const int err_in = c->slot_error;
+  int64_t t0 = 0, t1 = 0, t2 = 0, b0 = 0, b1 = 0;
+  uint64_t t3 = 0;
+  constexpr int kRound = 4;
+  for (int base = 0; base < G; base += kRound * kThreads) {
+    int64_t v[kRound][kPartWidth];
+#pragma unroll
+    for (int j = 0; j < kRound; j++) {
+      const int b = min(base + j * kThreads + tid, G - 1);
+#pragma unroll
+      for (int k = 0; k < kPartWidth; k++) v[j][k] = pin[b * kPartWidth + k];
+    }
+#pragma unroll
+    for (int j = 0; j < kRound; j++) {
+      const int b = base + j * kThreads + tid;
+      const int64_t live = b < G ? -1 : 0, pre = b < me ? -1 : 0;
+      t0 += v[j][0] & live;
+      t1 += v[j][1] & live;
+      t2 += v[j][2] & live;
+      t3 |= static_cast<uint64_t>(v[j][3] & live);
+      b0 += v[j][0] & pre;
+      b1 += v[j][1] & pre;
+    }
+  }
+  if (tid < kBHeadWords) L.sh.w[tid] = hw;
+  {
+    const int64_t r[6] = {wave_sum(t0), wave_sum(t1), wave_sum(t2), wave_sum(b0), wave_sum(b1),
+                          static_cast<int64_t>(wave_or(t3))};
+    if (lane_id() == 0) {
+#pragma unroll
+      for (int k = 0; k < 6; k++) L.red[k][tid >> 6] = r[k];
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {
+    int64_t sum[6] = {0, 0, 0, 0, 0, 0};
+    for (int w = 0; w < kThreads / 64; w++) {
+      for (int k = 0; k < 5; k++) sum[k] += L.red[k][w];
+      sum[5] |= L.red[5][w];
+    }
+    BHead& h = L.sh.h;
+    h.error |= err_in;
+    if (h.ran) post_update(a, h, me == 0 ? c : nullptr, sum[0], sum[1], sum[2], static_cast<uint64_t>(sum[5]));
+    h.ran = h.phase >= kBTD && h.phase <= kBWrite ? h.phase : 0;
+    L.base_c = sum[3];
+    L.base_d = sum[4];
+  }
+  __syncthreads();
+  if (me == 0 && tid < kBHeadWords) reinterpret_cast<long long*>(&c->h[parity ^ 1])[tid] = L.sh.w[tid];
+  const BHead& h = L.sh.h;
+  const int phase = h.ran, level = h.level;
+  if (phase == 0) return;
+  const BIo io = {h.acount, h.aedges,   h.live,   h.cur, &c->slot_error, a.part + parity * a.part_half,
+                  L.base_c, L.base_d};
+  switch (phase) {
+    case kBTD:
+      zero_next_next(a, level);
+      td_phase(a, io, lds.td, level);
+      break;
+    case kBBU:
+      zero_next_next(a, level);
+      bu_phase(a, io, lds.sm, level);
+      break;
+    case kBCount: count_or_write<false>(a, io, lds.sm, level); break;
+    default: count_or_write<true>(a, io, lds.sm, level); break;
+  }
 }
 
 // Level 0: F[0] = sources' lanes, F[1] cleared, seen cleared; active list =
@@ -649,7 +719,7 @@ __global__ void k_binit2(BArgs a, const int32_t* srcs, int nsrc) {
   // One wavefront, lane s = source s: lanes with the same local vertex
   // merge into its level-0 word; the first of them lists the vertex (if it
   // has out-edges), in source order, with the out-degree prefix.
-  BCtrl* c = a.ctrl;
+  BHead* c = &a.ctrl->h[0];
   const int s = threadIdx.x;
   const int32_t src = s < nsrc ? srcs[s] : -1;
   const int64_t lu = int64_t(src) - a.vbegin;
@@ -692,6 +762,9 @@ __global__ void k_binit2(BArgs a, const int32_t* srcs, int nsrc) {
   c->nlevels = 1;
   c->sweeps = 0;
   c->error = 0;
+  c->ran = 0;
+  c->used = 0;
+  a.ctrl->slot_error = 0;
   c->sweep_scanned_total = 0;
   if (cnt == 0) {
     c->phase = kBDone;
@@ -727,9 +800,9 @@ __device__ __forceinline__ uint64_t depth_bytes(const uint64_t* m, int g) {
 // lane s, 255 if none.  Levels are bit-sliced into eight planes (level L
 // sets lane s in plane j when bit j of L is set); an unreached lane gets
 // every plane bit, so its byte comes out as 255.
-__global__ __launch_bounds__(kThreads) void k_bdepth(BArgs a, uint8_t* out, int nsrc, const int32_t* perm) {
-  if (a.ctrl->done != 1) return;  // levels are missing: queued again behind them
-  const int nlev = a.ctrl->nlevels;
+__global__ __launch_bounds__(kThreads) void k_bdepth(BArgs a, const BHead* h, uint8_t* out, int nsrc, const int32_t* perm) {
+  if (h->done != 1) return;  // levels are missing: queued again behind them
+  const int nlev = h->nlevels;
   const int64_t gtid = int64_t(blockIdx.x) * kThreads + threadIdx.x;
   const int64_t gsize = int64_t(gridDim.x) * kThreads;
   for (int64_t v = gtid; v < a.nloc; v += gsize) {
@@ -760,10 +833,10 @@ __global__ __launch_bounds__(kThreads) void k_bdepth(BArgs a, uint8_t* out, int 
 }
 
 // Sum over lanes of the out-degrees of reached vertices (GTEPS numerator).
-__global__ __launch_bounds__(kThreads) void k_breach(BArgs a) {
+__global__ __launch_bounds__(kThreads) void k_breach(BArgs a, const BHead* h) {
   __shared__ int64_t red[kThreads / 64];
-  if (a.ctrl->done != 1) return;  // levels are missing, and a WRITE may need the partials
-  const int nlev = a.ctrl->nlevels;
+  if (h->done != 1) return;  // levels are missing, and the next slot needs the partials
+  const int nlev = h->nlevels;
   const int64_t gtid = int64_t(blockIdx.x) * kThreads + threadIdx.x;
   const int64_t gsize = int64_t(gridDim.x) * kThreads;
   int64_t acc = 0;
@@ -776,9 +849,9 @@ __global__ __launch_bounds__(kThreads) void k_breach(BArgs a) {
   if (threadIdx.x == 0) a.part[blockIdx.x * kPartWidth] = s;
 }
 
-__global__ __launch_bounds__(kThreads) void k_breach_sum(BArgs a, int nblocks, int64_t* out) {
+__global__ __launch_bounds__(kThreads) void k_breach_sum(BArgs a, const BHead* h, int nblocks, int64_t* out) {
   __shared__ int64_t red[kThreads / 64];
-  if (a.ctrl->done != 1) return;
+  if (h->done != 1) return;
   int64_t s = 0;
   for (int b = threadIdx.x; b < nblocks; b += kThreads) s += a.part[b * kPartWidth];
   s = block_sum<kThreads>(s, red);
@@ -803,6 +876,7 @@ BArgs make_args(dmm_ctx* ctx, int nsrc, int td_div) {
   a.aoff1 = ctx->d_baoff + ctx->nloc + 64;
   a.ctrl = reinterpret_cast<BCtrl*>(ctx->d_bctrl);
   a.part = ctx->d_part;
+  a.part_half = (ctx->part_cap / 2) * kPartWidth;
   a.lanes = nsrc >= 64 ? ~0ull : ((1ull << nsrc) - 1);
   a.m = std::max<int64_t>(1, ctx->m_out);
   a.td_div = std::max(1, td_div);
@@ -1289,62 +1363,70 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
   DMM_HIP_CHECK(ctx, hipMemcpyAsync(ctx->d_bsrc, ctx->h_bsrc, sizeof(int32_t) * 64, hipMemcpyHostToDevice,
                                     ctx->stream));
   for (int attempt = 0; attempt < 4; attempt++) {
-    const int gpc = p.grid_per_cu > 0 ? p.grid_per_cu : ctx->tuning.grid_per_cu;
+    const int gpc = std::min(kMaxGridPerCU, p.grid_per_cu > 0 ? p.grid_per_cu : ctx->tuning.grid_per_cu);
     const int64_t key = ((int64_t(p.td_div) * 4096 + p.graph_levels) * 128 + nsrc) * 64 + gpc;
     BArgs a = make_args(ctx, nsrc, p.td_div);
-    const int blocks = static_cast<int>(std::min<int64_t>(
-        int64_t(std::max(1, ctx->cu_count)) * std::max(1, std::min(kMaxGridPerCU, gpc)), ctx->part_cap));
-    if (!ctx->batch_graph || !ctx->batch_cont || ctx->batch_graph_key != key) {
+    const int64_t cus = std::max(1, ctx->cu_count);
+    const int blocks = static_cast<int>(
+        std::min({cus * std::max(1, gpc), ctx->part_cap / 2,
+                  std::max(cus, std::min(kBatchMostPerCU * cus, ceil_div(ctx->nloc, kBatchRows)))}));
+    // The first chain has the slots that the last runs used, and one for the
+    // last post (at most graph_levels + 1, as many as that before a run);
+    // the continuation an even number, which leaves the head's parity.
+    if (ctx->batch_graph_key != key) std::fill(std::begin(ctx->batch_recent), std::end(ctx->batch_recent), 0);
+    int most = 0;
+    for (int r : ctx->batch_recent) most = std::max(most, r);
+    const int want = most > 0 ? std::min(p.graph_levels, most) + 1 : p.graph_levels + 1;
+    if (!ctx->batch_graph || !ctx->batch_cont || ctx->batch_graph_key != key || ctx->batch_slots < want ||
+        ctx->batch_slots > want + 2) {
       if (ctx->batch_graph) (void)hipGraphExecDestroy(ctx->batch_graph);
       if (ctx->batch_cont) (void)hipGraphExecDestroy(ctx->batch_cont);
       ctx->batch_graph = ctx->batch_cont = nullptr;
-      hipGraph_t g = nullptr;
-      DMM_HIP_CHECK(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-      hipLaunchKernelGGL(k_binit, dim3(blocks), dim3(kThreads), 0, ctx->stream, a,
-                         static_cast<const int32_t*>(ctx->d_bsrc), nsrc);
-      hipLaunchKernelGGL(k_binit2, dim3(1), dim3(64), 0, ctx->stream, a,
-                         static_cast<const int32_t*>(ctx->d_bsrc), nsrc);
-      for (int i = 0; i < p.graph_levels; i++) {
-        hipLaunchKernelGGL(k_bstep, dim3(blocks), dim3(kThreads), 0, ctx->stream, a);
-        hipLaunchKernelGGL(k_bpost, dim3(1), dim3(kPostThreads), 0, ctx->stream, a, blocks);
+      for (int part = 0; part < 2; part++) {
+        constexpr int kCont = 6;
+        const int first = part == 0 ? 0 : want & 1;
+        hipGraph_t g = nullptr;
+        DMM_HIP_CHECK(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
+        if (part == 0) {
+          hipLaunchKernelGGL(k_binit, dim3(blocks), dim3(kThreads), 0, ctx->stream, a,
+                             static_cast<const int32_t*>(ctx->d_bsrc), nsrc);
+          hipLaunchKernelGGL(k_binit2, dim3(1), dim3(64), 0, ctx->stream, a,
+                             static_cast<const int32_t*>(ctx->d_bsrc), nsrc);
+        }
+        for (int i = 0; i < (part == 0 ? want : kCont); i++)
+          hipLaunchKernelGGL(k_bslot, dim3(blocks), dim3(kThreads), 0, ctx->stream, a, (first + i) & 1);
+        hipError_t e = hipStreamEndCapture(ctx->stream, &g);
+        if (e != hipSuccess) return set_err(ctx, DMM_ERR_HIP, "batch capture failed: %s", hipGetErrorString(e));
+        e = hipGraphInstantiate(part == 0 ? &ctx->batch_graph : &ctx->batch_cont, g, nullptr, nullptr, 0);
+        (void)hipGraphDestroy(g);
+        if (e != hipSuccess) return set_err(ctx, DMM_ERR_HIP, "batch instantiate failed: %s", hipGetErrorString(e));
       }
-      hipError_t e = hipStreamEndCapture(ctx->stream, &g);
-      if (e != hipSuccess) return set_err(ctx, DMM_ERR_HIP, "batch capture failed: %s", hipGetErrorString(e));
-      e = hipGraphInstantiate(&ctx->batch_graph, g, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(g);
-      if (e != hipSuccess) return set_err(ctx, DMM_ERR_HIP, "batch instantiate failed: %s", hipGetErrorString(e));
-      DMM_HIP_CHECK(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-      for (int i = 0; i < 6; i++) {
-        hipLaunchKernelGGL(k_bstep, dim3(blocks), dim3(kThreads), 0, ctx->stream, a);
-        hipLaunchKernelGGL(k_bpost, dim3(1), dim3(kPostThreads), 0, ctx->stream, a, blocks);
-      }
-      e = hipStreamEndCapture(ctx->stream, &g);
-      if (e != hipSuccess) return set_err(ctx, DMM_ERR_HIP, "batch capture failed: %s", hipGetErrorString(e));
-      e = hipGraphInstantiate(&ctx->batch_cont, g, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(g);
-      if (e != hipSuccess) return set_err(ctx, DMM_ERR_HIP, "batch instantiate failed: %s", hipGetErrorString(e));
       ctx->batch_graph_key = key;
+      ctx->batch_slots = want;
     }
-    BCtrl* h = reinterpret_cast<BCtrl*>(ctx->h_bctrl);
-    int64_t* h_reached = reinterpret_cast<int64_t*>(h + 1);
+    BCtrl* const hc = reinterpret_cast<BCtrl*>(ctx->h_bctrl);
+    int64_t* h_reached = reinterpret_cast<int64_t*>(hc + 1);
+    const int par = ctx->batch_slots & 1;  // the head that the last slot wrote
+    const BHead* const h = &hc->h[par];
+    const BHead* const d_head = &reinterpret_cast<const BCtrl*>(ctx->d_bctrl)->h[par];
     // What follows the levels is queued behind them, before it is known that
     // they are done (it reads only the state they left): one wait for all,
     // and again in the rare case that levels were missing.
     auto finish = [&]() -> int {
       DMM_HIP_CHECK(ctx, hipEventRecord(ctx->ev_b, ctx->stream));
       if (want_depth) {
-        hipLaunchKernelGGL(k_bdepth, dim3(blocks), dim3(kThreads), 0, ctx->stream, a, ctx->d_bdepth, nsrc,
+        hipLaunchKernelGGL(k_bdepth, dim3(blocks), dim3(kThreads), 0, ctx->stream, a, d_head, ctx->d_bdepth, nsrc,
                            ctx->relabeled ? static_cast<const int32_t*>(ctx->d_perm) : nullptr);
         DMM_HIP_CHECK(ctx, hipEventRecord(ctx->ev_b, ctx->stream));
       }
       if (stats) {
-        hipLaunchKernelGGL(k_breach, dim3(blocks), dim3(kThreads), 0, ctx->stream, a);
-        hipLaunchKernelGGL(k_breach_sum, dim3(1), dim3(kThreads), 0, ctx->stream, a, blocks, ctx->d_scratch64);
+        hipLaunchKernelGGL(k_breach, dim3(blocks), dim3(kThreads), 0, ctx->stream, a, d_head);
+        hipLaunchKernelGGL(k_breach_sum, dim3(1), dim3(kThreads), 0, ctx->stream, a, d_head, blocks, ctx->d_scratch64);
         DMM_HIP_CHECK(ctx, hipMemcpyAsync(h_reached, ctx->d_scratch64, sizeof(int64_t), hipMemcpyDeviceToHost,
                                           ctx->stream));
       }
       DMM_HIP_CHECK(ctx, hipGetLastError());
-      DMM_HIP_CHECK(ctx, hipMemcpyAsync(h, ctx->d_bctrl, sizeof(BCtrl), hipMemcpyDeviceToHost, ctx->stream));
+      DMM_HIP_CHECK(ctx, hipMemcpyAsync(hc, ctx->d_bctrl, sizeof(BCtrl), hipMemcpyDeviceToHost, ctx->stream));
       DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
       return DMM_OK;
     };
@@ -1379,8 +1461,8 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
       stats->sweeps = h->sweeps;
       const int nl = std::min(h->level, DMM_MAX_STEPS);
       for (int i = 0; i < nl; i++) {
-        stats->level_kind[i] = h->level_kind[i];
-        stats->level_active[i] = h->level_active[i];
+        stats->level_kind[i] = hc->level_kind[i];
+        stats->level_active[i] = hc->level_active[i];
       }
       // Sweep bytes: per sweep, seen + F[L][u] reads, offsets, F[L+1] and
       // seen writes (40 N + 8) plus 12 bytes per scanned edge (4 B ID +
@@ -1389,6 +1471,7 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
           h->sweeps * (40 * ctx->nloc + 8) + 12 * static_cast<int64_t>(h->sweep_scanned_total);
       stats->sweep_ms = 0;
     }
+    ctx->batch_recent[ctx->batch_recent_pos++ % kBatchRecent] = h->used;
     ctx->batch_valid = true;
     ctx->batch_last_level = h->level;
     if (stats) stats->reached_edges = *h_reached;

@@ -98,6 +98,7 @@ enum : int {
   kPhaseDone = 5,
 };
 
+constexpr int kBatchRecent = 8;  // batched runs sizing the next chain of slots
 constexpr int kReadSlots = 8;  // pieces of a read in flight (readout.hip)
 
 struct PrCtrl {
@@ -300,6 +301,9 @@ struct dmm_ctx {
   void* d_blkctrl = nullptr;        // block level control
   bool push_ready = false;
   int64_t batch_graph_key = -1;
+  int batch_slots = 0;              // slots of batch_graph
+  int batch_recent[dmm::kBatchRecent] = {};  // slots used by the last runs with its key
+  int batch_recent_pos = 0;
 
   dmm::Tuning tuning;
 };
