@@ -246,3 +246,21 @@ def test_batch_wide_rows_and_dead_lanes(dmm, orc, hub, directed):
             for i, s in enumerate(srcs):
                 ref = orc.bfs_depth(og, int(s))
                 assert np.array_equal(depth[i], np.where(ref < 0, 255, ref).astype(np.uint8)), (i, s, td_div)
+
+
+@pytest.mark.parametrize("graph_levels", [1, 6, 17])
+@pytest.mark.parametrize("td_div", [1, 1000000])
+def test_batch_chain_sized_by_the_last_runs(dmm, orc, graph_levels, td_div):
+    """Short and long searches in turn, past the number of runs that size the
+    launch chain: the chain grows, shrinks and is continued from either half
+    of the loop state, with the same depths and levels every time."""
+    n = 160
+    g = csr_from_pairs(dmm, np.stack((np.arange(n - 1), np.arange(1, n)), 1), n, symmetrize=False)
+    og = orc.CSR.of(g)
+    with dmm.Context(0) as c:
+        c.upload(g)
+        for first in [n - 1, 0, n - 2, n - 3, 100, n - 2] + [n - 4] * 9 + [3, n - 1, 90, 91, 0]:
+            srcs = np.array([first, n - 1, min(first + 7, n - 1)], np.int32)
+            depth, st = c.bfs_batch64(srcs, td_div=td_div, graph_levels=graph_levels)
+            assert np.array_equal(depth, expected(orc, og, srcs)), first
+            assert st.num_levels == n - first, first
