@@ -265,6 +265,13 @@ __device__ void td_phase(const BArgs& a, const BIo& io, TdLds& L, int level) {
 // reads kGroup edges (rows whose needed lanes are all found there stop
 // early), later rounds keep kUnroll frontier-word loads in flight per lane;
 // the group ORs them and the scan stops once every needed lane is found.
+// Up to kShort rounds stay short while those before found half of the needed
+// lanes: a dense frontier then gives the others to the next few edges.  Where
+// the words miss L2 (from kSweepFar vertices on; a sweep is bound by the lines
+// fetched, 1.86 ms for 118 M edges) every edge not read counts: 3.7 M uniform
+// vertices, 64 lanes, whole call with 1, 2, 4, 8 short rounds 7.60, 7.22,
+// 6.94, 7.00 ms.  Where they do not, the rounds' latency does: 120 K vertices
+// 308 us with one, 315 with four.  Kronecker graphs the same.
 // The whole-graph sweep uses kSweepUnroll (16 leaves registers for five
 // workgroups per CU; 32: four, 3% slower on Kronecker graphs); the PE-block
 // kernels, which probe the non-zero bitmaps first and stop earlier, use
@@ -275,7 +282,9 @@ __device__ void td_phase(const BArgs& a, const BIo& io, TdLds& L, int level) {
 // Returns the end of the examined range; *found = the needed lanes found.
 constexpr int kSweepUnroll = 16;
 constexpr int kBlockUnroll = 4;
-template <int kUnroll>
+constexpr int kSweepShort = 4;
+constexpr int64_t kSweepFar = int64_t(1) << 19;  // 4 MB of words
+template <int kUnroll, int kShort>
 __device__ __forceinline__ int64_t sweep_row(const int32_t* __restrict__ in_nbr, int64_t b, int64_t e,
                                              int sub, uint64_t need, const uint64_t* __restrict__ front,
                                              const uint64_t* __restrict__ nz, const uint64_t* __restrict__ nz2,
@@ -283,7 +292,8 @@ __device__ __forceinline__ int64_t sweep_row(const int32_t* __restrict__ in_nbr,
   uint64_t acc = 0;
   int64_t stop = e;
   int64_t k0 = b;
-  {
+  const int64_t least = min<int64_t>(e, b + kGroup * kShort);
+  do {
     const int64_t k = k0 + sub;
     int32_t v = k < e ? in_nbr[k] : -1;
     if (nz && v >= 0 && !((nz2[v >> 12] >> ((v >> 6) & 63)) & 1ull)) v = -1;
@@ -296,7 +306,7 @@ __device__ __forceinline__ int64_t sweep_row(const int32_t* __restrict__ in_nbr,
       *found = acc & need;
       return min<int64_t>(k0, e);
     }
-  }
+  } while (kShort > 1 && k0 < least && 2 * __popcll(acc & need) >= __popcll(need));
   for (; k0 < e; k0 += kGroup * kUnroll) {
     int32_t v[kUnroll];
 #pragma unroll
@@ -369,6 +379,7 @@ __device__ __forceinline__ int64_t wide_row(const int32_t* __restrict__ in_nbr, 
   return min(k0, e);
 }
 
+template <bool kFar>
 __device__ void bu_phase(const BArgs& a, const BIo& io, SmallLds& L, int level) {
   const uint64_t* __restrict__ Fl = a.levels + level * a.nloc;
   uint64_t* __restrict__ Fn = a.levels + (level + 1) * a.nloc;
@@ -445,7 +456,7 @@ __device__ void bu_phase(const BArgs& a, const BIo& io, SmallLds& L, int level) 
     const uint64_t need = lanes & ~s;
     uint64_t nxt = 0;
     if (need && h.e > h.b) {
-      const int64_t stop = sweep_row<kSweepUnroll>(in_nbr, h.b, h.e, sub, need, Fl, nullptr, nullptr, &nxt);
+      const int64_t stop = sweep_row<kSweepUnroll, kFar ? kSweepShort : 1>(in_nbr, h.b, h.e, sub, need, Fl, nullptr, nullptr, &nxt);
       if (sub == 0) scanned += stop - h.b;
     }
     // Out-degree of a found row: its in-row length when in-CSR == out-CSR.
@@ -625,6 +636,7 @@ struct SlotLds {
   int64_t base_c, base_d;
 };
 
+template <bool kFar>
 __global__ __launch_bounds__(kThreads, 4) void k_bslot(BArgs a, int parity) {
   __shared__ BLds lds;
   __shared__ SlotLds L;
@@ -696,7 +708,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_bslot(BArgs a, int parity) {
       break;
     case kBBU:
       zero_next_next(a, level);
-      bu_phase(a, io, lds.sm, level);
+      bu_phase<kFar>(a, io, lds.sm, level);
       break;
     case kBCount: count_or_write<false>(a, io, lds.sm, level); break;
     default: count_or_write<true>(a, io, lds.sm, level); break;
@@ -932,7 +944,7 @@ __global__ __launch_bounds__(kThreads) void k_block_sweep(const BlockCtrl* ctrl,
     const int64_t b = in_off[u], e = in_off[u + 1];
     uint64_t nxt = 0;
     if (need && e > b && e - b <= kBlockSplit) {
-      const int64_t stop = sweep_row<kBlockUnroll>(in_nbr, b, e, sub, need, front, fnz, fnz2, &nxt);
+      const int64_t stop = sweep_row<kBlockUnroll, 1>(in_nbr, b, e, sub, need, front, fnz, fnz2, &nxt);
       scanned += stop - b;
     }
     if (sub == 0) next[u] = nxt;
@@ -984,7 +996,7 @@ __global__ __launch_bounds__(kThreads) void k_block_segs(const BlockCtrl* ctrl, 
     const uint64_t need = ~seen[sg.row] & ~done;
     if (!need) continue;
     uint64_t nxt = 0;
-    const int64_t stop = sweep_row<kBlockUnroll>(in_nbr, sg.b, sg.e, sub, need, front, fnz, fnz2, &nxt);
+    const int64_t stop = sweep_row<kBlockUnroll, 1>(in_nbr, sg.b, sg.e, sub, need, front, fnz, fnz2, &nxt);
     scanned += stop - sg.b;
     if (sub == 0 && nxt)
       atomicOr(reinterpret_cast<unsigned long long*>(&next[sg.row]), static_cast<unsigned long long>(nxt));
@@ -1382,6 +1394,7 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
       if (ctx->batch_graph) (void)hipGraphExecDestroy(ctx->batch_graph);
       if (ctx->batch_cont) (void)hipGraphExecDestroy(ctx->batch_cont);
       ctx->batch_graph = ctx->batch_cont = nullptr;
+      const auto slot = ctx->nloc >= kSweepFar ? k_bslot<true> : k_bslot<false>;
       for (int part = 0; part < 2; part++) {
         constexpr int kCont = 6;
         const int first = part == 0 ? 0 : want & 1;
@@ -1394,7 +1407,7 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
                              static_cast<const int32_t*>(ctx->d_bsrc), nsrc);
         }
         for (int i = 0; i < (part == 0 ? want : kCont); i++)
-          hipLaunchKernelGGL(k_bslot, dim3(blocks), dim3(kThreads), 0, ctx->stream, a, (first + i) & 1);
+          hipLaunchKernelGGL(slot, dim3(blocks), dim3(kThreads), 0, ctx->stream, a, (first + i) & 1);
         hipError_t e = hipStreamEndCapture(ctx->stream, &g);
         if (e != hipSuccess) return set_err(ctx, DMM_ERR_HIP, "batch capture failed: %s", hipGetErrorString(e));
         e = hipGraphInstantiate(part == 0 ? &ctx->batch_graph : &ctx->batch_cont, g, nullptr, nullptr, 0);

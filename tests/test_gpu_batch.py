@@ -264,3 +264,23 @@ def test_batch_chain_sized_by_the_last_runs(dmm, orc, graph_levels, td_div):
             depth, st = c.bfs_batch64(srcs, td_div=td_div, graph_levels=graph_levels)
             assert np.array_equal(depth, expected(orc, og, srcs)), first
             assert st.num_levels == n - first, first
+
+
+@pytest.mark.parametrize("n", [(1 << 19) - 1, 1 << 19, 700001])
+@pytest.mark.parametrize("directed", [False, True])
+def test_batch_words_beyond_l2(dmm, orc, n, directed):
+    """The sweep of graphs whose frontier words miss L2, at its size limit:
+    rows of every class, and lanes found after any number of rounds."""
+    rng = np.random.default_rng([n, directed])
+    hub = np.stack((rng.integers(0, n, 6000), np.full(6000, 5)), 1)
+    mid = np.stack((rng.integers(0, n, 900), np.full(900, n - 7)), 1)
+    g = csr_from_pairs(dmm, np.concatenate((rng.integers(0, n, (6 * n, 2)), hub, mid)), n, symmetrize=not directed)
+    og = orc.CSR.of(g)
+    srcs = rng.integers(0, n, 64).astype(np.int32)
+    with dmm.Context(0) as c:
+        c.upload(g)
+        for td_div in (1, 20, 1000000):
+            depth, _ = c.bfs_batch64(srcs, td_div=td_div)
+            for i in (0, 1, 31, 62, 63):
+                ref = orc.bfs_depth(og, int(srcs[i]))
+                assert np.array_equal(depth[i], np.where(ref < 0, 255, ref).astype(np.uint8)), (i, td_div)
