@@ -69,7 +69,7 @@ struct BHead {
   int error;
   int ran;                            // the phase the slot ran, its post pending
   int used;                           // slots that ran one
-  int pad;
+  int nz_level;                       // the level whose non-zero words a COUNT marked
 };
 constexpr int kBHeadWords = sizeof(BHead) / 8;
 static_assert(sizeof(BHead) % 8 == 0 && kBHeadWords <= 64, "a head is copied as 8-byte words by one wave");
@@ -86,6 +86,7 @@ struct BCtrl {
 struct BIo {
   int64_t acount, aedges;
   uint64_t live;
+  const uint64_t* nz;                 // non-zero words of F[level], or NULL
   int cur;
   int* error;
   int64_t* part;                      // this slot's partials [gridDim.x][kPartWidth]
@@ -106,6 +107,7 @@ struct BArgs {
   int32_t* act1;
   int64_t* aoff0;
   int64_t* aoff1;
+  uint64_t* nz;       // bit per vertex
   BCtrl* ctrl;
   int64_t* part;      // [2][gridDim.x][kPartWidth], the slots' in turn
   int64_t part_half;  // offset of the second
@@ -276,13 +278,19 @@ __device__ void td_phase(const BArgs& a, const BIo& io, TdLds& L, int level) {
 // workgroups per CU; 32: four, 3% slower on Kronecker graphs); the PE-block
 // kernels, which probe the non-zero bitmaps first and stop earlier, use
 // kBlockUnroll.  nz (may be NULL) is a non-zero bitmap of the frontier words
-// (bit v), with a summary bitmap nz2 (bit w set iff nz word w != 0, so 256 KB
-// for 2^27 vertices, resident in L2); both are probed before a word load, so
-// sparse frontiers cost one L2 probe per edge.
+// (bit v), with a summary bitmap nz2 (may be NULL; bit w set iff nz word w
+// != 0, so 256 KB for 2^27 vertices, resident in L2); both are probed before a
+// word load, so sparse frontiers cost one L2 probe per edge.  The whole-graph
+// sweep probes nz where the words miss L2, the step before was a COUNT (which
+// reads the words and marks them) and fewer than kNzPart8 eighths of the rows are
+// listed: a probe costs a third of a far word (200 against 64 G/s).  3.7 M
+// uniform vertices, 43% listed at the first sweep: 1.86 -> 1.05 ms, whole
+// call 6.85 -> 6.1 ms; Kronecker 900 K 1.40 ms with and without.
 // Returns the end of the examined range; *found = the needed lanes found.
 constexpr int kSweepUnroll = 16;
 constexpr int kBlockUnroll = 4;
 constexpr int kSweepShort = 4;
+constexpr int kNzPart8 = 5;                         // eighths
 constexpr int64_t kSweepFar = int64_t(1) << 19;  // 4 MB of words
 template <int kUnroll, int kShort>
 __device__ __forceinline__ int64_t sweep_row(const int32_t* __restrict__ in_nbr, int64_t b, int64_t e,
@@ -296,7 +304,7 @@ __device__ __forceinline__ int64_t sweep_row(const int32_t* __restrict__ in_nbr,
   do {
     const int64_t k = k0 + sub;
     int32_t v = k < e ? in_nbr[k] : -1;
-    if (nz && v >= 0 && !((nz2[v >> 12] >> ((v >> 6) & 63)) & 1ull)) v = -1;
+    if (nz2 && v >= 0 && !((nz2[v >> 12] >> ((v >> 6) & 63)) & 1ull)) v = -1;
     if (nz && v >= 0 && !((nz[v >> 6] >> (v & 63)) & 1ull)) v = -1;
     if (v >= 0) acc |= front[v];
 #pragma unroll
@@ -316,7 +324,7 @@ __device__ __forceinline__ int64_t sweep_row(const int32_t* __restrict__ in_nbr,
     }
     if (nz) {
 #pragma unroll
-      for (int j = 0; j < kUnroll; j++)
+      for (int j = 0; nz2 && j < kUnroll; j++)
         if (v[j] >= 0 && !((nz2[v[j] >> 12] >> ((v[j] >> 6) & 63)) & 1ull)) v[j] = -1;
 #pragma unroll
       for (int j = 0; j < kUnroll; j++)
@@ -343,8 +351,8 @@ __device__ __forceinline__ int64_t sweep_row(const int32_t* __restrict__ in_nbr,
 constexpr int kWideUnroll = 8;
 template <int kWaves>
 __device__ __forceinline__ int64_t wide_row(const int32_t* __restrict__ in_nbr, int64_t b, int64_t e, uint64_t need,
-                                            const uint64_t* __restrict__ front, uint64_t (*red)[kThreads / 64],
-                                            int& buf, uint64_t* found) {
+                                            const uint64_t* __restrict__ front, const uint64_t* __restrict__ nz,
+                                            uint64_t (*red)[kThreads / 64], int& buf, uint64_t* found) {
   constexpr int64_t kRound = int64_t(kWaves) * 64 * kWideUnroll;
   const int t = kWaves == 1 ? lane_id() : static_cast<int>(threadIdx.x);
   uint64_t acc = 0;
@@ -357,8 +365,17 @@ __device__ __forceinline__ int64_t wide_row(const int32_t* __restrict__ in_nbr, 
       v[j] = in_nbr[min(k, e - 1)];  // past the end the last edge again
     }
     uint64_t x = 0;
+    if (nz) {
 #pragma unroll
-    for (int j = 0; j < kWideUnroll; j++) x |= front[v[j]];
+      for (int j = 0; j < kWideUnroll; j++)
+        if (!((nz[v[j] >> 6] >> (v[j] & 63)) & 1ull)) v[j] = -1;
+#pragma unroll
+      for (int j = 0; j < kWideUnroll; j++)
+        if (v[j] >= 0) x |= front[v[j]];
+    } else {
+#pragma unroll
+      for (int j = 0; j < kWideUnroll; j++) x |= front[v[j]];
+    }
     x = wave_or(x);
     if (kWaves > 1) {
       // The words alternate, so one barrier separates their uses.
@@ -404,7 +421,7 @@ __device__ void bu_phase(const BArgs& a, const BIo& io, SmallLds& L, int level) 
     int64_t ex = 0;
     if (need) {
       const int64_t b = in_off[u];
-      ex = wide_row<waves.value>(in_nbr, b, in_off[u + 1], need, Fl, L.found, buf, &nxt) - b;
+      ex = wide_row<waves.value>(in_nbr, b, in_off[u + 1], need, Fl, kFar ? io.nz : nullptr, L.found, buf, &nxt) - b;
     }
     if (writer) {
       scanned += ex;
@@ -456,7 +473,7 @@ __device__ void bu_phase(const BArgs& a, const BIo& io, SmallLds& L, int level) 
     const uint64_t need = lanes & ~s;
     uint64_t nxt = 0;
     if (need && h.e > h.b) {
-      const int64_t stop = sweep_row<kSweepUnroll, kFar ? kSweepShort : 1>(in_nbr, h.b, h.e, sub, need, Fl, nullptr, nullptr, &nxt);
+      const int64_t stop = sweep_row<kSweepUnroll, kFar ? kSweepShort : 1>(in_nbr, h.b, h.e, sub, need, Fl, kFar ? io.nz : nullptr, nullptr, &nxt);
       if (sub == 0) scanned += stop - h.b;
     }
     // Out-degree of a found row: its in-row length when in-CSR == out-CSR.
@@ -499,20 +516,25 @@ __device__ void bu_phase(const BArgs& a, const BIo& io, SmallLds& L, int level) 
 
 // COUNT / WRITE over the frontier words F[level]: contiguous vertex ranges
 // per workgroup in ascending order; listed = nonzero word and out-degree >= 1.
-template <bool kWrite>
+template <bool kWrite, bool kFar>
 __device__ void count_or_write(const BArgs& a, const BIo& io, SmallLds& L, int level) {
   // Workgroup b owns the contiguous range [v0, v1) and walks it in tiles
   // of kThreads consecutive vertices (coalesced); WRITE orders entries by
   // a block scan per tile on top of the workgroup's prefix.
   // Levels >= 1 have no lanes from bend on.
   const uint64_t* Fl = a.levels + level * a.nloc;
-  const int64_t vpb = (a.bend + gridDim.x - 1) / gridDim.x;
+  const int64_t vpb = (a.bend + int64_t(gridDim.x) * 64 - 1) / (int64_t(gridDim.x) * 64) * 64;
   const int64_t v0 = min(a.bend, int64_t(blockIdx.x) * vpb), v1 = min(a.bend, v0 + vpb);
   if (!kWrite) {
     int64_t cnt = 0, degs = 0;
     uint64_t any = 0;
-    for (int64_t u = v0 + threadIdx.x; u < v1; u += kThreads) {
-      const uint64_t f = Fl[u];
+    for (int64_t t = v0; t < v1; t += kThreads) {
+      const int64_t u = t + threadIdx.x;
+      const uint64_t f = u < v1 ? Fl[u] : 0;
+      if (kFar) {
+        const uint64_t w = __ballot(f != 0);
+        if (lane_id() == 0 && u < v1) a.nz[u >> 6] = w;
+      }
       any |= f;
       if (f) {
         const int64_t d = a.out_off[u + 1] - a.out_off[u];
@@ -608,6 +630,7 @@ __device__ void post_update(const BArgs& a, BHead& h, BCtrl* c, int64_t s0, int6
     return;
   }
   if (phase == kBCount) {
+    h.nz_level = level;
     h.live = s3;
     h.acount = s0;
     h.aedges = s1;
@@ -699,7 +722,8 @@ __global__ __launch_bounds__(kThreads, 4) void k_bslot(BArgs a, int parity) {
   const BHead& h = L.sh.h;
   const int phase = h.ran, level = h.level;
   if (phase == 0) return;
-  const BIo io = {h.acount, h.aedges,   h.live,   h.cur, &c->slot_error, a.part + parity * a.part_half,
+  const uint64_t* nz = kFar && h.nz_level == level && 8 * h.acount < kNzPart8 * a.bend ? a.nz : nullptr;
+  const BIo io = {h.acount, h.aedges,   h.live,   nz, h.cur, &c->slot_error, a.part + parity * a.part_half,
                   L.base_c, L.base_d};
   switch (phase) {
     case kBTD:
@@ -710,8 +734,8 @@ __global__ __launch_bounds__(kThreads, 4) void k_bslot(BArgs a, int parity) {
       zero_next_next(a, level);
       bu_phase<kFar>(a, io, lds.sm, level);
       break;
-    case kBCount: count_or_write<false>(a, io, lds.sm, level); break;
-    default: count_or_write<true>(a, io, lds.sm, level); break;
+    case kBCount: count_or_write<false, kFar>(a, io, lds.sm, level); break;
+    default: count_or_write<true, kFar>(a, io, lds.sm, level); break;
   }
 }
 
@@ -725,6 +749,8 @@ __global__ __launch_bounds__(kThreads) void k_binit(BArgs a, const int32_t* srcs
     a.levels[i] = 0;
     if (a.level_cap > 1) a.levels[a.nloc + i] = 0;
   }
+  // COUNT marks the words of rows below bend only.
+  for (int64_t i = gtid; i < (a.nloc + 63) / 64; i += gsize) a.nz[i] = 0;
 }
 
 __global__ void k_binit2(BArgs a, const int32_t* srcs, int nsrc) {
@@ -776,6 +802,7 @@ __global__ void k_binit2(BArgs a, const int32_t* srcs, int nsrc) {
   c->error = 0;
   c->ran = 0;
   c->used = 0;
+  c->nz_level = -1;
   a.ctrl->slot_error = 0;
   c->sweep_scanned_total = 0;
   if (cnt == 0) {
@@ -886,6 +913,7 @@ BArgs make_args(dmm_ctx* ctx, int nsrc, int td_div) {
   a.act1 = ctx->d_bact + ctx->nloc + 64;
   a.aoff0 = ctx->d_baoff;
   a.aoff1 = ctx->d_baoff + ctx->nloc + 64;
+  a.nz = ctx->d_seen + ctx->nloc;
   a.ctrl = reinterpret_cast<BCtrl*>(ctx->d_bctrl);
   a.part = ctx->d_part;
   a.part_half = (ctx->part_cap / 2) * kPartWidth;

@@ -311,7 +311,8 @@ int ensure_pr_state(dmm_ctx* ctx, int mode) {
 int ensure_batch_state(dmm_ctx* ctx) {
   int rc;
   if (!ctx->d_seen) {
-    if ((rc = dmm::dev_alloc(ctx, (void**)&ctx->d_seen, sizeof(uint64_t) * ctx->nloc, "batch seen"))) return rc;
+    if ((rc = dmm::dev_alloc(ctx, (void**)&ctx->d_seen, sizeof(uint64_t) * (ctx->nloc + dmm::ceil_div(ctx->nloc, 64)),
+                             "batch seen"))) return rc;
     if ((rc = dmm::dev_alloc(ctx, (void**)&ctx->d_bact, sizeof(int32_t) * 2 * (ctx->nloc + 64), "batch lists")))
       return rc;
     if ((rc = dmm::dev_alloc(ctx, (void**)&ctx->d_baoff, sizeof(int64_t) * 2 * (ctx->nloc + 64), "batch lists")))
