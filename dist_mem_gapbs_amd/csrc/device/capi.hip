@@ -883,7 +883,7 @@ int dmm_bfs_read(dmm_ctx* ctx, int32_t* parent, int32_t* depth) {
     return set_err(ctx, DMM_ERR_STATE, "the last BFS did not track depths (pass a depth buffer to dmm_bfs)");
   const int32_t* dp = ctx->relabeled ? ctx->d_parent_out : ctx->d_parent;
   const int32_t* dd = ctx->relabeled ? ctx->d_depth_out : ctx->d_depth;
-  const dmm::ReadPart parts[] = {{parent, dp, sizeof(int32_t) * ctx->nloc}, {depth, dd, sizeof(int32_t) * ctx->nloc, ctx->relabeled}};
+  const dmm::ReadPart parts[] = {{parent, dp, sizeof(int32_t) * ctx->nloc}, {depth, dd, sizeof(int32_t) * ctx->nloc}};
   return dmm::read_out(ctx, parts, 2);
 }
 

@@ -99,7 +99,8 @@ enum : int {
 };
 
 constexpr int kBatchRecent = 8;  // batched runs sizing the next chain of slots
-constexpr int kReadSlots = 8;  // pieces of a read in flight (readout.hip)
+constexpr int kReadSlots = 8;    // pieces of a read in flight (readout.hip)
+constexpr int kReadGroups = 32;  // workgroups that store them
 
 struct PrCtrl {
   double err;          // L1 change of the last iteration
@@ -248,7 +249,7 @@ struct dmm_ctx {
   dmm::PrCtrl* h_prctrl = nullptr;
   char* h_ring = nullptr;        // pinned staging of reads (readout.hip)
   size_t ring_bytes = 0;
-  hipEvent_t ring_events[dmm::kReadSlots] = {};
+  uint32_t read_seq = 0;         // the last piece read
   int32_t* d_heavy = nullptr;    // vertices with in-degree >= heavy threshold, longest class first
   int64_t n_heavy = 0;
   int64_t n_giant = 0, n_wide = 0;  // its leading rows of kSweepGiant and, after them, kSweepWide in-edges and more
@@ -330,7 +331,6 @@ struct ReadPart {
   void* dst;
   const void* src;
   size_t bytes;
-  bool joined = false;  // src follows the previous part's in the same allocation
 };
 int read_out(dmm_ctx* ctx, const ReadPart* parts, int nparts);
 void read_free(dmm_ctx* ctx);

@@ -2,14 +2,10 @@
 //
 // hipMemcpyAsync to pageable memory stages through the runtime's own pinned
 // buffer, a piece and a wait at a time (16 MB: 0.98 ms).  Here a read is cut
-// into pieces that come by DMA (45 GB/s) into a ring of pinned slots, all
-// queued at once as far as the ring goes, and go from there to the buffer by
-// up to kReaders threads while the next pieces arrive (0.48 ms).  The threads
-// matter most where the buffer's pages are new (64 MB of them: 16 ms by one
-// thread, 6.4 ms by four).  Whole calls before and after: depths of 64 sources
-// on 131 K vertices (8 MB) 760 -> 600 us, three level words of 3.7 M vertices
-// (89 MB) 12.4 -> 7.6 ms, 64 searches on Kronecker-22 with one result read
-// (32 MB) 17.4 -> 14.6 ms.
+// into pieces that a kernel stores into a ring of pinned slots, as far as the
+// ring goes in one launch; up to kReaders threads carry them to the buffer
+// while the next pieces arrive.  The threads matter most where the buffer's
+// pages are new (64 MB of them: 16 ms by one thread, 6.4 ms by four).
 #include <algorithm>
 #include <atomic>
 #include <cstring>
@@ -24,22 +20,65 @@ namespace dmm {
 
 namespace {
 
-// A piece: an eighth of the read, between these (a DMA takes some 10 us to set
-// up: 1.6 MB of a search's results in pieces of 256 KB, 512 KB, 1 MB: 260,
-// 224, 209 us for the whole call).  A context holds at most kReadSlots of
-// the larger, 16 MB, pinned.
-constexpr size_t kPieceLeast = size_t(1) << 20;
-constexpr size_t kSmallRead = size_t(512) << 10;  // up to here one wait for all of it
+// A piece: an eighth of the read, between these.  A context holds at most
+// kReadSlots of the larger, 16 MB, pinned.
+constexpr size_t kPieceLeast = size_t(256) << 10;
 constexpr size_t kPieceMost = size_t(2) << 20;
-constexpr size_t kThreadedRead = size_t(2) << 20;       // helpers from here on: starting one costs some 15 us
+constexpr size_t kSmallRead = size_t(512) << 10;    // up to here one wait for all of it
+constexpr size_t kThreadedRead = size_t(2) << 20;  // helpers from here on: starting one costs some 15 us
 constexpr int kReaders = 4;
+constexpr int64_t kGroupLeast = int64_t(16) << 10;  // of a small read, by each workgroup
+constexpr int kThreads = 256;
+constexpr int kUnroll = 4;
+constexpr size_t kFlagBytes = 4096;  // the slots behind them start on a page
+static_assert(sizeof(uint32_t) * kReadSlots * kReadGroups <= kFlagBytes, "flags of every workgroup and slot");
 
 struct Piece {
   char* dst;
   const char* src;
   size_t bytes;
-  bool joined;
 };
+
+struct ReadList {
+  const char* src[kReadSlots];
+  uint32_t bytes[kReadSlots];
+};
+
+// n pieces into the slots from `slot` on, one after the other, each by all
+// workgroups.  Bound by the link (PCIe, 56 GB/s).  A workgroup whose part of a
+// piece has been stored says so in its own pinned flag, so a piece needs
+// neither an event nor a copy command of its own: with those, every 2 MB
+// (37 us) were followed by 10 us in which nothing moved.  each: every piece
+// has its flags, else the last, for all.  Copy commands, then this: depths of
+// 64 sources on 131 K vertices (8 MB) 541 -> 448 us a call, path counts of
+// 480 K vertices (9.6 MB) 553 -> 467, a search's 32 MB 902 -> 780 (the read);
+// up to 512 KB the same.  16, 32, 64, 128 workgroups: 453, 448, 461, 490 us.
+__global__ __launch_bounds__(kThreads) void k_read(ReadList l, int n, char* slot, size_t slot_bytes, uint32_t* flags,
+                                                   uint32_t seq, bool each) {
+  const uint32_t t = blockIdx.x * kThreads + threadIdx.x;
+  const uint32_t step = gridDim.x * kThreads;
+  for (int p = 0; p < n; p++, slot += slot_bytes, flags += kReadGroups) {
+    const char* __restrict__ src = l.src[p];
+    const uint32_t words = l.bytes[p] / 16;
+    uint4* out = reinterpret_cast<uint4*>(slot);
+    for (uint32_t i = t; i < words; i += kUnroll * step) {
+      uint4 v[kUnroll];
+#pragma unroll
+      for (int j = 0; j < kUnroll; j++)  // a part may start at any byte
+        __builtin_memcpy(&v[j], src + size_t(min(i + j * step, words - 1)) * 16, 16);
+#pragma unroll
+      for (int j = 0; j < kUnroll; j++)
+        if (i + j * step < words) out[i + j * step] = v[j];
+    }
+    const uint32_t tail = words * 16 + t;
+    if (tail < l.bytes[p]) slot[tail] = src[tail];
+    if (!each && p + 1 < n) continue;
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0)
+      __hip_atomic_store(&flags[blockIdx.x], seq + p, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
 
 }  // namespace
 
@@ -47,10 +86,6 @@ void read_free(dmm_ctx* ctx) {
   if (ctx->h_ring) (void)hipHostFree(ctx->h_ring);
   ctx->h_ring = nullptr;
   ctx->ring_bytes = 0;
-  for (auto& e : ctx->ring_events) {
-    if (e) (void)hipEventDestroy(e);
-    e = nullptr;
-  }
 }
 
 static int read_pieces(dmm_ctx* ctx, const ReadPart* parts, int nparts) {
@@ -67,9 +102,7 @@ static int read_pieces(dmm_ctx* ctx, const ReadPart* parts, int nparts) {
     if (!parts[i].dst) continue;
     char* d = static_cast<char*>(parts[i].dst);
     const char* s = static_cast<const char*>(parts[i].src);
-    const bool joined = parts[i].joined && i > 0 && parts[i - 1].dst;
-    for (size_t o = 0; o < parts[i].bytes; o += slot)
-      pieces.push_back({d + o, s + o, std::min(slot, parts[i].bytes - o), joined && o == 0});
+    for (size_t o = 0; o < parts[i].bytes; o += slot) pieces.push_back({d + o, s + o, std::min(slot, parts[i].bytes - o)});
   }
   const int n = static_cast<int>(pieces.size());
   // Slot s holds the pieces s, s + slots, ...  The ring grows to what a read
@@ -78,56 +111,72 @@ static int read_pieces(dmm_ctx* ctx, const ReadPart* parts, int nparts) {
   if (ctx->ring_bytes < slots * slot) {
     DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
     read_free(ctx);
-    if (hipHostMalloc(reinterpret_cast<void**>(&ctx->h_ring), slots * slot, hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc(reinterpret_cast<void**>(&ctx->h_ring), kFlagBytes + slots * slot, hipHostMallocDefault) !=
+        hipSuccess) {
       ctx->h_ring = nullptr;
       (void)hipGetLastError();
     } else {
       ctx->ring_bytes = slots * slot;
+      std::memset(ctx->h_ring, 0, kFlagBytes);
+      ctx->read_seq = 0;
     }
   }
-  for (auto& e : ctx->ring_events)
-    if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-      e = nullptr;
-      (void)hipGetLastError();
-    }
-  bool direct = !ctx->h_ring;
-  for (auto& e : ctx->ring_events) direct = direct || !e;
-  if (direct) {  // no pinned memory to be had: the runtime's own path
+  if (!ctx->h_ring) {  // no pinned memory to be had: the runtime's own path
     for (int i = 0; i < nparts; i++)
       if (parts[i].dst && parts[i].bytes)
         DMM_HIP_CHECK(ctx, hipMemcpyAsync(parts[i].dst, parts[i].src, parts[i].bytes, hipMemcpyDeviceToHost, ctx->stream));
     DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
     return DMM_OK;
   }
-  if (total <= kSmallRead) {
-    // Joined parts come in one piece.  (That two parts' addresses follow one
-    // another does not say so: a copy must not span allocations.)
-    size_t at = 0;
-    for (int i = 0; i < n;) {
-      size_t run = pieces[i].bytes;
-      int j = i + 1;
-      for (; j < n && pieces[j].joined; j++) run += pieces[j].bytes;
-      DMM_HIP_CHECK(ctx, hipMemcpyAsync(ctx->h_ring + at, pieces[i].src, run, hipMemcpyDeviceToHost, ctx->stream));
-      at += run;
-      i = j;
-    }
+  uint32_t* const flags = reinterpret_cast<uint32_t*>(ctx->h_ring);
+  char* const ring = ctx->h_ring + kFlagBytes;
+  // Piece i is there once its slot's flags hold seq + i; no other piece of
+  // the slot before or after it has that number.
+  if (ctx->read_seq > UINT32_MAX - static_cast<uint32_t>(n) - 1) {
     DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-    at = 0;
-    for (const Piece& p : pieces) {
-      std::memcpy(p.dst, ctx->h_ring + at, p.bytes);
-      at += p.bytes;
-    }
-    return DMM_OK;
+    std::memset(flags, 0, kFlagBytes);
+    ctx->read_seq = 0;
   }
-  std::vector<std::atomic<int>> queued(n);  // 1: its DMA and event are on the stream, 2: they could not be
+  const bool each = total > kSmallRead;
+  const int groups = each ? kReadGroups : static_cast<int>(std::min<size_t>(kReadGroups, ceil_div(total, kGroupLeast)));
+  const uint32_t seq = ctx->read_seq + 1;
+  ctx->read_seq += static_cast<uint32_t>(n);
+  std::vector<std::atomic<int>> queued(n);  // 1: its copy is on the stream, 2: it could not be
   for (auto& q : queued) q.store(0, std::memory_order_relaxed);
   std::atomic<int> next{0}, error{0};
-  auto queue = [&](int i) {
-    char* at = ctx->h_ring + (i % slots) * slot;
-    hipError_t e = hipMemcpyAsync(at, pieces[i].src, pieces[i].bytes, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipEventRecord(ctx->ring_events[i % slots], ctx->stream);
+  auto queue = [&](int i, int count) {
+    ReadList l{};
+    for (int k = 0; k < count; k++) {
+      l.src[k] = pieces[i + k].src;
+      l.bytes[k] = static_cast<uint32_t>(pieces[i + k].bytes);
+    }
+    const int s = i % slots;
+    hipLaunchKernelGGL(k_read, dim3(groups), dim3(kThreads), 0, ctx->stream, l, count, ring + s * slot, slot,
+                       flags + s * kReadGroups, seq + static_cast<uint32_t>(i), each);
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) error.store(static_cast<int>(e));
-    queued[i].store(e == hipSuccess ? 1 : 2, std::memory_order_release);
+    for (int k = 0; k < count; k++) queued[i + k].store(e == hipSuccess ? 1 : 2, std::memory_order_release);
+  };
+  auto stored = [&](int i) {
+    const uint32_t* f = flags + (i % slots) * kReadGroups;
+    for (int g = 0; g < groups; g++)
+      if (__atomic_load_n(&f[g], __ATOMIC_ACQUIRE) != seq + static_cast<uint32_t>(i)) return false;
+    return true;
+  };
+  // A stream that has ended, well or not, without the flags set ends the wait.
+  auto wait = [&](int i) -> hipError_t {
+    for (int spins = 1;; spins++) {
+      if (stored(i)) return hipSuccess;
+      if (spins % 65536 == 0) {
+        const hipError_t e = hipStreamQuery(ctx->stream);
+        if (e == hipErrorNotReady) {
+          (void)hipGetLastError();
+          std::this_thread::yield();
+        } else if (!stored(i)) {
+          return e == hipSuccess ? hipErrorUnknown : e;
+        }
+      }
+    }
   };
   // Every piece is taken once; a slot's next piece is queued by the thread
   // that emptied it, so every wait here is for a piece some thread is past.
@@ -139,16 +188,16 @@ static int read_pieces(dmm_ctx* ctx, const ReadPart* parts, int nparts) {
       int q;
       while ((q = queued[i].load(std::memory_order_acquire)) == 0) std::this_thread::yield();
       if (q == 1) {
-        const hipError_t e = hipEventSynchronize(ctx->ring_events[i % slots]);
+        const hipError_t e = wait(each ? i : n - 1);
         if (e == hipSuccess)
-          std::memcpy(pieces[i].dst, ctx->h_ring + (i % slots) * slot, pieces[i].bytes);
+          std::memcpy(pieces[i].dst, ring + (i % slots) * slot, pieces[i].bytes);
         else
           error.store(static_cast<int>(e));
       }
-      if (i + slots < n) queue(i + slots);
+      if (i + slots < n) queue(i + slots, 1);
     }
   };
-  for (int i = 0; i < slots; i++) queue(i);
+  queue(0, slots);
   std::thread helpers[kReaders - 1];
   if (total >= kThreadedRead) {
     for (int k = 0; k < kReaders - 1; k++) {
