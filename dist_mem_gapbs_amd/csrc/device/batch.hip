@@ -53,6 +53,7 @@ constexpr int kGroup = 8;  // lanes per vertex in the bottom-up sweep
 // 3.7 M uniform 5.00, 4.41, 4.36, 4.55, 4.62 ms.
 constexpr int64_t kBatchRows = 256;
 constexpr int kBatchMostPerCU = 4;
+constexpr int kBatchMostSlots = 64;  // of a captured chain, but for one
 
 enum : int { kBTD = 1, kBBU = 2, kBCount = 3, kBWrite = 4, kBDone = 5 };
 
@@ -1411,12 +1412,14 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
         std::min({cus * std::max(1, gpc), ctx->part_cap / 2,
                   std::max(cus, std::min(kBatchMostPerCU * cus, ceil_div(ctx->nloc, kBatchRows)))}));
     // The first chain has the slots that the last runs used, and one for the
-    // last post (at most graph_levels + 1, as many as that before a run);
-    // the continuation an even number, which leaves the head's parity.
+    // last post (before a run graph_levels + 1); the continuation an even
+    // number, which leaves the head's parity.  A run that needs it pays a wait
+    // and what follows the levels a second time (Kronecker 900 K, 19 slots used:
+    // 530 us a call with a chain of 17, 483 with 20).
     if (ctx->batch_graph_key != key) std::fill(std::begin(ctx->batch_recent), std::end(ctx->batch_recent), 0);
     int most = 0;
     for (int r : ctx->batch_recent) most = std::max(most, r);
-    const int want = most > 0 ? std::min(p.graph_levels, most) + 1 : p.graph_levels + 1;
+    const int want = (most > 0 ? std::min(kBatchMostSlots, most) : p.graph_levels) + 1;
     if (!ctx->batch_graph || !ctx->batch_cont || ctx->batch_graph_key != key || ctx->batch_slots < want ||
         ctx->batch_slots > want + 2) {
       if (ctx->batch_graph) (void)hipGraphExecDestroy(ctx->batch_graph);
