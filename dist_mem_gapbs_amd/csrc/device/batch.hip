@@ -169,11 +169,11 @@ __device__ __forceinline__ uint64_t block_or(uint64_t x, uint64_t* scratch) {
   return x;
 }
 
-__device__ void zero_next_next(const BArgs& a, int level) {
-  // F[level + 2] is written by atomics if level + 1 runs top-down.  Its
-  // words from bend on stay zero (cleared when the storage was allocated).
-  if (level + 2 >= a.level_cap) return;
-  uint64_t* z = a.levels + (level + 2) * a.nloc;
+// F[level + 1] of a top-down level is written by atomics (a sweep overwrites
+// it whole).  Its words from bend on stay zero (cleared when the storage was
+// allocated).
+__device__ void zero_next(const BArgs& a, int level) {
+  uint64_t* z = a.levels + (level + 1) * a.nloc;
   const int64_t gtid = int64_t(blockIdx.x) * kThreads + threadIdx.x;
   const int64_t gsize = int64_t(gridDim.x) * kThreads;
   for (int64_t i = gtid; i < a.bend; i += gsize) z[i] = 0;
@@ -517,7 +517,7 @@ __device__ void bu_phase(const BArgs& a, const BIo& io, SmallLds& L, int level) 
 
 // COUNT / WRITE over the frontier words F[level]: contiguous vertex ranges
 // per workgroup in ascending order; listed = nonzero word and out-degree >= 1.
-template <bool kWrite, bool kFar>
+template <bool kWrite>
 __device__ void count_or_write(const BArgs& a, const BIo& io, SmallLds& L, int level) {
   // Workgroup b owns the contiguous range [v0, v1) and walks it in tiles
   // of kThreads consecutive vertices (coalesced); WRITE orders entries by
@@ -532,10 +532,8 @@ __device__ void count_or_write(const BArgs& a, const BIo& io, SmallLds& L, int l
     for (int64_t t = v0; t < v1; t += kThreads) {
       const int64_t u = t + threadIdx.x;
       const uint64_t f = u < v1 ? Fl[u] : 0;
-      if (kFar) {
-        const uint64_t w = __ballot(f != 0);
-        if (lane_id() == 0 && u < v1) a.nz[u >> 6] = w;
-      }
+      const uint64_t w = __ballot(f != 0);
+      if (lane_id() == 0 && u < v1) a.nz[u >> 6] = w;
       any |= f;
       if (f) {
         const int64_t d = a.out_off[u + 1] - a.out_off[u];
@@ -562,10 +560,23 @@ __device__ void count_or_write(const BArgs& a, const BIo& io, SmallLds& L, int l
   int64_t* oqoff = cur ? a.aoff0 : a.aoff1;
   int64_t pos = io.base_c;
   int64_t run = io.base_d;
+  // The COUNT marked the words: most tiles of a top-down level have none.
+  constexpr int kTileWords = kThreads / 64;
   for (int64_t t = v0; t < v1; t += kThreads) {
+    uint64_t w[kTileWords], some = 0;
+#pragma unroll
+    for (int j = 0; j < kTileWords; j++) {
+      w[j] = t + j * 64 < v1 ? a.nz[(t >> 6) + j] : 0;
+      some |= w[j];
+    }
+    if (!some) continue;
     const int64_t u = t + threadIdx.x;
+    uint64_t mine = w[0];
+#pragma unroll
+    for (int j = 1; j < kTileWords; j++)
+      if ((threadIdx.x >> 6) == j) mine = w[j];
     int64_t d = 0;
-    if (u < v1 && Fl[u]) d = a.out_off[u + 1] - a.out_off[u];
+    if ((mine >> lane_id()) & 1ull) d = a.out_off[u + 1] - a.out_off[u];
     const int64_t f = d > 0 ? 1 : 0;
     int64_t tc, td;
     const int64_t ec = block_excl_scan<kThreads>(f, L.scan_c, &tc);
@@ -727,16 +738,13 @@ __global__ __launch_bounds__(kThreads, 4) void k_bslot(BArgs a, int parity) {
   const BIo io = {h.acount, h.aedges,   h.live,   nz, h.cur, &c->slot_error, a.part + parity * a.part_half,
                   L.base_c, L.base_d};
   switch (phase) {
-    case kBTD:
-      zero_next_next(a, level);
-      td_phase(a, io, lds.td, level);
+    case kBTD: td_phase(a, io, lds.td, level); break;
+    case kBBU: bu_phase<kFar>(a, io, lds.sm, level); break;
+    case kBCount: count_or_write<false>(a, io, lds.sm, level); break;
+    default:  // a top-down level comes next
+      zero_next(a, level);
+      count_or_write<true>(a, io, lds.sm, level);
       break;
-    case kBBU:
-      zero_next_next(a, level);
-      bu_phase<kFar>(a, io, lds.sm, level);
-      break;
-    case kBCount: count_or_write<false, kFar>(a, io, lds.sm, level); break;
-    default: count_or_write<true, kFar>(a, io, lds.sm, level); break;
   }
 }
 
