@@ -284,3 +284,27 @@ def test_batch_words_beyond_l2(dmm, orc, n, directed):
             for i in (0, 1, 31, 62, 63):
                 ref = orc.bfs_depth(og, int(srcs[i]))
                 assert np.array_equal(depth[i], np.where(ref < 0, 255, ref).astype(np.uint8)), (i, td_div)
+
+
+@pytest.mark.parametrize("td_div", [1, 20, 1000000])
+@pytest.mark.parametrize("layout", [L.DMM_LAYOUT_NATURAL, L.DMM_LAYOUT_DEGREE])
+def test_batch_reached_edges_of_every_source(dmm, orc, td_div, layout):
+    """Out-edges of the reached vertices, for sources without in-edges,
+    without out-edges and without either, after any kind of last level."""
+    n = 3000
+    rng = np.random.default_rng(n)
+    pairs = rng.integers(100, n - 100, (9000, 2))  # 0 .. 99 and the last 100: no edges
+    pairs[:, 0][pairs[:, 0] < 200] += 200           # 100 .. 199: no out-edges
+    pairs[:, 1][pairs[:, 1] > n - 200] -= 200       # the 99 before the last 100: no in-edges
+    g = csr_from_pairs(dmm, pairs, n, symmetrize=False)
+    og = orc.CSR.of(g)
+    deg = np.diff(og.oo)
+    with dmm.Context(0) as c:
+        c.set_layout(layout)
+        c.upload(g)
+        for srcs in ([5], [150], [n - 150], [n - 5], [1500, 150, n - 150, 7], list(range(90, n - 90, 45))):
+            srcs = np.array(srcs, np.int32)
+            depth, st = c.bfs_batch64(srcs, td_div=td_div)
+            exp = expected(orc, og, srcs)
+            assert np.array_equal(depth, exp), srcs
+            assert st.reached_edges == sum(int(deg[e != 255].sum()) for e in exp), srcs
