@@ -1525,7 +1525,7 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
           h->sweeps * (40 * ctx->nloc + 8) + 12 * static_cast<int64_t>(h->sweep_scanned_total);
       stats->sweep_ms = 0;
     }
-    ctx->batch_recent[ctx->batch_recent_pos++ % kBatchRecent] = h->used;
+    ctx->batch_recent[ctx->batch_recent_pos++ % kRecentRuns] = h->used;
     ctx->batch_valid = true;
     ctx->batch_last_level = h->level;
     if (stats) stats->reached_edges = *h_reached;

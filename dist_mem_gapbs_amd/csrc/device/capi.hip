@@ -73,11 +73,12 @@ void drop_graphs(dmm_ctx* ctx) {
     ctx->bfs_graph_steps[d] = 0;
   }
   if (ctx->pr_graph) (void)hipGraphExecDestroy(ctx->pr_graph);
+  if (ctx->pr_rest) (void)hipGraphExecDestroy(ctx->pr_rest);
   if (ctx->bc_graph) (void)hipGraphExecDestroy(ctx->bc_graph);
   ctx->bc_graph = nullptr;
   if (ctx->batch_graph) (void)hipGraphExecDestroy(ctx->batch_graph);
   if (ctx->batch_cont) (void)hipGraphExecDestroy(ctx->batch_cont);
-  ctx->pr_graph = ctx->batch_graph = ctx->batch_cont = nullptr;
+  ctx->pr_graph = ctx->pr_rest = ctx->batch_graph = ctx->batch_cont = nullptr;
   ctx->pr_graph_key = -1;
   ctx->batch_graph_key = -1;
 }

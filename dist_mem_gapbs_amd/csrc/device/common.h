@@ -98,7 +98,7 @@ enum : int {
   kPhaseDone = 5,
 };
 
-constexpr int kBatchRecent = 8;  // batched runs sizing the next chain of slots
+constexpr int kRecentRuns = 8;  // runs sizing the next captured chain
 constexpr int kReadSlots = 8;    // pieces of a read in flight (readout.hip)
 constexpr int kReadGroups = 32;  // workgroups that store them
 
@@ -269,6 +269,10 @@ struct dmm_ctx {
   hipGraphExec_t pr_graph = nullptr;
   hipGraphExec_t bc_graph = nullptr;  // Brandes: a fixed number of levels
   int pr_graph_key = -1;
+  hipGraphExec_t pr_rest = nullptr;  // the iterations after pr_graph's (none: NULL)
+  int pr_chain = 0;                  // iterations of pr_graph
+  int pr_recent[dmm::kRecentRuns] = {};  // iterations of the last runs with its key
+  int pr_recent_pos = 0;
   int pr_mode = -1;
 
   // Batched BFS state.
@@ -303,7 +307,7 @@ struct dmm_ctx {
   bool push_ready = false;
   int64_t batch_graph_key = -1;
   int batch_slots = 0;              // slots of batch_graph
-  int batch_recent[dmm::kBatchRecent] = {};  // slots used by the last runs with its key
+  int batch_recent[dmm::kRecentRuns] = {};  // slots used by the last runs with its key
   int batch_recent_pos = 0;
 
   dmm::Tuning tuning;

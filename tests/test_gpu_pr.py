@@ -233,3 +233,25 @@ def test_pr_kahan_tiled_equals_host_replay(dmm, graph, scale, uniform):
         got, pst = c.PageRankPull(1, 0.0, MODES["kahan"])
     assert pst.iters == 1
     assert np.array_equal(got, expect)
+
+
+@pytest.mark.parametrize("mode", sorted(MODES.values()))
+def test_pr_chain_sized_by_the_last_runs(dmm, graph, mode):
+    """Runs of few and many iterations in turn, past the number that size the
+    captured chain: each equals, bit for bit, a fresh context's first run,
+    whose chain has every iteration."""
+    g = graph(13, 16, False)
+    first = {}
+    for eps in (1.0, 1e-3, 1e-5, 0.0):
+        with dmm.Context(0) as c:
+            c.upload(g)
+            first[eps] = c.PageRankPull(25, eps, mode)
+    assert len({st.iters for _, st in first.values()}) == 4
+    with dmm.Context(0) as c:
+        c.upload(g)
+        for eps in [1e-3, 1e-3, 0.0, 1e-5] + [1.0] * 9 + [1e-5, 1e-3, 0.0] + [1e-3] * 9 + [1.0, 0.0]:
+            scores, st = c.PageRankPull(25, eps, mode)
+            exp, est = first[eps]
+            assert st.iters == est.iters, eps
+            assert list(st.err[:st.iters]) == list(est.err[:est.iters]), eps
+            assert np.array_equal(scores, exp), eps
