@@ -84,6 +84,25 @@ struct PrPrev {
   const PrParams* prm;
 };
 
+// Constants and control block of a block iteration, written by its first
+// kernel, where they are not there yet (prm NULL: they are).
+struct PrHead {
+  PrParams* prm;
+  PrCtrl* ctrl;
+  PrParams p;
+};
+
+__device__ __forceinline__ void write_head(const PrHead& h) {
+  *h.prm = h.p;
+  h.ctrl->err = 0;
+  h.ctrl->ticket = 0;
+  h.ctrl->pad = 0;
+}
+
+__global__ void k_head(PrHead h) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) write_head(h);
+}
+
 // Start of an iteration's first kernel: every workgroup sums the previous
 // iteration's error partials in the same order and stops if that iteration
 // converged (src/pr.cc:66-68); workgroup 0 records the error and the stop
@@ -1237,10 +1256,10 @@ __device__ __forceinline__ float fx_value(unsigned long long lo, long long hi) {
 // up to its edge, counted in the group's mask.  The next round's source
 // offsets and masks are loaded before this round's stores.
 __global__ __launch_bounds__(kBPropThreads) void k_bprop(BpArgs b, const float* __restrict__ cin, int64_t n_gather,
-                                                         const PrCtrl* ctrl) {
+                                                         PrHead head) {
   __shared__ float win[kBWin];
   __shared__ int32_t sd[kBSegMax];
-  if (ctrl->pad) return;
+  if (head.prm && blockIdx.x == 0 && threadIdx.x == 0) write_head(head);  // for the kernels that follow
   const int lane = lane_id();
   const int wv = threadIdx.x >> 6;
   constexpr int kRound = 64 * kBPer;                         // edges per wavefront round
@@ -1684,10 +1703,30 @@ __global__ __launch_bounds__(kBSumThreads) void k_bsum(PrArgs a, BpArgs b, float
 
 // The one-row buckets in parts: each row's partial sums (exact) in slot
 // order, then the row finishes.
+// The last iteration's error (the others' are reduced by the kernel that
+// follows them, pr_begin), by one workgroup; partial `own` is `mine`.
+__device__ __forceinline__ void reduce_error(const PrArgs& a, int own, double mine, double* red) {
+  PrCtrl* c = a.ctrl;
+  const int np = a.main_blocks + a.super_blocks;
+  double x = 0;
+  for (int i = threadIdx.x; i < np; i += kThreads) x += i == own ? mine : a.err_part[i];
+  double t = block_err_sum(x, red);
+  if (threadIdx.x == 0) {
+    const unsigned it = c->ticket;
+    c->err = t;
+    if (it < DMM_MAX_PR_ITERS) a.err_trace[it] = t;
+    if (a.err_out) *a.err_out = t;
+    c->ticket = it + 1;
+    if (t < a.prm->eps) c->pad = 1;
+  }
+}
+
+// With one workgroup (up to kThreads split rows) also the reduction of the
+// error, 4 us of a launch less.
 __global__ __launch_bounds__(kThreads) void k_bsplit(PrArgs a, BpArgs b, float* __restrict__ cout,
                                                      float* __restrict__ score) {
   __shared__ double red[kThreads / 64];
-  if (a.ctrl->pad) return;
+  __shared__ double mine;
   double err = 0;
   const int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x;
   if (i < b.n_splits) {
@@ -1700,29 +1739,21 @@ __global__ __launch_bounds__(kThreads) void k_bsplit(PrArgs a, BpArgs b, float* 
     err = finish_f32(a, sp.row, fx_value(lo, hi), score, cout);
   }
   const double t = block_err_sum(err, red);
-  if (threadIdx.x == 0) a.err_part[a.main_blocks + blockIdx.x] = t;
+  if (gridDim.x > 1) {
+    if (threadIdx.x == 0) a.err_part[a.main_blocks + blockIdx.x] = t;
+    return;
+  }
+  if (threadIdx.x == 0) mine = t;
+  __syncthreads();
+  reduce_error(a, a.main_blocks, mine, red);
 }
 
 // ---- iteration bookkeeping --------------------------------------------------
 
-// The last iteration's error (the others' are reduced by the kernel that
-// follows them, pr_begin).
 __global__ __launch_bounds__(kThreads) void k_reduce(PrArgs a) {
   __shared__ double red[kThreads / 64];
-  PrCtrl* c = a.ctrl;
-  if (c->pad) return;
-  const int np = a.main_blocks + a.super_blocks;
-  double x = 0;
-  for (int i = threadIdx.x; i < np; i += kThreads) x += a.err_part[i];
-  double t = block_err_sum(x, red);
-  if (threadIdx.x == 0) {
-    const unsigned it = c->ticket;
-    c->err = t;
-    if (it < DMM_MAX_PR_ITERS) a.err_trace[it] = t;
-    if (a.err_out) *a.err_out = t;
-    c->ticket = it + 1;
-    if (t < a.prm->eps) c->pad = 1;
-  }
+  if (a.ctrl->pad) return;
+  reduce_error(a, -1, 0.0, red);
 }
 
 __global__ __launch_bounds__(kThreads) void k_init_f32(PrArgs a, float* score, float* contrib) {
@@ -1809,8 +1840,10 @@ int pr_error_parts(dmm_ctx* ctx, int mode, bool block) {
 // the block's new contributions to score_out / contrib_out instead of the
 // context's own buffers.
 void launch_iteration(dmm_ctx* ctx, PrArgs a, int mode, int it, bool last, const void* gcontrib,
-                      float* score_out = nullptr, float* contrib_out = nullptr) {
+                      float* score_out = nullptr, float* contrib_out = nullptr, const PrHead* head = nullptr) {
   hipStream_t s = ctx->stream;
+  const bool block_path = mode == DMM_PR_FP32_KAHAN && ctx->bp_ready && gcontrib;
+  if (head && !block_path) hipLaunchKernelGGL(k_head, dim3(1), dim3(64), 0, s, *head);
   const int sb = a.super_blocks;
   // The error partials alternate between two halves: a kernel that writes its
   // own may still be reading the previous iteration's.
@@ -1833,7 +1866,7 @@ void launch_iteration(dmm_ctx* ctx, PrArgs a, int mode, int it, bool last, const
       double* cout = ctx->d_contrib64[(it + 1) & 1];
       hipLaunchKernelGGL(k_fused<double>, dim3(fb), dim3(kFusedThreads), 0, s, a, prev, cin, cout, ctx->d_score64);
       hipLaunchKernelGGL(k_f64_super, dim3(sb), dim3(kThreads), 0, s, a, cout, ctx->d_score64);
-    } else if (ctx->bp_ready && gcontrib) {
+    } else if (block_path) {
       const float* cin = static_cast<const float*>(gcontrib);
       float* cout = contrib_out ? contrib_out : ctx->d_contrib[(it + 1) & 1];
       BpArgs b;
@@ -1857,7 +1890,7 @@ void launch_iteration(dmm_ctx* ctx, PrArgs a, int mode, int it, bool last, const
       b.n_units = ctx->n_bp_units;
       b.n_splits = ctx->n_bp_splits;
       hipLaunchKernelGGL(k_bprop, dim3(std::max(1, ctx->cu_count)), dim3(kBPropThreads), 0, s, b, cin, a.n_gather,
-                         a.ctrl);
+                         head ? *head : PrHead{});
       a.main_blocks = pr_bsum_blocks(ctx);
       a.super_blocks = pr_bsplit_blocks(ctx);
       if (ctx->bp_fine)
@@ -1900,7 +1933,8 @@ void launch_iteration(dmm_ctx* ctx, PrArgs a, int mode, int it, bool last, const
       hipLaunchKernelGGL(k_kahan_super, dim3(sb), dim3(kThreads), 0, s, a, cout, score_f);
     }
   }
-  if (last) hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kThreads), 0, s, a);
+  // A block's one iteration with a single k_bsplit workgroup is reduced by that.
+  if (last && !(block_path && a.super_blocks == 1)) hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kThreads), 0, s, a);
 }
 
 }  // namespace
@@ -2162,16 +2196,6 @@ constexpr int kMaxScratchDevices = 64;
 std::mutex g_scratch_mu;
 unsigned char* g_scratch_ptr[kMaxScratchDevices] = {};
 
-__global__ void k_scratch_prep(unsigned char* base, PrParams p) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    *reinterpret_cast<PrParams*>(base + kScratchParams) = p;
-    PrCtrl* c = reinterpret_cast<PrCtrl*>(base + kScratchCtrl);
-    c->err = 0;
-    c->ticket = 0;
-    c->pad = 0;
-  }
-}
-
 }  // namespace
 
 int scratch_init(dmm_ctx* ctx) {
@@ -2209,7 +2233,10 @@ int pr_block_iteration_noalloc(dmm_ctx* ctx, const float* d_gcontrib, float* d_s
   a.partial = reinterpret_cast<double2*>(base + kScratchSegs);
   // Constants as the reference computes them in float (src/pr.cc:39, 45-46);
   // no convergence test (one iteration).
-  PrParams p;
+  PrHead head;
+  head.prm = reinterpret_cast<PrParams*>(base + kScratchParams);
+  head.ctrl = a.ctrl;
+  PrParams& p = head.p;
   const float kDamp = 0.85f;
   const float nf = static_cast<float>(ctx->n);
   p.eps = -1.0;
@@ -2220,8 +2247,7 @@ int pr_block_iteration_noalloc(dmm_ctx* ctx, const float* d_gcontrib, float* d_s
   p.base_d = static_cast<double>(p.base_f);
   p.init_d = static_cast<double>(p.init_f);
   p.pad = 0;
-  hipLaunchKernelGGL(k_scratch_prep, dim3(1), dim3(64), 0, ctx->stream, base, p);
-  launch_iteration(ctx, a, mode, 0, true, d_gcontrib, d_scores, d_contrib_out);
+  launch_iteration(ctx, a, mode, 0, true, d_gcontrib, d_scores, d_contrib_out, &head);
   DMM_HIP_CHECK(ctx, hipGetLastError());
   DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
   return DMM_OK;
