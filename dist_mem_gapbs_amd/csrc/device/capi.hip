@@ -612,6 +612,7 @@ int dmm_graph_upload(dmm_ctx* ctx, int64_t num_nodes, int64_t vbegin, int64_t ve
   DMM_HIP_CHECK(ctx, hipSetDevice(ctx->device));
   DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
   free_graph_state(ctx);
+  const dmm::ReadWarm warm(ctx, 64 * rows, 16 * rows);  // a batch; anything else
   ctx->n = num_nodes;
   ctx->vbegin = vbegin;
   ctx->vend = vend;

@@ -88,6 +88,39 @@ void read_free(dmm_ctx* ctx) {
   ctx->ring_bytes = 0;
 }
 
+// A ring of `bytes` of slots (none if there is no pinned memory to be had).
+static void ring_alloc(dmm_ctx* ctx, size_t bytes) {
+  read_free(ctx);
+  if (hipHostMalloc(reinterpret_cast<void**>(&ctx->h_ring), kFlagBytes + bytes, hipHostMallocDefault) != hipSuccess) {
+    ctx->h_ring = nullptr;
+    (void)hipGetLastError();
+    return;
+  }
+  ctx->ring_bytes = bytes;
+  std::memset(ctx->h_ring, 0, kFlagBytes);
+  ctx->read_seq = 0;
+}
+
+ReadWarm::ReadWarm(dmm_ctx* ctx, int64_t bytes, int64_t usual) {
+  const size_t most = kReadSlots * kPieceMost;
+  const size_t want = std::min(most, static_cast<size_t>(bytes) + kReadSlots * (size_t(1) << 16));
+  if (ctx->ring_bytes >= want) return;
+  const size_t touch = std::min(want, std::max(2 * kThreadedRead, static_cast<size_t>(usual)));
+  try {
+    thread = std::thread([ctx, want, touch] {
+      (void)hipSetDevice(ctx->device);
+      ring_alloc(ctx, want);
+      if (!ctx->h_ring) return;
+      for (size_t i = 0; i < touch; i += 4096) reinterpret_cast<volatile char*>(ctx->h_ring)[kFlagBytes + i] = 0;
+    });
+  } catch (const std::system_error&) {  // the first read allocates
+  }
+}
+
+ReadWarm::~ReadWarm() {
+  if (thread.joinable()) thread.join();
+}
+
 static int read_pieces(dmm_ctx* ctx, const ReadPart* parts, int nparts) {
   size_t total = 0;
   for (int i = 0; i < nparts; i++) total += parts[i].dst ? parts[i].bytes : 0;
@@ -110,16 +143,7 @@ static int read_pieces(dmm_ctx* ctx, const ReadPart* parts, int nparts) {
   const int slots = std::min(n, kReadSlots);
   if (ctx->ring_bytes < slots * slot) {
     DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-    read_free(ctx);
-    if (hipHostMalloc(reinterpret_cast<void**>(&ctx->h_ring), kFlagBytes + slots * slot, hipHostMallocDefault) !=
-        hipSuccess) {
-      ctx->h_ring = nullptr;
-      (void)hipGetLastError();
-    } else {
-      ctx->ring_bytes = slots * slot;
-      std::memset(ctx->h_ring, 0, kFlagBytes);
-      ctx->read_seq = 0;
-    }
+    ring_alloc(ctx, slots * slot);
   }
   if (!ctx->h_ring) {  // no pinned memory to be had: the runtime's own path
     for (int i = 0; i < nparts; i++)
