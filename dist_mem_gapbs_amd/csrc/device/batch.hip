@@ -274,7 +274,9 @@ __device__ void td_phase(const BArgs& a, const BIo& io, TdLds& L, int level) {
 // fetched, 1.86 ms for 118 M edges) every edge not read counts: 3.7 M uniform
 // vertices, 64 lanes, whole call with 1, 2, 4, 8 short rounds 7.60, 7.22,
 // 6.94, 7.00 ms.  Where they do not, the rounds' latency does: 120 K vertices
-// 308 us with one, 315 with four.  Kronecker graphs the same.
+// 308 us with one, 315 with four.  Kronecker graphs the same, but from
+// kSweepFarMost vertices on slower: Kronecker-24 5.92 ms with one, 6.02 with
+// four (uniform the same).
 // The whole-graph sweep uses kSweepUnroll (16 leaves registers for five
 // workgroups per CU; 32: four, 3% slower on Kronecker graphs); the PE-block
 // kernels, which probe the non-zero bitmaps first and stop earlier, use
@@ -286,13 +288,16 @@ __device__ void td_phase(const BArgs& a, const BIo& io, TdLds& L, int level) {
 // reads the words and marks them) and fewer than kNzPart8 eighths of the rows are
 // listed: a probe costs a third of a far word (200 against 64 G/s).  3.7 M
 // uniform vertices, 43% listed at the first sweep: 1.86 -> 1.05 ms, whole
-// call 6.85 -> 6.1 ms; Kronecker 900 K 1.40 ms with and without.
+// call 6.85 -> 6.1 ms; the levels of Kronecker-22 2.19 -> 2.07 ms, -23 4.98 ->
+// 4.62, but -24 6.02 -> 6.75: not beyond kSweepFarMost either, where the bits
+// crowd the words out of L2.
 // Returns the end of the examined range; *found = the needed lanes found.
 constexpr int kSweepUnroll = 16;
 constexpr int kBlockUnroll = 4;
 constexpr int kSweepShort = 4;
 constexpr int kNzPart8 = 5;                         // eighths
-constexpr int64_t kSweepFar = int64_t(1) << 19;  // 4 MB of words
+constexpr int64_t kSweepFar = int64_t(1) << 19;      // 4 MB of words
+constexpr int64_t kSweepFarMost = int64_t(1) << 23;  // 1 MB of their bits
 template <int kUnroll, int kShort>
 __device__ __forceinline__ int64_t sweep_row(const int32_t* __restrict__ in_nbr, int64_t b, int64_t e,
                                              int sub, uint64_t need, const uint64_t* __restrict__ front,
@@ -1435,7 +1440,7 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
       if (ctx->batch_graph) (void)hipGraphExecDestroy(ctx->batch_graph);
       if (ctx->batch_cont) (void)hipGraphExecDestroy(ctx->batch_cont);
       ctx->batch_graph = ctx->batch_cont = nullptr;
-      const auto slot = ctx->nloc >= kSweepFar ? k_bslot<true> : k_bslot<false>;
+      const auto slot = ctx->nloc >= kSweepFar && ctx->nloc <= kSweepFarMost ? k_bslot<true> : k_bslot<false>;
       for (int part = 0; part < 2; part++) {
         constexpr int kCont = 6;
         const int first = part == 0 ? 0 : want & 1;
