@@ -351,36 +351,37 @@ __device__ __forceinline__ int64_t sweep_row(const int32_t* __restrict__ in_nbr,
 }
 
 // Rows beyond kSweepWide in-edges: by a wavefront (kWaves 1) or a workgroup
-// (its kWaves), kWideUnroll edges per lane and round, stopping as soon as
-// every needed lane is found.  An 8-lane group took 256 edges a round, so a
-// hub's row was the sweep: 318 us for one level of a Kronecker-17 batch.
+// (its kWaves), one edge per lane and then kWideUnroll per lane and round,
+// stopping as soon as every needed lane is found.  An 8-lane group took 256
+// edges a round, so a hub's row was the sweep: 318 us for one level of a
+// Kronecker-17 batch.  A dense frontier gives the lanes in the first round;
+// with kWideUnroll edges a lane in that too, Kronecker-24 5.89 ms instead of
+// 5.53, Kronecker-22 1.94 instead of 1.87.
 constexpr int kWideUnroll = 8;
 template <int kWaves>
 __device__ __forceinline__ int64_t wide_row(const int32_t* __restrict__ in_nbr, int64_t b, int64_t e, uint64_t need,
                                             const uint64_t* __restrict__ front, const uint64_t* __restrict__ nz,
                                             uint64_t (*red)[kThreads / 64], int& buf, uint64_t* found) {
-  constexpr int64_t kRound = int64_t(kWaves) * 64 * kWideUnroll;
+  constexpr int kLanes = kWaves * 64;
   const int t = kWaves == 1 ? lane_id() : static_cast<int>(threadIdx.x);
   uint64_t acc = 0;
   int64_t k0 = b;
-  for (; k0 < e; k0 += kRound) {
-    int32_t v[kWideUnroll];
+  auto round = [&](auto unroll) {
+    constexpr int kUnroll = unroll.value;
+    int32_t v[kUnroll];
 #pragma unroll
-    for (int j = 0; j < kWideUnroll; j++) {
-      const int64_t k = k0 + j * (kWaves * 64) + t;
-      v[j] = in_nbr[min(k, e - 1)];  // past the end the last edge again
-    }
+    for (int j = 0; j < kUnroll; j++) v[j] = in_nbr[min(k0 + j * kLanes + t, e - 1)];  // past the end the last edge again
     uint64_t x = 0;
     if (nz) {
 #pragma unroll
-      for (int j = 0; j < kWideUnroll; j++)
+      for (int j = 0; j < kUnroll; j++)
         if (!((nz[v[j] >> 6] >> (v[j] & 63)) & 1ull)) v[j] = -1;
 #pragma unroll
-      for (int j = 0; j < kWideUnroll; j++)
+      for (int j = 0; j < kUnroll; j++)
         if (v[j] >= 0) x |= front[v[j]];
     } else {
 #pragma unroll
-      for (int j = 0; j < kWideUnroll; j++) x |= front[v[j]];
+      for (int j = 0; j < kUnroll; j++) x |= front[v[j]];
     }
     x = wave_or(x);
     if (kWaves > 1) {
@@ -393,11 +394,12 @@ __device__ __forceinline__ int64_t wide_row(const int32_t* __restrict__ in_nbr, 
       buf ^= 1;
     }
     acc |= x;
-    if ((acc & need) == need) {
-      k0 += kRound;
-      break;
+    k0 += kLanes * kUnroll;
+    return (acc & need) == need;
+  };
+  if (!round(std::integral_constant<int, 1>()))
+    while (k0 < e && !round(std::integral_constant<int, kWideUnroll>())) {
     }
-  }
   *found = acc & need;
   return min(k0, e);
 }

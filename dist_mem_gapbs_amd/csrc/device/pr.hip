@@ -772,7 +772,7 @@ __global__ __launch_bounds__(kFusedThreads) void k_fused(PrArgs a, PrPrev prev, 
         a.partial[it.slot] = acc.partial();
     }
   }
-  // Light rows, one per 8-lane group; every lane of a wavefront runs the
+  // Light rows, one per kGroup-lane group; every lane of a wavefront runs the
   // same number of rounds so the group shuffles stay convergent.  A row is a
   // chain of bounds, neighbours, contributions and its old score; while one
   // row's contributions arrive, the next row's neighbours (kLightUnroll a

@@ -260,12 +260,12 @@ def test_pr_chain_sized_by_the_last_runs(dmm, graph, mode):
 @pytest.mark.parametrize("n", [9001, 40011])  # every source in the LDS hub, or not
 @pytest.mark.parametrize("mode", ["kahan", "fp64"])
 def test_pr_row_lengths_of_the_fused_sums(dmm, orc, n, mode):
-    """Rows at the edges of a light step (32 edges), of the heavy rows (64),
+    """Rows at the edges of a light step (16 edges), of the heavy rows (64),
     of an item's steps (256, 512) and of its size (2048).  FP64: 10 iterations
     of sums of up to L non-negative terms differ from another order's by at
     most 10 * L * 2^-52 of their size; compensated: 4e-7."""
     rng = np.random.default_rng([n, len(mode)])
-    lengths = [1, 7, 8, 9, 31, 32, 33, 62, 63, 64, 65, 255, 256, 257, 319, 320, 321, 511, 512, 513, 575, 576, 577,
+    lengths = [1, 3, 4, 5, 7, 8, 9, 15, 16, 17, 31, 32, 33, 62, 63, 64, 65, 255, 256, 257, 319, 320, 321, 511, 512, 513, 575, 576, 577,
                767, 768, 769, 1023, 1024, 1025, 2047, 2048, 2049, 4096, 4097, 8192]
     pairs = [np.stack((rng.choice(n, k, replace=False), np.full(k, i * 3 + 1)), 1) for i, k in enumerate(lengths)]
     pairs.append(rng.integers(0, n, (4 * n, 2)))
