@@ -104,6 +104,25 @@ __global__ void k_head(PrHead h) {
   if (blockIdx.x == 0 && threadIdx.x == 0) write_head(h);
 }
 
+// The sum of an iteration's error partials by a workgroup of kBlock threads,
+// in one order whoever takes it: what a run reports, and where it stops, must
+// not depend on which kernel of which captured chain sums an iteration.  The
+// order is that of the kThreads threads of k_reduce; the others of a larger
+// workgroup add nothing.  Partial `own` (-1: none) is `mine`.  The sum is every
+// thread's; scratch (one double per wavefront) is in use until the next barrier.
+template <int kBlock>
+__device__ __forceinline__ double error_sum(const double* part, int parts, int own, double mine, double* scratch) {
+  double x = 0;
+  if (threadIdx.x < kThreads)
+    for (int i = threadIdx.x; i < parts; i += kThreads) x += i == own ? mine : part[i];
+  x = wave_sum(x);
+  if (lane_id() == 0) scratch[threadIdx.x >> 6] = x;
+  __syncthreads();
+  double t = 0;
+  for (int w = 0; w < kThreads / 64; w++) t += scratch[w];
+  return t;
+}
+
 // Start of an iteration's first kernel: every workgroup sums the previous
 // iteration's error partials in the same order and stops if that iteration
 // converged (src/pr.cc:66-68); workgroup 0 records the error and the stop
@@ -114,16 +133,9 @@ __global__ void k_head(PrHead h) {
 template <int kBlock>
 __device__ __forceinline__ bool pr_begin(const PrPrev& p, double* scratch) {
   if (p.it == 0) return true;
-  double x = 0;
-  for (int i = threadIdx.x; i < p.parts; i += kBlock) x += p.part[i];
   // Workgroup 0 may be writing the mark: one thread reads it for all.
-  const double mark = threadIdx.x == 0 && p.ctrl->pad ? 1.0 : 0.0;
-  x = wave_sum(x);
-  if (lane_id() == 0) scratch[threadIdx.x >> 6] = x;
-  if (threadIdx.x == 0) scratch[kBlock / 64] = mark;
-  __syncthreads();
-  double t = 0;
-  for (int w = 0; w < kBlock / 64; w++) t += scratch[w];
+  if (threadIdx.x == 0) scratch[kBlock / 64] = p.ctrl->pad ? 1.0 : 0.0;
+  const double t = error_sum<kBlock>(p.part, p.parts, -1, 0.0, scratch);
   const bool over = scratch[kBlock / 64] != 0.0;
   __syncthreads();
   if (over) return false;
@@ -1794,10 +1806,7 @@ __global__ __launch_bounds__(kBSumThreads) void k_bsum(PrArgs a, BpArgs b, float
 // follows them, pr_begin), by one workgroup; partial `own` is `mine`.
 __device__ __forceinline__ void reduce_error(const PrArgs& a, int own, double mine, double* red) {
   PrCtrl* c = a.ctrl;
-  const int np = a.main_blocks + a.super_blocks;
-  double x = 0;
-  for (int i = threadIdx.x; i < np; i += kThreads) x += i == own ? mine : a.err_part[i];
-  double t = block_err_sum(x, red);
+  const double t = error_sum<kThreads>(a.err_part, a.main_blocks + a.super_blocks, own, mine, red);
   if (threadIdx.x == 0) {
     const unsigned it = c->ticket;
     c->err = t;

@@ -278,3 +278,30 @@ def test_pr_row_lengths_of_the_fused_sums(dmm, orc, n, mode):
     ref, it, _ = orc.pr_f64(og, 10, 0.0)
     assert st.iters == it == 10
     assert np.allclose(s, ref, rtol=10 * 8300 * 2.0 ** -52 if mode == "fp64" else 4e-7, atol=0)
+
+
+@pytest.mark.parametrize("layout", [0, 1])  # natural: untiled; degree: the compensated mode tiled
+@pytest.mark.parametrize("mode", ["serial", "kahan", "fp64"])
+def test_pr_error_of_an_iteration_is_one_value(dmm, mode, layout):
+    """The error of iteration k is the same 64 bits in a run that ends there
+    and in one that goes on, and in every repeat of either: the error partials
+    (here more than a reducing workgroup has threads, split rows among them)
+    are summed in one order."""
+    n = 120011
+    rng = np.random.default_rng(n)
+    hubs = [np.stack((rng.integers(0, n, 5000), np.full(5000, h)), 1) for h in (3, n // 2, n - 1)]
+    g = csr_from_pairs(dmm, np.concatenate([rng.integers(0, n, (8 * n, 2))] + hubs), n)
+    with dmm.Context(0) as c:
+        c.set_layout(layout)
+        c.upload(g)
+        whole = c.PageRankPull(14, 0.0, MODES[mode], read=False)[1]
+        errs = list(whole.err[:14])
+        for k in range(1, 14):
+            st = c.PageRankPull(k, 0.0, MODES[mode], read=False)[1]
+            assert st.iters == k and list(st.err[:k]) == errs[:k], k
+        # Stopped by the tolerance, from chains of every iteration and of the last runs'.
+        for k in (2, 5, 9):
+            eps = (errs[k - 1] + errs[k - 2]) / 2
+            for _ in range(12):
+                st = c.PageRankPull(14, eps, MODES[mode], read=False)[1]
+                assert st.iters == k and list(st.err[:k]) == errs[:k], k
