@@ -10,10 +10,10 @@
 #include <atomic>
 #include <cstring>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <vector>
 
+#include "../host/threads.h"
 #include "common.h"
 
 namespace dmm {
@@ -106,15 +106,13 @@ ReadWarm::ReadWarm(dmm_ctx* ctx, int64_t bytes, int64_t usual) {
   const size_t want = std::min(most, static_cast<size_t>(bytes) + kReadSlots * (size_t(1) << 16));
   if (ctx->ring_bytes >= want) return;
   const size_t touch = std::min(want, std::max(2 * kThreadedRead, static_cast<size_t>(usual)));
-  try {
-    thread = std::thread([ctx, want, touch] {
-      (void)hipSetDevice(ctx->device);
-      ring_alloc(ctx, want);
-      if (!ctx->h_ring) return;
-      for (size_t i = 0; i < touch; i += 4096) reinterpret_cast<volatile char*>(ctx->h_ring)[kFlagBytes + i] = 0;
-    });
-  } catch (const std::system_error&) {  // the first read allocates
-  }
+  // Without a thread the first read allocates.
+  (void)start_thread(&thread, [ctx, want, touch] {
+    (void)hipSetDevice(ctx->device);
+    ring_alloc(ctx, want);
+    if (!ctx->h_ring) return;
+    for (size_t i = 0; i < touch; i += 4096) reinterpret_cast<volatile char*>(ctx->h_ring)[kFlagBytes + i] = 0;
+  });
 }
 
 ReadWarm::~ReadWarm() {
@@ -224,13 +222,8 @@ static int read_pieces(dmm_ctx* ctx, const ReadPart* parts, int nparts) {
   queue(0, slots);
   std::thread helpers[kReaders - 1];
   if (total >= kThreadedRead) {
-    for (int k = 0; k < kReaders - 1; k++) {
-      try {
-        helpers[k] = std::thread(work);
-      } catch (const std::system_error&) {
-        break;  // the caller reads alone
-      }
-    }
+    for (int k = 0; k < kReaders - 1; k++)
+      if (!start_thread(&helpers[k], work)) break;  // those that there are read alone
   }
   work();
   for (auto& t : helpers)
