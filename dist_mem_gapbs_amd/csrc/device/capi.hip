@@ -126,7 +126,7 @@ void free_graph_state(dmm_ctx* ctx) {
   void* bufs[] = {ctx->d_out_off, ctx->d_out_nbr, ctx->d_parent, ctx->d_depth, ctx->d_queue,
                   ctx->d_qoff,    ctx->d_bm[0],   ctx->d_bm[1],  ctx->d_bm[2],
                   ctx->d_score,   ctx->d_contrib[0], ctx->d_contrib[1], ctx->d_score64,
-                  ctx->d_contrib64[0], ctx->d_contrib64[1], ctx->d_err_part, ctx->d_heavy, ctx->d_sitems, ctx->d_sstart,
+                  ctx->d_contrib64[0], ctx->d_contrib64[1], ctx->d_err_part, ctx->d_sitems,
                   ctx->d_gcontrib, ctx->d_seen, ctx->d_levels, ctx->d_bact, ctx->d_baoff,
                   ctx->d_bdepth, ctx->d_items, ctx->d_supers, ctx->d_partial, ctx->d_perm, ctx->d_inv,
                   ctx->d_parent_out, ctx->d_score_out, ctx->d_score64_out,
@@ -612,7 +612,7 @@ int dmm_graph_upload(dmm_ctx* ctx, int64_t num_nodes, int64_t vbegin, int64_t ve
   DMM_HIP_CHECK(ctx, hipSetDevice(ctx->device));
   DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
   free_graph_state(ctx);
-  const dmm::ReadWarm warm(ctx, 64 * rows, 16 * rows);  // a batch; anything else
+  const dmm::ReadWarm warm(ctx, rows);
   ctx->n = num_nodes;
   ctx->vbegin = vbegin;
   ctx->vend = vend;
@@ -730,20 +730,20 @@ int dmm_graph_upload(dmm_ctx* ctx, int64_t num_nodes, int64_t vbegin, int64_t ve
         ctx->n_wide++;
     }
   }
-  if ((rc = A((void**)&ctx->d_heavy, sizeof(int32_t) * std::max<size_t>(1, heavy.size()), "heavy list"))) return rc;
-  if (!heavy.empty())
-    DMM_HIP_CHECK(ctx, hipMemcpy(ctx->d_heavy, by_class.data(), sizeof(int32_t) * heavy.size(), hipMemcpyHostToDevice));
   std::vector<dmm::SerialItem> sitems;
   std::vector<int32_t> sstart;
-  dmm::serial_plan(rows, ctx->pr_light_begin, ctx->pr_zero_begin, ioff, by_class, ctx->heavy_threshold,
-                   dmm::pr_serial_blocks(ctx), &sitems, &sstart);
-  if ((rc = A(&ctx->d_sitems, sizeof(dmm::SerialItem) * std::max<size_t>(1, sitems.size()), "serial items")) ||
-      (rc = A((void**)&ctx->d_sstart, sizeof(int32_t) * sstart.size(), "serial items")))
-    return rc;
-  if (!sitems.empty())
-    DMM_HIP_CHECK(ctx, hipMemcpy(ctx->d_sitems, sitems.data(), sizeof(dmm::SerialItem) * sitems.size(),
-                                 hipMemcpyHostToDevice));
-  DMM_HIP_CHECK(ctx, hipMemcpy(ctx->d_sstart, sstart.data(), sizeof(int32_t) * sstart.size(), hipMemcpyHostToDevice));
+  dmm::serial_plan(rows, ctx->pr_light_begin, ctx->pr_zero_begin, ioff, heavy, by_class, dmm::pr_serial_blocks(ctx),
+                   &sitems, &sstart);
+  // One allocation and one copy: the items, their starts, the heavy list.
+  std::vector<int32_t> lists(2 * sitems.size());
+  static_assert(sizeof(dmm::SerialItem) == 2 * sizeof(int32_t), "items are copied as pairs of words");
+  if (!sitems.empty()) std::memcpy(lists.data(), sitems.data(), sizeof(dmm::SerialItem) * sitems.size());
+  lists.insert(lists.end(), sstart.begin(), sstart.end());
+  lists.insert(lists.end(), by_class.begin(), by_class.end());
+  if ((rc = A(&ctx->d_sitems, sizeof(int32_t) * lists.size(), "row lists"))) return rc;
+  ctx->d_sstart = static_cast<int32_t*>(ctx->d_sitems) + 2 * sitems.size();
+  ctx->d_heavy = ctx->d_sstart + sstart.size();
+  DMM_HIP_CHECK(ctx, hipMemcpy(ctx->d_sitems, lists.data(), sizeof(int32_t) * lists.size(), hipMemcpyHostToDevice));
   // Work items of the compensated / FP64 modes: heavy rows whole, rows with
   // more than kPrSplit in-edges cut into kPrSegment-edge segments.
   std::vector<dmm::PrItem> items;

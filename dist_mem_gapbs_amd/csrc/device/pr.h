@@ -50,8 +50,9 @@ struct SerialItem {
   int32_t first;
   int32_t kind;
 };
-void serial_plan(int64_t rows, int64_t light_begin, int64_t zero_begin, const int64_t* off, const std::vector<int32_t>& by_class,
-                 int64_t heavy_threshold, int blocks, std::vector<SerialItem>* items, std::vector<int32_t>* start);
+void serial_plan(int64_t rows, int64_t light_begin, int64_t zero_begin, const int64_t* off,
+                 const std::vector<int32_t>& heavy, const std::vector<int32_t>& by_class, int blocks,
+                 std::vector<SerialItem>* items, std::vector<int32_t>* start);
 
 // Window-tiled compensated PageRank (degree-ordered whole graphs).
 // Sources are cut into windows of `pr_window` vertices (a tuning value:

@@ -101,21 +101,28 @@ static void ring_alloc(dmm_ctx* ctx, size_t bytes) {
   ctx->read_seq = 0;
 }
 
-ReadWarm::ReadWarm(dmm_ctx* ctx, int64_t bytes, int64_t usual) {
-  const size_t most = kReadSlots * kPieceMost;
-  const size_t want = std::min(most, static_cast<size_t>(bytes) + kReadSlots * (size_t(1) << 16));
+ReadWarm::ReadWarm(dmm_ctx* ctx, int64_t rows) {
+  const size_t search = 8 * static_cast<size_t>(rows);  // a parent and a depth, or an FP64 rank
+  // A larger ring is an allocation of its own in the driver, which holds up
+  // the upload's: no more than a search needs where that is a small read (a
+  // batch then enlarges it), else what a batch can use of it.
+  const size_t want = search <= kSmallRead
+                          ? 2 * kPieceLeast
+                          : std::min(kReadSlots * kPieceMost, 8 * search + kReadSlots * (size_t(1) << 16));
   if (ctx->ring_bytes >= want) return;
-  const size_t touch = std::min(want, std::max(2 * kThreadedRead, static_cast<size_t>(usual)));
+  const size_t touch = std::min(want, std::max(2 * kThreadedRead, 2 * search));
   // Without a thread the first read allocates.
-  (void)start_thread(&thread, [ctx, want, touch] {
+  (void)start_thread(&thread, [this, ctx, want, touch] {
     (void)hipSetDevice(ctx->device);
     ring_alloc(ctx, want);
     if (!ctx->h_ring) return;
-    for (size_t i = 0; i < touch; i += 4096) reinterpret_cast<volatile char*>(ctx->h_ring)[kFlagBytes + i] = 0;
+    for (size_t i = 0; i < touch && !done.load(std::memory_order_relaxed); i += 4096)
+      reinterpret_cast<volatile char*>(ctx->h_ring)[kFlagBytes + i] = 0;
   });
 }
 
 ReadWarm::~ReadWarm() {
+  done.store(true, std::memory_order_relaxed);
   if (thread.joinable()) thread.join();
 }
 

@@ -1,0 +1,81 @@
+"""What the library asks of the HIP runtime on the host: pinned memory of an
+upload.  Each scenario runs in a process of its own that maps, ahead of the
+library, a shared object whose functions count the calls and pass them on."""
+import json
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = [pytest.mark.gpu, pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")]
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+COUNTS = r"""
+#include <atomic>
+#include <cstddef>
+#include <dlfcn.h>
+
+static void* runtime(const char* name) {
+  static void* lib = dlopen("libamdhip64.so.7", RTLD_NOW | RTLD_LOCAL);
+  return lib ? dlsym(lib, name) : nullptr;
+}
+static std::atomic<long> pinned_bytes{0};
+
+extern "C" long count_pinned_bytes() { return pinned_bytes.exchange(0); }
+extern "C" int hipHostMalloc(void** p, size_t n, unsigned flags) {
+  static auto next = reinterpret_cast<int (*)(void**, size_t, unsigned)>(runtime("hipHostMalloc"));
+  pinned_bytes += static_cast<long>(n);
+  return next(p, n, flags);
+}
+"""
+PRELUDE = """
+import ctypes, json, sys
+counts = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+counts.count_pinned_bytes.restype = ctypes.c_long
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+import dist_mem_gapbs_amd as dmm
+def graph(n, degree=8):
+    return dmm.from_edgelist(np.random.default_rng(n).integers(0, n, (degree * n, 2)).astype(np.int32), n)
+out = []
+"""
+
+
+@pytest.fixture(scope="module")
+def counted(tmp_path_factory):
+    d = tmp_path_factory.mktemp("counts")
+    (d / "counts.cc").write_text(COUNTS)
+    so = d / "counts.so"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", str(d / "counts.cc"), "-o", str(so), "-ldl"],
+                   check=True)
+
+    def run(scenario):
+        p = subprocess.run([sys.executable, "-c", PRELUDE + scenario + "\nprint(json.dumps(out))", str(so), ROOT],
+                           capture_output=True, text=True, timeout=100)
+        assert p.returncode == 0, p.stderr
+        return json.loads(p.stdout)
+    return run
+
+
+def test_an_upload_pins_what_a_search_reads(counted):
+    """The ring for reads: of a small graph the slots of a search's two small
+    parts, of a larger one at most 64 bytes a row beside the slots' rounding,
+    and none for a graph of the same size again."""
+    sizes = [100, 1000, 32768, 65536, 65537, 131072, 600001]
+    got = counted("""
+for n in %r:
+    g = graph(n, 2)
+    with dmm.Context(0) as c:
+        counts.count_pinned_bytes()
+        c.upload(g)
+        first = counts.count_pinned_bytes()
+        c.upload(g)
+        out.append((n, first, counts.count_pinned_bytes()))
+""" % sizes)
+    assert [n for n, _, _ in got] == sizes
+    for n, first, again in got:
+        most = 512 << 10 if 8 * n <= 512 << 10 else min(16 << 20, 64 * n + (512 << 10))
+        assert 0 < first <= most + 4096, n
+        assert again == 0, n
