@@ -332,7 +332,9 @@ int dev_alloc(dmm_ctx* ctx, void** p, size_t bytes, const char* what);
 void dev_free(void* p);
 
 // Copies results to the caller's buffers (a part without one is skipped)
-// behind everything queued on the stream; returns when they have arrived.
+// behind everything queued on the stream; returns when they have arrived.  Up
+// to four threads poll for them from the start, so that what is queued before
+// it should be short.
 struct ReadPart {
   void* dst;
   const void* src;

@@ -1,5 +1,5 @@
 """What the library asks of the HIP runtime on the host: pinned memory of an
-upload.  Each scenario runs in a process of its own that maps, ahead of the
+upload, waits before a read.  Each scenario runs in a process of its own that maps, ahead of the
 library, a shared object whose functions count the calls and pass them on."""
 import json
 import os
@@ -29,11 +29,28 @@ extern "C" int hipHostMalloc(void** p, size_t n, unsigned flags) {
   pinned_bytes += static_cast<long>(n);
   return next(p, n, flags);
 }
+
+struct Dim { unsigned x, y, z; };
+static std::atomic<long> queued{0};  // kernels launched since the stream was last waited for
+static std::atomic<long> before_last{0};  // ... before the last one
+
+extern "C" long count_before_last_launch() { return before_last; }
+extern "C" int hipLaunchKernel(const void* f, Dim grid, Dim block, void** args, size_t lds, void* stream) {
+  static auto next =
+      reinterpret_cast<int (*)(const void*, Dim, Dim, void**, size_t, void*)>(runtime("hipLaunchKernel"));
+  before_last = queued.fetch_add(1);
+  return next(f, grid, block, args, lds, stream);
+}
+extern "C" int hipStreamSynchronize(void* stream) {
+  static auto next = reinterpret_cast<int (*)(void*)>(runtime("hipStreamSynchronize"));
+  queued = 0;
+  return next(stream);
+}
 """
 PRELUDE = """
 import ctypes, json, sys
 counts = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
-counts.count_pinned_bytes.restype = ctypes.c_long
+counts.count_pinned_bytes.restype = counts.count_before_last_launch.restype = ctypes.c_long
 sys.path.insert(0, sys.argv[2])
 import numpy as np
 import dist_mem_gapbs_amd as dmm
@@ -79,3 +96,25 @@ for n in %r:
         most = 512 << 10 if 8 * n <= 512 << 10 else min(16 << 20, 64 * n + (512 << 10))
         assert 0 < first <= most + 4096, n
         assert again == 0, n
+
+
+@pytest.mark.parametrize("n", [3000, 400001])
+def test_a_block_level_is_waited_for_before_its_read(counted, n):
+    """The last kernel of a block's level is the read's, and it is launched
+    when the level is done: the read's threads do not poll for the level."""
+    got = counted("""
+n = %d
+g = graph(n)
+off = g.out_offsets
+b, e = n // 3, n
+with dmm.Context(0) as c:
+    c.set_layout(0)
+    c.upload(num_nodes=n, out_offsets=off[b:] - off[b], out_neighs=g.out_neighs[off[b]:], vbegin=b, vend=e)
+    front = np.zeros(n, np.uint64)
+    for density in (1, n // 2):  # swept and pushed
+        front[:] = 0
+        front[::density] = 3
+        c.batch_block_level(front, np.zeros(e - b, np.uint64))
+        out.append(counts.count_before_last_launch())
+""" % n)
+    assert got == [0, 0]
