@@ -54,6 +54,7 @@ constexpr int kGroup = 8;  // lanes per vertex in the bottom-up sweep
 constexpr int64_t kBatchRows = 256;
 constexpr int kBatchMostPerCU = 4;
 constexpr int kBatchMostSlots = 64;  // of a captured chain, but for one
+constexpr int kBatchMoreSlots = 6;   // of its continuation
 
 enum : int { kBTD = 1, kBBU = 2, kBCount = 3, kBWrite = 4, kBDone = 5 };
 
@@ -1429,41 +1430,32 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
         std::min({cus * std::max(1, gpc), ctx->part_cap / 2,
                   std::max(cus, std::min(kBatchMostPerCU * cus, ceil_div(ctx->nloc, kBatchRows)))}));
     // The first chain has the slots that the last runs used, and one for the
-    // last post (before a run graph_levels + 1); the continuation an even
-    // number, which leaves the head's parity.  A run that needs it pays a wait
-    // and what follows the levels a second time (Kronecker 900 K, 19 slots used:
-    // 530 us a call with a chain of 17, 483 with 20).
-    if (ctx->batch_graph_key != key) std::fill(std::begin(ctx->batch_recent), std::end(ctx->batch_recent), 0);
-    int most = 0;
-    for (int r : ctx->batch_recent) most = std::max(most, r);
+    // last post (at first graph_levels + 1); the continuation, captured once a
+    // run needs it, an even number, which leaves the head's parity.  A run that
+    // needs it pays a wait and what follows the levels a second time (Kronecker
+    // 900 K, 19 slots used: 530 us a call with a chain of 17, 483 with 20).
+    if (ctx->batch_graph_key != key) ctx->batch_runs = ChainRuns();
+    const int most = ctx->batch_runs.most();
     const int want = (most > 0 ? std::min(kBatchMostSlots, most) : p.graph_levels) + 1;
-    if (!ctx->batch_graph || !ctx->batch_cont || ctx->batch_graph_key != key || ctx->batch_slots < want ||
-        ctx->batch_slots > want + 2) {
-      if (ctx->batch_graph) (void)hipGraphExecDestroy(ctx->batch_graph);
-      if (ctx->batch_cont) (void)hipGraphExecDestroy(ctx->batch_cont);
-      ctx->batch_graph = ctx->batch_cont = nullptr;
-      const auto slot = ctx->nloc >= kSweepFar && ctx->nloc <= kSweepFarMost ? k_bslot<true> : k_bslot<false>;
-      for (int part = 0; part < 2; part++) {
-        constexpr int kCont = 6;
-        const int first = part == 0 ? 0 : want & 1;
-        hipGraph_t g = nullptr;
-        DMM_HIP_CHECK(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-        if (part == 0) {
-          hipLaunchKernelGGL(k_binit, dim3(blocks), dim3(kThreads), 0, ctx->stream, a,
-                             static_cast<const int32_t*>(ctx->d_bsrc), nsrc);
-          hipLaunchKernelGGL(k_binit2, dim3(1), dim3(64), 0, ctx->stream, a,
-                             static_cast<const int32_t*>(ctx->d_bsrc), nsrc);
-        }
-        for (int i = 0; i < (part == 0 ? want : kCont); i++)
-          hipLaunchKernelGGL(slot, dim3(blocks), dim3(kThreads), 0, ctx->stream, a, (first + i) & 1);
-        hipError_t e = hipStreamEndCapture(ctx->stream, &g);
-        if (e != hipSuccess) return set_err(ctx, DMM_ERR_HIP, "batch capture failed: %s", hipGetErrorString(e));
-        e = hipGraphInstantiate(part == 0 ? &ctx->batch_graph : &ctx->batch_cont, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        if (e != hipSuccess) return set_err(ctx, DMM_ERR_HIP, "batch instantiate failed: %s", hipGetErrorString(e));
-      }
+    const auto slot = ctx->nloc >= kSweepFar && ctx->nloc <= kSweepFarMost ? k_bslot<true> : k_bslot<false>;
+    auto slots = [&](int first, int count) {
+      for (int i = 0; i < count; i++)
+        hipLaunchKernelGGL(slot, dim3(blocks), dim3(kThreads), 0, ctx->stream, a, (first + i) & 1);
+    };
+    OldGraphs old;
+    if (!ctx->batch_graph || ctx->batch_graph_key != key || ctx->batch_runs.anew(want, ctx->batch_slots)) {
+      old.take(ctx->batch_graph, ctx->batch_cont);
+      rc = capture_chain(ctx, "batch", &ctx->batch_graph, [&] {
+        hipLaunchKernelGGL(k_binit, dim3(blocks), dim3(kThreads), 0, ctx->stream, a,
+                           static_cast<const int32_t*>(ctx->d_bsrc), nsrc);
+        hipLaunchKernelGGL(k_binit2, dim3(1), dim3(64), 0, ctx->stream, a,
+                           static_cast<const int32_t*>(ctx->d_bsrc), nsrc);
+        slots(0, want);
+      });
+      if (rc) return rc;
       ctx->batch_graph_key = key;
       ctx->batch_slots = want;
+      ctx->batch_runs.lost = 0;
     }
     BCtrl* const hc = reinterpret_cast<BCtrl*>(ctx->h_bctrl);
     int64_t* h_reached = reinterpret_cast<int64_t*>(hc + 1);
@@ -1493,10 +1485,14 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
     };
     DMM_HIP_CHECK(ctx, hipEventRecord(ctx->ev_a, ctx->stream));
     DMM_HIP_CHECK(ctx, hipGraphLaunch(ctx->batch_graph, ctx->stream));
+    old.drop();
     if ((rc = finish())) return rc;
-    int guard = 0;
+    int waits = 0;
     while (h->done == 0 && !h->error) {
-      if (++guard > 100000) return set_err(ctx, DMM_ERR_STATE, "batched BFS did not terminate");
+      if (++waits > 100000) return set_err(ctx, DMM_ERR_STATE, "batched BFS did not terminate");
+      if (!ctx->batch_cont &&
+          (rc = capture_chain(ctx, "batch", &ctx->batch_cont, [&] { slots(ctx->batch_slots & 1, kBatchMoreSlots); })))
+        return rc;
       DMM_HIP_CHECK(ctx, hipGraphLaunch(ctx->batch_cont, ctx->stream));
       if ((rc = finish())) return rc;
     }
@@ -1532,7 +1528,7 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
           h->sweeps * (40 * ctx->nloc + 8) + 12 * static_cast<int64_t>(h->sweep_scanned_total);
       stats->sweep_ms = 0;
     }
-    ctx->batch_recent[ctx->batch_recent_pos++ % kRecentRuns] = h->used;
+    ctx->batch_runs.add(h->used, ctx->batch_slots - 1, 1, waits);
     ctx->batch_valid = true;
     ctx->batch_last_level = h->level;
     if (stats) stats->reached_edges = *h_reached;

@@ -51,6 +51,33 @@ void dev_free(void* p) {
   if (p) (void)hipFree(p);
 }
 
+int ChainRuns::most() const { return *std::max_element(std::begin(used), std::end(used)); }
+
+void ChainRuns::add(int steps, int chain, int launches, int waits) {
+  used[pos++ % kRecentRuns] = steps;
+  lost += std::max(0, chain - steps) * launches + waits * kWaitLaunches;
+}
+
+bool ChainRuns::anew(int want, int chain) {
+  if (lost < kCaptureLaunches) return false;
+  lost = 0;
+  return want != chain;
+}
+
+void OldGraphs::take(hipGraphExec_t& a, hipGraphExec_t& b) {
+  drop();
+  g[0] = a;
+  g[1] = b;
+  a = b = nullptr;
+}
+
+void OldGraphs::drop() {
+  for (hipGraphExec_t& x : g) {
+    if (x) (void)hipGraphExecDestroy(x);
+    x = nullptr;
+  }
+}
+
 }  // namespace dmm
 
 using dmm::set_err;

@@ -100,7 +100,38 @@ enum : int {
   kPhaseDone = 5,
 };
 
-constexpr int kRecentRuns = 8;  // runs sizing the next captured chain
+// The length of a captured chain of launches.  The first holds all that a run
+// may need (or is tuned to); after that the last kRecentRuns runs say what is
+// needed.  A launch that finds nothing to do takes 5 us and going on past the
+// chain's end a wait, some 40; capturing anew costs the run that does it 50 to
+// 100 us (400 if the old graph is destroyed first: its memory is taken up
+// again), so that what was lost has to come to that.  16 K Kronecker vertices,
+// us of runs 1, 2, 3, ... of an FP64 rank: 375 250 245 295 212 ...; capturing as
+// soon as a run used less 750 710 227 216 ..., chains of one length 450 305 300
+// ...; of a batch 380 230 225 ... 217, 710 680 220 ..., 555 375 ...
+constexpr int kRecentRuns = 8;
+constexpr int kWaitLaunches = 8;      // a wait, in launches without work
+constexpr int kCaptureLaunches = 24;  // a capture
+struct ChainRuns {
+  int used[kRecentRuns] = {};  // steps of the last runs (0: none yet)
+  int pos = 0;
+  int lost = 0;                // by the chain's length since it was captured, in launches
+  int most() const;
+  // A run used `steps` of a chain of `chain`, each of `launches` kernels, and
+  // went on past its end `waits` times.
+  void add(int steps, int chain, int launches, int waits);
+  // Whether to capture a chain of `want` in place of one of `chain`.
+  bool anew(int want, int chain);
+};
+
+// Graphs that another took the place of: destroyed behind its launch.
+struct OldGraphs {
+  hipGraphExec_t g[2] = {};
+  void take(hipGraphExec_t& a, hipGraphExec_t& b);
+  void drop();
+  ~OldGraphs() { drop(); }
+};
+
 constexpr int kReadSlots = 8;    // pieces of a read in flight (readout.hip)
 constexpr int kReadGroups = 32;  // workgroups that store them
 
@@ -271,10 +302,9 @@ struct dmm_ctx {
   hipGraphExec_t pr_graph = nullptr;
   hipGraphExec_t bc_graph = nullptr;  // Brandes: a fixed number of levels
   int pr_graph_key = -1;
-  hipGraphExec_t pr_rest = nullptr;  // the iterations after pr_graph's (none: NULL)
+  hipGraphExec_t pr_rest = nullptr;  // the iterations after pr_graph's (NULL: not needed yet)
   int pr_chain = 0;                  // iterations of pr_graph
-  int pr_recent[dmm::kRecentRuns] = {};  // iterations of the last runs with its key
-  int pr_recent_pos = 0;
+  dmm::ChainRuns pr_runs;            // runs with its key
   int pr_mode = -1;
 
   // Batched BFS state.
@@ -309,8 +339,7 @@ struct dmm_ctx {
   bool push_ready = false;
   int64_t batch_graph_key = -1;
   int batch_slots = 0;              // slots of batch_graph
-  int batch_recent[dmm::kRecentRuns] = {};  // slots used by the last runs with its key
-  int batch_recent_pos = 0;
+  dmm::ChainRuns batch_runs;        // runs with its key
 
   dmm::Tuning tuning;
 };
@@ -328,6 +357,26 @@ int set_err(dmm_ctx* ctx, int code, const char* fmt, ...);
   } while (0)
 
 // Device allocation that records failures as DMM_ERR_NOMEM.
+// Captures what launch() queues on ctx->stream; *exec is NULL on an error.
+template <typename F>
+int capture_chain(dmm_ctx* ctx, const char* what, hipGraphExec_t* exec, F launch) {
+  *exec = nullptr;
+  hipGraph_t g = nullptr;
+  hipError_t e = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal);
+  if (e == hipSuccess) {
+    launch();
+    e = hipStreamEndCapture(ctx->stream, &g);
+  }
+  if (e != hipSuccess) return set_err(ctx, DMM_ERR_HIP, "%s capture failed: %s", what, hipGetErrorString(e));
+  e = hipGraphInstantiate(exec, g, nullptr, nullptr, 0);
+  (void)hipGraphDestroy(g);
+  if (e != hipSuccess) {
+    *exec = nullptr;
+    return set_err(ctx, DMM_ERR_HIP, "%s instantiate failed: %s", what, hipGetErrorString(e));
+  }
+  return DMM_OK;
+}
+
 int dev_alloc(dmm_ctx* ctx, void** p, size_t bytes, const char* what);
 void dev_free(void* p);
 

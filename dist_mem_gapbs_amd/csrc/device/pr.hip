@@ -2127,8 +2127,6 @@ int pr_super_blocks(dmm_ctx* ctx) {
   return static_cast<int>(std::max<int64_t>(1, ceil_div(ctx->n_super, kThreads)));
 }
 
-constexpr int kPrChainSlack = 2;  // iterations too many that a captured chain may have
-
 int pr_run(dmm_ctx* ctx, int32_t max_iters, double epsilon, int32_t mode, dmm_pr_stats* stats) {
   // Constants exactly as the reference computes them in float
   // (src/pr.cc:39, 45-46), widened for the FP64 mode.
@@ -2146,27 +2144,20 @@ int pr_run(dmm_ctx* ctx, int32_t max_iters, double epsilon, int32_t mode, dmm_pr
   DMM_HIP_CHECK(ctx, hipMemcpyAsync(ctx->d_prparams, ctx->h_prparams, sizeof(PrParams),
                                     hipMemcpyHostToDevice, ctx->stream));
   // Two captured graphs per (mode, max_iters): init and the iterations that
-  // the last runs took (before a run max_iters), and what is left up to
-  // max_iters, launched if the first did not converge.  Iterations after
-  // convergence return at once, but their launches take 5 us a kernel: 16 K
-  // Kronecker vertices, 9 iterations of at most 20: 279 -> 251 us a call.  A
-  // run that needs the second graph pays one more wait, some 30 us.
+  // the last runs took (at first max_iters), and what is left up to max_iters,
+  // captured and launched once a run does not converge within the first.
+  // Iterations after convergence return at once, but their launches take 5 us
+  // a kernel: 16 K Kronecker vertices, 9 iterations of at most 20: 279 -> 251
+  // us a call.
   const int key = mode * 100000 + max_iters;
-  if (ctx->pr_graph_key != key) std::fill(std::begin(ctx->pr_recent), std::end(ctx->pr_recent), 0);
-  int most = 0;
-  for (int r : ctx->pr_recent) most = std::max(most, r);
+  if (ctx->pr_graph_key != key) ctx->pr_runs = ChainRuns();
+  const int most = ctx->pr_runs.most();
   const int want = most > 0 ? std::min(most, max_iters) : max_iters;
-  if (!ctx->pr_graph || ctx->pr_graph_key != key || ctx->pr_chain < want || ctx->pr_chain > want + kPrChainSlack) {
-    if (ctx->pr_graph) (void)hipGraphExecDestroy(ctx->pr_graph);
-    if (ctx->pr_rest) (void)hipGraphExecDestroy(ctx->pr_rest);
-    ctx->pr_graph = ctx->pr_rest = nullptr;
-    const PrArgs a = make_args(ctx);
-    const int ib = pr_light_blocks(ctx);
-    for (int part = 0; part < (want < max_iters ? 2 : 1); part++) {
-      hipGraph_t g = nullptr;
-      DMM_HIP_CHECK(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-      const int first = part == 0 ? 0 : want, end = part == 0 ? want : max_iters;
-      if (part == 0) {
+  const PrArgs a = make_args(ctx);
+  auto capture = [&](hipGraphExec_t* exec, int first, int end) {
+    return capture_chain(ctx, "PR", exec, [&] {
+      const int ib = pr_light_blocks(ctx);
+      if (first == 0) {
         if (mode == DMM_PR_FP64)
           hipLaunchKernelGGL(k_init_f64, dim3(ib), dim3(kThreads), 0, ctx->stream, a, ctx->d_score64,
                              ctx->d_contrib64[0]);
@@ -2182,24 +2173,28 @@ int pr_run(dmm_ctx* ctx, int32_t max_iters, double epsilon, int32_t mode, dmm_pr
         else
           launch_map_scores_f32(ctx);
       }
-      hipError_t e = hipStreamEndCapture(ctx->stream, &g);
-      if (e != hipSuccess) return set_err(ctx, DMM_ERR_HIP, "PR capture failed: %s", hipGetErrorString(e));
-      e = hipGraphInstantiate(part == 0 ? &ctx->pr_graph : &ctx->pr_rest, g, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(g);
-      if (e != hipSuccess) {
-        if (ctx->pr_graph && part == 1) (void)hipGraphExecDestroy(ctx->pr_graph);
-        ctx->pr_graph = ctx->pr_rest = nullptr;
-        return set_err(ctx, DMM_ERR_HIP, "PR instantiate failed: %s", hipGetErrorString(e));
-      }
-    }
+    });
+  };
+  OldGraphs old;
+  if (!ctx->pr_graph || ctx->pr_graph_key != key || ctx->pr_runs.anew(want, ctx->pr_chain)) {
+    old.take(ctx->pr_graph, ctx->pr_rest);
+    int rc = capture(&ctx->pr_graph, 0, want);
+    if (rc) return rc;
     ctx->pr_graph_key = key;
     ctx->pr_chain = want;
+    ctx->pr_runs.lost = 0;
   }
   double* h_trace = reinterpret_cast<double*>(ctx->h_prctrl + 1);
   const int trace = std::min(max_iters, DMM_MAX_PR_ITERS);
   DMM_HIP_CHECK(ctx, hipEventRecord(ctx->ev_a, ctx->stream));
+  int waits = 0;
   for (int part = 0; part < 2; part++) {
+    if (part == 1 && !ctx->pr_rest) {
+      int rc = capture(&ctx->pr_rest, ctx->pr_chain, max_iters);
+      if (rc) return rc;
+    }
     DMM_HIP_CHECK(ctx, hipGraphLaunch(part == 0 ? ctx->pr_graph : ctx->pr_rest, ctx->stream));
+    old.drop();
     DMM_HIP_CHECK(ctx, hipEventRecord(ctx->ev_b, ctx->stream));
     DMM_HIP_CHECK(ctx, hipMemcpyAsync(ctx->h_prctrl, ctx->d_prctrl, sizeof(PrCtrl), hipMemcpyDeviceToHost,
                                       ctx->stream));
@@ -2208,9 +2203,10 @@ int pr_run(dmm_ctx* ctx, int32_t max_iters, double epsilon, int32_t mode, dmm_pr
       DMM_HIP_CHECK(ctx, hipMemcpyAsync(h_trace, ctx->d_err_trace, sizeof(double) * trace, hipMemcpyDeviceToHost,
                                         ctx->stream));
     DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+    waits = part;
     if (ctx->pr_chain == max_iters || ctx->h_prctrl->pad) break;
   }
-  ctx->pr_recent[ctx->pr_recent_pos++ % kRecentRuns] = static_cast<int>(ctx->h_prctrl->ticket);
+  ctx->pr_runs.add(static_cast<int>(ctx->h_prctrl->ticket), ctx->pr_chain, mode == DMM_PR_FP32_SERIAL ? 1 : 2, waits);
   ctx->pr_mode = mode;
   if (stats) {
     float ms = 0;

@@ -1,5 +1,5 @@
 """What the library asks of the HIP runtime on the host: pinned memory of an
-upload, waits before a read.  Each scenario runs in a process of its own that maps, ahead of the
+upload, waits before a read, graphs instantiated.  Each scenario runs in a process of its own that maps, ahead of the
 library, a shared object whose functions count the calls and pass them on."""
 import json
 import os
@@ -46,11 +46,26 @@ extern "C" int hipStreamSynchronize(void* stream) {
   queued = 0;
   return next(stream);
 }
+
+static std::atomic<long> graphs{0};
+static std::atomic<long> fail_in{-1};  // this many graphs from now on one cannot be had
+
+extern "C" long count_graphs() { return graphs.exchange(0); }
+extern "C" void fail_graph(long in) { fail_in = in; }
+extern "C" int hipGraphInstantiate(void** exec, void* graph, void** node, char* log, size_t size) {
+  static auto next =
+      reinterpret_cast<int (*)(void**, void*, void**, char*, size_t)>(runtime("hipGraphInstantiate"));
+  if (fail_in.fetch_sub(1) == 0) return 2;  // out of memory
+  graphs++;
+  return next(exec, graph, node, log, size);
+}
 """
 PRELUDE = """
 import ctypes, json, sys
 counts = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
-counts.count_pinned_bytes.restype = counts.count_before_last_launch.restype = ctypes.c_long
+for f in (counts.count_pinned_bytes, counts.count_before_last_launch, counts.count_graphs):
+    f.restype = ctypes.c_long
+counts.fail_graph.argtypes = [ctypes.c_long]
 sys.path.insert(0, sys.argv[2])
 import numpy as np
 import dist_mem_gapbs_amd as dmm
@@ -118,3 +133,59 @@ with dmm.Context(0) as c:
         out.append(counts.count_before_last_launch())
 """ % n)
     assert got == [0, 0]
+
+
+RUNS = """
+g = dmm.build_graph(14, 16, False)
+srcs = dmm.pick_sources(g, 64)
+with dmm.Context(0) as c:
+    c.upload(g)
+    def rank(eps):
+        return c.PageRankPull(20, eps, %d)[0]
+    def batch(k):
+        return c.bfs_batch64(srcs[:k])[0]
+"""
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_a_chain_is_captured_when_that_pays(counted, mode):
+    """One graph for a first run, none for a second like it; a chain that is
+    longer than the runs need is captured anew once, and one that is too short
+    not by every run that it is too short for."""
+    got = counted(RUNS % mode + """
+    for call in [lambda: rank(1e-4)] * 30 + [lambda: batch(64)] * 30:
+        counts.count_graphs()
+        call()
+        out.append(counts.count_graphs())
+    counts.count_graphs()
+    for eps in [1e-2, 1e-5] * 20:
+        rank(eps)
+    out.append(counts.count_graphs())
+""")
+    for runs in (got[:30], got[30:60]):
+        assert runs[0] == 1 and runs[1] == 0 and sum(runs) <= 2, runs
+    assert got[60] <= 8
+
+
+def test_a_graph_that_cannot_be_had(counted):
+    """The call that needs it reports the error; the calls after it are whole."""
+    got = counted(RUNS % 2 + """
+    want = [rank(eps) for eps in (1e-2, 1e-6)] + [batch(64)]
+    for fail in range(4):
+        c.upload(g)
+        errors = 0
+        counts.fail_graph(fail)
+        for k in range(40):
+            try:
+                # Chains of every, of few and of more iterations; of a batch
+                # with one length of chain and then another.
+                r = [rank(1e-6 if k %% 12 == 11 else 1e-2)] + ([batch(64)] if k %% 3 == 0 else [])
+            except RuntimeError:
+                errors += 1
+                continue
+            assert np.array_equal(r[0], want[1 if k %% 12 == 11 else 0]), (fail, k)
+            assert len(r) == 1 or np.array_equal(r[1], want[2]), (fail, k)
+        counts.fail_graph(-1)
+        out.append(errors)
+""".replace("%%", "%"))
+    assert got[:3] == [1, 1, 1] and got[3] <= 1
