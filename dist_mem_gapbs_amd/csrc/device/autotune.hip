@@ -5,7 +5,7 @@
 //                 1024 edges), both at the reference thresholds alpha = 15,
 //                 beta = 18 (src/bfs.cc:142); then alpha x beta
 //   batched BFS : top-down divisor x its own workgroups per CU, then the
-//                 levels per captured graph
+//                 slots of the chain that the first run captures
 //   PageRank    : the compensated mode's tile window (16384 / 32768
 //                 sources), on a degree-ordered whole graph
 // The best values are installed on the ctx.
@@ -52,11 +52,23 @@ extern "C" int dmm_autotune(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, 
     *ms = best;
     return DMM_OK;
   };
+  // Runs that capture: later ones have chains sized by the runs before them.
+  auto time_first_batch = [&](const dmm_tuning& t, double* ms) -> int {
+    *ms = 1e30;
+    for (int r = 0; r < reps + 1; r++) {
+      dmm_batch_stats st;
+      int e = dmm_set_tuning(ctx, &t);  // drops the graphs
+      if (!e) e = dmm_bfs_batch64(ctx, sources, ns, nullptr, &ctx->tuning.batch, &st);
+      if (e) return e;
+      *ms = std::min(*ms, st.total_ms);
+    }
+    return DMM_OK;
+  };
   dmm_tuning best = base;
   best.plain_ms = 1e30;
   const int alphas[] = {5, 10, 15, 20, 30, 60};
   const int betas[] = {9, 18, 36, 72};
-  const int gpcs[] = {2, 4, 8, 16};
+  const int gpcs[] = {4, 2, 1};  // the searches take no more than 4
   const int chunks[] = {256, 512, 1024};
   // Workgroups per CU, then the top-down chunk, at the reference
   // thresholds; then alpha x beta.
@@ -118,19 +130,19 @@ extern "C" int dmm_autotune(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, 
     }
   }
   const int levels[] = {2, 4, 8, 16, 32};
+  double best_first = 1e30;
+  int best_levels = best.batch.graph_levels;
   for (int lv : levels) {
     dmm_tuning t = best;
     t.batch.graph_levels = lv;
-    if ((rc = dmm_set_tuning(ctx, &t))) return rc;
     double ms;
-    if ((rc = time_batch(&ms))) return rc;
-    if (ms < best.batch_ms) {
-      const double pm = best.plain_ms;
-      best = t;
-      best.plain_ms = pm;
-      best.batch_ms = ms;
+    if ((rc = time_first_batch(t, &ms))) return rc;
+    if (ms < best_first) {
+      best_first = ms;
+      best_levels = lv;
     }
   }
+  best.batch.graph_levels = best_levels;
   // Compensated PageRank tile window (tiled only on a degree-ordered whole
   // graph): a few iterations per window.
   best.pr_ms = 0;

@@ -967,6 +967,11 @@ constexpr int kHeavyStage = 1024;     // heavy push lists staged in LDS per roun
 // kBlockSplit-edge segments are swept by k_block_segs, so one hub row does
 // not hold a group for its whole length when no lane exits early.
 constexpr int64_t kBlockSplit = 512;
+// Workgroups per CU of a block level, at least (a search's tuned number is at
+// most 4).  Kernels of a swept level with 1, 2, 4, 8, 16 per CU: 2 M rows of
+// Kronecker-22 3.5, 2.2, 1.43, 1.02, 1.18 ms, of a uniform graph 1.71, 1.03,
+// 0.74, 0.73, 0.74; pushed levels the same from 4 on.
+constexpr int kBlockPerCU = 8;
 struct BlockSeg {
   int64_t row, b, e;
 };
@@ -1583,9 +1588,8 @@ int batch_block_level(dmm_ctx* ctx, const uint64_t* front, const uint64_t* seen,
     return rc;
   DMM_HIP_CHECK(ctx, hipMemcpyAsync(ctx->d_gfront, front, sizeof(uint64_t) * ctx->n, hipMemcpyHostToDevice, ctx->stream));
   DMM_HIP_CHECK(ctx, hipMemcpyAsync(ctx->d_bseen, seen, sizeof(uint64_t) * ctx->nloc, hipMemcpyHostToDevice, ctx->stream));
-  const int blocks = static_cast<int>(std::min<int64_t>(
-      int64_t(std::max(1, ctx->cu_count)) * std::max(1, std::min(kMaxGridPerCU, ctx->tuning.grid_per_cu)),
-      ctx->part_cap / 2));
+  const int per_cu = std::min(kMaxGridPerCU, std::max(kBlockPerCU, ctx->tuning.grid_per_cu));
+  const int blocks = static_cast<int>(std::min<int64_t>(int64_t(std::max(1, ctx->cu_count)) * per_cu, ctx->part_cap / 2));
   // Long rows' segments, built once per upload from the block's offsets.
   if (!ctx->bsegs_ready) {
     std::vector<int64_t> off(ctx->nloc + 1);

@@ -14,8 +14,8 @@
 //   part    int64[G][4]      per-workgroup partial results of the last step
 //   ctrl    BfsCtrl          window, loop state and the step trace
 //
-// A step is one grid-stride kernel (k_step) over G = CUs x grid_per_cu
-// workgroups, followed by a one-workgroup kernel (k_post) that reduces the
+// A step is one grid-stride kernel (k_step) over G workgroups (grid_blocks:
+// CUs x grid_per_cu, at most 4 per CU and one per 1024 rows), followed by a one-workgroup kernel (k_post) that reduces the
 // partials and -- in the device-resident loop -- applies the reference's
 // direction heuristic (src/bfs.cc:160-186) to schedule the next phase.
 // Kernel boundaries are the only grid-wide synchronisation: no workgroup

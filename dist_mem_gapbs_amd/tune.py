@@ -7,7 +7,7 @@ library searches, on the GPU:
                 thresholds (alpha 15, beta 18, src/bfs.cc:142), then
                 alpha x beta;
   batched BFS   the top-down divisor x the batch kernels' workgroups per CU,
-                then the levels per captured graph;
+                then the steps of the chain that a first run captures;
   PageRank      the compensated mode's tile window.
 bench.py installs the launch and tile shapes and the batch settings from
 this file;

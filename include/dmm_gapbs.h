@@ -314,8 +314,11 @@ int dmm_state_set_level(dmm_ctx* ctx, int32_t level);
 typedef struct dmm_batch_params {
   int32_t td_div;        /* top-down while active edges < M / td_div       */
   int32_t grid_per_cu;   /* workgroups per CU of the batched kernels
-                            (<= 0: the ctx's grid_per_cu)                 */
-  int32_t graph_levels;  /* levels per captured hipGraph chunk             */
+                            (<= 0: the ctx's grid_per_cu; at most 4 are
+                            taken, and one per 256 rows)                  */
+  int32_t graph_levels;  /* steps of the launch chain that a first run
+                            captures; later ones are sized by the runs
+                            before them                                   */
   int32_t flags;         /* DMM_BATCH_* bits                               */
 } dmm_batch_params;
 
@@ -484,7 +487,9 @@ int dmm_pr_blocks_check(int64_t n, int64_t n_gather, const int64_t* in_offsets,
 typedef struct dmm_tuning {
   int32_t alpha;
   int32_t beta;
-  int32_t grid_per_cu;     /* workgroups per CU of the grid-stride steps   */
+  int32_t grid_per_cu;     /* workgroups per CU of the grid-stride steps (a
+                              search takes at most 4, and one per 1024
+                              rows; a block's batched level at least 8)   */
   int32_t td_edges_per_block; /* top-down edges per workgroup chunk: 256,
                               512 or 1024 (0 = keep)                       */
   dmm_batch_params batch;
@@ -499,8 +504,8 @@ typedef struct dmm_tuning {
 /* Searches the direction thresholds, launch and tile shapes on this ctx's
  * graph using the given sample sources: plain DOBFS workgroups per CU and
  * top-down chunk at the reference's alpha = 15 / beta = 18, then alpha x
- * beta; batched BFS top-down divisor x workgroups per CU, then levels per
- * captured graph; on a degree-ordered whole graph the compensated
+ * beta; batched BFS top-down divisor x workgroups per CU, then the steps of
+ * the first captured chain; on a degree-ordered whole graph the compensated
  * PageRank's tile window.  Writes the best into *out and installs it on the
  * ctx.  No reference counterpart (src/bfs.cc:142 fixes alpha and beta). */
 int dmm_autotune(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc,

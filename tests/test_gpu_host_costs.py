@@ -1,5 +1,5 @@
 """What the library asks of the HIP runtime on the host: pinned memory of an
-upload, waits before a read, graphs instantiated.  Each scenario runs in a process of its own that maps, ahead of the
+upload, waits before a read, launch sizes, graphs instantiated.  Each scenario runs in a process of its own that maps, ahead of the
 library, a shared object whose functions count the calls and pass them on."""
 import json
 import os
@@ -34,11 +34,15 @@ struct Dim { unsigned x, y, z; };
 static std::atomic<long> queued{0};  // kernels launched since the stream was last waited for
 static std::atomic<long> before_last{0};  // ... before the last one
 
+static std::atomic<long> largest{0};  // workgroups of a launch
+
 extern "C" long count_before_last_launch() { return before_last; }
+extern "C" long count_largest_grid() { return largest.exchange(0); }
 extern "C" int hipLaunchKernel(const void* f, Dim grid, Dim block, void** args, size_t lds, void* stream) {
   static auto next =
       reinterpret_cast<int (*)(const void*, Dim, Dim, void**, size_t, void*)>(runtime("hipLaunchKernel"));
   before_last = queued.fetch_add(1);
+  if (grid.x > largest) largest = grid.x;
   return next(f, grid, block, args, lds, stream);
 }
 extern "C" int hipStreamSynchronize(void* stream) {
@@ -63,7 +67,8 @@ extern "C" int hipGraphInstantiate(void** exec, void* graph, void** node, char* 
 PRELUDE = """
 import ctypes, json, sys
 counts = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
-for f in (counts.count_pinned_bytes, counts.count_before_last_launch, counts.count_graphs):
+for f in (counts.count_pinned_bytes, counts.count_before_last_launch, counts.count_graphs,
+          counts.count_largest_grid):
     f.restype = ctypes.c_long
 counts.fail_graph.argtypes = [ctypes.c_long]
 sys.path.insert(0, sys.argv[2])
@@ -189,3 +194,23 @@ def test_a_graph_that_cannot_be_had(counted):
         out.append(errors)
 """.replace("%%", "%"))
     assert got[:3] == [1, 1, 1] and got[3] <= 1
+
+
+def test_a_block_level_fills_the_card_whatever_a_search_is_tuned_to(counted):
+    """Workgroups per CU that a search is tuned to (1 to 4, which make no
+    difference to a small graph's) are not a block level's."""
+    got = counted("""
+g = graph(5000)
+with dmm.Context(0) as c:
+    c.set_layout(0)
+    c.upload(g)
+    for per_cu in (8, 1, 2, 4):
+        t = c.get_tuning()
+        t.grid_per_cu = per_cu
+        c.set_tuning(t)
+        c.batch_block_level(np.ones(5000, np.uint64), np.zeros(5000, np.uint64))
+        counts.count_largest_grid()
+        c.batch_block_level(np.ones(5000, np.uint64), np.zeros(5000, np.uint64))
+        out.append(counts.count_largest_grid())
+""")
+    assert got[0] > 0 and got == got[:1] * 4

@@ -95,3 +95,18 @@ def test_set_tuning_rejects_bad_values(dmm):
         after = c.get_tuning()
         for f in ("alpha", "beta", "grid_per_cu", "td_edges_per_block", "pr_window"):
             assert getattr(after, f) == getattr(good, f)
+
+
+@pytest.mark.parametrize("uniform", [False, True])
+def test_autotune_picks_among_launches_that_differ(dmm, graph, uniform):
+    """Workgroups per CU beyond 4 are the same launch as 4: no candidates, so
+    that what is reported is what ran; the batch settings that it installs
+    keep the depths."""
+    g = graph(13, 16, uniform)
+    srcs = dmm.pick_sources(g, 64)
+    with dmm.Context(0) as c:
+        c.upload(g)
+        want = c.bfs_batch64(srcs)[0]
+        t = c.autotune(srcs, 1)
+        assert t.grid_per_cu in (1, 2, 4) and t.batch.grid_per_cu in (1, 2, 4)
+        assert np.array_equal(c.bfs_batch64(srcs)[0], want)
