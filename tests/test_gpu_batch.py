@@ -308,3 +308,27 @@ def test_batch_reached_edges_of_every_source(dmm, orc, td_div, layout):
             exp = expected(orc, og, srcs)
             assert np.array_equal(depth, exp), srcs
             assert st.reached_edges == sum(int(deg[e != 255].sum()) for e in exp), srcs
+
+
+@pytest.mark.parametrize("n", [1 << 23, (1 << 23) + 1])
+def test_batch_beyond_the_far_sweep(dmm, orc, n):
+    """The last size whose sweep probes the frontier's bitmap, and the first
+    beyond it: rows of every class, pushed and swept levels."""
+    rng = np.random.default_rng(n)
+    hub = np.stack((rng.integers(0, n, 6000), np.full(6000, 5)), 1)
+    mid = np.stack((rng.integers(0, n, 900), np.full(900, n - 7)), 1)
+    pairs = np.concatenate((rng.integers(0, n, (3 * n, 2)), hub, mid)).astype(np.int32)
+    srcs = np.concatenate((rng.integers(0, n, 14), [5, n - 1])).astype(np.int32)
+    with dmm.Context(0) as c:
+        g = c.build_graph(pairs, n)
+        del pairs
+        og = orc.CSR.of(g)
+        c.upload(g)
+        refs = {}
+        for i in (0, 13, 14, 15):
+            ref = orc.bfs_depth(og, int(srcs[i]))
+            refs[i] = np.where(ref < 0, 255, ref).astype(np.uint8)
+        for td_div in (1, 20, 1000000):
+            depth, _ = c.bfs_batch64(srcs, td_div=td_div)
+            for i, ref in refs.items():
+                assert np.array_equal(depth[i], ref), (i, td_div)

@@ -137,3 +137,28 @@ def test_bc_forward_unsorted_rows(natural, dmm, orc):
     natural.upload(num_nodes=og.n, out_offsets=og.oo, out_neighs=on)
     for s in dmm.pick_sources(g, 4):
         _check(natural, orc, shuffled, int(s))
+
+
+# 2048 compaction wavefronts of 16 bitmap words: up to here every workgroup of
+# the write pass sums their counts itself, beyond a launch of its own scans them
+# and the count is apart from the successor bits.
+@pytest.mark.parametrize("n,directed", [(1 << 21, False), ((1 << 21) + 1, False), ((1 << 21) + 70001, True)])
+def test_bc_forward_around_the_scanned_size(dmm, orc, n, directed):
+    """Pulled and pushed levels, more of them than a captured chain has, and
+    the vertices of the last partial."""
+    rng = np.random.default_rng([n, directed])
+    tail = 40
+    m = n - tail
+    path = np.arange(m - 1, n)
+    hub = np.full(6000, 12345)
+    pairs = [rng.integers(0, m, (2 * n, 2)), np.stack((hub, rng.integers(0, m, 6000)), 1),
+             np.stack((path[:-1], path[1:]), 1)]
+    if directed:
+        pairs.append(np.stack((path[1:], path[:-1]), 1))  # both ways: the tail reaches the rest
+    g = dmm.from_edgelist(np.concatenate(pairs).astype(np.int32), n, symmetrize=not directed)
+    og = orc.CSR.of(g)
+    with dmm.Context(0) as c:
+        c.set_layout(L.DMM_LAYOUT_NATURAL)
+        c.upload(g)
+        for s in (12345, n - 1, int(rng.integers(0, m))):
+            _check(c, orc, og, s)

@@ -64,3 +64,38 @@ def test_serial_sums_bit_exact(dmm, n, kind):
             total = np.add.accumulate(np.concatenate((np.zeros(1, np.float32), x)), dtype=np.float32)[-1]
             want = np.float32(base + np.float32(np.float32(0.85) * total))
             assert got[r] == want or (np.isnan(got[r]) and np.isnan(want)), (r, lengths[r], got[r], want)
+
+
+# Where a workgroup takes over from a wavefront: 32768 in-edges, halved down to
+# 2048 while a graph has less than that many edges for each of 256 workgroups.
+TAKEOVER = [1026, 1536, 1537, 2047, 2048, 2049, 4095, 4096, 4097, 5003, 8191, 8192, 8193, 16383, 16384, 16385, 20011,
+            32767, 32768, 32769, 40961]
+
+
+@pytest.mark.parametrize("n,edges", [(20011, 500_000), (90001, 2_200_000), (20011, 8_600_000)])
+@pytest.mark.parametrize("kind", ["rank", "halves", "ones", "big_halves", "wide", "tiny", "signed", "special"])
+def test_serial_rows_around_the_takeover(dmm, n, edges, kind):
+    """The same rows in graphs of more and more edges (the rest in short rows):
+    the longest go to workgroups from 2048, from 8192 and from 32768 in-edges
+    on, those below to a wavefront each."""
+    rng = np.random.default_rng([n, edges, len(kind)])
+    lengths = np.zeros(n, np.int64)
+    fill = max(0, edges - sum(TAKEOVER))
+    lengths[:] = rng.integers(0, 2 * fill // n + 1, n)
+    rows = rng.permutation(n)[:len(TAKEOVER)]
+    lengths[rows] = TAKEOVER
+    off = np.concatenate(([0], np.cumsum(lengths)))
+    src = rng.integers(0, n, off[-1]).astype(np.int32)
+    contrib = _values(kind, n, rng)
+    with dmm.Context(0) as c:
+        c.set_layout(L.DMM_LAYOUT_NATURAL)
+        c.upload(num_nodes=n, out_offsets=np.arange(n + 1), out_neighs=np.zeros(n, np.int32), in_offsets=off,
+                 in_neighs=src)
+        got, _, _ = c.pr_block_iteration(contrib, np.zeros(n, np.float32), L.DMM_PR_FP32_SERIAL)
+    base = (np.float32(1) - np.float32(0.85)) / np.float32(n)
+    with np.errstate(all="ignore"):
+        for r in np.concatenate((rows, rng.integers(0, n, 60))):
+            x = contrib[src[off[r]:off[r + 1]]]
+            total = np.add.accumulate(np.concatenate((np.zeros(1, np.float32), x)), dtype=np.float32)[-1]
+            want = np.float32(base + np.float32(np.float32(0.85) * total))
+            assert got[r] == want or (np.isnan(got[r]) and np.isnan(want)), (r, lengths[r], got[r], want)
