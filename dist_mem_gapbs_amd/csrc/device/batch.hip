@@ -9,8 +9,12 @@
 //   F[L]   uint64[nloc] per level L   lanes whose BFS reaches u at depth L;
 //                                     kept for every level (depth output)
 //   seen   uint64[nloc]               lanes that have reached u at a depth
-//                                     < current level (committed lazily: a
-//                                     step at level L folds F[L] in)
+//                                     < current level, and some or all of
+//                                     those at later ones: a step at level L
+//                                     folds F[L] in where it looks at u, a
+//                                     sweep F[L+1] too.  When the levels end,
+//                                     every vertex with out-edges has its
+//                                     lanes there (k_breach counts on it)
 //   act    int32[2][nloc], aoff int64[2][nloc]
 //                                     active vertices (F[L][u] != 0) with an
 //                                     out-degree prefix, for top-down levels
@@ -1488,18 +1492,22 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
       DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
       return DMM_OK;
     };
+    const ReadPart part = {depth, ctx->d_bdepth, static_cast<size_t>(int64_t(nsrc) * ctx->nloc)};
+    int waits = 0;
     DMM_HIP_CHECK(ctx, hipEventRecord(ctx->ev_a, ctx->stream));
     DMM_HIP_CHECK(ctx, hipGraphLaunch(ctx->batch_graph, ctx->stream));
-    old.drop();
-    if ((rc = finish())) return rc;
-    int waits = 0;
-    while (h->done == 0 && !h->error) {
-      if (++waits > 100000) return set_err(ctx, DMM_ERR_STATE, "batched BFS did not terminate");
-      if (!ctx->batch_cont &&
-          (rc = capture_chain(ctx, "batch", &ctx->batch_cont, [&] { slots(ctx->batch_slots & 1, kBatchMoreSlots); })))
-        return rc;
-      DMM_HIP_CHECK(ctx, hipGraphLaunch(ctx->batch_cont, ctx->stream));
+    {
+      const ReadWarm warm(ctx, &part, 1);
+      old.drop();
       if ((rc = finish())) return rc;
+      while (h->done == 0 && !h->error) {
+        if (++waits > 100000) return set_err(ctx, DMM_ERR_STATE, "batched BFS did not terminate");
+        if (!ctx->batch_cont &&
+            (rc = capture_chain(ctx, "batch", &ctx->batch_cont, [&] { slots(ctx->batch_slots & 1, kBatchMoreSlots); })))
+          return rc;
+        DMM_HIP_CHECK(ctx, hipGraphLaunch(ctx->batch_cont, ctx->stream));
+        if ((rc = finish())) return rc;
+      }
     }
     if (h->error) return set_err(ctx, DMM_ERR_STATE, "batched BFS active list invariant violated");
     if (h->done == 3) {
@@ -1511,7 +1519,6 @@ int batch_run(dmm_ctx* ctx, const int32_t* sources, int32_t nsrc, uint8_t* depth
       continue;
     }
     if (want_depth) {
-      const ReadPart part = {depth, ctx->d_bdepth, static_cast<size_t>(int64_t(nsrc) * ctx->nloc)};
       if (depth && (rc = read_out(ctx, &part, 1))) return rc;
       ctx->bdepth_nsrc = nsrc;
     }

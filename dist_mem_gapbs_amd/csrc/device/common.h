@@ -281,8 +281,11 @@ struct dmm_ctx {
   dmm::PrCtrl* d_prctrl = nullptr;
   dmm::PrCtrl* h_prctrl = nullptr;
   char* h_ring = nullptr;        // pinned staging of reads (readout.hip)
+  char* h_ring_old = nullptr;    // the one before
+  size_t ring_touched = 0;       // its leading bytes that the host has used
   size_t ring_bytes = 0;
   uint32_t read_seq = 0;         // the last piece read
+  int short_reads = 0;           // reads that the ring was too small for
   int32_t* d_heavy = nullptr;    // vertices with in-degree >= heavy threshold, longest class first
   int64_t n_heavy = 0;
   int64_t n_giant = 0, n_wide = 0;  // its leading rows of kSweepGiant and, after them, kSweepWide in-edges and more
@@ -393,15 +396,19 @@ int read_out(dmm_ctx* ctx, const ReadPart* parts, int nparts);
 void read_free(dmm_ctx* ctx);
 
 // Allocates the ring that reads use and touches its pages, by a thread of its
-// own beside an upload of `rows` rows, and no longer than that takes: what is
-// not touched when this ends, the first read touches.  A page of pinned memory
-// costs 1.4 us when the host first touches it: a context's first search with
-// 1.6 MB read took 1.3 ms instead of 0.4.  An upload whose contexts stay, with
-// all of a larger ring touched before it ends: 32 K rows 1.2 ms, 0.66 so, 0.62
-// without a ring (and the first search 0.26, 0.26, 0.30).
+// own and no longer than what it is beside takes: an upload of `rows` rows (a
+// ring for what a search reads), or the search whose `parts` are read next, if
+// the ring is to grow for them.  What is not touched when this ends, the read
+// touches.  A page of pinned memory costs 1.4 us when the host first touches it,
+// and the allocation holds up others: a context's first search with 1.6 MB read
+// took 1.3 ms without this and 0.4 with it; but an upload of 32 K rows, of
+// contexts that stay, 1.2 ms with the ring of a batch (64 bytes a row) touched
+// whole, 0.64 so and 0.60 without a ring.
 struct ReadWarm {
   ReadWarm(dmm_ctx* ctx, int64_t rows);
+  ReadWarm(dmm_ctx* ctx, const ReadPart* parts, int nparts);
   ~ReadWarm();
+  void start(dmm_ctx* ctx, size_t want);
   std::atomic<bool> done{false};  // the upload: no page is touched any more
   std::thread thread;
 };

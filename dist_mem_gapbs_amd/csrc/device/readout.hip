@@ -25,7 +25,16 @@ namespace {
 constexpr size_t kPieceLeast = size_t(256) << 10;
 constexpr size_t kPieceMost = size_t(2) << 20;
 constexpr size_t kSmallRead = size_t(512) << 10;    // up to here one wait for all of it
-constexpr size_t kThreadedRead = size_t(2) << 20;  // helpers from here on: starting one costs some 15 us
+constexpr size_t kThreadedRead = size_t(2) << 20;  // helpers from here on: starting one costs some 15 us; also on new pages
+// A ring that is too small for a read: pieces of a quarter of it, for this many
+// reads.  After them it grows, beside the levels where there are some.  A whole
+// batch of 64 sources, the first through the search's ring, the second, the one
+// that enlarges it, later ones: 20 K vertices (1.3 MB) 389, 251, 489, 188 us; 131
+// K (8.4 MB) 952, 621, 1512, 450; enlarged by the upload 419, 254, 197 and 1405,
+// 506, 450, and the uploads 0.4 and 0.3 ms longer.
+constexpr int kShortSlots = 4;
+constexpr int kShortReads = 2;
+static_assert(kShortSlots <= kReadSlots, "flags");
 constexpr int kReaders = 4;
 constexpr int64_t kGroupLeast = int64_t(16) << 10;  // of a small read, by each workgroup
 constexpr int kThreads = 256;
@@ -84,40 +93,71 @@ __global__ __launch_bounds__(kThreads) void k_read(ReadList l, int n, char* slot
 
 void read_free(dmm_ctx* ctx) {
   if (ctx->h_ring) (void)hipHostFree(ctx->h_ring);
-  ctx->h_ring = nullptr;
+  if (ctx->h_ring_old) (void)hipHostFree(ctx->h_ring_old);
+  ctx->h_ring = ctx->h_ring_old = nullptr;
   ctx->ring_bytes = 0;
 }
 
-// A ring of `bytes` of slots (none if there is no pinned memory to be had).
+// A ring of `bytes` of slots in place of a smaller one, which stays in use if
+// there is no pinned memory to be had, and is freed with the next one replaced
+// otherwise (65 us, which is not for this read).
 static void ring_alloc(dmm_ctx* ctx, size_t bytes) {
-  read_free(ctx);
-  if (hipHostMalloc(reinterpret_cast<void**>(&ctx->h_ring), kFlagBytes + bytes, hipHostMallocDefault) != hipSuccess) {
-    ctx->h_ring = nullptr;
+  char* ring = nullptr;
+  if (hipHostMalloc(reinterpret_cast<void**>(&ring), kFlagBytes + bytes, hipHostMallocDefault) != hipSuccess) {
     (void)hipGetLastError();
     return;
   }
+  std::memset(ring, 0, kFlagBytes);
+  if (ctx->h_ring_old) (void)hipHostFree(ctx->h_ring_old);
+  ctx->h_ring_old = ctx->h_ring;
+  ctx->h_ring = ring;
   ctx->ring_bytes = bytes;
-  std::memset(ctx->h_ring, 0, kFlagBytes);
+  ctx->ring_touched = 0;
+  ctx->short_reads = 0;
   ctx->read_seq = 0;
 }
 
+// The slots of a read: an eighth of it each, between the least and the most.
+static size_t slot_bytes(size_t total) {
+  return std::min(kPieceMost, std::max(kPieceLeast, (total / kReadSlots + (size_t(1) << 16) - 1) >> 16 << 16));
+}
+
+static size_t total_bytes(const ReadPart* parts, int nparts) {
+  size_t total = 0;
+  for (int i = 0; i < nparts; i++) total += parts[i].dst ? parts[i].bytes : 0;
+  return total;
+}
+
+// The ring that a read can use.
+static size_t ring_of(const ReadPart* parts, int nparts) {
+  const size_t slot = slot_bytes(total_bytes(parts, nparts));
+  size_t slots = 0;
+  for (int i = 0; i < nparts; i++) slots += parts[i].dst ? (parts[i].bytes + slot - 1) / slot : 0;
+  return std::min<size_t>(slots, kReadSlots) * slot;
+}
+
 ReadWarm::ReadWarm(dmm_ctx* ctx, int64_t rows) {
-  const size_t search = 8 * static_cast<size_t>(rows);  // a parent and a depth, or an FP64 rank
-  // A larger ring is an allocation of its own in the driver, which holds up
-  // the upload's: no more than a search needs where that is a small read (a
-  // batch then enlarges it), else what a batch can use of it.
-  const size_t want = search <= kSmallRead
-                          ? 2 * kPieceLeast
-                          : std::min(kReadSlots * kPieceMost, 8 * search + kReadSlots * (size_t(1) << 16));
+  // A parent and a depth; an FP64 rank needs no more.
+  const size_t bytes = sizeof(int32_t) * static_cast<size_t>(rows);
+  const ReadPart search[] = {{ctx, nullptr, bytes}, {ctx, nullptr, bytes}};
+  start(ctx, ring_of(search, 2));
+}
+
+ReadWarm::ReadWarm(dmm_ctx* ctx, const ReadPart* parts, int nparts) {
+  if (ctx->short_reads >= kShortReads) start(ctx, ring_of(parts, nparts));
+}
+
+void ReadWarm::start(dmm_ctx* ctx, size_t want) {
   if (ctx->ring_bytes >= want) return;
-  const size_t touch = std::min(want, std::max(2 * kThreadedRead, 2 * search));
-  // Without a thread the first read allocates.
-  (void)start_thread(&thread, [this, ctx, want, touch] {
+  // Without a thread the read allocates.
+  (void)start_thread(&thread, [this, ctx, want] {
     (void)hipSetDevice(ctx->device);
     ring_alloc(ctx, want);
-    if (!ctx->h_ring) return;
-    for (size_t i = 0; i < touch && !done.load(std::memory_order_relaxed); i += 4096)
+    if (ctx->ring_bytes < want) return;
+    size_t i = 0;
+    for (; i < want && !done.load(std::memory_order_relaxed); i += 4096)
       reinterpret_cast<volatile char*>(ctx->h_ring)[kFlagBytes + i] = 0;
+    ctx->ring_touched = i;
   });
 }
 
@@ -127,30 +167,48 @@ ReadWarm::~ReadWarm() {
 }
 
 static int read_pieces(dmm_ctx* ctx, const ReadPart* parts, int nparts) {
-  size_t total = 0;
-  for (int i = 0; i < nparts; i++) total += parts[i].dst ? parts[i].bytes : 0;
+  const size_t total = total_bytes(parts, nparts);
   if (total == 0) {
     DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
     return DMM_OK;
   }
-  const size_t slot =
-      std::min(kPieceMost, std::max(kPieceLeast, (total / kReadSlots + (size_t(1) << 16) - 1) >> 16 << 16));
   std::vector<Piece> pieces;
-  for (int i = 0; i < nparts; i++) {
-    if (!parts[i].dst) continue;
-    char* d = static_cast<char*>(parts[i].dst);
-    const char* s = static_cast<const char*>(parts[i].src);
-    for (size_t o = 0; o < parts[i].bytes; o += slot) pieces.push_back({d + o, s + o, std::min(slot, parts[i].bytes - o)});
-  }
-  const int n = static_cast<int>(pieces.size());
+  auto cut = [&](size_t slot) {
+    pieces.clear();
+    for (int i = 0; i < nparts; i++) {
+      if (!parts[i].dst) continue;
+      char* d = static_cast<char*>(parts[i].dst);
+      const char* s = static_cast<const char*>(parts[i].src);
+      for (size_t o = 0; o < parts[i].bytes; o += slot)
+        pieces.push_back({d + o, s + o, std::min(slot, parts[i].bytes - o)});
+    }
+    return static_cast<int>(pieces.size());
+  };
   // Slot s holds the pieces s, s + slots, ...  The ring grows to what a read
-  // can use of it.
-  const int slots = std::min(n, kReadSlots);
+  // can use of it, but not for the first few that it is too small for, nor for
+  // one that smaller pieces get through it at once.
+  size_t slot = slot_bytes(total);
+  int n = cut(slot);
+  int slots = std::min(n, kReadSlots);
   if (ctx->ring_bytes < slots * slot) {
-    DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-    ring_alloc(ctx, slots * slot);
+    const size_t whole = slots * slot;
+    const auto quarters = [&] {
+      slot = ctx->ring_bytes / kShortSlots / 4096 * 4096;
+      n = cut(slot);
+      slots = std::min(n, kShortSlots);
+    };
+    if (ctx->ring_bytes > 0) quarters();
+    if (ctx->ring_bytes == 0 || (n > slots && ++ctx->short_reads > kShortReads)) {
+      DMM_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+      ring_alloc(ctx, whole);
+      if (ctx->ring_bytes >= whole) {
+        slot = slot_bytes(total);
+        n = cut(slot);
+        slots = std::min(n, kReadSlots);
+      }
+    }
   }
-  if (!ctx->h_ring) {  // no pinned memory to be had: the runtime's own path
+  if (ctx->ring_bytes == 0) {  // no pinned memory to be had: the runtime's own path
     for (int i = 0; i < nparts; i++)
       if (parts[i].dst && parts[i].bytes)
         DMM_HIP_CHECK(ctx, hipMemcpyAsync(parts[i].dst, parts[i].src, parts[i].bytes, hipMemcpyDeviceToHost, ctx->stream));
@@ -166,7 +224,7 @@ static int read_pieces(dmm_ctx* ctx, const ReadPart* parts, int nparts) {
     std::memset(flags, 0, kFlagBytes);
     ctx->read_seq = 0;
   }
-  const bool each = total > kSmallRead;
+  const bool each = total > kSmallRead || n > slots;
   const int groups = each ? kReadGroups : static_cast<int>(std::min<size_t>(kReadGroups, ceil_div(total, kGroupLeast)));
   const uint32_t seq = ctx->read_seq + 1;
   ctx->read_seq += static_cast<uint32_t>(n);
@@ -228,13 +286,15 @@ static int read_pieces(dmm_ctx* ctx, const ReadPart* parts, int nparts) {
   };
   queue(0, slots);
   std::thread helpers[kReaders - 1];
-  if (total >= kThreadedRead) {
+  const size_t used = slots * slot;
+  if (total >= kThreadedRead || (each && used > ctx->ring_touched)) {
     for (int k = 0; k < kReaders - 1; k++)
       if (!start_thread(&helpers[k], work)) break;  // those that there are read alone
   }
   work();
   for (auto& t : helpers)
     if (t.joinable()) t.join();
+  ctx->ring_touched = std::max(ctx->ring_touched, used);
   if (error.load()) {
     (void)hipStreamSynchronize(ctx->stream);
     return set_err(ctx, DMM_ERR_HIP, "reading results failed: %s", hipGetErrorString(static_cast<hipError_t>(error.load())));

@@ -113,7 +113,7 @@ for n in %r:
 """ % sizes)
     assert [n for n, _, _ in got] == sizes
     for n, first, again in got:
-        most = 512 << 10 if 8 * n <= 512 << 10 else min(16 << 20, 64 * n + (512 << 10))
+        most = min(16 << 20, max(512 << 10, 8 * n + (1 << 20)))  # eight slots, rounded to 64 KB
         assert 0 < first <= most + 4096, n
         assert again == 0, n
 

@@ -59,3 +59,28 @@ def test_parts_of_separate_allocations(dmm, orc, n):
         assert counts[s] == 1 and (counts[depth > 0] > 0).all()
         parent, depth, _ = c.DOBFS(s)
         assert np.array_equal(depth, orc.bfs_depth(og, s)) and orc.bfs_verify(og, s, parent)[0]
+
+
+# Up to 65536 rows the ring has two slots of 256 KB after the upload: results of
+# several parts that fill it, that need more of its quarters than it has, and
+# batches (64 bytes a row) that go through it and then enlarge it.
+@pytest.mark.parametrize("n", [9000, 21000, 22000, 30000, 33000, 33500, 44000, 65536])
+def test_reads_larger_than_the_ring(dmm, orc, n):
+    g = _graph(dmm, n)
+    og = orc.CSR.of(g)
+    srcs = dmm.pick_sources(g, 64)
+    s = int(srcs[0])
+    counts = orc.bc_forward(og, s)
+    depths = np.array([np.where(r < 0, 255, r) for r in (orc.bfs_depth(og, int(x)) for x in srcs[:8])], np.uint8)
+    ref = orc.bfs_depth(og, s)
+    for first in ("counts", "batch"):
+        with dmm.Context(0) as c:
+            c.set_layout(L.DMM_LAYOUT_NATURAL)
+            c.upload(g)
+            for k in range(6):
+                if first == "counts" or k > 3:
+                    for got, want in zip(c.bc_forward(s)[:3], counts):
+                        assert np.array_equal(got, want), (first, k)
+                if first == "batch" or k > 3:
+                    assert np.array_equal(c.bfs_batch64(srcs)[0][:8], depths), (first, k)
+                assert np.array_equal(c.DOBFS(s)[1], ref), (first, k)
