@@ -2,7 +2,9 @@
 #ifndef DMM_DEVICE_PR_H_
 #define DMM_DEVICE_PR_H_
 
+#include <memory>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "common.h"
@@ -160,17 +162,37 @@ struct BlockSplit {  // a one-row bucket in parts: partial slots [first, first +
   int32_t count;
   int32_t pad;
 };
+// An array whose elements hold nothing until they are written.
+template <typename T>
+class RawArray {
+ public:
+  RawArray() = default;
+  explicit RawArray(int64_t n) : p_(new T[static_cast<size_t>(n)]), n_(static_cast<size_t>(n)) {}
+  T& operator[](int64_t i) { return p_[i]; }
+  const T& operator[](int64_t i) const { return p_[i]; }
+  T* data() { return p_.get(); }
+  const T* data() const { return p_.get(); }
+  size_t size() const { return n_; }
+  void swap(RawArray& o) {
+    p_.swap(o.p_);
+    std::swap(n_, o.n_);
+  }
+
+ private:
+  std::unique_ptr<T[]> p_;
+  size_t n_ = 0;
+};
 struct BlockHost {
-  std::vector<uint16_t> src;       // window-major source offsets (window starts padded to kBPer)
+  RawArray<uint16_t> src;          // window-major source offsets (window starts padded to kBPer)
   std::vector<int64_t> wstart;     // window starts (+ end)
   std::vector<int32_t> wlen;       // window edge counts
   std::vector<int64_t> wseg;       // first segment of each window (+ end)
-  std::vector<int32_t> seg_e;      // segment start inside its window
-  std::vector<int32_t> seg_d;      // segment destination minus seg_e
+  RawArray<int32_t> seg_e;         // segment start inside its window
+  RawArray<int32_t> seg_d;         // segment destination minus seg_e
   std::vector<int64_t> wgroup;     // first group of 64 edges of each window (+ end)
-  std::vector<BlockGroup> groups;  // per group: where segments start in it
-  std::vector<uint16_t> brow_off;  // bucket-major; coarse: row offset inside the bucket, fine: place, rows by length
-  std::vector<FineRow> rows;       // fine: per bucket (from its first row on), longest class first
+  RawArray<BlockGroup> groups;     // per group: where segments start in it
+  RawArray<uint16_t> brow_off;     // bucket-major; coarse: row offset inside the bucket, fine: place, rows by length
+  RawArray<FineRow> rows;          // fine: per bucket (from its first row on), longest class first
   std::vector<BlockUnit> units;
   std::vector<BlockSplit> splits;
   int32_t n_slots = 0, n_windows = 0;

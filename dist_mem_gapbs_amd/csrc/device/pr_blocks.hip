@@ -32,6 +32,32 @@
 
 namespace dmm {
 
+namespace {
+
+// Buckets of the shape: their first rows (+ end).
+std::vector<int32_t> cut_buckets(int64_t n, const int64_t* off, const BlockShape& shape) {
+  std::vector<int32_t> brow{0};
+  int64_t rows = 0, edges = 0;
+  for (int64_t r = 0; r < n; r++) {
+    const int64_t d = off[r + 1] - off[r];
+    if (rows > 0 && (rows == shape.rows || edges + d > shape.edges)) {
+      brow.push_back(static_cast<int32_t>(r));
+      rows = edges = 0;
+    }
+    rows++;
+    edges += d;
+  }
+  if (n > 0) brow.push_back(static_cast<int32_t>(n));
+  return brow;
+}
+
+}  // namespace
+
+// Host time counts: a block's first iteration waits for this.  With many
+// windows the (window, bucket) tables are the larger part, so a bucket's entries
+// lie together, every pass over them is shared out, and nothing is filled
+// before it is written (33 M edges from 2^27 sources, fine: 297 ms for the first
+// iteration with window-major tables, serial passes and zeroed vectors).
 int build_blocks_host(int64_t n, int64_t n_gather, const int64_t* off, const int32_t* nbr, const BlockShape& shape,
                       BlockHost* out, std::string* err) {
   const int nt = resolve_threads(0);
@@ -42,80 +68,76 @@ int build_blocks_host(int64_t n, int64_t n_gather, const int64_t* off, const int
   }
   const int32_t nwin = static_cast<int32_t>(std::max<int64_t>(1, (n_gather + kBWin - 1) / kBWin));
   // 1. Buckets.
-  std::vector<int32_t> brow{0};
-  {
-    int64_t rows = 0, edges = 0;
-    for (int64_t r = 0; r < n; r++) {
-      const int64_t d = off[r + 1] - off[r];
-      if (rows > 0 && (rows == shape.rows || edges + d > shape.edges)) {
-        brow.push_back(static_cast<int32_t>(r));
-        rows = edges = 0;
-      }
-      rows++;
-      edges += d;
-    }
-    if (n > 0) brow.push_back(static_cast<int32_t>(n));
-  }
+  const std::vector<int32_t> brow = cut_buckets(n, off, shape);
   const int64_t nb = static_cast<int64_t>(brow.size()) - 1;
   if (nb > kBSegMax) {
     *err = "PE block has more row buckets than a window's segment table holds";
     return DMM_ERR_CAPACITY;
   }
-  // 2. Edges per (window, bucket), cnt[w * nb + b].
-  std::vector<int32_t> cnt(static_cast<size_t>(nwin) * std::max<int64_t>(1, nb), 0);
-  parallel_dynamic(nb, nt, 16, [&](int64_t b) {
-    for (int64_t e = off[brow[b]]; e < off[brow[b + 1]]; e++) {
-      const int32_t u = nbr[e];
-      cnt[static_cast<size_t>(u / kBWin) * nb + b]++;
+  // 2. Bucket-major: a segment's start inside its bucket, boff[b * pitch + w]
+  // (+ end).
+  const int64_t pitch = int64_t(nwin) + 1;
+  RawArray<uint32_t> boff(nb * pitch);
+  auto window = [](int32_t u) { return static_cast<uint32_t>(u) / kBWin; };
+  parallel_dynamic(nb, nt, 4, [&](int64_t b) {
+    uint32_t* o = &boff[b * pitch];
+    std::fill(o, o + pitch, 0u);
+    for (int64_t e = off[brow[b]]; e < off[brow[b + 1]]; e++) o[window(nbr[e]) + 1]++;
+    for (int32_t w = 0; w < nwin; w++) o[w + 1] += o[w];
+  });
+  std::vector<int64_t> bstart(nb + 1, 0);
+  for (int64_t b = 0; b < nb; b++) bstart[b + 1] = off[brow[b + 1]];
+  // 3. Window-major: its start inside its window, wrel[b * nwin + w]; a cache
+  // line of windows at a time.
+  constexpr int32_t kLine = 16;
+  const int64_t lines = (nwin + kLine - 1) / kLine;
+  RawArray<uint32_t> wrel(nb * nwin);
+  std::vector<int32_t> wlen(nwin, 0);
+  std::vector<int64_t> wseg(nwin + 1, 0);
+  parallel_dynamic(lines, nt, 1, [&](int64_t l) {
+    const int32_t w0 = static_cast<int32_t>(l) * kLine, w1 = std::min(nwin, w0 + kLine);
+    uint32_t run[kLine] = {};
+    int32_t segs[kLine] = {};
+    for (int64_t b = 0; b < nb; b++) {
+      const uint32_t* o = &boff[b * pitch];
+      uint32_t* r = &wrel[b * nwin];
+      for (int32_t w = w0; w < w1; w++) {
+        const uint32_t d = o[w + 1] - o[w];
+        r[w] = run[w - w0];
+        run[w - w0] += d;
+        segs[w - w0] += d > 0;
+      }
+    }
+    for (int32_t w = w0; w < w1; w++) {
+      wlen[w] = static_cast<int32_t>(run[w - w0]);
+      wseg[w + 1] = segs[w - w0];
     }
   });
-  // 3. Window-major starts (padded) and bucket-major starts per segment.
-  std::vector<int64_t> wstart(nwin + 1, 0);
-  std::vector<int32_t> wlen(nwin, 0);
+  std::vector<int64_t> wstart(nwin + 1, 0), wgroup(nwin + 1, 0);  // window starts padded
   for (int32_t w = 0; w < nwin; w++) {
-    int64_t len = 0;
-    for (int64_t b = 0; b < nb; b++) len += cnt[static_cast<size_t>(w) * nb + b];
-    wlen[w] = static_cast<int32_t>(len);
-    wstart[w + 1] = wstart[w] + (len + kBPer - 1) / kBPer * kBPer;
+    wstart[w + 1] = wstart[w] + (int64_t(wlen[w]) + kBPer - 1) / kBPer * kBPer;
+    wgroup[w + 1] = wgroup[w] + (wlen[w] + 63) / 64;
+    wseg[w + 1] += wseg[w];
   }
-  std::vector<int64_t> bstart(nb + 1, 0);
-  for (int64_t b = 0; b < nb; b++) bstart[b + 1] = bstart[b] + (off[brow[b + 1]] - off[brow[b]]);
-  // Segment (w, b): start in the window-major array, destination in the
-  // bucket-major array.
-  std::vector<int64_t> wpos(static_cast<size_t>(nwin) * std::max<int64_t>(1, nb)),
-      bpos(static_cast<size_t>(nwin) * std::max<int64_t>(1, nb));
-  for (int32_t w = 0; w < nwin; w++) {
-    int64_t p = wstart[w];
+  // 4. Segment tables per window (non-empty segments, bucket order), and where
+  // segments start, per group of 64 edges.
+  RawArray<int32_t> seg_e(wseg[nwin]), seg_d(wseg[nwin]);
+  parallel_dynamic(lines, nt, 1, [&](int64_t l) {
+    const int32_t w0 = static_cast<int32_t>(l) * kLine, w1 = std::min(nwin, w0 + kLine);
+    int64_t at[kLine];
+    for (int32_t w = w0; w < w1; w++) at[w - w0] = wseg[w];
     for (int64_t b = 0; b < nb; b++) {
-      wpos[static_cast<size_t>(w) * nb + b] = p;
-      p += cnt[static_cast<size_t>(w) * nb + b];
+      const uint32_t* o = &boff[b * pitch];
+      const uint32_t* r = &wrel[b * nwin];
+      for (int32_t w = w0; w < w1; w++) {
+        if (o[w + 1] == o[w]) continue;
+        const int64_t k = at[w - w0]++;
+        seg_e[k] = static_cast<int32_t>(r[w]);
+        seg_d[k] = static_cast<int32_t>(bstart[b] + o[w] - r[w]);
+      }
     }
-  }
-  for (int64_t b = 0; b < nb; b++) {
-    int64_t p = bstart[b];
-    for (int32_t w = 0; w < nwin; w++) {
-      bpos[static_cast<size_t>(w) * nb + b] = p;
-      p += cnt[static_cast<size_t>(w) * nb + b];
-    }
-  }
-  // 4. Segment tables per window (non-empty segments, bucket order).
-  std::vector<int64_t> wseg(nwin + 1, 0);
-  std::vector<int32_t> seg_e;
-  std::vector<int32_t> seg_d;
-  for (int32_t w = 0; w < nwin; w++) {
-    for (int64_t b = 0; b < nb; b++) {
-      const size_t k = static_cast<size_t>(w) * nb + b;
-      if (!cnt[k]) continue;
-      const int64_t e = wpos[k] - wstart[w];
-      seg_e.push_back(static_cast<int32_t>(e));
-      seg_d.push_back(static_cast<int32_t>(bpos[k] - e));
-    }
-    wseg[w + 1] = static_cast<int64_t>(seg_e.size());
-  }
-  // Where segments start, per group of 64 edges.
-  std::vector<int64_t> wgroup(nwin + 1, 0);
-  for (int32_t w = 0; w < nwin; w++) wgroup[w + 1] = wgroup[w] + (wlen[w] + 63) / 64;
-  std::vector<BlockGroup> groups(wgroup[nwin]);
+  });
+  RawArray<BlockGroup> groups(wgroup[nwin]);
   parallel_dynamic(nwin, nt, 1, [&](int64_t w) {
     int32_t k = 0;
     const int32_t* se = seg_e.data() + wseg[w];
@@ -130,12 +152,15 @@ int build_blocks_host(int64_t n, int64_t n_gather, const int64_t* off, const int
   // 5. Fine buckets: rows by length, longest first (row order inside a length
   // class of powers of two, so that the rows of a wavefront are alike), and
   // their runs of places in that order.
-  std::vector<FineRow> rows(shape.fine ? n : 0);
-  std::vector<int32_t> place(shape.fine ? n : 0, 0);  // each row's next place
+  RawArray<FineRow> rows(shape.fine ? n : 0);
+  RawArray<int32_t> place(shape.fine ? n : 0);  // each row's next place
   std::vector<int32_t> nlong(nb, 0), nmid(nb, 0);
   if (shape.fine)
     parallel_dynamic(nb, nt, 16, [&](int64_t b) {
-      if (brow[b + 1] - brow[b] == 1) return;  // one-row units need no order
+      if (brow[b + 1] - brow[b] == 1) {  // one-row units need no order
+        rows[brow[b]] = {};
+        return;
+      }
       auto len = [&](int64_t r) { return off[r + 1] - off[r]; };
       auto cls = [&](int64_t r) {  // 0: longest, 64: empty
         return len(r) == 0 ? 64 : __builtin_clzll(static_cast<unsigned long long>(len(r)));
@@ -156,17 +181,22 @@ int build_blocks_host(int64_t n, int64_t n_gather, const int64_t* off, const int
         next += rows[i].len;
       }
     });
-  // 6. Fill both arrays, bucket by bucket (disjoint segments).
-  std::vector<uint16_t> src(std::max<int64_t>(1, wstart[nwin]), 0);
-  std::vector<uint16_t> brow_off(std::max<int64_t>(1, m), 0);
-  parallel_dynamic(nb, nt, 16, [&](int64_t b) {
+  // 6. Fill both arrays, bucket by bucket (disjoint segments); the tables' words
+  // are each segment's next place in them.
+  RawArray<uint16_t> src(std::max<int64_t>(1, wstart[nwin]));
+  RawArray<uint16_t> brow_off(std::max<int64_t>(1, m));
+  src[0] = brow_off[0] = 0;
+  for (int32_t w = 0; w < nwin; w++) std::fill(&src[0] + wstart[w] + wlen[w], &src[0] + wstart[w + 1], uint16_t(0));
+  parallel_dynamic(nb, nt, 4, [&](int64_t b) {
     const bool places = shape.fine && brow[b + 1] - brow[b] > 1;
+    uint32_t* o = &boff[b * pitch];
+    uint32_t* p = &wrel[b * nwin];
+    uint16_t* const to = &brow_off[0] + bstart[b];
     for (int64_t r = brow[b]; r < brow[b + 1]; r++)
       for (int64_t e = off[r]; e < off[r + 1]; e++) {
-        const int32_t u = nbr[e];
-        const size_t k = static_cast<size_t>(u / kBWin) * nb + b;
-        src[wpos[k]++] = static_cast<uint16_t>(u % kBWin);
-        brow_off[bpos[k]++] = static_cast<uint16_t>(places ? place[r]++ : r - brow[b]);
+        const uint32_t w = window(nbr[e]);
+        src[wstart[w] + p[w]++] = static_cast<uint16_t>(static_cast<uint32_t>(nbr[e]) % kBWin);
+        to[o[w]++] = static_cast<uint16_t>(places ? place[r]++ : r - brow[b]);
       }
   });
   // 7. Units: a bucket whole, or a one-row bucket beyond shape.edges in parts
@@ -205,11 +235,12 @@ int build_blocks_host(int64_t n, int64_t n_gather, const int64_t* off, const int
 
 namespace {
 
-template <typename T>
-int upload_vec(dmm_ctx* ctx, void** dst, const std::vector<T>& v, const char* what) {
-  int rc = dev_alloc(ctx, dst, sizeof(T) * std::max<size_t>(1, v.size()), what);
+template <typename Array>
+int upload_vec(dmm_ctx* ctx, void** dst, const Array& v, const char* what) {
+  const size_t bytes = sizeof(*v.data()) * v.size();
+  int rc = dev_alloc(ctx, dst, std::max(sizeof(*v.data()), bytes), what);
   if (rc) return rc;
-  if (!v.empty()) DMM_HIP_CHECK(ctx, hipMemcpy(*dst, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
+  if (bytes) DMM_HIP_CHECK(ctx, hipMemcpy(*dst, v.data(), bytes, hipMemcpyHostToDevice));
   return DMM_OK;
 }
 
@@ -230,8 +261,8 @@ BlockShape fine_shape(int64_t m, int cus) {
 int pr_blocks_build(dmm_ctx* ctx) {
   const int64_t n = ctx->nloc;
   const int64_t m = ctx->m_in;
-  std::vector<int64_t> off(n + 1);
-  std::vector<int32_t> nbr(std::max<int64_t>(1, m));
+  RawArray<int64_t> off(n + 1);
+  RawArray<int32_t> nbr(std::max<int64_t>(1, m));
   DMM_HIP_CHECK(ctx, hipMemcpy(off.data(), ctx->d_in_off, sizeof(int64_t) * (n + 1), hipMemcpyDeviceToHost));
   if (m > 0) DMM_HIP_CHECK(ctx, hipMemcpy(nbr.data(), ctx->d_in_nbr, sizeof(int32_t) * m, hipMemcpyDeviceToHost));
   BlockHost bh;
@@ -242,8 +273,8 @@ int pr_blocks_build(dmm_ctx* ctx) {
   ctx->bp_fine = rc == DMM_OK;
   if (rc == DMM_ERR_CAPACITY) rc = build_blocks_host(n, ctx->n, off.data(), nbr.data(), kCoarse, &bh, &err);
   if (rc) return set_err(ctx, rc, "%s", err.c_str());
-  std::vector<int64_t>().swap(off);
-  std::vector<int32_t>().swap(nbr);
+  RawArray<int64_t>().swap(off);
+  RawArray<int32_t>().swap(nbr);
   if ((rc = upload_vec(ctx, &ctx->d_bp_src, bh.src, "PR block sources")) ||
       (rc = upload_vec(ctx, &ctx->d_bp_wstart, bh.wstart, "PR block window starts")) ||
       (rc = upload_vec(ctx, &ctx->d_bp_wlen, bh.wlen, "PR block window lengths")) ||
