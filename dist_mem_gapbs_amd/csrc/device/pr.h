@@ -116,10 +116,11 @@ int pr_tiles_build(dmm_ctx* ctx);
 //   fine    a bucket's contributions fit LDS: pass 2 sorts them there by row
 //           (static places) and sums each row's run in registers
 //   coarse  a bucket's row accumulators fit LDS: pass 2 adds every
-//           contribution with LDS atomics.  Only for blocks with more fine
-//           buckets than a window's segment table holds (some 125 M
-//           in-edges): the atomics run at about 350 G/s, and a block that does
-//           not fill the CUs with buckets of 2^19 edges waits for the largest.
+//           contribution with LDS atomics, at about 350 G/s, and a block that
+//           does not fill the CUs with buckets of 2^19 edges waits for the
+//           largest.  For blocks with more fine buckets than a window's segment
+//           table holds (from some 125 M in-edges or 16 M rows on), and where
+//           the fine buckets' shorter segments cost more (fine_is_faster).
 //           Kronecker-23, block 3 of 8, pass 1 + pass 2: coarse 52 + 281 us,
 //           fine 61 + 75 us.
 constexpr int kBWin = 32768;             // sources per window (128 KB of LDS)

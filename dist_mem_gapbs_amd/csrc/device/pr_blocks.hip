@@ -258,6 +258,80 @@ BlockShape fine_shape(int64_t m, int cus) {
   return shape;
 }
 
+// Whether a block's iteration is faster with the fine buckets of fine_shape
+// than with coarse ones, from what the two shapes take beyond what they have in
+// common (us; each term fitted to blocks of 2 to 126 M edges from 2^23 to 2^27
+// sources):
+//   fine    3.5 per M edges (both passes), 13 per M segments: pass 1 writes a
+//           segment at a time, and the more windows, the shorter they are
+//   coarse  1.6 per M edges (pass 1), 13 per M segments (few), and the edges of
+//           the workgroup that has most (pass 2): 0.42 ns for each, and 0.37
+//           for one that follows another of its row in a segment, whose LDS
+//           atomics wait for each other; 0.1 ns for those of one-row units
+// So blocks of like rows are better coarse from some 50 M edges on, or 30 M from
+// many windows (uniform, 2^23 sources, 67 M: fine 272 us, coarse 225; 2^25, 126
+// M: 645, 467; 2^27, 34 M: 321, 286; 2^25, 34 M: 179, 198), Kronecker blocks,
+// whose hubs crowd one coarse unit, only where the fine buckets hardly fit
+// (Kronecker-24, an eighth, 66 M: 321, 437; -26, a 32nd: 452, 548; -25, a ninth,
+// 117 M: 648, 641).  Of 60 blocks measured both ways none was 5% slower than
+// the better.
+constexpr double kFineEdgeUs = 3.5e-6, kCoarseEdgeUs = 1.6e-6, kSegmentUs = 13e-6;
+constexpr double kAtomicUs = 0.42e-3, kRepeatUs = 0.37e-3, kOneRowUs = 0.1e-3;
+
+bool fine_is_faster(int64_t n, int64_t n_gather, const int64_t* off, const int32_t* nbr, int cus, double* us) {
+  const double m = static_cast<double>(off[n]);
+  const double nwin = static_cast<double>(std::max<int64_t>(1, ceil_div(n_gather, kBWin)));
+  const BlockShape fine = fine_shape(off[n], cus);
+  const double nb_fine = static_cast<double>(cut_buckets(n, off, fine).size()) - 1;
+  us[0] = kFineEdgeUs * m;
+  us[1] = kCoarseEdgeUs * m;
+  if (nb_fine > kBSegMax) return false;
+  const std::vector<int32_t> coarse = cut_buckets(n, off, kCoarse);
+  const int64_t nb_coarse = static_cast<int64_t>(coarse.size()) - 1;
+  // Pass 2 of the coarse units, dealt in turn.
+  std::vector<double> load(std::max(1, cus), 0.0);
+  size_t unit = 0;
+  for (int64_t b = 0; b < nb_coarse; b++) {
+    const int64_t edges = off[coarse[b + 1]] - off[coarse[b]];
+    if (coarse[b + 1] - coarse[b] == 1) {
+      for (int64_t e = 0; e < std::max<int64_t>(1, edges); e += kCoarse.edges)
+        load[unit++ % load.size()] += kOneRowUs * static_cast<double>(std::min(kCoarse.edges, edges - e));
+      continue;
+    }
+    double repeats = 0;
+    for (int64_t r = coarse[b]; r < coarse[b + 1]; r++) {
+      const double d = static_cast<double>(off[r + 1] - off[r]);
+      // Edges less the segments that they fall into.
+      if (d > 1) repeats += d - nwin * -std::expm1(-d / nwin);
+    }
+    load[unit++ % load.size()] += kAtomicUs * static_cast<double>(edges) + kRepeatUs * std::max(0.0, repeats);
+  }
+  us[1] += *std::max_element(load.begin(), load.end());
+  // At most a segment per edge, and per window and bucket.
+  if (us[0] + kSegmentUs * std::min(m, nb_fine * nwin) <= us[1]) return true;
+  if (us[0] > us[1] + kSegmentUs * std::min(m, static_cast<double>(nb_coarse) * nwin)) return false;
+  // Else those of buckets of the same size: a window that has the share p of
+  // the edges is met by 1 - (1 - p)^(edges) of them.
+  const int nt = resolve_threads(0);
+  std::vector<std::vector<uint32_t>> part(nt);
+  parallel_dynamic(nt, nt, 1, [&](int64_t t) {
+    std::vector<uint32_t>& c = part[t];
+    c.assign(static_cast<size_t>(nwin), 0);
+    for (int64_t e = off[n] * t / nt; e < off[n] * (t + 1) / nt; e++) c[static_cast<uint32_t>(nbr[e]) / kBWin]++;
+  });
+  double segs_fine = 0, segs_coarse = 0;
+  for (size_t w = 0; w < static_cast<size_t>(nwin); w++) {
+    double p = 0;
+    for (const auto& c : part) p += c[w];
+    p /= m;
+    segs_fine += nb_fine * -std::expm1(-m / nb_fine * p);
+    segs_coarse += static_cast<double>(nb_coarse) * -std::expm1(-m / static_cast<double>(nb_coarse) * p);
+  }
+  us[0] += kSegmentUs * segs_fine;
+  us[1] += kSegmentUs * segs_coarse;
+  return us[0] <= us[1];
+}
+
 int pr_blocks_build(dmm_ctx* ctx) {
   const int64_t n = ctx->nloc;
   const int64_t m = ctx->m_in;
@@ -268,10 +342,10 @@ int pr_blocks_build(dmm_ctx* ctx) {
   BlockHost bh;
   std::string err;
   const int64_t held = ctx->dev_bytes;
-  // Fine buckets where a window's segment table holds them.
-  int rc = build_blocks_host(n, ctx->n, off.data(), nbr.data(), fine_shape(m, ctx->cu_count), &bh, &err);
-  ctx->bp_fine = rc == DMM_OK;
-  if (rc == DMM_ERR_CAPACITY) rc = build_blocks_host(n, ctx->n, off.data(), nbr.data(), kCoarse, &bh, &err);
+  double us[2];
+  ctx->bp_fine = m < (int64_t(1) << 31) && fine_is_faster(n, ctx->n, off.data(), nbr.data(), ctx->cu_count, us);
+  int rc = build_blocks_host(n, ctx->n, off.data(), nbr.data(), ctx->bp_fine ? fine_shape(m, ctx->cu_count) : kCoarse,
+                             &bh, &err);
   if (rc) return set_err(ctx, rc, "%s", err.c_str());
   RawArray<int64_t>().swap(off);
   RawArray<int32_t>().swap(nbr);
@@ -496,4 +570,17 @@ extern "C" int dmm_pr_blocks_check(int64_t n, int64_t n_gather, const int64_t* o
   stats[4] = static_cast<int64_t>(bh.seg_e.size());
   stats[5] = bh.n_slots;
   return DMM_OK;
+}
+
+// Host check of the choice between the shapes: 1 if a block's iteration on a
+// GPU of `cus` CUs would take fine buckets; us[2]: the estimates that decided
+// it, as far as they were needed.
+extern "C" int dmm_pr_blocks_shape(int64_t n, int64_t n_gather, const int64_t* off, const int32_t* nbr, int32_t cus,
+                                   double* us) {
+  using namespace dmm;
+  if (n < 0 || !off || (off[n] > 0 && !nbr) || !us || cus < 1)
+    return set_err(nullptr, DMM_ERR_INVALID, "dmm_pr_blocks_shape: bad arguments");
+  for (int64_t e = 0; e < off[n]; e++)
+    if (nbr[e] < 0 || nbr[e] >= n_gather) return set_err(nullptr, DMM_ERR_GRAPH, "source outside [0, n_gather)");
+  return fine_is_faster(n, n_gather, off, nbr, cus, us) ? 1 : 0;
 }

@@ -479,6 +479,12 @@ int dmm_pr_tiles_check(int64_t n, int64_t zb, int64_t n_gather, const int64_t* i
 int dmm_pr_blocks_check(int64_t n, int64_t n_gather, const int64_t* in_offsets,
                         const int32_t* in_neighs, const float* contrib, float* incoming,
                         int64_t* stats);
+/* Host check of which of its two layouts such a block's iteration uses on a
+ * GPU of `cus` CUs: 1 for the one of fine buckets, 0 for the one of coarse
+ * ones; us[2]: what the two were estimated to take (as far as the choice
+ * needed it).  No reference counterpart. */
+int dmm_pr_blocks_shape(int64_t n, int64_t n_gather, const int64_t* in_offsets,
+                        const int32_t* in_neighs, int32_t cus, double* us);
 
 /* ======================================================================== */
 /* Autotuner                                                                 */

@@ -60,3 +60,33 @@ def test_block_sums_exact(dmm, kind, n_gather):
         for _ in range(2):  # the first call builds the layout
             got, _, _ = c.pr_block_iteration(contrib, np.zeros(rows, np.float32), L.DMM_PR_FP32_KAHAN)
             assert np.array_equal(got, expect)
+
+
+def test_coarse_block_sums_exact(dmm):
+    """A block of like rows from many windows, which takes coarse buckets: every
+    row as the host's replay of the layout, bit for bit."""
+    n_gather, m = 1 << 26, 36 << 20
+    rng = np.random.default_rng(26)
+    rows = m // 32
+    lengths = np.full(rows, 32)
+    lengths[:4000] = rng.integers(0, 65, 4000)
+    lengths[100] = 600000  # in parts
+    lengths[-1] += 5
+    off = np.concatenate(([0], np.cumsum(lengths)))
+    src = rng.integers(0, n_gather, off[-1], dtype=np.int32)
+    contrib = (rng.random(n_gather, np.float32) / np.float32(n_gather)).astype(np.float32)
+    lib = L.load()
+    us, inc, st = np.zeros(2), np.empty(rows, np.float32), np.zeros(6, np.int64)
+    assert lib.dmm_pr_blocks_shape(rows, n_gather, L.ptr(off, C.c_int64), L.ptr(src, C.c_int32), 256,
+                                   L.ptr(us, C.c_double)) == 0
+    assert lib.dmm_pr_blocks_check(rows, n_gather, L.ptr(off, C.c_int64), L.ptr(src, C.c_int32),
+                                   L.ptr(contrib, C.c_float), L.ptr(inc, C.c_float), L.ptr(st, C.c_int64)) == 0
+    base = (np.float32(1.0) - np.float32(0.85)) / np.float32(n_gather)
+    expect = (base + (np.float32(0.85) * inc).astype(np.float32)).astype(np.float32)
+    with dmm.Context(0) as c:
+        c.set_layout(L.DMM_LAYOUT_NATURAL)
+        c.upload(num_nodes=n_gather, out_offsets=np.arange(rows + 1), out_neighs=np.zeros(rows, np.int32),
+                 in_offsets=off, in_neighs=src, vbegin=7, vend=7 + rows)
+        for _ in range(2):
+            got, _, _ = c.pr_block_iteration(contrib, np.zeros(rows, np.float32), L.DMM_PR_FP32_KAHAN)
+            assert np.array_equal(got, expect)

@@ -112,3 +112,33 @@ def test_blocks_hub_row_summed_in_parts():
 
 def test_blocks_empty():
     check(np.zeros(5, np.int64), np.zeros(0, np.int32), 10, np.ones(10, np.float32))
+
+
+def _shape(lengths, n_gather, src, cus=256):
+    off = np.concatenate(([0], np.cumsum(lengths))).astype(np.int64)
+    us = np.zeros(2)
+    rc = L.load().dmm_pr_blocks_shape(len(lengths), n_gather, L.ptr(off, C.c_int64),
+                                      L.ptr(np.ascontiguousarray(src, np.int32), C.c_int32), cus, L.ptr(us, C.c_double))
+    assert rc in (0, 1), L.load().dmm_last_error(None)
+    return rc
+
+
+def test_blocks_shape_by_rows_and_windows():
+    """Fine buckets for small blocks and for those whose hubs crowd one coarse
+    bucket, coarse ones for large blocks of like rows, from fewer edges on the
+    more windows their segments are cut by, and for more rows or edges than the
+    fine ones' segment table holds."""
+    rng = np.random.default_rng(7)
+    assert _shape([], 10, []) == 1 and _shape([0, 0, 0], 10, []) == 1
+    assert _shape([32] * 1000, 1 << 27, rng.integers(0, 1 << 27, 32000)) == 1
+    m = 36 << 20
+    lengths = np.full(m // 32, 32)
+    one = rng.integers(0, 1 << 27, m, dtype=np.int32)
+    assert _shape(lengths, 1 << 27, one) == 0
+    assert _shape(lengths, 1 << 22, one >> 5) == 1
+    hub = lengths.copy()
+    hub[5] = 400000
+    hub[6:6 + (400000 - 32) // 32 + 1] = 0
+    hub[-1] += m - hub.sum()
+    assert hub.sum() == m and _shape(hub, 1 << 22, one >> 5) == 1
+    assert _shape(np.zeros(8001 * 2048, np.int64), 100, []) == 0
