@@ -665,7 +665,7 @@ int dmm_graph_upload(dmm_ctx* ctx, int64_t num_nodes, int64_t vbegin, int64_t ve
         (rc = A((void**)&ctx->d_inv, sizeof(int32_t) * rows, "layout inverse")) ||
         (rc = A((void**)&ctx->d_parent_out, 2 * sizeof(int32_t) * rows, "parent and depth (original IDs)")))
       return rc;
-    ctx->d_depth_out = ctx->d_parent_out + rows;  // read out in one piece
+    ctx->d_depth_out = ctx->d_parent_out + rows;  // one allocation
     DMM_HIP_CHECK(ctx, hipMemcpy(ctx->d_perm, ctx->h_perm.data(), sizeof(int32_t) * rows, hipMemcpyHostToDevice));
     DMM_HIP_CHECK(ctx, hipMemcpy(ctx->d_inv, inv.data(), sizeof(int32_t) * rows, hipMemcpyHostToDevice));
     if ((rc = dmm::relabel_upload(ctx, out_offsets, out_neighs, inv, &new_out_off, &ctx->d_out_off, &ctx->d_out_nbr)))

@@ -65,7 +65,7 @@ struct PrArgs {
   int64_t light_begin, light_end; // light-row range (heavy rows inside are skipped)
   int64_t zero_begin;             // rows [zero_begin, nloc) have no in-edges
   int heavy_threshold;
-  double* err_part;               // [light | heavy-or-items | super] blocks
+  double* err_part;               // [main | super] blocks
   int serial_hub;                     // contributions [0, serial_hub) go to LDS (serial mode)
   int super_blocks;
   int main_blocks;                // error partials written before the combine
@@ -272,11 +272,12 @@ __device__ __forceinline__ void hub_gathers(const T* hub, int hub_n, const T* __
 //                on by a workgroup, by exact composition (serial_fold)
 // What bounds it: the gathers beyond the LDS hub, some 200 G/s (a cache line
 // into L1 for each), and per CU about 1/256 of that, so items are dealt to
-// the CUs by their edges (serial_plan).  Kronecker-21, per iteration: 260 us;
-// 2150 us with a wavefront per heavy row adding shuffled values one by one
-// (the longest row, some 10^5 edges, took that long), 340 us with these
-// items strided over small workgroups without the hub, 327 us with the hub
-// and strided.
+// the CUs by their edges (serial_plan).  Kronecker-21, per iteration that runs:
+// 262 us (242 G edges/s, those that the hub serves included); 6.12 ms with a
+// wavefront per heavy row adding shuffled values one by one (the longest row,
+// some 10^5 edges, took that long).  A whole rank of 7 iterations, when the
+// items came: 2.42 ms, strided over small workgroups without the hub 2.67,
+// strided with it 2.9.
 //
 // Long rows by composition.  While the running sum S stays inside one binade
 // [2^E, 2^(E+1)), S is an integer multiple of u = 2^(E-23), and adding x >= 0
@@ -1800,8 +1801,6 @@ __global__ __launch_bounds__(kBSumThreads) void k_bsum(PrArgs a, BpArgs b, float
   if (threadIdx.x == 0) a.err_part[blockIdx.x] = t;
 }
 
-// The one-row buckets in parts: each row's partial sums (exact) in slot
-// order, then the row finishes.
 // The last iteration's error (the others' are reduced by the kernel that
 // follows them, pr_begin), by one workgroup; partial `own` is `mine`.
 __device__ __forceinline__ void reduce_error(const PrArgs& a, int own, double mine, double* red) {
@@ -1817,8 +1816,9 @@ __device__ __forceinline__ void reduce_error(const PrArgs& a, int own, double mi
   }
 }
 
-// With one workgroup (up to kThreads split rows) also the reduction of the
-// error, 4 us of a launch less.
+// The one-row buckets in parts: each row's partial sums (exact) in slot order,
+// then the row finishes.  With one workgroup (up to kThreads split rows) also
+// the reduction of the error, 4 us of a launch less.
 __global__ __launch_bounds__(kThreads) void k_bsplit(PrArgs a, BpArgs b, float* __restrict__ cout,
                                                      float* __restrict__ score) {
   __shared__ double red[kThreads / 64];

@@ -97,9 +97,9 @@ def counted(tmp_path_factory):
 
 
 def test_an_upload_pins_what_a_search_reads(counted):
-    """The ring for reads: of a small graph the slots of a search's two small
-    parts, of a larger one at most 64 bytes a row beside the slots' rounding,
-    and none for a graph of the same size again."""
+    """The ring for reads: a parent and a depth in at most eight slots, each
+    rounded to 64 KB, of 256 KB at least; none for a graph of the same size
+    again."""
     sizes = [100, 1000, 32768, 65536, 65537, 131072, 600001]
     got = counted("""
 for n in %r:
