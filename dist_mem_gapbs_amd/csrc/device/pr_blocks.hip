@@ -313,10 +313,9 @@ bool fine_is_faster(int64_t n, int64_t n_gather, const int64_t* off, const int32
   // Else those of buckets of the same size: a window that has the share p of
   // the edges is met by 1 - (1 - p)^(edges) of them.
   const int nt = resolve_threads(0);
-  std::vector<std::vector<uint32_t>> part(nt);
+  std::vector<std::vector<uint32_t>> part(nt, std::vector<uint32_t>(static_cast<size_t>(nwin), 0));
   parallel_dynamic(nt, nt, 1, [&](int64_t t) {
     std::vector<uint32_t>& c = part[t];
-    c.assign(static_cast<size_t>(nwin), 0);
     for (int64_t e = off[n] * t / nt; e < off[n] * (t + 1) / nt; e++) c[static_cast<uint32_t>(nbr[e]) / kBWin]++;
   });
   double segs_fine = 0, segs_coarse = 0;
