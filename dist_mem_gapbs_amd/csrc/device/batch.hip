@@ -54,7 +54,8 @@ constexpr int kGroup = 8;  // lanes per vertex in the bottom-up sweep
 // registers leave room for five, and every workgroup reads every partial.
 // 64 lanes with 1, 2, 4, 8, 16 per CU: 22 K Kronecker vertices 173, 180, 200,
 // 264, 455 us; 131 K 221, 200, 203, 258, 428; 900 K 788, 565, 497, 589, 849;
-// 3.7 M uniform 5.00, 4.41, 4.36, 4.55, 4.62 ms.
+// 3.7 M uniform 5.00, 4.41, 4.36, 4.55, 4.62 ms.  4 and 8, sweeps alone:
+// Kronecker-24 5.31, 5.30 ms, uniform-25 49.3, 49.2, Kronecker-26 23.5, 23.1.
 constexpr int64_t kBatchRows = 256;
 constexpr int kBatchMostPerCU = 4;
 constexpr int kBatchMostSlots = 64;  // of a captured chain, but for one
@@ -122,7 +123,8 @@ struct BArgs {
   int td_div;
   int undirected;     // in-CSR == out-CSR
   const int32_t* heavy;       // rows by in-degree class, longest first:
-  int64_t n_giant, n_wide;    // the leading ones of kSweepGiant and, after them, kSweepWide in-edges and more
+  int64_t n_giant, n_wide;    // the leading giant and, after them, the other wide ones
+  int64_t wide;               // wide rows: of this many in-edges and more
 };
 
 struct TdLds {
@@ -355,7 +357,7 @@ __device__ __forceinline__ int64_t sweep_row(const int32_t* __restrict__ in_nbr,
   return stop;
 }
 
-// Rows beyond kSweepWide in-edges: by a wavefront (kWaves 1) or a workgroup
+// Wide rows (see kSweepWide): by a wavefront (kWaves 1) or a workgroup
 // (its kWaves), one edge per lane and then kWideUnroll per lane and round,
 // stopping as soon as every needed lane is found.  An 8-lane group took 256
 // edges a round, so a hub's row was the sweep: 318 us for one level of a
@@ -481,7 +483,7 @@ __device__ void bu_phase(const BArgs& a, const BIo& io, SmallLds& L, int level) 
   };
   auto row = [&](int64_t u, const RowHead& h, RowHead& hn) {
     hn = load_head(u + ngrp);
-    if (h.e - h.b >= kSweepWide) return;  // a wide row
+    if (h.e - h.b >= a.wide) return;  // a wide row
     const uint64_t s = h.seen | h.fl;
     const uint64_t need = lanes & ~s;
     uint64_t nxt = 0;
@@ -947,6 +949,7 @@ BArgs make_args(dmm_ctx* ctx, int nsrc, int td_div) {
   a.heavy = ctx->d_heavy;
   a.n_giant = ctx->n_giant;
   a.n_wide = ctx->n_wide;
+  a.wide = ctx->sweep_wide;
   return a;
 }
 

@@ -748,12 +748,14 @@ int dmm_graph_upload(dmm_ctx* ctx, int64_t num_nodes, int64_t vbegin, int64_t ve
     for (int32_t r : heavy) at[cls(r) + 1]++;
     for (int c = 0; c < 64; c++) at[c + 1] += at[c];
     ctx->n_giant = ctx->n_wide = 0;
+    ctx->sweep_wide = rows < dmm::kSweepHuge ? dmm::kSweepWide : dmm::kSweepHugeWide;
+    const int64_t giant = rows < dmm::kSweepHuge ? dmm::kSweepGiant : dmm::kSweepHugeGiant;
     for (int32_t r : heavy) {
       by_class[at[cls(r)]++] = r;
       const int64_t d = ioff[r + 1] - ioff[r];
-      if (d >= dmm::kSweepGiant)
+      if (d >= giant)
         ctx->n_giant++;
-      else if (d >= dmm::kSweepWide)
+      else if (d >= ctx->sweep_wide)
         ctx->n_wide++;
     }
   }

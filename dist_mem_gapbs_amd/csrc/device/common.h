@@ -29,9 +29,18 @@ constexpr int kHeadNbrs = 4;        // in-neighbours per row in the head array
 // two, so that they lead the list by classes).  64 lanes on Kronecker graphs,
 // whole call: 131 K vertices 1108 us with 8-lane groups for all rows, 769
 // with 512 / 16384, 755 with 512 / 4096; 900 K vertices 4.29, 1.91, 1.87 ms.
-// 256 or 1024 for the first: within 2%.
+// 256 or 1024 for the first: within 2%.  From kSweepHuge vertices on, where most
+// words come from HBM, what a round reads beyond the lanes' last word costs more
+// than its latency, and a wavefront waits for each of the many wide rows that
+// late sweeps find without need: with 512 / 4096, 8192 / 65536 (and with groups
+// for all rows) 10 M Kronecker vertices 2.60, 3.10 (9.9) ms, 13 M 3.37, 3.42
+// (7.0), 16.7 M 4.45, 4.35 (11.1), Kronecker-24 5.32, 5.09 (5.85), -25 12.1, 11.6
+// (17.4), -26 23.8, 21.7 (21.9).
 constexpr int64_t kSweepWide = 512;
 constexpr int64_t kSweepGiant = 4096;
+constexpr int64_t kSweepHuge = int64_t(7) << 21;
+constexpr int64_t kSweepHugeWide = 8192;
+constexpr int64_t kSweepHugeGiant = 65536;
 
 // What the host needs of a finished device-loop search, written by its
 // last kernel into mapped host memory (no copy back).
@@ -288,7 +297,8 @@ struct dmm_ctx {
   int short_reads = 0;           // reads that the ring was too small for
   int32_t* d_heavy = nullptr;    // vertices with in-degree >= heavy threshold, longest class first
   int64_t n_heavy = 0;
-  int64_t n_giant = 0, n_wide = 0;  // its leading rows of kSweepGiant and, after them, kSweepWide in-edges and more
+  int64_t sweep_wide = 0;           // the batched sweep's wide rows: of this many in-edges and more
+  int64_t n_giant = 0, n_wide = 0;  // the list's leading giant ones and, after them, the other wide ones
   void* d_sitems = nullptr;      // serial mode: work items by workgroup
   int32_t* d_sstart = nullptr;   // ... first item of each workgroup (+ end)
   void* d_items = nullptr;       // PrItem list (compensated / FP64 modes)

@@ -332,3 +332,28 @@ def test_batch_beyond_the_far_sweep(dmm, orc, n):
             depth, _ = c.bfs_batch64(srcs, td_div=td_div)
             for i, ref in refs.items():
                 assert np.array_equal(depth[i], ref), (i, td_div)
+
+
+@pytest.mark.parametrize("n", [(7 << 21) - 1, 7 << 21])
+def test_batch_wide_rows_of_the_largest_graphs(dmm, orc, n):
+    """From 7 * 2^21 vertices on rows are wide from 8192 in-edges on, giant from
+    65536: rows around all four limits, below and at that size."""
+    rng = np.random.default_rng(n)
+    hubs = [511, 512, 513, 4095, 4096, 8191, 8192, 8193, 65535, 65536, 66000]
+    pairs = [np.stack((rng.permutation(3 * k)[:k] * 11 % n,
+                       np.full(k, n - 1 - 3 * i)), 1) for i, k in enumerate(hubs)]
+    pairs = np.concatenate([rng.integers(0, n, (2 * n, 2))] + pairs).astype(np.int32)
+    srcs = np.concatenate((rng.integers(0, n, 10), [n - 1 - 3 * i for i in range(len(hubs))])).astype(np.int32)
+    with dmm.Context(0) as c:
+        g = c.build_graph(pairs, n, symmetrize=False)
+        del pairs
+        og = orc.CSR.of(g)
+        c.upload(g)
+        refs = {}
+        for i in (0, 9, 10, 20):
+            ref = orc.bfs_depth(og, int(srcs[i]))
+            refs[i] = np.where(ref < 0, 255, ref).astype(np.uint8)
+        for td_div in (1, 1000000):
+            depth, _ = c.bfs_batch64(srcs, td_div=td_div)
+            for i, ref in refs.items():
+                assert np.array_equal(depth[i], ref), (i, td_div)
